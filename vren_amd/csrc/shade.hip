@@ -727,26 +727,45 @@ __device__ __forceinline__ void light_adjoint(const Surface& s, const LightTerm&
     gl[6] += g_att * datt_dx * (-t.x * t.inv_r);
 }
 
-// Sums each of the 7 values over the wave with 10 shuffles instead of 42: the first three butterfly stages (lane
-// bits 5, 4, 3) each keep half of the remaining components, so lane l ends with component (l >> 3) & 7 summed
-// over its 8-lane group, and three more stages sum the group. Every lane of the wave must be active.
+// Sums each of the 7 values over the wave: the first three butterfly stages (lane bits 5, 4, 3) each keep half of the
+// remaining components, so lane l ends with component (l >> 3) & 7 summed over its 8-lane group, and three more
+// stages sum the group. A permlane swap of two registers puts the two halves that a stage adds side by side (one
+// swap and one add for two components); the stages inside a row of 16 lanes are DPP moves. No LDS permute: 18 VALU
+// operations in place of 10 permutes and 22 selects and adds. Every lane of the wave must be active.
+template <int CTRL>
+__device__ __forceinline__ float dpp_move_f32(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
 __device__ __forceinline__ float wave_sum_components(const float g[7])
 {
-    const uint32_t lane = lane_id();
     const float v[8] = {g[0], g[1], g[2], g[3], g[4], g[5], g[6], 0.0f};
-    const bool h32 = (lane & 32u) != 0, h16 = (lane & 16u) != 0, h8 = (lane & 8u) != 0;
     float w4[4], w2[2];
 #pragma unroll
-    for (int i = 0; i < 4; i++) w4[i] = (h32 ? v[i + 4] : v[i]) + shfl_xor(h32 ? v[i] : v[i + 4], 32);
+    for (int i = 0; i < 4; i++) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 4]), false, false);
+        w4[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
 #pragma unroll
-    for (int i = 0; i < 2; i++) w2[i] = (h16 ? w4[i + 2] : w4[i]) + shfl_xor(h16 ? w4[i] : w4[i + 2], 16);
-    float w = (h8 ? w2[1] : w2[0]) + shfl_xor(h8 ? w2[0] : w2[1], 8);
-    w += shfl_xor(w, 4);
-    w += shfl_xor(w, 2);
-    w += shfl_xor(w, 1);
+    for (int i = 0; i < 2; i++) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(w4[i]), __float_as_uint(w4[i + 2]), false, false);
+        w2[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    const bool h8 = (lane_id() & 8u) != 0;
+    float w = (h8 ? w2[1] : w2[0]) + dpp_move_f32<0x128>(h8 ? w2[0] : w2[1]); // row_ror:8
+    w += dpp_move_f32<0x141>(w); // row_half_mirror
+    w += dpp_move_f32<0xB1>(w);  // quad_perm [1,0,3,2]
+    w += dpp_move_f32<0x4E>(w);  // quad_perm [2,3,0,1]
     return w;
 }
 
+constexpr int kSumRounds = 8;  // distinct entries of one step that a wave sums; lanes past them add one by one
+
+// One 32x8 strip of a tile per workgroup. On a 1920x1080 frame with 4096 lights (4.7 M pairs) it took 228 us: 95 us in
+// LDS adds of 64 lanes to one slot (every wave that covers two clusters took them, since it summed over the wave only
+// when all its lanes were at one entry) and 50 us in the gradients' global atomics, seven instructions each of whose
+// lanes hit another cache line. Summing once per distinct entry and one term per lane in the global adds: 91 us.
+// Larger workgroups (two and four strips, fewer global adds) are slower, 97 and 115 us.
 __global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev* __restrict__ frames, uint32_t F,
                                                              uint32_t total_tiles, const float* grad_out,
                                                              float* g_pos, float* g_light, float* g_ar)
@@ -934,13 +953,21 @@ __global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev* __r
         const uint64_t lm = ballot(live);
         if (lm == 0) continue;
         if (staged) {
-            const uint32_t first = (uint32_t)__builtin_ctzll(lm);
-            const uint32_t ef = __builtin_amdgcn_readlane(e, first);
-            if (ballot(live && e != ef) == 0) {
-                const float sum = wave_sum_components(gl);
-                const uint32_t c = (lane >> 3) & 7u;
+            // one round per distinct entry among the live lanes (the lanes of a cluster are at the same entry): the
+            // wave sums that entry's terms and seven lanes add them to its slot
+            const uint32_t c = (lane >> 3) & 7u;
+            uint64_t rem = lm;
+            for (int round = 0; round < kSumRounds && rem != 0; round++) {
+                const uint32_t ef = __builtin_amdgcn_readlane(e, (uint32_t)__builtin_ctzll(rem));
+                const bool mine = live && e == ef;
+                rem &= ~ballot(mine);
+                float gm[7];
+#pragma unroll
+                for (int i = 0; i < 7; i++) gm[i] = mine ? gl[i] : 0.0f;
+                const float sum = wave_sum_components(gm);
                 if ((lane & 7u) == 0 && c < 7 && sum != 0.0f) atomicAdd(&s_g[(ef - start) * 7 + c], sum);
-            } else if (live) {
+            }
+            if ((rem >> lane) & 1ull) {
                 float* slot = s_g + (e - start) * 7;
 #pragma unroll
                 for (int i = 0; i < 7; i++) atomicAdd(&slot[i], gl[i]);
@@ -962,14 +989,12 @@ __global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev* __r
     }
     __syncthreads();
     if (staged) {
-        for (uint32_t i = tid; i < nstage; i += 256) {
-            const uint32_t li = s_li[i];
-            if (li >= fd.L) continue;
-            const float* slot = s_g + i * 7;
-            for (int c = 0; c < 3; c++)
-                if (slot[c] != 0.0f) atomicAdd(&g_pos[4 * li + c], slot[c]);
-            for (int c = 0; c < 4; c++)
-                if (slot[3 + c] != 0.0f) atomicAdd(&g_light[4 * li + c], slot[3 + c]);
+        // one term per lane, so that a light's terms leave as neighbouring addresses of one instruction
+        for (uint32_t i = tid; i < nstage * 7; i += 256) {
+            const float v = s_g[i];
+            const uint32_t n = i / 7, c = i - n * 7, li = s_li[n];
+            if (v == 0.0f || li >= fd.L) continue;
+            atomicAdd(c < 3 ? &g_pos[4 * li + c] : &g_light[4 * li + (c - 3)], v);
         }
     }
 }
