@@ -26,7 +26,7 @@ struct vren_batch {
     ChainWork w;                    // batch-wide
     std::vector<ChainWork> w_frame; // per-frame views of the same memory
     std::vector<uint32_t> leaf_slots;
-    std::vector<uint32_t> live_slots; // per frame: leaf slots of the groups that hold lights (256-aligned)
+    std::vector<uint32_t> live_slots; // per frame: leaf slots of the leaf kernel (256-aligned; none for one chunk)
     uint32_t total_live_slots = 0;
     uint32_t* d_tile_frame = nullptr; // frame of every flattened tile
     hipGraph_t graph = nullptr;
@@ -89,8 +89,8 @@ void set_batch_shape(vren_batch* b, const vren_chain_shape& s)
     b->graph = nullptr;
 }
 
-// live_slots: the leaf-kernel grid over the frames' light-holding leaf groups (their padding groups were written
-// when the batch was created). With a concurrent light stage (and no per-kernel timing), the lights and their BVH
+// live_slots: the leaf-kernel grid over the light-holding leaf groups of the frames of more than one light chunk (the
+// padding groups were written when the batch was created). With a concurrent light stage (and no per-kernel timing), the lights and their BVH
 // run on the batch's second stream between a fork and a join while `s` keys the clusters: the two stages share no
 // buffer, and light assignment, the first consumer of both, waits for the join. The join is recorded even when a
 // light-stage launch fails, so a capture always ends with both streams joined.
@@ -103,14 +103,14 @@ int run_chain(vren_batch* b, hipStream_t s, const FrameDev* table, uint32_t F, c
         VREN_HIP(ctx, hipEventRecord(b->fork, s));
         VREN_HIP(ctx, hipStreamWaitEvent(b->side, b->fork, 0));
         int sl = launch_lights(ctx, b->side, table, F, w);
-        if (!sl && live_slots) sl = launch_bvh(ctx, b->side, table, F, live_slots, true, &w, kLeavesLive);
+        if (!sl) sl = launch_bvh(ctx, b->side, table, F, live_slots, true, &w, kLeavesLive);
         VREN_HIP(ctx, hipEventRecord(b->join, b->side));
         st = launch_clusters(ctx, s, table, F, w);
         VREN_HIP(ctx, hipStreamWaitEvent(s, b->join, 0));
         if (!st) st = sl;
     } else {
         if (!st) st = launch_lights(ctx, s, table, F, w);
-        if (!st && live_slots) st = launch_bvh(ctx, s, table, F, live_slots, true, &w, kLeavesLive);
+        if (!st) st = launch_bvh(ctx, s, table, F, live_slots, true, &w, kLeavesLive);
         if (!st) st = launch_clusters(ctx, s, table, F, w);
     }
     if (!st) st = launch_assign(ctx, s, table, F, w);
@@ -156,7 +156,7 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
     b->leaf_slots.resize(n_frames);
     b->live_slots.resize(n_frames);
     // sizes and arena layout
-    uint32_t tile_base = 0, leaf_base = 0, live_base = 0, offs_base = 0, max_L = 0, any_materials = 0;
+    uint32_t tile_base = 0, leaf_base = 0, live_base = 0, offs_base = 0, chunk_base = 0, max_L = 0, any_materials = 0;
     std::vector<size_t> off(n_frames * 14);
     size_t arena = 0;
     for (uint32_t i = 0; i < n_frames; i++) {
@@ -174,6 +174,9 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         f.leaf_base = leaf_base;
         f.live_leaf_base = live_base;
         f.offs_base = offs_base;
+        f.light_chunk_base = chunk_base;
+        const uint32_t chunks = (L + VREN_LIGHT_CHUNK - 1) / VREN_LIGHT_CHUNK;
+        chunk_base += chunks;
         f.L = L;
         f.light_pos = d.light_positions;
         f.lights = d.point_lights;
@@ -197,7 +200,8 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         f.bvh_length = L ? vren_calc_bvh_buffer_length(L) : 0;
         const uint32_t slots = L ? (f.bvh_padded + VREN_LEAF_ALIGN - 1) / VREN_LEAF_ALIGN * VREN_LEAF_ALIGN : 0;
         b->leaf_slots[i] = slots;
-        const uint32_t live = (std::min(slots, (L + 31u) & ~31u) + VREN_LEAF_ALIGN - 1) / VREN_LEAF_ALIGN * VREN_LEAF_ALIGN;
+        const uint32_t live = chunks <= 1 ? 0u // lights_kernel writes these frames' leaves
+            : (std::min(slots, (L + 31u) & ~31u) + VREN_LEAF_ALIGN - 1) / VREN_LEAF_ALIGN * VREN_LEAF_ALIGN;
         b->live_slots[i] = live;
         tile_base += (tiles + VREN_TILE_GROUP - 1) / VREN_TILE_GROUP * VREN_TILE_GROUP;
         leaf_base += slots;
@@ -210,7 +214,7 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         size_t* o = &off[i * 14];
         o[0] = arena; arena += a256((size_t)L * 16);                 // view_pos
         o[1] = arena; arena += a256((size_t)L * 8);                  // codes
-        o[2] = arena; arena += a256(L > 4096 ? (size_t)L * 8 : 0);   // codes_tmp
+        o[2] = arena; arena += a256(chunks > 1 ? (size_t)L * 8 + (size_t)chunks * VREN_CHUNK_BOX_BYTES : 0); // codes_tmp, chunk_box
         o[3] = arena; arena += a256((size_t)f.bvh_length * 32);      // bvh
         o[4] = arena; arena += a256((size_t)key_cap * 4);            // keys
         o[5] = arena; arena += 256;                                  // cluster_count
@@ -247,7 +251,10 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         size_t* o = &off[i * 14];
         f.view_pos = reinterpret_cast<float*>(b->arena + o[0]);
         f.codes = reinterpret_cast<uint32_t*>(b->arena + o[1]);
-        f.codes_tmp = f.L > 4096 ? reinterpret_cast<uint32_t*>(b->arena + o[2]) : nullptr;
+        if (f.L > VREN_LIGHT_CHUNK) {
+            f.codes_tmp = reinterpret_cast<uint32_t*>(b->arena + o[2]);
+            f.chunk_box = reinterpret_cast<uint32_t*>(b->arena + o[2] + (size_t)f.L * 8);
+        }
         f.bvh = reinterpret_cast<vren_bvh_node*>(b->arena + o[3]);
         f.keys = reinterpret_cast<uint32_t*>(b->arena + o[4]);
         f.cluster_count = reinterpret_cast<uint32_t*>(b->arena + o[5]);
@@ -264,6 +271,7 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
     b->w.total_leaf_slots = leaf_base;
     b->total_live_slots = live_base;
     b->w.max_L = max_L;
+    b->w.light_chunks = chunk_base;
     b->w.any_materials = any_materials;
     {
         uint64_t pixels = 0;
@@ -277,12 +285,14 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         single[i].tile_base = 0;
         single[i].leaf_base = 0;
         single[i].live_leaf_base = 0;
+        single[i].light_chunk_base = 0;
         single[i].offs_base = 0;
         ChainWork& wf = b->w_frame[i];
         chain_work_bind(&wf, b->work, single[i].Sx * single[i].Sy, (single[i].key_cap + VREN_SCAN_TILE - 1) / VREN_SCAN_TILE,
                         1);
         wf.total_leaf_slots = b->leaf_slots[i];
         wf.max_L = single[i].L;
+        wf.light_chunks = (single[i].L + VREN_LIGHT_CHUNK - 1) / VREN_LIGHT_CHUNK;
         wf.any_materials = single[i].texcoords != nullptr;
     }
     {

@@ -12,6 +12,9 @@ void vren_frame_set_materials(FrameDev* f, const vren_material_set* m);
 FrameDev* vren_next_frame_slot(vren_ctx* ctx);
 
 #define VREN_LEAF_ALIGN 256u
+// lights that one workgroup sorts (lights.hip); a frame of at most this many has its BVH from that workgroup
+#define VREN_LIGHT_CHUNK 4096u
+#define VREN_CHUNK_BOX_BYTES 24u
 // a frame's 32x32 tiles start at a multiple of this in the flattened tile numbering of a table (the clusters kernel
 // chains its look-back over groups of this many tiles, one workgroup each); tiles of the padding do nothing
 #define VREN_TILE_GROUP 8u
@@ -30,6 +33,7 @@ struct ChainWork {
     uint32_t total_offs_tiles;
     uint32_t total_leaf_slots;
     uint32_t max_L;
+    uint32_t light_chunks;  // chunks of VREN_LIGHT_CHUNK lights over the table's frames (light_chunk_base numbering)
     uint32_t any_materials; // some frame of the table takes the material path (shade picks its kernel by it)
     // launch shape (vren_chain_shape; 0 = the default): shade strips per workgroup, persistent assignment waves
     // per CU, digit width of the light sort
@@ -69,7 +73,8 @@ void chain_work_bind(ChainWork* w, void* mem, uint32_t total_tiles, uint32_t tot
 
 // stage launchers; d_frames is a device table of F FrameDev records
 int launch_chain_init(vren_ctx* ctx, hipStream_t s, const ChainWork& w);
-int launch_lights(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w);
+int launch_lights(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
+                  uint32_t pad_blocks = 0);
 // which 32-leaf groups the leaf kernel writes: all, those holding a light, or the all-padding ones
 enum : uint32_t { kLeavesAll = 0, kLeavesLive = 1, kLeavesPadding = 2 };
 int launch_bvh(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, uint32_t total_leaf_slots,

@@ -20,7 +20,8 @@ struct FrameDev {
     uint32_t W, H, Sx, Sy;
     uint32_t tile_base;     // first flattened 32x32 tile of this frame in the table
     uint32_t leaf_base;     // first flattened leaf slot (256-aligned) of this frame's BVH leaves
-    uint32_t live_leaf_base; // the same over the leaf groups that hold lights only (a batch's chain launch)
+    uint32_t live_leaf_base; // the same over the light-holding leaf groups of frames of more than one light chunk
+    uint32_t light_chunk_base; // first flattened chunk of VREN_LIGHT_CHUNK lights of this frame
     uint32_t offs_base;     // first flattened tile of this frame's light-offset scan
     // camera constants
     float view[16];         // camera::get_view()
@@ -50,7 +51,8 @@ struct FrameDev {
     const float* dir_lights;  // {dir, pad, rgb, pad}[n_dir]
     float* view_pos;          // float4[L]
     uint32_t* codes;          // uint2[L] (code, light index), sorted by code
-    uint32_t* codes_tmp;      // uint2[L] scratch for the sort
+    uint32_t* codes_tmp;      // uint2[L] the chunks' sorted runs (more than one chunk)
+    uint32_t* chunk_box;      // the chunks' view-space boxes, six words each (more than one chunk)
     vren_bvh_node* bvh;
     uint32_t bvh_padded, bvh_root, bvh_levels, bvh_length;
     float* leaf_pos;          // optional float4[L]: view position of sorted leaf i (= view_pos[codes[i].y])

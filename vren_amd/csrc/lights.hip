@@ -2,210 +2,124 @@
 //
 // Reference: 8 recorded steps and ~10 dispatches per frame (view transform, two vec4 reduce trees, a copy,
 // Morton codes, a 65 536-bucket atomic bucket sort with a fixed 2^16 scan, leaf init, then one dispatch per BVH
-// level). Here, per frame:
-//   lights_kernel   one workgroup: view transform, AABB (order-independent min/max), Morton codes, and a stable
-//                   LSD radix sort of (code, light index) in LDS (global ping-pong above 4096 lights);
-//   bvh_leaf_kernel every leaf of every frame (flattened grid): leaf AABB = view position -+ radius, and the first
-//                   parent level straight from registers (32-lane min/max over half-waves);
-//   bvh_upper_kernel one workgroup per frame for the remaining (<= 32^k / 32) parent levels.
-// A batch of frames runs the same three launches with one workgroup (or leaf range) per frame.
+// level). Here a frame's lights are cut into chunks of 4096, one workgroup each:
+//   lights_kernel        view transform, AABB (order-independent min/max), Morton codes and a stable LSD radix sort of
+//                        (code, light index) in LDS. A frame of one chunk also builds its whole BVH there, from the
+//                        sorted lights in LDS, so it takes one launch; a chunk of a larger frame leaves its sorted
+//                        run in global memory.
+// and for the frames of more than one chunk:
+//   lights_bounds_kernel (ahead) view transform and the AABB of each chunk;
+//   lights_merge_kernel  each light's rank in the frame: its place in its own run plus the number of lights that sort
+//                        before it in every other run (binary searches), which is the stable order;
+//   bvh_leaf_kernel      every leaf: leaf AABB = view position -+ radius, and the first parent level straight from
+//                        registers (32-lane min/max over half-waves);
+//   bvh_upper_kernel     one workgroup per frame for the remaining (<= 32^k / 32) parent levels.
+// A batch of frames runs the same launches with the chunks (or leaf ranges) of every frame side by side.
 #include "chain.hpp"
 #include "radix_device.hpp"
 #include "scan_device.hpp"
 
 namespace {
 
-constexpr int kLT = 1024;           // threads of the per-frame light workgroup
-constexpr int kLKPT = 4;            // keys per thread per sort chunk
-constexpr int kLChunk = kLT * kLKPT;
-constexpr uint32_t kLdsCap = 4096;  // lights sorted entirely in LDS
+constexpr int kLT = 1024;            // threads of a chunk's workgroup
+constexpr int kLWaves = kLT / VREN_WAVE;
+constexpr int kLKPT = 4;             // lights per thread of a full chunk
+constexpr uint32_t kLChunk = VREN_LIGHT_CHUNK;
+static_assert(kLChunk == kLT * kLKPT, "a chunk is what one workgroup sorts");
+constexpr uint32_t kMergeThreads = 256;
+constexpr uint32_t kMergeParts = kLChunk / kMergeThreads; // merge workgroups per chunk
 
+// every third bit of the result holds one of the low 10 bits of q
+__device__ __forceinline__ uint32_t spread3(uint32_t q)
+{
+    q = (q | (q << 16)) & 0x030000FFu;
+    q = (q | (q << 8)) & 0x0300F00Fu;
+    q = (q | (q << 4)) & 0x030C30C3u;
+    return (q | (q << 2)) & 0x09249249u;
+}
+
+// bits <= 10 per axis: x at bit 3 i, y at 3 i + 1, z at 3 i + 2 (what lies above an axis' bits is dropped)
 __device__ __forceinline__ uint32_t morton_interleave(uint32_t qx, uint32_t qy, uint32_t qz, uint32_t bits)
 {
-    uint32_t code = 0;
-    for (uint32_t i = 0; i < bits; i++) {
-        code |= ((qx >> i) & 1u) << (i * 3);
-        code |= ((qy >> i) & 1u) << (i * 3 + 1);
-        code |= ((qz >> i) & 1u) << (i * 3 + 2);
-    }
-    return code;
+    const uint32_t m = (1u << bits) - 1u;
+    return spread3(qx & m) | (spread3(qy & m) << 1) | (spread3(qz & m) << 2);
 }
 
-// one stable LSD pass of a BITS-bit digit (BITS <= 8) over a segment of L (code, index) pairs, src -> dst (generic
-// pointers: LDS or global)
-template <int BITS>
-__device__ void block_sort_pass(const uint2* src, uint2* dst, uint32_t L, uint32_t shift, uint32_t width,
-                                uint32_t* s_whist, uint32_t* s_base, uint32_t* s_cnt, uint32_t* s_scan)
+// floats as integers of the same order (-0 below +0), so that min and max of any number of them are integer minima
+__device__ __forceinline__ uint32_t ordered_bits(float x)
 {
-    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / VREN_WAVE;
-    const uint32_t mask = (1u << width) - 1u;
-    if (tid < 256) s_cnt[tid] = 0u;
-    __syncthreads();
-    for (uint32_t i = tid; i < L; i += kLT) atomicAdd(&s_cnt[(src[i].x >> shift) & mask], 1u);
-    __syncthreads();
-    uint32_t tot;
-    uint32_t ex = block_exclusive_sum<kLT>(tid < 256 ? s_cnt[tid] : 0u, s_scan, &tot);
-    if (tid < 256) s_base[tid] = ex;
-    __syncthreads();
-    for (uint32_t c0 = 0; c0 < L; c0 += kLChunk) {
-        const uint32_t cnt = min((uint32_t)kLChunk, L - c0);
-        for (uint32_t i = tid; i < (uint32_t)(kLT / VREN_WAVE) * 256; i += kLT) s_whist[i] = 0u;
-        __syncthreads();
-        const uint32_t wbase = wave * kLKPT * VREN_WAVE;
-        uint2 e[kLKPT];
-        uint32_t digit[kLKPT], local[kLKPT];
+    const uint32_t u = __float_as_uint(x);
+    return u ^ ((u >> 31) ? 0xFFFFFFFFu : 0x80000000u);
+}
+__device__ __forceinline__ float from_ordered(uint32_t o) { return __uint_as_float(o ^ ((o >> 31) ? 0x80000000u : 0xFFFFFFFFu)); }
+
+// The AABB of view-space positions as six minima: ordered_bits of the three lower corners, and the complements of
+// the three upper ones'. A NaN coordinate widens neither corner. Start: the reduce identities +-1e35.
+struct BoxKeys {
+    uint32_t k[6];
+};
+__device__ __forceinline__ BoxKeys empty_box()
+{
+    BoxKeys b;
 #pragma unroll
-        for (int j = 0; j < kLKPT; j++) {
-            uint32_t pos = wbase + j * VREN_WAVE + lane;
-            e[j] = pos < cnt ? src[c0 + pos] : make_uint2(0u, 0u);
-            digit[j] = (e[j].x >> shift) & mask;
-        }
-        rank_wave_keys<BITS, kLKPT>(digit, wbase, cnt, &s_whist[wave * 256], local);
-        __syncthreads();
-        if (tid < 256) {
-            uint32_t run = 0;
-            for (int w = 0; w < kLT / VREN_WAVE; w++) {
-                uint32_t c = s_whist[w * 256 + tid];
-                s_whist[w * 256 + tid] = run;
-                run += c;
-            }
-            s_cnt[tid] = run;
-        }
-        __syncthreads();
+    for (int a = 0; a < 3; a++) {
+        b.k[a] = ordered_bits(1e35f);
+        b.k[3 + a] = ~ordered_bits(-1e35f);
+    }
+    return b;
+}
+__device__ __forceinline__ void add_to_box(BoxKeys& b, const float r[3])
+{
 #pragma unroll
-        for (int j = 0; j < kLKPT; j++) {
-            uint32_t pos = wbase + j * VREN_WAVE + lane;
-            if (pos < cnt) {
-                uint32_t d = digit[j];
-                dst[s_base[d] + s_whist[wave * 256 + d] + local[j]] = e[j];
-            }
-        }
-        __syncthreads();
-        if (tid < 256) s_base[tid] += s_cnt[tid];
-        __syncthreads();
+    for (int a = 0; a < 3; a++) {
+        const uint32_t o = ordered_bits(r[a]);
+        const bool num = r[a] == r[a];
+        b.k[a] = min(b.k[a], num ? o : 0xFFFFFFFFu);
+        b.k[3 + a] = min(b.k[3 + a], num ? ~o : 0xFFFFFFFFu);
     }
 }
 
-// BITS: digit width of the Morton-code sort (8 by default; 4 is a chain-shape choice)
-template <int BITS>
-__global__ __launch_bounds__(kLT) void lights_kernel(const FrameDev* __restrict__ frames)
+// minimum over each row of 16 lanes, in every lane of the row
+__device__ __forceinline__ uint32_t row_min(uint32_t v)
 {
-    __shared__ uint2 s_a[kLdsCap];
-    __shared__ uint2 s_b[kLdsCap];
-    __shared__ uint32_t s_whist[(kLT / VREN_WAVE) * 256];
-    __shared__ uint32_t s_base[256], s_cnt[256], s_scan[kLT / VREN_WAVE];
-    __shared__ float s_red[6][kLT / VREN_WAVE];
-    __shared__ float s_box[6];
-
-    const FrameDev& fd = frames[blockIdx.x];
-    const uint32_t L = fd.L;
-    if (L == 0) return;
-    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / VREN_WAVE;
-    const float4* pos = reinterpret_cast<const float4*>(fd.light_pos);
-    float4* vpos = reinterpret_cast<float4*>(fd.view_pos);
-
-    // 1. view transform (point_light_position_to_view_space.comp:26-32) + AABB partials
-    float mn[3] = {1e35f, 1e35f, 1e35f}, mx[3] = {-1e35f, -1e35f, -1e35f};
-    for (uint32_t i = tid; i < L; i += kLT) {
-        float4 p = pos[i];
-        float v[4] = {p.x, p.y, p.z, 1.0f}, r[4];
-        vren_mat4_mul_vec4(fd.view, v, r);
-        vpos[i] = make_float4(r[0], r[1], r[2], r[3]);
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-            mn[a] = tmin(mn[a], r[a]);
-            mx[a] = tmax(mx[a], r[a]);
-        }
-    }
-    // 2. AABB (reduce_vec4 min/max of clustered_shading.cpp:137-191; min/max are exact in any order)
-    if (fd.morton_aabb_mode == VREN_MORTON_GIVEN_AABB) {
-        if (tid < 3) {
-            s_box[tid] = fd.morton_min[tid];
-            s_box[3 + tid] = fd.morton_max[tid];
-        }
-    } else {
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) {
-#pragma unroll
-            for (int a = 0; a < 3; a++) {
-                mn[a] = tmin(mn[a], shfl_xor(mn[a], m));
-                mx[a] = tmax(mx[a], shfl_xor(mx[a], m));
-            }
-        }
-        if (lane == 0) {
-            for (int a = 0; a < 3; a++) {
-                s_red[a][wave] = mn[a];
-                s_red[3 + a][wave] = mx[a];
-            }
-        }
-        __syncthreads();
-        if (tid < 3) {
-            float m0 = 1e35f, m1 = -1e35f;
-            for (int w = 0; w < kLT / VREN_WAVE; w++) {
-                m0 = tmin(m0, s_red[tid][w]);
-                m1 = tmax(m1, s_red[3 + tid][w]);
-            }
-            s_box[tid] = m0;
-            s_box[3 + tid] = m1;
-        }
-    }
-    __syncthreads();
-
-    // 3. Morton codes (discretize_point_light_positions.comp:26-43), paired with the light index
-    const uint32_t bits = fd.morton_bits;
-    const uint32_t total_bits = 3 * bits;
-    const uint32_t passes = (total_bits + BITS - 1) / BITS;
-    const float scale = (float)(1u << bits);
-    const bool in_lds = L <= kLdsCap;
-    uint2* A;
-    uint2* B;
-    if (in_lds) {
-        A = s_a;
-        B = s_b;
-    } else {
-        // end the even/odd ping-pong in fd.codes
-        A = reinterpret_cast<uint2*>((passes & 1) ? fd.codes_tmp : fd.codes);
-        B = reinterpret_cast<uint2*>((passes & 1) ? fd.codes : fd.codes_tmp);
-    }
-    for (uint32_t i = tid; i < L; i += kLT) {
-        float4 p = pos[i];
-        float v[4] = {p.x, p.y, p.z, 1.0f}, r[4];
-        vren_mat4_mul_vec4(fd.view, v, r);
-        uint32_t q[3];
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-            float t = (r[a] - s_box[a]) / (s_box[3 + a] - s_box[a]) * scale;
-            q[a] = vren_f2u_sat(vren_floorf(t));
-        }
-        A[i] = make_uint2(morton_interleave(q[0], q[1], q[2], bits), i);
-    }
-    __syncthreads();
-    // 4. stable sort by code (ties keep light-index order)
-    uint2* src = A;
-    uint2* dst = B;
-    for (uint32_t p = 0; p < passes; p++) {
-        uint32_t shift = BITS * p;
-        block_sort_pass<BITS>(src, dst, L, shift, min((uint32_t)BITS, total_bits - shift), s_whist, s_base, s_cnt,
-                              s_scan);
-        uint2* t = src;
-        src = dst;
-        dst = t;
-    }
-    if (in_lds) {
-        uint2* out = reinterpret_cast<uint2*>(fd.codes);
-        for (uint32_t i = tid; i < L; i += kLT) out[i] = src[i];
-    }
+    v = min(v, dpp_fill<0xB1, 0xF>(v, v));  // quad_perm [1,0,3,2]
+    v = min(v, dpp_fill<0x4E, 0xF>(v, v));  // quad_perm [2,3,0,1]
+    v = min(v, dpp_fill<0x141, 0xF>(v, v)); // row_half_mirror
+    return min(v, dpp_fill<0x140, 0xF>(v, v)); // row_mirror
 }
 
-__device__ __forceinline__ void half_wave_minmax(float (&mn)[3], float (&mx)[3])
+// The box of a whole workgroup of kLWaves waves, in every thread: the waves' minima meet in LDS, and every wave reads
+// them all and reduces them by rows of 16 lanes (one barrier). s_red: 6 * 16 words.
+__device__ __forceinline__ void block_box(BoxKeys& b, uint32_t* s_red)
+{
+    static_assert(kLWaves == 16, "a row of lanes holds one minimum per wave");
+    const uint32_t lane = lane_id(), wave = wave_id();
+#pragma unroll
+    for (int a = 0; a < 6; a++) {
+        const uint32_t m = wave_min_u32(b.k[a]);
+        if (lane == 0) s_red[a * kLWaves + wave] = m;
+    }
+    __syncthreads();
+    const uint32_t p = row_min(s_red[lane]), q = row_min(s_red[64 + (lane & 31)]);
+    b.k[0] = __builtin_amdgcn_readlane(p, 0);
+    b.k[1] = __builtin_amdgcn_readlane(p, 16);
+    b.k[2] = __builtin_amdgcn_readlane(p, 32);
+    b.k[3] = __builtin_amdgcn_readlane(p, 48);
+    b.k[4] = __builtin_amdgcn_readlane(q, 0);
+    b.k[5] = __builtin_amdgcn_readlane(q, 16);
+}
+
+// 32-lane AABB of the half-wave's leaves or nodes, in its last lane (31 or 63). Lanes without a box pass the empty
+// one (min = +inf, max = -inf); min and max are exact in any order.
+__device__ __forceinline__ void half_wave_box(float (&mn)[3], float (&mx)[3])
 {
 #pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) {
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-            mn[a] = tmin(mn[a], shfl_xor(mn[a], m));
-            mx[a] = tmax(mx[a], shfl_xor(mx[a], m));
-        }
+    for (int a = 0; a < 3; a++) {
+        uint32_t lo = row_min(ordered_bits(mn[a])), hi = row_min(~ordered_bits(mx[a]));
+        lo = min(lo, dpp_fill<0x142, 0xA>(lo, lo)); // row_bcast:15
+        hi = min(hi, dpp_fill<0x142, 0xA>(hi, hi));
+        mn[a] = from_ordered(lo);
+        mx[a] = from_ordered(~hi);
     }
 }
 
@@ -214,6 +128,389 @@ __device__ __forceinline__ void store_node(vren_bvh_node* n, const float (&mn)[3
     float4* q = reinterpret_cast<float4*>(n);
     q[0] = make_float4(mn[0], mn[1], mn[2], __uint_as_float(next));
     q[1] = make_float4(mx[0], mx[1], mx[2], 0.0f);
+}
+
+__device__ __forceinline__ void store_invalid(vren_bvh_node* n)
+{
+    const float inf[3] = {VREN_F32_INF, VREN_F32_INF, VREN_F32_INF};
+    const float ninf[3] = {-VREN_F32_INF, -VREN_F32_INF, -VREN_F32_INF};
+    store_node(n, inf, ninf, VREN_BVH_INVALID_NODE);
+}
+
+// the frame and the chunk of a flattened chunk number
+__device__ __forceinline__ const FrameDev& frame_of_chunk(const FrameDev* __restrict__ frames, uint32_t F, uint32_t c,
+                                                          uint32_t* chunk)
+{
+    const uint32_t f = F > 1 ? find_frame_wave(frames, F, c, [](const FrameDev& d) { return d.light_chunk_base; }) : 0u;
+    *chunk = c - frames[f].light_chunk_base;
+    return frames[f];
+}
+
+// Frames of more than one chunk: the chunk's view positions (point_light_position_to_view_space.comp:26-32) and box.
+__global__ __launch_bounds__(kLT) void lights_bounds_kernel(const FrameDev* __restrict__ frames, uint32_t F)
+{
+    __shared__ uint32_t s_red[6 * kLWaves];
+    uint32_t chunk;
+    const FrameDev& fd = frame_of_chunk(frames, F, blockIdx.x, &chunk);
+    if (fd.L <= kLChunk) return; // the whole workgroup
+    const uint32_t first = chunk * kLChunk;
+    BoxKeys box = empty_box();
+#pragma unroll
+    for (int j = 0; j < kLKPT; j++) {
+        const uint32_t i = first + j * kLT + threadIdx.x;
+        if (i < fd.L) {
+            const float4 p = reinterpret_cast<const float4*>(fd.light_pos)[i];
+            const float v[4] = {p.x, p.y, p.z, 1.0f};
+            float r[4];
+            vren_mat4_mul_vec4(fd.view, v, r);
+            reinterpret_cast<float4*>(fd.view_pos)[i] = make_float4(r[0], r[1], r[2], r[3]);
+            add_to_box(box, r);
+        }
+    }
+    block_box(box, s_red);
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int a = 0; a < 6; a++) fd.chunk_box[chunk * 6 + a] = box.k[a];
+    }
+}
+
+// One chunk: its lights' Morton codes, sorted stably with the light indices by an LSD radix sort on BITS-bit digits
+// (8 by default; 4 is a chain-shape choice). Keys stay in registers, warp-striped over kpt keys per thread (as few as
+// the chunk needs, so that a small frame's keys are spread over all the waves), and go through one LDS array between
+// passes; three barriers per pass: each wave ranks its keys in its own row of digit counters (which it clears itself),
+// one thread per digit turns the rows into wave prefixes, and the digits' starts across the four waves of digit
+// threads are added by the readers. Blocks at and past `chunks` write the frame's padding leaves (single-frame calls).
+// A frame of one chunk then builds its BVH from the sorted lights: leaves, the first parent level over half-waves, the
+// rest from LDS. 4096 lights and their BVH took 34 us in three launches (21.7 + 6 + 6.8) and take one of 22 us
+// (256 lights: 21 -> 7 us), bound by the vector issue of its one CU; 65 536 lights took 292 us in one workgroup that
+// sorted in global memory and take 36 us (bounds 6, chunks 12.5, merge 17).
+template <int BITS>
+__global__ __launch_bounds__(kLT) void lights_kernel(const FrameDev* __restrict__ frames, uint32_t F, uint32_t chunks)
+{
+    constexpr uint32_t RADIX = 1u << BITS;
+    __shared__ uint2 s_pair[kLChunk];              // (code, light index)
+    __shared__ float4 s_light[kLChunk];            // view position, radius (frames of one chunk)
+    __shared__ uint32_t s_row[kLWaves * RADIX];    // per wave: digit counts, then the digit's prefix
+    __shared__ uint32_t s_digits[4];               // keys per group of 64 digits
+    __shared__ uint32_t s_red[6 * kLWaves];
+    __shared__ float s_node[kLChunk / 32][6];      // the first parent level, then the second one
+    __shared__ float s_node2[kLChunk / 1024][6];
+
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+    if (blockIdx.x >= chunks) {
+        const FrameDev& fd = frames[0];
+        const uint32_t i = (blockIdx.x - chunks) * kLT + tid, padded = fd.bvh_padded;
+        if (i < ((fd.L + 31u) & ~31u) || i >= padded) return;
+        store_invalid(&fd.bvh[i]);
+        if ((i & 31u) == 0) store_invalid(&fd.bvh[padded + i / 32]);
+        return;
+    }
+    uint32_t chunk;
+    const FrameDev& fd = frame_of_chunk(frames, F, blockIdx.x, &chunk);
+    const uint32_t L = fd.L, first = chunk * kLChunk;
+    const bool whole = L <= kLChunk; // the frame is this chunk
+    const uint32_t n = min(kLChunk, L - first);
+    const uint32_t kpt = (n + kLT - 1) / kLT;
+    const uint32_t wbase = wave * kpt * VREN_WAVE;
+
+    // view positions and the frame's box (reduce_vec4 min/max of clustered_shading.cpp:137-191)
+    float r[kLKPT][3];
+    BoxKeys box = empty_box();
+#pragma unroll
+    for (int j = 0; j < kLKPT; j++) {
+        const uint32_t i = wbase + j * VREN_WAVE + lane;
+        if (j < (int)kpt && i < n) {
+            float q[4];
+            if (whole) {
+                const vf4 p = *((gvf4*)fd.light_pos + i);
+                const float radius = *((gfloat*)fd.lights + 4 * i + 3);
+                const float v[4] = {p.x, p.y, p.z, 1.0f};
+                vren_mat4_mul_vec4(fd.view, v, q);
+                reinterpret_cast<float4*>(fd.view_pos)[i] = make_float4(q[0], q[1], q[2], q[3]);
+                s_light[i] = make_float4(q[0], q[1], q[2], radius);
+                add_to_box(box, q);
+            } else {
+                const vf4 p = *((gvf4*)fd.view_pos + first + i);
+                q[0] = p.x;
+                q[1] = p.y;
+                q[2] = p.z;
+            }
+#pragma unroll
+            for (int a = 0; a < 3; a++) r[j][a] = q[a];
+        }
+    }
+    float lo[3], hi[3];
+    if (fd.morton_aabb_mode == VREN_MORTON_GIVEN_AABB) {
+        for (int a = 0; a < 3; a++) {
+            lo[a] = fd.morton_min[a];
+            hi[a] = fd.morton_max[a];
+        }
+    } else {
+        if (whole) {
+            block_box(box, s_red);
+        } else {
+            const uint32_t n_chunks = (L + kLChunk - 1) / kLChunk;
+            for (uint32_t c = lane; c < n_chunks; c += VREN_WAVE)
+#pragma unroll
+                for (int a = 0; a < 6; a++) box.k[a] = min(box.k[a], *((guint*)fd.chunk_box + c * 6 + a));
+#pragma unroll
+            for (int a = 0; a < 6; a++) box.k[a] = wave_min_u32(box.k[a]);
+        }
+        for (int a = 0; a < 3; a++) {
+            lo[a] = from_ordered(box.k[a]);
+            hi[a] = from_ordered(~box.k[3 + a]);
+        }
+    }
+
+    // Morton codes (discretize_point_light_positions.comp:26-43), paired with the light index
+    const uint32_t bits = fd.morton_bits, total_bits = 3 * bits;
+    const float scale = (float)(1u << bits);
+    uint2 e[kLKPT];
+#pragma unroll
+    for (int j = 0; j < kLKPT; j++) {
+        const uint32_t i = wbase + j * VREN_WAVE + lane;
+        e[j] = make_uint2(0u, 0u);
+        if (j < (int)kpt && i < n) {
+            uint32_t q[3];
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                const float t = (r[j][a] - lo[a]) / (hi[a] - lo[a]) * scale;
+                q[a] = vren_f2u_sat(vren_floorf(t));
+            }
+            e[j] = make_uint2(morton_interleave(q[0], q[1], q[2], bits), first + i);
+        }
+    }
+
+    // the stable sort by code (ties keep light-index order)
+    uint32_t* row = s_row + wave * RADIX;
+    for (uint32_t shift = 0; shift < total_bits; shift += BITS) {
+        const uint32_t width = min((uint32_t)BITS, total_bits - shift);
+        for (uint32_t i = lane; i < RADIX; i += VREN_WAVE) row[i] = 0u;
+        __builtin_amdgcn_wave_barrier();
+        uint32_t digit[kLKPT], local[kLKPT];
+#pragma unroll
+        for (int j = 0; j < kLKPT; j++) {
+            digit[j] = __builtin_amdgcn_ubfe(e[j].x, shift, width);
+            local[j] = 0u;
+            if (j < (int)kpt) { // uniform
+                const bool valid = wbase + j * VREN_WAVE + lane < n;
+                const uint64_t vm = ballot(valid);
+                uint32_t plo = (uint32_t)vm, phi = (uint32_t)(vm >> 32);
+                const uint32_t before = valid ? row[digit[j]] : 0u;
+                match_digit<BITS>(digit[j], plo, phi);
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(phi, __builtin_amdgcn_mbcnt_lo(plo, 0u));
+                const uint64_t peers = ((uint64_t)phi << 32) | plo;
+                if (valid && (peers >> lane) == 1ull) row[digit[j]] = before + rank + 1u; // the highest peer lane
+                local[j] = before + rank;
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+        __syncthreads();
+        if (tid < ((RADIX + 63u) & ~63u)) { // whole waves
+            uint32_t c[kLWaves], sum = 0;
+#pragma unroll
+            for (int w = 0; w < kLWaves; w++) {
+                c[w] = tid < RADIX ? s_row[w * RADIX + tid] : 0u;
+                sum += c[w];
+            }
+            const uint32_t incl = wave_inclusive_sum(sum);
+            if (lane == VREN_WAVE - 1) s_digits[wave] = incl;
+            uint32_t run = incl - sum;
+            if (tid < RADIX) {
+#pragma unroll
+                for (int w = 0; w < kLWaves; w++) {
+                    s_row[w * RADIX + tid] = run;
+                    run += c[w];
+                }
+            }
+        }
+        __syncthreads();
+        uint32_t d1 = 0, d2 = 0, d3 = 0; // keys in the digit groups before groups 1, 2, 3
+        if (RADIX > 64) {
+            d1 = s_digits[0];
+            d2 = d1 + s_digits[1];
+            d3 = d2 + s_digits[2];
+        }
+#pragma unroll
+        for (int j = 0; j < kLKPT; j++) {
+            if (j < (int)kpt && wbase + j * VREN_WAVE + lane < n) {
+                const uint32_t d = digit[j], g = d >> 6;
+                const uint32_t before = g == 0 ? 0u : (g == 1 ? d1 : (g == 2 ? d2 : d3));
+                s_pair[before + row[d] + local[j]] = e[j];
+            }
+        }
+        __syncthreads();
+        if (shift + BITS < total_bits) {
+#pragma unroll
+            for (int j = 0; j < kLKPT; j++)
+                if (j < (int)kpt && wbase + j * VREN_WAVE + lane < n) e[j] = s_pair[wbase + j * VREN_WAVE + lane];
+        }
+    }
+    uint2* out = reinterpret_cast<uint2*>(whole ? fd.codes : fd.codes_tmp) + first;
+    if (!whole) {
+        for (uint32_t i = tid; i < n; i += kLT) out[i] = s_pair[i];
+        return;
+    }
+
+    // leaves (init_light_array_bvh.comp:42-65) in light-holding groups of 32, and their parents
+    const uint32_t padded = fd.bvh_padded;
+    const uint32_t groups = (n + 31) / 32;
+#pragma unroll
+    for (int k = 0; k < kLKPT; k++) {
+        const uint32_t i = k * kLT + tid;
+        if (i >= groups * 32) break; // whole half-waves leave together; the others' lanes do not read them
+        float mn[3] = {VREN_F32_INF, VREN_F32_INF, VREN_F32_INF};
+        float mx[3] = {-VREN_F32_INF, -VREN_F32_INF, -VREN_F32_INF};
+        if (i < n) {
+            const uint2 pr = s_pair[i];
+            const float4 v = s_light[pr.y];
+            out[i] = pr;
+            if (fd.leaf_pos) reinterpret_cast<float4*>(fd.leaf_pos)[i] = v;
+            mn[0] = v.x - v.w;
+            mn[1] = v.y - v.w;
+            mn[2] = v.z - v.w;
+            mx[0] = v.x + v.w;
+            mx[1] = v.y + v.w;
+            mx[2] = v.z + v.w;
+        }
+        store_node(&fd.bvh[i], mn, mx, i < n ? VREN_BVH_LEAF_NODE : VREN_BVH_INVALID_NODE);
+        half_wave_box(mn, mx);
+        if ((lane & 31) == 31) {
+            const uint32_t g = i / 32;
+            store_node(&fd.bvh[padded + g], mn, mx, g * 32);
+            for (int a = 0; a < 3; a++) {
+                s_node[g][a] = mn[a];
+                s_node[g][3 + a] = mx[a];
+            }
+        }
+    }
+    if (padded < 1024) return; // 32 leaves: the first parent is the root
+    __syncthreads();
+    // second parent level: padded / 1024 nodes, the first n2 of them over first-level nodes that hold lights
+    const uint32_t level1 = padded, level2 = level1 + padded / 32, size2 = padded / 1024;
+    const uint32_t n2 = (groups + 31) / 32;
+    if (tid < n2 * 32) {
+        float mn[3] = {VREN_F32_INF, VREN_F32_INF, VREN_F32_INF};
+        float mx[3] = {-VREN_F32_INF, -VREN_F32_INF, -VREN_F32_INF};
+        if (tid < groups) {
+            for (int a = 0; a < 3; a++) {
+                mn[a] = s_node[tid][a];
+                mx[a] = s_node[tid][3 + a];
+            }
+        }
+        half_wave_box(mn, mx);
+        if ((lane & 31) == 31) {
+            const uint32_t g = tid / 32;
+            store_node(&fd.bvh[level2 + g], mn, mx, level1 + g * 32);
+            for (int a = 0; a < 3; a++) {
+                s_node2[g][a] = mn[a];
+                s_node2[g][3 + a] = mx[a];
+            }
+        }
+    }
+    if (tid >= n2 && tid < size2) store_invalid(&fd.bvh[level2 + tid]);
+    if (size2 == 1) return; // 1024 leaves: that was the root
+    __syncthreads();
+    if (tid < 32) { // the root over the 32 second-level nodes of 32768 leaves
+        float mn[3] = {VREN_F32_INF, VREN_F32_INF, VREN_F32_INF};
+        float mx[3] = {-VREN_F32_INF, -VREN_F32_INF, -VREN_F32_INF};
+        if (tid < n2) {
+            for (int a = 0; a < 3; a++) {
+                mn[a] = s_node2[tid][a];
+                mx[a] = s_node2[tid][3 + a];
+            }
+        }
+        half_wave_box(mn, mx);
+        if (tid == 31) store_node(&fd.bvh[level2 + 32], mn, mx, level2);
+    }
+}
+
+// Frames of more than one chunk: codes[rank] for every light of the chunks' sorted runs. A light's rank is its place in
+// its run plus, for every other run, the number of its lights that sort before it: codes up to and including the
+// light's in the runs before its own (their light indices are lower), codes below it in the runs after. A workgroup
+// takes kMergeThreads neighbouring lights of a run, whose bounds fall into a short range of every other run: one wave
+// finds the range from every 64th code of the run (one load and two ballots) and stages it in LDS, kMergeRuns runs at
+// a time, and each thread searches the staged codes. A range that is longer than the stage (a run that lies inside the
+// workgroup's range of codes, as when light indices follow their places) is searched in global memory. 65 536 lights
+// took 34 us with every search in global memory (26 dependent loads that miss the L2 of their XCD) and take 17 us.
+constexpr uint32_t kMergeRuns = 16;   // runs staged at a time
+constexpr uint32_t kMergeStage = 512; // codes staged per run (two workgroups' worth)
+constexpr uint32_t kMergeWaves = kMergeThreads / VREN_WAVE;
+
+// the number of codes below `bound` among codes[0 .. len), ascending, len <= 2 * top (a power of 2)
+template <typename Get>
+__device__ __forceinline__ uint32_t count_below(Get code, uint32_t len, uint32_t bound, uint32_t top)
+{
+    uint32_t pos = 0;
+    // the halving steps reach 2 top - 1, the last one 2 top
+    for (uint32_t step = top; step >= 1; step >>= 1)
+        if (pos + step <= len && code(pos + step - 1u) < bound) pos += step;
+    if (pos < len && code(pos) < bound) pos++;
+    return pos;
+}
+
+__global__ __launch_bounds__(kMergeThreads) void lights_merge_kernel(const FrameDev* __restrict__ frames, uint32_t F)
+{
+    __shared__ uint32_t s_code[kMergeRuns][kMergeStage];
+    __shared__ uint32_t s_first[kMergeRuns], s_len[kMergeRuns]; // the staged range of each run; 0xFFFFFFFF: not staged
+    uint32_t chunk;
+    const FrameDev& fd = frame_of_chunk(frames, F, blockIdx.x / kMergeParts, &chunk);
+    const uint32_t L = fd.L;
+    const uint32_t p0 = (blockIdx.x % kMergeParts) * kMergeThreads;
+    const uint32_t own_len = min(kLChunk, L - chunk * kLChunk);
+    if (L <= kLChunk || p0 >= own_len) return; // the whole workgroup
+    const uint32_t lane = lane_id(), wave = wave_id();
+    gvu2* runs = (gvu2*)fd.codes_tmp;
+    const uint32_t p = p0 + threadIdx.x;
+    const vu2 mine = runs[chunk * kLChunk + min(p, own_len - 1u)];
+    // the lowest and the highest code of the workgroup's lights
+    const uint32_t low = runs[chunk * kLChunk + p0].x;
+    const uint32_t high = runs[chunk * kLChunk + min(p0 + kMergeThreads, own_len) - 1u].x;
+    const uint32_t n_chunks = (L + kLChunk - 1) / kLChunk;
+    uint32_t rank = p;
+    for (uint32_t c0 = 0; c0 < n_chunks; c0 += kMergeRuns) {
+        __syncthreads(); // the previous stage's readers are done
+        uint32_t first[kMergeRuns / kMergeWaves], len[kMergeRuns / kMergeWaves];
+#pragma unroll
+        for (uint32_t k = 0; k < kMergeRuns / kMergeWaves; k++) {
+            const uint32_t c = c0 + k * kMergeWaves + wave;
+            const uint32_t n = c < n_chunks ? min(kLChunk, L - c * kLChunk) : 0u;
+            static_assert(kLChunk == VREN_WAVE * VREN_WAVE, "one sample per lane");
+            const uint32_t sample = lane * VREN_WAVE < n ? runs[c * kLChunk + lane * VREN_WAVE].x : 0xFFFFFFFFu;
+            // every bound of the workgroup is in [low, high + 1]: of the codes in front of the first range are all
+            // below it, and of the codes past the last sample below high + 1 at most the rest of its 64
+            const uint32_t m1 = (uint32_t)__popcll(ballot(sample < low)), m2 = (uint32_t)__popcll(ballot(sample < high + 1u));
+            first[k] = m1 ? (m1 - 1u) * VREN_WAVE : 0u;
+            len[k] = min(n, m2 * VREN_WAVE) - min(first[k], min(n, m2 * VREN_WAVE));
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kMergeRuns / kMergeWaves; k++) {
+            const uint32_t u = k * kMergeWaves + wave, c = c0 + u;
+            if (len[k] <= kMergeStage)
+                for (uint32_t i = lane; i < len[k]; i += VREN_WAVE) s_code[u][i] = runs[c * kLChunk + first[k] + i].x;
+            if (lane == 0) {
+                s_first[u] = first[k];
+                s_len[u] = len[k] <= kMergeStage ? len[k] : 0xFFFFFFFFu;
+            }
+        }
+        __syncthreads();
+        const uint32_t m = min(kMergeRuns, n_chunks - c0);
+#pragma unroll 8
+        for (uint32_t u = 0; u < m; u++) {
+            const uint32_t c = c0 + u;
+            if (c == chunk) continue; // uniform
+            const uint32_t bound = mine.x + (c < chunk ? 1u : 0u); // codes have at most 30 bits
+            const uint32_t n = s_len[u];
+            if (n != 0xFFFFFFFFu) {
+                const uint32_t* codes = s_code[u];
+                rank += s_first[u] + count_below([&](uint32_t i) { return codes[i]; }, n, bound, kMergeStage / 2);
+            } else {
+                rank += count_below([&](uint32_t i) { return (uint32_t)runs[c * kLChunk + i].x; },
+                                    min(kLChunk, L - c * kLChunk), bound, kLChunk / 2);
+            }
+        }
+    }
+    if (p < own_len) reinterpret_cast<uint2*>(fd.codes)[rank] = make_uint2(mine.x, mine.y);
 }
 
 // leaves (init_light_array_bvh.comp:42-65) + the first parent level (build_bvh.comp:32-55). `span` selects the
@@ -236,10 +533,8 @@ __global__ __launch_bounds__(256) void bvh_leaf_kernel(const FrameDev* __restric
     if (span == kLeavesLive && i >= live_end) return;
     if (span == kLeavesPadding) {
         if (i < live_end) return;
-        const float inf[3] = {VREN_F32_INF, VREN_F32_INF, VREN_F32_INF};
-        const float ninf[3] = {-VREN_F32_INF, -VREN_F32_INF, -VREN_F32_INF};
-        store_node(&fd.bvh[i], inf, ninf, VREN_BVH_INVALID_NODE);
-        if ((lane_id() & 31) == 0) store_node(&fd.bvh[padded + i / 32], inf, ninf, VREN_BVH_INVALID_NODE);
+        store_invalid(&fd.bvh[i]);
+        if ((lane_id() & 31) == 0) store_invalid(&fd.bvh[padded + i / 32]);
         return;
     }
     float mn[3], mx[3];
@@ -273,30 +568,35 @@ __global__ __launch_bounds__(256) void bvh_leaf_kernel(const FrameDev* __restric
     const uint64_t vm = ballot(valid);
     const uint32_t half = (lane_id() >> 5) << 5;
     const bool any = ((vm >> half) & 0xFFFFFFFFull) != 0ull;
-    half_wave_minmax(mn, mx);
-    if ((lane_id() & 31) == 0) {
+    half_wave_box(mn, mx);
+    if ((lane_id() & 31) == 31) {
         uint32_t gi = i / 32;
-        store_node(&fd.bvh[padded + gi], mn, mx, any ? i : VREN_BVH_INVALID_NODE);
+        store_node(&fd.bvh[padded + gi], mn, mx, any ? gi * 32 : VREN_BVH_INVALID_NODE);
     }
 }
 
-// remaining parent levels, one workgroup per frame
-__global__ __launch_bounds__(1024) void bvh_upper_kernel(const FrameDev* __restrict__ frames)
+// Remaining parent levels, one workgroup per frame. from_lights: only the first ceil(L / 32) nodes of the first
+// parent level hold lights (the rest are INVALID), so only they and their ancestors are read; the padding parents are
+// INVALID without reading their children (65 536 lights in 2^20 padded leaves: 94 -> 6.6 us). Frames of one chunk
+// have their whole BVH from lights_kernel.
+__global__ __launch_bounds__(1024) void bvh_upper_kernel(const FrameDev* __restrict__ frames, bool from_lights)
 {
     const FrameDev& fd = frames[blockIdx.x];
+    if (from_lights && fd.L <= kLChunk) return;
     const uint32_t padded = fd.bvh_padded;
     uint32_t src = padded, size = padded / 32;
+    uint32_t live = from_lights ? (fd.L + 31) / 32 : size; // nodes of the level that may be valid
     const uint32_t tid = threadIdx.x;
     while (size > 1) {
-        const uint32_t dst = src + size;
+        const uint32_t dst = src + size, parents = size / 32, live_parents = (live + 31) / 32;
         // one half-wave per parent
-        for (uint32_t base = 0; base < size; base += 1024) {
-            uint32_t c = base + tid;
-            bool in = c < size;
+        for (uint32_t base = 0; base < live_parents * 32; base += 1024) {
+            const uint32_t c = base + tid;
+            const bool in = c < live_parents * 32; // whole half-waves
             float mn[3] = {VREN_F32_INF, VREN_F32_INF, VREN_F32_INF};
             float mx[3] = {-VREN_F32_INF, -VREN_F32_INF, -VREN_F32_INF};
             bool valid = false;
-            if (in) {
+            if (c < live) {
                 const float4* q = reinterpret_cast<const float4*>(&fd.bvh[src + c]);
                 float4 lo = q[0], hi = q[1];
                 valid = __float_as_uint(lo.w) != VREN_BVH_INVALID_NODE;
@@ -312,36 +612,58 @@ __global__ __launch_bounds__(1024) void bvh_upper_kernel(const FrameDev* __restr
             const uint64_t vm = ballot(valid);
             const uint32_t half = (lane_id() >> 5) << 5;
             const bool any = ((vm >> half) & 0xFFFFFFFFull) != 0ull;
-            half_wave_minmax(mn, mx);
-            if (in && (lane_id() & 31) == 0) store_node(&fd.bvh[dst + c / 32], mn, mx, any ? src + c : VREN_BVH_INVALID_NODE);
+            half_wave_box(mn, mx);
+            if (in && (lane_id() & 31) == 31)
+                store_node(&fd.bvh[dst + c / 32], mn, mx, any ? src + (c & ~31u) : VREN_BVH_INVALID_NODE);
         }
+        for (uint32_t p = live_parents + tid; p < parents; p += 1024) store_invalid(&fd.bvh[dst + p]);
         __syncthreads();
         src = dst;
-        size /= 32;
+        size = parents;
+        live = live_parents;
     }
 }
 
 } // namespace
 
-int launch_lights(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w)
+// pad_blocks: workgroups of a single-frame call that write the padding leaves of a frame of one chunk
+int launch_lights(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
+                  uint32_t pad_blocks)
 {
-    if (w.light_bits == 4) lights_kernel<4><<<F, kLT, 0, s>>>(d_frames);
-    else lights_kernel<8><<<F, kLT, 0, s>>>(d_frames);
-    VREN_LAUNCH_CHECK(ctx);
+    const uint32_t chunks = w.light_chunks;
+    if (chunks) {
+        if (w.max_L > kLChunk) {
+            lights_bounds_kernel<<<chunks, kLT, 0, s>>>(d_frames, F);
+            VREN_LAUNCH_CHECK(ctx);
+        }
+        const uint32_t grid = chunks + pad_blocks;
+        if (w.light_bits == 4) lights_kernel<4><<<grid, kLT, 0, s>>>(d_frames, F, chunks);
+        else lights_kernel<8><<<grid, kLT, 0, s>>>(d_frames, F, chunks);
+        VREN_LAUNCH_CHECK(ctx);
+        if (w.max_L > kLChunk) {
+            lights_merge_kernel<<<chunks * kMergeParts, kMergeThreads, 0, s>>>(d_frames, F);
+            VREN_LAUNCH_CHECK(ctx);
+        }
+    }
     chain_mark(w, s);
     return VREN_OK;
 }
 
-// total_leaf_slots: the grid in leaf slots, the frames' live slots (live_leaf_base numbering) for kLeavesLive
+// total_leaf_slots: the grid in leaf slots, the frames' live slots (live_leaf_base numbering) for kLeavesLive; none
+// when no frame has more than one chunk of lights (lights_kernel has built their BVHs)
 int launch_bvh(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, uint32_t total_leaf_slots,
                bool leaves_from_lights, const ChainWork* w, uint32_t span)
 {
-    bvh_leaf_kernel<<<total_leaf_slots / 256, 256, 0, s>>>(d_frames, F, leaves_from_lights, span);
-    VREN_LAUNCH_CHECK(ctx);
+    if (total_leaf_slots) {
+        bvh_leaf_kernel<<<total_leaf_slots / 256, 256, 0, s>>>(d_frames, F, leaves_from_lights, span);
+        VREN_LAUNCH_CHECK(ctx);
+    }
     if (span == kLeavesPadding) return VREN_OK;
     if (w) chain_mark(*w, s);
-    bvh_upper_kernel<<<F, 1024, 0, s>>>(d_frames);
-    VREN_LAUNCH_CHECK(ctx);
+    if (total_leaf_slots) {
+        bvh_upper_kernel<<<F, 1024, 0, s>>>(d_frames, leaves_from_lights);
+        VREN_LAUNCH_CHECK(ctx);
+    }
     if (w) chain_mark(*w, s);
     return VREN_OK;
 }
@@ -405,18 +727,24 @@ VREN_EXPORT int vren_construct_point_light_bvh(vren_ctx* ctx, vren_stream_t stre
     f.bvh_root = vren_calc_bvh_root_index(light_count);
     f.bvh_levels = vren_calc_bvh_level_count(light_count);
     f.bvh_length = vren_calc_bvh_buffer_length(light_count);
-    if (light_count > kLdsCap) {
-        st = vren_ensure_scratch(ctx, (size_t)light_count * 8, s);
+    const uint32_t chunks = (light_count + kLChunk - 1) / kLChunk;
+    if (chunks > 1) {
+        const size_t runs = (size_t)light_count * 8;
+        st = vren_ensure_scratch(ctx, runs + (size_t)chunks * VREN_CHUNK_BOX_BYTES, s);
         if (st) return st;
         f.codes_tmp = static_cast<uint32_t*>(ctx->scratch);
+        f.chunk_box = reinterpret_cast<uint32_t*>(static_cast<char*>(ctx->scratch) + runs);
     }
     FrameDev* slot = vren_next_frame_slot(ctx);
     st = vren_upload_frames(ctx, s, slot, &f, 1);
     if (st) return st;
     ChainWork w;
     memset(&w, 0, sizeof(w));
-    st = launch_lights(ctx, s, slot, 1, w);
-    if (st) return st;
+    w.max_L = light_count;
+    w.light_chunks = chunks;
+    const bool padding = chunks == 1 && f.bvh_padded > ((light_count + 31u) & ~31u);
+    st = launch_lights(ctx, s, slot, 1, w, padding ? (f.bvh_padded + kLT - 1) / kLT : 0u);
+    if (st || chunks == 1) return st;
     uint32_t slots = (f.bvh_padded + VREN_LEAF_ALIGN - 1) / VREN_LEAF_ALIGN * VREN_LEAF_ALIGN;
     return launch_bvh(ctx, s, slot, 1, slots, true, nullptr, kLeavesAll);
 }
