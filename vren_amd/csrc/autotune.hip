@@ -15,21 +15,20 @@
 
 namespace {
 
-// defaults when nothing is tuned or forced: 8-bit digits, 23 keys per thread, 16 waves, onesweep (the fastest on
-// MI355X at 2^26 key-value pairs)
-constexpr int kDefaultBits = 8, kDefaultKpt = 23, kDefaultWaves = 16, kDefaultAlgorithm = 0;
-
 uint64_t bucket_key(uint64_t n, bool vals, uint32_t key_bits)
 {
     return ((uint64_t)ilog2_u64(n) << 8) | ((uint64_t)(vals ? 1 : 0) << 7) | key_bits;
 }
 
-int default_config()
+// the configuration when nothing is tuned or forced: onesweep with the default tile of n keys
+int default_config(uint64_t n, int num_cus)
 {
+    const int shape[][2] = {{8, 8}, {8, 16}, {15, 16}, {23, 16}}; // (keys per thread, waves), in RadixTile order
+    const int* d = shape[vren_radix_default_tile(n, num_cus)];
     for (int i = 0; i < vren_radix_config_count(); i++) {
         int b, k, w, a;
         vren_radix_config_info(i, &b, &k, &w, &a);
-        if (b == kDefaultBits && k == kDefaultKpt && w == kDefaultWaves && a == kDefaultAlgorithm) return i;
+        if (b == 8 && k == d[0] && w == d[1] && a == 0) return i;
     }
     return 0;
 }
@@ -55,7 +54,7 @@ int vren_radix_pick_config(vren_ctx* ctx, hipStream_t s, uint64_t n, bool vals, 
     auto it = ctx->radix_tuned.find(bucket_key(n, vals, key_bits));
     if (it != ctx->radix_tuned.end()) return it->second;
     (void)s;
-    return default_config();
+    return default_config(n, ctx->num_cus);
 }
 
 extern "C" {

@@ -175,11 +175,8 @@ __global__ __launch_bounds__(kLT) void lights_bounds_kernel(const FrameDev* __re
 }
 
 // One chunk: its lights' Morton codes, sorted stably with the light indices by an LSD radix sort on BITS-bit digits
-// (8 by default; 4 is a chain-shape choice). Keys stay in registers, warp-striped over kpt keys per thread (as few as
-// the chunk needs, so that a small frame's keys are spread over all the waves), and go through one LDS array between
-// passes; three barriers per pass: each wave ranks its keys in its own row of digit counters (which it clears itself),
-// one thread per digit turns the rows into wave prefixes, and the digits' starts across the four waves of digit
-// threads are added by the readers. Blocks at and past `chunks` write the frame's padding leaves (single-frame calls).
+// (8 by default; 4 is a chain-shape choice), as few keys per thread as the chunk needs, so that a small frame's keys are
+// spread over all the waves (block_sort). Blocks at and past `chunks` write the frame's padding leaves (single-frame calls).
 // A frame of one chunk then builds its BVH from the sorted lights: leaves, the first parent level over half-waves, the
 // rest from LDS. 4096 lights and their BVH took 34 us in three launches (21.7 + 6 + 6.8) and take one of 22 us
 // (256 lights: 21 -> 7 us), bound by the vector issue of its one CU; 65 536 lights took 292 us in one workgroup that
@@ -187,11 +184,9 @@ __global__ __launch_bounds__(kLT) void lights_bounds_kernel(const FrameDev* __re
 template <int BITS>
 __global__ __launch_bounds__(kLT) void lights_kernel(const FrameDev* __restrict__ frames, uint32_t F, uint32_t chunks)
 {
-    constexpr uint32_t RADIX = 1u << BITS;
     __shared__ uint2 s_pair[kLChunk];              // (code, light index)
     __shared__ float4 s_light[kLChunk];            // view position, radius (frames of one chunk)
-    __shared__ uint32_t s_row[kLWaves * RADIX];    // per wave: digit counts, then the digit's prefix
-    __shared__ uint32_t s_digits[4];               // keys per group of 64 digits
+    __shared__ BlockSortLds<BITS, kLWaves> s_sort;
     __shared__ uint32_t s_red[6 * kLWaves];
     __shared__ float s_node[kLChunk / 32][6];      // the first parent level, then the second one
     __shared__ float s_node2[kLChunk / 1024][6];
@@ -282,70 +277,7 @@ __global__ __launch_bounds__(kLT) void lights_kernel(const FrameDev* __restrict_
     }
 
     // the stable sort by code (ties keep light-index order)
-    uint32_t* row = s_row + wave * RADIX;
-    for (uint32_t shift = 0; shift < total_bits; shift += BITS) {
-        const uint32_t width = min((uint32_t)BITS, total_bits - shift);
-        for (uint32_t i = lane; i < RADIX; i += VREN_WAVE) row[i] = 0u;
-        __builtin_amdgcn_wave_barrier();
-        uint32_t digit[kLKPT], local[kLKPT];
-#pragma unroll
-        for (int j = 0; j < kLKPT; j++) {
-            digit[j] = __builtin_amdgcn_ubfe(e[j].x, shift, width);
-            local[j] = 0u;
-            if (j < (int)kpt) { // uniform
-                const bool valid = wbase + j * VREN_WAVE + lane < n;
-                const uint64_t vm = ballot(valid);
-                uint32_t plo = (uint32_t)vm, phi = (uint32_t)(vm >> 32);
-                const uint32_t before = valid ? row[digit[j]] : 0u;
-                match_digit<BITS>(digit[j], plo, phi);
-                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(phi, __builtin_amdgcn_mbcnt_lo(plo, 0u));
-                const uint64_t peers = ((uint64_t)phi << 32) | plo;
-                if (valid && (peers >> lane) == 1ull) row[digit[j]] = before + rank + 1u; // the highest peer lane
-                local[j] = before + rank;
-                __builtin_amdgcn_wave_barrier();
-            }
-        }
-        __syncthreads();
-        if (tid < ((RADIX + 63u) & ~63u)) { // whole waves
-            uint32_t c[kLWaves], sum = 0;
-#pragma unroll
-            for (int w = 0; w < kLWaves; w++) {
-                c[w] = tid < RADIX ? s_row[w * RADIX + tid] : 0u;
-                sum += c[w];
-            }
-            const uint32_t incl = wave_inclusive_sum(sum);
-            if (lane == VREN_WAVE - 1) s_digits[wave] = incl;
-            uint32_t run = incl - sum;
-            if (tid < RADIX) {
-#pragma unroll
-                for (int w = 0; w < kLWaves; w++) {
-                    s_row[w * RADIX + tid] = run;
-                    run += c[w];
-                }
-            }
-        }
-        __syncthreads();
-        uint32_t d1 = 0, d2 = 0, d3 = 0; // keys in the digit groups before groups 1, 2, 3
-        if (RADIX > 64) {
-            d1 = s_digits[0];
-            d2 = d1 + s_digits[1];
-            d3 = d2 + s_digits[2];
-        }
-#pragma unroll
-        for (int j = 0; j < kLKPT; j++) {
-            if (j < (int)kpt && wbase + j * VREN_WAVE + lane < n) {
-                const uint32_t d = digit[j], g = d >> 6;
-                const uint32_t before = g == 0 ? 0u : (g == 1 ? d1 : (g == 2 ? d2 : d3));
-                s_pair[before + row[d] + local[j]] = e[j];
-            }
-        }
-        __syncthreads();
-        if (shift + BITS < total_bits) {
-#pragma unroll
-            for (int j = 0; j < kLKPT; j++)
-                if (j < (int)kpt && wbase + j * VREN_WAVE + lane < n) e[j] = s_pair[wbase + j * VREN_WAVE + lane];
-        }
-    }
+    block_sort<BITS, kLKPT, kLWaves>(e, kpt, n, 0, total_bits, s_pair, s_sort, [](const uint2& x) { return x.x; });
     uint2* out = reinterpret_cast<uint2*>(whole ? fd.codes : fd.codes_tmp) + first;
     if (!whole) {
         for (uint32_t i = tid; i < n; i += kLT) out[i] = s_pair[i];

@@ -1,4 +1,5 @@
-// radix_device.hpp -- the stable tile ranking shared by the onesweep radix sort and the per-frame light sort.
+// radix_device.hpp -- the stable tile ranking of the onesweep radix sort, and the stable sort of one workgroup's elements
+// in LDS that the light stage and the sorts of a few thousand keys share.
 //
 // Keys are held warp-striped: key j of lane l of wave w sits at tile position (w * KPT + j) * 64 + l, so the
 // order (w, j, l) is the input order and ranking in that order is stable. A key's digit peers inside the wave
@@ -95,5 +96,93 @@ __device__ __forceinline__ void rank_wave_keys(const uint32_t (&digit)[KPT], uin
         if (valid && (peers >> lane) == 1ull) s_wave_row[d] = before + rank + 1u;
         local[j] = before + rank;
         __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// LDS of block_sort: per-wave digit rows and the digit counts of every 64 digits
+template <int BITS, int WAVES>
+struct BlockSortLds {
+    uint32_t row[WAVES << BITS];
+    uint32_t digits[4];
+};
+
+// Stable LSD sort of the n elements that a workgroup of WAVES waves holds, on key bits [begin_bit, end_bit) in BITS-bit
+// digits, one pass at least; s_elem[0 .. n) holds them in order afterwards (every thread may read it at once). Elements
+// are warp-striped, kpt <= KPT per thread (uniform): e[j] of lane l of wave w is element (w kpt + j) 64 + l. They stay in
+// registers within a pass and go through s_elem between passes. Three barriers per pass: each wave ranks its elements
+// in its own row of digit counters, which it clears itself; one thread per digit turns the rows into wave prefixes;
+// what lies in the groups of 64 digits before a digit's is added by the readers.
+template <int BITS, int KPT, int WAVES, typename E, typename Key>
+__device__ __forceinline__ void block_sort(E (&e)[KPT], uint32_t kpt, uint32_t n, uint32_t begin_bit, uint32_t end_bit,
+                                           E* s_elem, BlockSortLds<BITS, WAVES>& lds, Key key)
+{
+    constexpr uint32_t RADIX = 1u << BITS;
+    static_assert(BITS <= 8 && WAVES * VREN_WAVE >= (int)RADIX, "one thread per digit");
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+    const uint32_t wbase = wave * kpt * VREN_WAVE;
+    uint32_t* row = lds.row + wave * RADIX;
+    uint32_t shift = begin_bit;
+    for (;;) {
+        const uint32_t width = min((uint32_t)BITS, end_bit - shift);
+        for (uint32_t i = lane; i < RADIX; i += VREN_WAVE) row[i] = 0u;
+        __builtin_amdgcn_wave_barrier();
+        uint32_t digit[KPT], local[KPT];
+#pragma unroll
+        for (int j = 0; j < KPT; j++) {
+            digit[j] = __builtin_amdgcn_ubfe(key(e[j]), shift, width);
+            local[j] = 0u;
+            if (j < (int)kpt) {
+                const bool valid = wbase + j * VREN_WAVE + lane < n;
+                const uint64_t vm = ballot(valid);
+                uint32_t lo = (uint32_t)vm, hi = (uint32_t)(vm >> 32);
+                const uint32_t before = valid ? row[digit[j]] : 0u;
+                match_digit<BITS>(digit[j], lo, hi);
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+                const uint64_t peers = ((uint64_t)hi << 32) | lo;
+                if (valid && (peers >> lane) == 1ull) row[digit[j]] = before + rank + 1u; // the highest peer lane
+                local[j] = before + rank;
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+        __syncthreads();
+        if (tid < ((RADIX + 63u) & ~63u)) { // whole waves
+            uint32_t c[WAVES], sum = 0;
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) {
+                c[w] = tid < RADIX ? lds.row[w * RADIX + tid] : 0u;
+                sum += c[w];
+            }
+            const uint32_t incl = wave_inclusive_sum(sum);
+            if (lane == VREN_WAVE - 1) lds.digits[wave] = incl;
+            uint32_t run = incl - sum;
+            if (tid < RADIX) {
+#pragma unroll
+                for (int w = 0; w < WAVES; w++) {
+                    lds.row[w * RADIX + tid] = run;
+                    run += c[w];
+                }
+            }
+        }
+        __syncthreads();
+        uint32_t d1 = 0, d2 = 0, d3 = 0; // elements in the digit groups before groups 1, 2, 3
+        if (RADIX > 64) {
+            d1 = lds.digits[0];
+            d2 = d1 + lds.digits[1];
+            d3 = d2 + lds.digits[2];
+        }
+#pragma unroll
+        for (int j = 0; j < KPT; j++) {
+            if (j < (int)kpt && wbase + j * VREN_WAVE + lane < n) {
+                const uint32_t d = digit[j], g = d >> 6;
+                const uint32_t before = g == 0 ? 0u : (g == 1 ? d1 : (g == 2 ? d2 : d3));
+                s_elem[before + row[d] + local[j]] = e[j];
+            }
+        }
+        __syncthreads();
+        shift += BITS;
+        if (shift >= end_bit) return;
+#pragma unroll
+        for (int j = 0; j < KPT; j++)
+            if (j < (int)kpt && wbase + j * VREN_WAVE + lane < n) e[j] = s_elem[wbase + j * VREN_WAVE + lane];
     }
 }

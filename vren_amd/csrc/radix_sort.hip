@@ -12,6 +12,7 @@
 // workgroup are template parameters chosen by the autotuner (autotune.hip).
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "radix_device.hpp"
 #include "radix_sort.hpp"
@@ -37,13 +38,17 @@ __global__ void rs_init_kernel(uint32_t* hist, uint32_t n_hist, uint32_t* counte
 // atomics that all land in a few cache lines, so the number of workgroups is kept small
 constexpr uint32_t kHistThreads = 1024;
 
-// PAIRS: the keys are the first words of interleaved (key, value) pairs (key i at keys[2 i])
-template <int BITS, bool PAIRS = false>
+// PAIRS: the keys are the first words of interleaved (key, value) pairs (key i at keys[2 i]).
+// PARTS: every workgroup stores its own counts, pass by pass (hist[(pass * gridDim.x + blockIdx.x) * RADIX + digit]), and
+// workgroup 0 clears the passes' tile tickets; otherwise the counts are added to one histogram, which rs_init_kernel has cleared with the tickets.
+template <int BITS, bool PAIRS, bool PARTS>
 __global__ __launch_bounds__(kHistThreads) void rs_hist_kernel(const uint32_t* __restrict__ keys, uint64_t n,
                                                                uint32_t begin_bit, uint32_t end_bit, uint32_t passes,
                                                                uint32_t* __restrict__ hist,
-                                                               uint32_t* __restrict__ clear, uint64_t clear_words)
+                                                               uint32_t* __restrict__ clear, uint64_t clear_words,
+                                                               uint32_t* __restrict__ counters)
 {
+    if (PARTS && blockIdx.x == 0 && threadIdx.x < passes) counters[threadIdx.x] = 0u;
     constexpr uint32_t KPV = PAIRS ? 2 : 4; // keys per 16-byte load
     constexpr int RADIX = 1 << BITS;
     __shared__ uint32_t s_h[8 * RADIX];
@@ -107,7 +112,8 @@ __global__ __launch_bounds__(kHistThreads) void rs_hist_kernel(const uint32_t* _
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < passes * RADIX; i += kHistThreads) {
         uint32_t c = s_h[i];
-        if (c) atomic_add_agent(&hist[i], c);
+        if (PARTS) hist[(i / RADIX * gridDim.x + blockIdx.x) * RADIX + i % RADIX] = c;
+        else if (c) atomic_add_agent(&hist[i], c);
     }
 }
 
@@ -192,6 +198,27 @@ struct BucketStarts {
     uint32_t shift, mask;
 };
 
+// The histogram workgroups' counts of one pass (rs_hist_kernel with PARTS), n of them; n = 0: the pass reads scanned
+// digit bases. Up to kPartsMaxKeys keys, each tile sums and scans the few parts itself, beside its
+// key loads, which saves the clearing launch ahead of the histogram and the scanning one after it (2^16 pairs: 45.3
+// -> 38.9 us); tile 0 leaves the bases for whoever reads them after the pass. Above, the sum would take each tile longer
+// than the two launches take all of them.
+struct HistParts {
+    const uint32_t* counts;
+    uint32_t n;
+};
+constexpr uint64_t kPartsMaxKeys = 1ull << 19;
+constexpr uint32_t kPartsMaxBlocks = 16;
+// the tiles that take them: those of few keys per thread, whose registers have room
+constexpr bool takes_parts(int kpt) { return kpt <= 8; }
+
+// the scratch has room for them at every size, so that a scratch sized for more keys is always enough for fewer
+uint32_t parts_room(uint64_t n)
+{
+    return (uint32_t)std::min<uint64_t>(kPartsMaxBlocks, ceil_div_u64(std::max<uint64_t>(n, 1), 4096));
+}
+uint32_t parts_blocks(uint64_t n) { return n <= kPartsMaxKeys ? parts_room(n) : 0u; }
+
 template <int BITS, int KPT, int WAVES, bool VALS, bool RTS = false, bool IN_PAIRS = false, bool OUT_PAIRS = false,
           bool BSTARTS = false>
 __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t* __restrict__ keys_in,
@@ -199,10 +226,10 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
                                                                  uint32_t* __restrict__ keys_out,
                                                                  uint32_t* __restrict__ vals_out, uint64_t n,
                                                                  uint32_t shift, uint32_t width,
-                                                                 const uint32_t* __restrict__ digit_base,
+                                                                 uint32_t* __restrict__ digit_base,
                                                                  uint32_t* status, uint32_t* counter,
                                                                  uint32_t* __restrict__ clear_next,
-                                                                 const BucketStarts bs)
+                                                                 const BucketStarts bs, const HistParts parts)
 {
     constexpr int THREADS = WAVES * 64;
     constexpr int RADIX = 1 << BITS;
@@ -256,6 +283,14 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
             key[j] = wbase + j * VREN_WAVE + lane < tile_count ? __builtin_nontemporal_load(kin + j * VREN_WAVE)
                                                                : 0xFFFFFFFFu;
     }
+    // the histogram's parts of this thread's digit are requested with the keys and summed after the ranking
+    constexpr bool PARTS = !RTS && takes_parts(KPT);
+    uint32_t part[PARTS ? kPartsMaxBlocks : 1];
+    if constexpr (PARTS) {
+#pragma unroll
+        for (uint32_t b = 0; b < kPartsMaxBlocks; b++)
+            part[b] = tid < (uint32_t)RADIX && b < parts.n ? parts.counts[b * RADIX + tid] : 0u;
+    }
 #pragma unroll
     for (int j = 0; j < KPT; j++) digit[j] = __builtin_amdgcn_ubfe(key[j], shift, width);
     rank_wave_keys<BITS, KPT, false>(digit, wbase, tile_count, &s_whist[wave * RADIX], local);
@@ -281,8 +316,17 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
     // padding, and no tile looks back at the last one) are published before the block scan
     if (!RTS && tid < (uint32_t)RADIX)
         st_agent_u32(status + (uint64_t)tile * RADIX + tid, (tile == 0 ? RS_INCL : RS_AGG) | dcount);
-    uint32_t total;
+    uint32_t total, base = 0;
     uint32_t dstart = block_exclusive_sum<THREADS>(dcount, s_scan, &total);
+    if constexpr (PARTS) {
+        if (parts.n) {
+            uint32_t c = 0;
+#pragma unroll
+            for (uint32_t b = 0; b < kPartsMaxBlocks; b++) c += part[b];
+            base = block_exclusive_sum<THREADS>(c, s_scan, &total);
+            if (tile == 0 && tid < (uint32_t)RADIX) digit_base[tid] = base;
+        }
+    }
     uint32_t prefix = 0;
     if (tid < (uint32_t)RADIX) {
         uint32_t run = dstart;
@@ -323,7 +367,7 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
             const uint32_t tiles = (uint32_t)((n + TILE - 1) / TILE);
             s_goff[tid] = digit_base[(uint64_t)tid * tiles + tile] - dstart;
         } else {
-            s_goff[tid] = digit_base[tid] + prefix - dstart;
+            s_goff[tid] = (PARTS && parts.n ? base : digit_base[tid]) + prefix - dstart;
         }
     }
     __syncthreads();
@@ -424,10 +468,13 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
     }
 }
 
+// words of one histogram part: every pass's digits (at most four passes of 256, six of 64 or eight of 16)
+constexpr uint32_t kPartWords = 1024;
+
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct Layout {
-    size_t tmp_keys, tmp_vals, hist, counters, status_a, status_b, total;
+    size_t tmp_keys, tmp_vals, hist, counters, status_a, status_b, parts, total;
 };
 
 Layout layout_for(uint64_t n, bool vals, uint32_t min_tile, uint32_t max_radix)
@@ -447,6 +494,8 @@ Layout layout_for(uint64_t n, bool vals, uint32_t min_tile, uint32_t max_radix)
     off += align256(tiles * max_radix * 4);
     l.status_b = off;
     off += align256(tiles * max_radix * 4);
+    l.parts = off;
+    off += (size_t)parts_room(n) * kPartWords * 4;
     l.total = off;
     return l;
 }
@@ -478,10 +527,11 @@ int run_sort_rts(vren_ctx* ctx, hipStream_t s, uint32_t* keys, uint32_t* vals, u
         if (st) return st;
         if (vals) {
             rs_onesweep_kernel<BITS, KPT, WAVES, true, true><<<tiles, WAVES * 64, 0, s>>>(
-                ksrc, vsrc, kdst, vdst, n, shift, width, tile_hist, nullptr, nullptr, nullptr, BucketStarts{});
+                ksrc, vsrc, kdst, vdst, n, shift, width, tile_hist, nullptr, nullptr, nullptr, BucketStarts{}, HistParts{});
         } else {
             rs_onesweep_kernel<BITS, KPT, WAVES, false, true><<<tiles, WAVES * 64, 0, s>>>(
-                ksrc, nullptr, kdst, nullptr, n, shift, width, tile_hist, nullptr, nullptr, nullptr, BucketStarts{});
+                ksrc, nullptr, kdst, nullptr, n, shift, width, tile_hist, nullptr, nullptr, nullptr, BucketStarts{},
+                HistParts{});
         }
         VREN_LAUNCH_CHECK(ctx);
         std::swap(ksrc, kdst);
@@ -492,6 +542,43 @@ int run_sort_rts(vren_ctx* ctx, hipStream_t s, uint32_t* keys, uint32_t* vals, u
         if (vals) VREN_HIP(ctx, hipMemcpyAsync(vals, vsrc, n * 4, hipMemcpyDeviceToDevice, s));
     }
     return VREN_OK;
+}
+
+// The digit counts of every pass, ready for the passes: parts that the tiles sum (few keys), or scanned digit bases in
+// `hist`; the look-back statuses of the first pass and the tickets are cleared too.
+template <int BITS, int KPT, bool PAIRS>
+int run_hist(vren_ctx* ctx, hipStream_t s, const uint32_t* keys, uint64_t n, uint32_t begin_bit, uint32_t end_bit,
+             uint32_t passes, uint64_t tiles, char* scratch, const Layout& L, HistParts* parts)
+{
+    constexpr uint32_t RADIX = 1u << BITS;
+    uint32_t* hist = reinterpret_cast<uint32_t*>(scratch + L.hist);
+    uint32_t* counters = reinterpret_cast<uint32_t*>(scratch + L.counters);
+    uint32_t* status = reinterpret_cast<uint32_t*>(scratch + L.status_a);
+    const uint32_t blocks = takes_parts(KPT) ? parts_blocks(n) : 0u;
+    if (blocks) {
+        uint32_t* counts = reinterpret_cast<uint32_t*>(scratch + L.parts);
+        rs_hist_kernel<BITS, PAIRS, true><<<blocks, kHistThreads, 0, s>>>(keys, n, begin_bit, end_bit, passes, counts, status,
+                                                                          tiles * RADIX, counters);
+        VREN_LAUNCH_CHECK(ctx);
+        *parts = HistParts{counts, blocks};
+        return VREN_OK;
+    }
+    rs_init_kernel<<<1, 256, 0, s>>>(hist, passes * RADIX, counters, passes);
+    VREN_LAUNCH_CHECK(ctx);
+    const uint32_t hb = (uint32_t)std::min<uint64_t>((uint64_t)ctx->num_cus, std::max<uint64_t>(1, ceil_div_u64(n, 16384)));
+    rs_hist_kernel<BITS, PAIRS, false><<<hb, kHistThreads, 0, s>>>(keys, n, begin_bit, end_bit, passes, hist, status,
+                                                                   tiles * RADIX, counters);
+    VREN_LAUNCH_CHECK(ctx);
+    rs_hexscan_kernel<BITS><<<1, 256, 0, s>>>(hist, passes);
+    VREN_LAUNCH_CHECK(ctx);
+    *parts = HistParts{nullptr, 0};
+    return VREN_OK;
+}
+
+// the counts of pass p
+inline HistParts pass_parts(const HistParts& parts, uint32_t p, uint32_t radix)
+{
+    return HistParts{parts.n ? parts.counts + p * parts.n * radix : nullptr, parts.n};
 }
 
 template <int BITS, int KPT, int WAVES>
@@ -509,13 +596,9 @@ int run_sort(vren_ctx* ctx, hipStream_t s, uint32_t* keys, uint32_t* vals, uint6
     uint32_t* tk = reinterpret_cast<uint32_t*>(scratch + L.tmp_keys);
     uint32_t* tv = vals ? reinterpret_cast<uint32_t*>(scratch + L.tmp_vals) : nullptr;
 
-    rs_init_kernel<<<1, 256, 0, s>>>(hist, passes * RADIX, counters, passes);
-    VREN_LAUNCH_CHECK(ctx);
-    uint32_t hb = (uint32_t)std::min<uint64_t>((uint64_t)ctx->num_cus, std::max<uint64_t>(1, ceil_div_u64(n, 16384)));
-    rs_hist_kernel<BITS><<<hb, kHistThreads, 0, s>>>(keys, n, begin_bit, end_bit, passes, hist, st[0], tiles * RADIX);
-    VREN_LAUNCH_CHECK(ctx);
-    rs_hexscan_kernel<BITS><<<1, 256, 0, s>>>(hist, passes);
-    VREN_LAUNCH_CHECK(ctx);
+    HistParts parts;
+    const int err = run_hist<BITS, KPT, false>(ctx, s, keys, n, begin_bit, end_bit, passes, tiles, scratch, L, &parts);
+    if (err) return err;
     uint32_t *ksrc = keys, *vsrc = vals, *kdst = tk, *vdst = tv;
     for (uint32_t p = 0; p < passes; p++) {
         uint32_t shift = begin_bit + p * BITS;
@@ -524,11 +607,11 @@ int run_sort(vren_ctx* ctx, hipStream_t s, uint32_t* keys, uint32_t* vals, uint6
         if (vals) {
             rs_onesweep_kernel<BITS, KPT, WAVES, true><<<(uint32_t)tiles, WAVES * 64, 0, s>>>(
                 ksrc, vsrc, kdst, vdst, n, shift, width, hist + p * RADIX, st[p & 1], counters + p, clear_next,
-                BucketStarts{});
+                BucketStarts{}, pass_parts(parts, p, RADIX));
         } else {
             rs_onesweep_kernel<BITS, KPT, WAVES, false><<<(uint32_t)tiles, WAVES * 64, 0, s>>>(
                 ksrc, nullptr, kdst, nullptr, n, shift, width, hist + p * RADIX, st[p & 1], counters + p, clear_next,
-                BucketStarts{});
+                BucketStarts{}, pass_parts(parts, p, RADIX));
         }
         VREN_LAUNCH_CHECK(ctx);
         std::swap(ksrc, kdst);
@@ -569,6 +652,23 @@ __global__ __launch_bounds__(256) void bucket_run_starts_kernel(const uint32_t* 
     }
 }
 
+// The bucket starts of sorted pairs by binary search, one thread per bucket: for fewer pairs than buckets, where the
+// passes would write most starts one after the other in the gaps between neighbouring keys (1000 pairs into 65536
+// buckets: 66 -> 9.7 us, 20000: 45 -> 24).
+__global__ __launch_bounds__(256) void bucket_search_kernel(const uint32_t* __restrict__ pairs, uint32_t n,
+                                                            const BucketStarts bs, uint32_t n_buckets)
+{
+    const uint32_t b = blockIdx.x * 256 + threadIdx.x;
+    if (b >= n_buckets) return;
+    uint32_t lo = 0, hi = n; // the first position whose bucket is at least b
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (((pairs[2 * (uint64_t)mid] >> bs.shift) & bs.mask) < b) lo = mid + 1;
+        else hi = mid;
+    }
+    bs.offsets[b] = lo;
+}
+
 // stable sort of interleaved (key, value) pairs on bits [begin_bit, end_bit), at most two digit passes: the first
 // pass reads the pairs and the last one writes them (a single pass does both); between two passes the keys and
 // values sit split in the scratch. Per pair: 8 B histogram read + 16 B per pass. With bucket_offsets, the final
@@ -589,33 +689,30 @@ int run_sort_pairs(vren_ctx* ctx, hipStream_t s, const uint32_t* in, uint32_t* o
     uint32_t* tk = reinterpret_cast<uint32_t*>(scratch + L.tmp_keys);
     uint32_t* tv = reinterpret_cast<uint32_t*>(scratch + L.tmp_vals);
 
-    rs_init_kernel<<<1, 256, 0, s>>>(hist, passes * RADIX, counters, passes);
-    VREN_LAUNCH_CHECK(ctx);
-    uint32_t hb = (uint32_t)std::min<uint64_t>((uint64_t)ctx->num_cus, std::max<uint64_t>(1, ceil_div_u64(n, 16384)));
-    rs_hist_kernel<BITS, true><<<hb, kHistThreads, 0, s>>>(in, n, begin_bit, end_bit, passes, hist, st[0], tiles * RADIX);
-    VREN_LAUNCH_CHECK(ctx);
-    rs_hexscan_kernel<BITS><<<1, 256, 0, s>>>(hist, passes);
-    VREN_LAUNCH_CHECK(ctx);
+    HistParts parts;
+    const int err = run_hist<BITS, KPT, true>(ctx, s, in, n, begin_bit, end_bit, passes, tiles, scratch, L, &parts);
+    if (err) return err;
+    const HistParts parts1 = pass_parts(parts, 1, RADIX);
     const BucketStarts bs{bucket_offsets, begin_bit, n_buckets ? n_buckets - 1u : 0u};
     if (passes == 1) {
         if (bucket_offsets)
             rs_onesweep_kernel<BITS, KPT, WAVES, true, false, true, true, true><<<(uint32_t)tiles, WAVES * 64, 0, s>>>(
-                in, nullptr, out, nullptr, n, begin_bit, end_bit - begin_bit, hist, st[0], counters, nullptr, bs);
+                in, nullptr, out, nullptr, n, begin_bit, end_bit - begin_bit, hist, st[0], counters, nullptr, bs, parts);
         else
             rs_onesweep_kernel<BITS, KPT, WAVES, true, false, true, true><<<(uint32_t)tiles, WAVES * 64, 0, s>>>(
-                in, nullptr, out, nullptr, n, begin_bit, end_bit - begin_bit, hist, st[0], counters, nullptr, bs);
+                in, nullptr, out, nullptr, n, begin_bit, end_bit - begin_bit, hist, st[0], counters, nullptr, bs, parts);
         VREN_LAUNCH_CHECK(ctx);
     } else {
         const uint32_t shift1 = begin_bit + BITS;
         rs_onesweep_kernel<BITS, KPT, WAVES, true, false, true, false><<<(uint32_t)tiles, WAVES * 64, 0, s>>>(
-            in, nullptr, tk, tv, n, begin_bit, BITS, hist, st[0], counters, st[1], BucketStarts{});
+            in, nullptr, tk, tv, n, begin_bit, BITS, hist, st[0], counters, st[1], BucketStarts{}, parts);
         VREN_LAUNCH_CHECK(ctx);
         if (bucket_offsets)
             rs_onesweep_kernel<BITS, KPT, WAVES, true, false, false, true, true><<<(uint32_t)tiles, WAVES * 64, 0, s>>>(
-                tk, tv, out, nullptr, n, shift1, end_bit - shift1, hist + RADIX, st[1], counters + 1, nullptr, bs);
+                tk, tv, out, nullptr, n, shift1, end_bit - shift1, hist + RADIX, st[1], counters + 1, nullptr, bs, parts1);
         else
             rs_onesweep_kernel<BITS, KPT, WAVES, true, false, false, true><<<(uint32_t)tiles, WAVES * 64, 0, s>>>(
-                tk, tv, out, nullptr, n, shift1, end_bit - shift1, hist + RADIX, st[1], counters + 1, nullptr, bs);
+                tk, tv, out, nullptr, n, shift1, end_bit - shift1, hist + RADIX, st[1], counters + 1, nullptr, bs, parts1);
         VREN_LAUNCH_CHECK(ctx);
     }
     if (bucket_offsets) {
@@ -625,6 +722,73 @@ int run_sort_pairs(vren_ctx* ctx, hipStream_t s, const uint32_t* in, uint32_t* o
         VREN_LAUNCH_CHECK(ctx);
     }
     return VREN_OK;
+}
+
+// ---- a few thousand keys: one workgroup, one launch ----------------------------------------------------------------
+// Every pass in LDS (block_sort). Up to kBlockSortMax keys the launches of the multi-tile sort, each with its own loads
+// and its own wait for the previous one, take longer than one CU takes to rank the keys: 4096 pairs on 32 bits 64.7 us
+// (29.2 with its best configuration) -> 13.7, 8192 pairs 66.1 (30.4) -> 21.7.
+constexpr uint32_t kBlockSortMax = 8192;
+constexpr int kBlockSortThreads = 1024, kBlockSortWaves = kBlockSortThreads / VREN_WAVE;
+
+template <int KPT, bool VALS>
+__global__ __launch_bounds__(kBlockSortThreads) void rs_block_kernel(uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
+                                                                     uint32_t n, uint32_t begin_bit, uint32_t end_bit)
+{
+    typedef std::conditional_t<VALS, uint2, uint32_t> E;
+    __shared__ E s_elem[KPT * kBlockSortThreads];
+    __shared__ BlockSortLds<8, kBlockSortWaves> s_sort;
+    const uint32_t kpt = (n + kBlockSortThreads - 1) / kBlockSortThreads;
+    const uint32_t first = wave_id() * kpt * VREN_WAVE + lane_id();
+    E e[KPT];
+#pragma unroll
+    for (int j = 0; j < KPT; j++) {
+        const uint32_t i = first + j * VREN_WAVE;
+        e[j] = E{};
+        if (j < (int)kpt && i < n) {
+            if constexpr (VALS) e[j] = make_uint2(keys[i], vals[i]);
+            else e[j] = keys[i];
+        }
+    }
+    block_sort<8, KPT, kBlockSortWaves>(e, kpt, n, begin_bit, end_bit, s_elem, s_sort, [](const E& x) {
+        if constexpr (VALS) return x.x;
+        else return x;
+    });
+    for (uint32_t i = threadIdx.x; i < n; i += kBlockSortThreads) {
+        if constexpr (VALS) {
+            keys[i] = s_elem[i].x;
+            vals[i] = s_elem[i].y;
+        } else {
+            keys[i] = s_elem[i];
+        }
+    }
+}
+
+// the same for interleaved pairs, with the bucket starts: position i writes the starts of the buckets after its
+// predecessor's up to its own, the last position also those after it
+template <int KPT>
+__global__ __launch_bounds__(kBlockSortThreads) void rs_block_pairs_kernel(const uint2* __restrict__ in, uint2* __restrict__ out,
+                                                                           uint32_t n, uint32_t begin_bit, uint32_t end_bit,
+                                                                           const BucketStarts bs, uint32_t n_buckets)
+{
+    __shared__ uint2 s_elem[KPT * kBlockSortThreads];
+    __shared__ BlockSortLds<8, kBlockSortWaves> s_sort;
+    const uint32_t kpt = (n + kBlockSortThreads - 1) / kBlockSortThreads;
+    const uint32_t first = wave_id() * kpt * VREN_WAVE + lane_id();
+    uint2 e[KPT];
+#pragma unroll
+    for (int j = 0; j < KPT; j++) {
+        const uint32_t i = first + j * VREN_WAVE;
+        e[j] = j < (int)kpt && i < n ? in[i] : make_uint2(0u, 0u);
+    }
+    block_sort<8, KPT, kBlockSortWaves>(e, kpt, n, begin_bit, end_bit, s_elem, s_sort, [](const uint2& x) { return x.x; });
+    for (uint32_t i = threadIdx.x; i < n; i += kBlockSortThreads) out[i] = s_elem[i];
+    if (!bs.offsets) return;
+    const auto bucket = [&](uint32_t i) { return (s_elem[i].x >> bs.shift) & bs.mask; };
+    for (uint32_t i = threadIdx.x; i <= n; i += kBlockSortThreads) {
+        const uint32_t from = i == 0 ? 0u : bucket(i - 1) + 1u, to = i == n ? n_buckets : bucket(i) + 1u;
+        for (uint32_t c = from; c < to; c++) bs.offsets[c] = i;
+    }
 }
 
 typedef int (*sort_fn)(vren_ctx*, hipStream_t, uint32_t*, uint32_t*, uint64_t, uint32_t, uint32_t, char*, const Layout&);
@@ -647,6 +811,20 @@ const SortConfig kConfigs[] = {
 };
 
 } // namespace
+
+// Untuned sorts use 8-bit digits and the smallest tile that still gives no CU more than one tile per pass: a pass then
+// takes one tile's time, which is what its size makes it, and above that the largest tile, whose digit runs are the
+// longest stores. The smallest one stops at half the CUs, since the look-back over more tiles costs what the tile saves.
+// 2^16 pairs on 32 bits: 38.9 us in 4096-key tiles, 45.6 in 8192, 83.5 in 23552; 2^20: 79.5, 76.6, 101; 3 M: 142, 125,
+// 115 and 103 in 15360; 4.2 M: 173, 147, 123 and 148.
+RadixTile vren_radix_default_tile(uint64_t n, int num_cus)
+{
+    const uint64_t cus = (uint64_t)num_cus;
+    if (n <= 4096 * cus / 2) return kRadixTile4096;
+    if (n <= 8192 * cus) return kRadixTile8192;
+    if (n <= 15360 * cus) return kRadixTile15360;
+    return kRadixTile23552;
+}
 
 int vren_radix_config_count() { return (int)(sizeof(kConfigs) / sizeof(kConfigs[0])); }
 
@@ -681,13 +859,35 @@ int vren_radix_sort_pairs_interleaved(vren_ctx* ctx, hipStream_t s, const uint32
         VREN_HIP(ctx, hipMemcpyAsync(out_pairs, in_pairs, n * 8, hipMemcpyDeviceToDevice, s));
         return VREN_OK;
     }
-    // the default configuration's tile (8-bit digits, 23 keys per thread, 16 waves); below 2^21 pairs, 11 keys per
-    // thread (more tiles to spread over the CUs: 2^20 pairs in 54 instead of 73 us for 65536 buckets)
-    if (n < (1u << 21))
-        return run_sort_pairs<8, 11, 16>(ctx, s, in_pairs, out_pairs, n, begin_bit, end_bit,
-                                         static_cast<char*>(scratch), L, bucket_offsets, n_buckets);
-    return run_sort_pairs<8, 23, 16>(ctx, s, in_pairs, out_pairs, n, begin_bit, end_bit, static_cast<char*>(scratch), L,
-                                     bucket_offsets, n_buckets);
+    // fewer pairs than buckets: the starts by search, after a sort without them
+    const bool search = bucket_offsets && n < n_buckets;
+    uint32_t* starts = search ? nullptr : bucket_offsets;
+    const BucketStarts bs{bucket_offsets, begin_bit, n_buckets ? n_buckets - 1u : 0u};
+    int st = VREN_OK;
+    if (n <= kBlockSortMax) {
+        const uint2* in = reinterpret_cast<const uint2*>(in_pairs);
+        uint2* out = reinterpret_cast<uint2*>(out_pairs);
+        const BucketStarts own{starts, bs.shift, bs.mask};
+        if (n <= 2048)
+            rs_block_pairs_kernel<2><<<1, kBlockSortThreads, 0, s>>>(in, out, (uint32_t)n, begin_bit, end_bit, own, n_buckets);
+        else
+            rs_block_pairs_kernel<8><<<1, kBlockSortThreads, 0, s>>>(in, out, (uint32_t)n, begin_bit, end_bit, own, n_buckets);
+        VREN_LAUNCH_CHECK(ctx);
+    } else {
+        const auto sort = [&](auto run) {
+            return run(ctx, s, in_pairs, out_pairs, n, begin_bit, end_bit, static_cast<char*>(scratch), L, starts, n_buckets);
+        };
+        switch (vren_radix_default_tile(n, ctx->num_cus)) {
+        case kRadixTile4096: st = sort(run_sort_pairs<8, 8, 8>); break;
+        case kRadixTile8192: st = sort(run_sort_pairs<8, 8, 16>); break;
+        case kRadixTile15360: st = sort(run_sort_pairs<8, 15, 16>); break;
+        default: st = sort(run_sort_pairs<8, 23, 16>);
+        }
+    }
+    if (st || !search) return st;
+    bucket_search_kernel<<<(n_buckets + 255) / 256, 256, 0, s>>>(out_pairs, (uint32_t)n, bs, n_buckets);
+    VREN_LAUNCH_CHECK(ctx);
+    return VREN_OK;
 }
 
 extern "C" {
@@ -708,6 +908,19 @@ VREN_EXPORT int vren_radix_sort(vren_ctx* ctx, vren_stream_t stream, uint32_t* k
         return vren_fail(ctx, VREN_EINVAL, "radix_sort: scratch of %zu bytes, %zu required", scratch_bytes,
                          vren_radix_sort_scratch_bytes(n, vals != nullptr));
     if (ctx->device < 0) return vren_fail(ctx, VREN_EINVAL, "radix_sort: context has no device");
+    if (n <= kBlockSortMax && begin_bit < end_bit && ctx->radix_forced < 0) {
+        hipStream_t s = (hipStream_t)stream;
+        const uint32_t m = (uint32_t)n;
+        if (vals) {
+            if (m <= 2048) rs_block_kernel<2, true><<<1, kBlockSortThreads, 0, s>>>(keys, vals, m, begin_bit, end_bit);
+            else rs_block_kernel<8, true><<<1, kBlockSortThreads, 0, s>>>(keys, vals, m, begin_bit, end_bit);
+        } else {
+            if (m <= 2048) rs_block_kernel<2, false><<<1, kBlockSortThreads, 0, s>>>(keys, vals, m, begin_bit, end_bit);
+            else rs_block_kernel<8, false><<<1, kBlockSortThreads, 0, s>>>(keys, vals, m, begin_bit, end_bit);
+        }
+        VREN_LAUNCH_CHECK(ctx);
+        return VREN_OK;
+    }
     int cfg = vren_radix_pick_config(ctx, (hipStream_t)stream, n, vals != nullptr, end_bit - begin_bit);
     return vren_radix_sort_with_config(ctx, (hipStream_t)stream, cfg, keys, vals, n, begin_bit, end_bit, scratch,
                                        scratch_bytes);
