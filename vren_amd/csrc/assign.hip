@@ -426,10 +426,8 @@ __device__ __forceinline__ uint32_t emit_bitmask(uint32_t* bitmask, uint32_t* su
 // counting its hit lights and keeping the first VREN_LIST_SLOT of them in the half's LDS list; a list of at most
 // VREN_LIST_SLOT lights is sorted (the rank of each index among the list) into the cluster's slot, so the writing
 // pass copies it instead of traversing again.
-__global__ __launch_bounds__(256, 8) void assign_count_kernel(const FrameDev* __restrict__ frames, uint32_t F,
-                                                             uint32_t mask_words)
+__device__ __forceinline__ void assign_count_body(const FrameDev* __restrict__ frames, uint32_t F, uint32_t* s_mem)
 {
-    extern __shared__ uint32_t s_mem[];
     const uint32_t wpb = blockDim.x / VREN_WAVE;
     const uint32_t wave = wave_id();
     const uint32_t lane = lane_id();
@@ -474,7 +472,7 @@ __global__ __launch_bounds__(256, 8) void assign_count_kernel(const FrameDev* __
 // exclusive scan of counts[0 .. min(cluster_count, key_cap)) -> offsets and assigned_total: one workgroup per
 // frame walks its counts 4096 at a time with a running carry (no cross-workgroup chaining, no tickets; a frame
 // holds a few thousand clusters, at most key_cap)
-__global__ __launch_bounds__(1024) void assign_offsets_kernel(const FrameDev* __restrict__ frames)
+__device__ __forceinline__ void assign_offsets_body(const FrameDev* __restrict__ frames)
 {
     __shared__ uint32_t s_wave[16];
     const FrameDev& fd = frames[blockIdx.x];
@@ -511,9 +509,9 @@ struct ListBounds {
 
 // WRITE: each cluster's list at its offset: copied from the slot the counting pass kept, or traversed again
 // (bitmask, emitted in ascending light index) when it was longer than a slot
-__global__ __launch_bounds__(256, 8) void assign_write_kernel(const FrameDev* __restrict__ frames, uint32_t F, uint32_t mask_words)
+__device__ __forceinline__ void assign_write_body(const FrameDev* __restrict__ frames, uint32_t F, uint32_t mask_words,
+                                                  uint32_t* s_mem)
 {
-    extern __shared__ uint32_t s_mem[];
     const uint32_t wpb = blockDim.x / VREN_WAVE;
     const uint32_t wave = wave_id();
     const uint32_t lane = lane_id();
@@ -551,6 +549,68 @@ __global__ __launch_bounds__(256, 8) void assign_write_kernel(const FrameDev* __
         });
 }
 
+// [begin, end) of the index-buffer entries of a tile's light lists, for shade: the tile's clusters are the consecutive
+// indices [c0, c0 + u) (clusters kernel) and their lists are consecutive in the index buffer, so the range runs from the
+// first cluster's offset to the end of the last list (both clamped to the capacities like the per-pixel lists). One
+// thread per tile, ahead of the writing pass's lists, which it does not depend on.
+struct TileRanges {
+    const uint32_t* tile_frame;
+    const uint2* tile_cl;
+    uint2* tile_range; // null: no ranges
+    uint32_t total_tiles;
+};
+
+__device__ __forceinline__ void write_tile_ranges(const FrameDev* __restrict__ frames, const TileRanges& r)
+{
+    if (!r.tile_range) return;
+    for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < r.total_tiles; g += gridDim.x * blockDim.x) {
+        const FrameDev& fd = frames[frame_of_tile(r.tile_frame, g)];
+        const uint2 c = r.tile_cl[g];
+        uint32_t a = 0, b = 0;
+        if (g - fd.tile_base < fd.Sx * fd.Sy && fd.L > 0 && c.y > 0 && c.x < fd.key_cap) { // not a padding tile
+            const uint32_t c1 = min(c.x + c.y, fd.key_cap) - 1u;
+            a = min(fd.offsets[c.x], fd.index_cap);
+            const uint64_t e = (uint64_t)fd.offsets[c1] + fd.counts[c1];
+            b = e > fd.index_cap ? fd.index_cap : (uint32_t)e;
+        }
+        r.tile_range[g] = make_uint2(a, b);
+    }
+}
+
+// clear: the cluster stage's tickets and statuses, which nothing reads after it, left zero for the chain's next run
+__global__ __launch_bounds__(256, 8) void assign_count_kernel(const FrameDev* __restrict__ frames, uint32_t F,
+                                                             uint32_t* __restrict__ clear, uint32_t clear_words)
+{
+    extern __shared__ uint32_t s_mem[];
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < clear_words; i += gridDim.x * 256) clear[i] = 0u;
+    assign_count_body(frames, F, s_mem);
+}
+__global__ __launch_bounds__(256, 8) void assign_count_one_kernel(const FrameDev one)
+{
+    extern __shared__ uint32_t s_mem[];
+    assign_count_body(inline_frame(), 1, s_mem);
+}
+__global__ __launch_bounds__(1024) void assign_offsets_kernel(const FrameDev* __restrict__ frames) { assign_offsets_body(frames); }
+__global__ __launch_bounds__(1024) void assign_offsets_one_kernel(const FrameDev one) { assign_offsets_body(inline_frame()); }
+__global__ __launch_bounds__(256, 8) void assign_write_kernel(const FrameDev* __restrict__ frames, uint32_t F,
+                                                             uint32_t mask_words, const TileRanges ranges)
+{
+    extern __shared__ uint32_t s_mem[];
+    write_tile_ranges(frames, ranges);
+    assign_write_body(frames, F, mask_words, s_mem);
+}
+__global__ __launch_bounds__(256, 8) void assign_write_one_kernel(const FrameDev one, uint32_t mask_words)
+{
+    extern __shared__ uint32_t s_mem[];
+    assign_write_body(inline_frame(), 1, mask_words, s_mem);
+}
+
+__global__ void empty_lists_kernel(uint32_t* counts, uint32_t* offsets, uint32_t n, uint32_t* total)
+{
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) counts[i] = offsets[i] = 0u;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *total = 0u;
+}
+
 // enough resident waves per CU (32 by default, the chain shape's choice otherwise) to hide the dependent node loads
 // of the traversals
 uint32_t persistent_blocks(vren_ctx* ctx, uint32_t wpb, uint32_t waves_per_cu)
@@ -561,9 +621,10 @@ uint32_t persistent_blocks(vren_ctx* ctx, uint32_t wpb, uint32_t waves_per_cu)
 
 } // namespace
 
-int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w)
+int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
+                  const FrameDev* one)
 {
-    if (w.max_L == 0) return VREN_OK;
+    if (w.max_L == 0) return one ? VREN_OK : launch_chain_init(ctx, s, w); // no lists; the next run finds cleared words
     const uint32_t mask_words = (w.max_L + 31) / 32;
     const size_t per_wave = (size_t)(kStack + mask_words + (mask_words + 31) / 32) * 4;
     uint32_t wpb = 4;
@@ -572,15 +633,25 @@ int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32
     // two stacks and two lists per wave (one per half), the chunk's boxes and cluster frames
     constexpr size_t count_per_wave = (size_t)2 * (kStackHalf + VREN_LIST_SLOT) * 4 + VREN_WAVE * (sizeof(float) * 6 + 4);
     static_assert(count_per_wave * 4 <= 160 * 1024 / 8, "assign_count: 8 workgroups of 4 waves must fit a CU's LDS");
-    assign_count_kernel<<<persistent_blocks(ctx, 4, w.assign_wpc), 4 * VREN_WAVE, count_per_wave * 4, s>>>(d_frames, F,
-                                                                                                    mask_words);
+    const uint32_t count_blocks = persistent_blocks(ctx, 4, w.assign_wpc), write_blocks = persistent_blocks(ctx, wpb, w.assign_wpc);
+    if (one) {
+        assign_count_one_kernel<<<count_blocks, 4 * VREN_WAVE, count_per_wave * 4, s>>>(*one);
+        VREN_LAUNCH_CHECK(ctx);
+        assign_offsets_one_kernel<<<1, 1024, 0, s>>>(*one);
+        VREN_LAUNCH_CHECK(ctx);
+        assign_write_one_kernel<<<write_blocks, wpb * VREN_WAVE, per_wave * wpb, s>>>(*one, mask_words);
+        VREN_LAUNCH_CHECK(ctx);
+        return VREN_OK;
+    }
+    assign_count_kernel<<<count_blocks, 4 * VREN_WAVE, count_per_wave * 4, s>>>(
+        d_frames, F, w.tickets, (uint32_t)(chain_work_clear_bytes(w.total_tiles) / 4));
     VREN_LAUNCH_CHECK(ctx);
     chain_mark(w, s);
     assign_offsets_kernel<<<F, 1024, 0, s>>>(d_frames);
     VREN_LAUNCH_CHECK(ctx);
     chain_mark(w, s);
-    assign_write_kernel<<<persistent_blocks(ctx, wpb, w.assign_wpc), wpb * VREN_WAVE, per_wave * wpb, s>>>(d_frames, F,
-                                                                                                   mask_words);
+    const TileRanges ranges{F > 1 ? w.tile_frame : nullptr, w.tile_cl, w.tile_range, w.total_tiles};
+    assign_write_kernel<<<write_blocks, wpb * VREN_WAVE, per_wave * wpb, s>>>(d_frames, F, mask_words, ranges);
     VREN_LAUNCH_CHECK(ctx);
     chain_mark(w, s);
     return VREN_OK;
@@ -627,24 +698,15 @@ extern "C" VREN_EXPORT int vren_assign_lights(vren_ctx* ctx, vren_stream_t strea
     f.index_cap = index_capacity;
     f.assigned_total = assigned_total;
     f.flags = ctx->d_flags;
-    f.offs_base = 0;
-    ChainWork w;
-    memset(&w, 0, sizeof(w));
-    const uint32_t offs_tiles = (key_capacity + VREN_SCAN_TILE - 1) / VREN_SCAN_TILE;
-    st = vren_ensure_scratch(ctx, chain_work_bytes(0, offs_tiles, 0), s);
-    if (st) return st;
-    chain_work_bind(&w, ctx->scratch, 0, offs_tiles, 0);
-    w.max_L = light_count;
-    FrameDev* slot = vren_next_frame_slot(ctx);
-    st = vren_upload_frames(ctx, s, slot, &f, 1);
-    if (!st) st = launch_chain_init(ctx, s, w);
-    if (st) return st;
     if (light_count == 0) {
         // no lights: every list is empty
-        VREN_HIP(ctx, hipMemsetAsync(light_counts, 0, (size_t)key_capacity * 4, s));
-        VREN_HIP(ctx, hipMemsetAsync(light_offsets, 0, (size_t)key_capacity * 4, s));
-        VREN_HIP(ctx, hipMemsetAsync(assigned_total, 0, 4, s));
+        empty_lists_kernel<<<std::min<uint32_t>(256, (key_capacity + 255) / 256), 256, 0, s>>>(light_counts, light_offsets,
+                                                                                            key_capacity, assigned_total);
+        VREN_LAUNCH_CHECK(ctx);
         return VREN_OK;
     }
-    return launch_assign(ctx, s, slot, 1, w);
+    ChainWork w;
+    memset(&w, 0, sizeof(w));
+    w.max_L = light_count;
+    return launch_assign(ctx, s, nullptr, 1, w, &f);
 }

@@ -37,6 +37,7 @@ struct vren_batch {
     // the second stream of a concurrent light stage, with its fork and join events (created with the batch)
     hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
+    bool dirty = false;             // the work memory's cleared words may not be (a run that was not launched whole)
 };
 
 namespace {
@@ -98,7 +99,10 @@ int run_chain(vren_batch* b, hipStream_t s, const FrameDev* table, uint32_t F, c
               uint32_t live_slots)
 {
     vren_ctx* ctx = b->ctx;
-    int st = launch_chain_init(ctx, s, w);
+    // a run leaves the tickets and statuses cleared for the next one (launch_assign); one that failed half-way may not
+    int st = b->dirty ? launch_chain_init(ctx, s, b->w) : VREN_OK;
+    b->dirty = true;
+    chain_mark(w, s);
     if (!st && w.light_concurrent && !w.events && b->side) {
         VREN_HIP(ctx, hipEventRecord(b->fork, s));
         VREN_HIP(ctx, hipStreamWaitEvent(b->side, b->fork, 0));
@@ -114,6 +118,7 @@ int run_chain(vren_batch* b, hipStream_t s, const FrameDev* table, uint32_t F, c
         if (!st) st = launch_clusters(ctx, s, table, F, w);
     }
     if (!st) st = launch_assign(ctx, s, table, F, w);
+    if (!st) b->dirty = false;
     if (!st) st = launch_shade(ctx, s, table, F, w);
     return st;
 }
@@ -156,7 +161,7 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
     b->leaf_slots.resize(n_frames);
     b->live_slots.resize(n_frames);
     // sizes and arena layout
-    uint32_t tile_base = 0, leaf_base = 0, live_base = 0, offs_base = 0, chunk_base = 0, max_L = 0, any_materials = 0;
+    uint32_t tile_base = 0, leaf_base = 0, live_base = 0, chunk_base = 0, max_L = 0, any_materials = 0;
     std::vector<size_t> off(n_frames * 14);
     size_t arena = 0;
     for (uint32_t i = 0; i < n_frames; i++) {
@@ -173,7 +178,6 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         f.tile_base = tile_base;
         f.leaf_base = leaf_base;
         f.live_leaf_base = live_base;
-        f.offs_base = offs_base;
         f.light_chunk_base = chunk_base;
         const uint32_t chunks = (L + VREN_LIGHT_CHUNK - 1) / VREN_LIGHT_CHUNK;
         chunk_base += chunks;
@@ -206,7 +210,6 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         tile_base += (tiles + VREN_TILE_GROUP - 1) / VREN_TILE_GROUP * VREN_TILE_GROUP;
         leaf_base += slots;
         live_base += live;
-        offs_base += (key_cap + VREN_SCAN_TILE - 1) / VREN_SCAN_TILE;
         max_L = std::max(max_L, L);
         // list slots for the first 32 768 clusters of the frame (768 B each); clusters past them are traversed again
         const uint32_t slot_cap = std::min<uint32_t>(key_cap, 1u << 15);
@@ -228,8 +231,9 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
     }
     hipError_t e = hipMalloc(&b->arena, std::max<size_t>(arena, 256));
     if (e == hipSuccess) e = hipMemset(b->arena, 0, std::max<size_t>(arena, 256));
-    const size_t wbytes = chain_work_bytes(tile_base, offs_base, n_frames);
+    const size_t wbytes = chain_work_bytes(tile_base, n_frames);
     if (e == hipSuccess) e = hipMalloc(&b->work, wbytes);
+    if (e == hipSuccess) e = hipMemset(b->work, 0, chain_work_clear_bytes(tile_base));
     if (e == hipSuccess) e = hipMalloc(&b->d_table, sizeof(FrameDev) * n_frames);
     if (e == hipSuccess) e = hipMalloc(&b->d_single, sizeof(FrameDev) * n_frames);
     if (e == hipSuccess) e = hipMalloc(&b->d_tile_frame, sizeof(uint32_t) * std::max<uint32_t>(tile_base, 1));
@@ -266,7 +270,7 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         f.leaf_pos = f.L ? reinterpret_cast<float*>(b->arena + o[11]) : nullptr;
         f.list_slots = f.slot_cap ? reinterpret_cast<uint32_t*>(b->arena + o[12]) : nullptr;
     }
-    chain_work_bind(&b->w, b->work, tile_base, offs_base, n_frames);
+    chain_work_bind(&b->w, b->work, tile_base);
     b->w.tile_frame = b->d_tile_frame;
     b->w.total_leaf_slots = leaf_base;
     b->total_live_slots = live_base;
@@ -278,7 +282,8 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         for (uint32_t i = 0; i < n_frames; i++) pixels += (uint64_t)frames[i].width * frames[i].height;
         b->size_class = batch_size_class(pixels, max_L, n_frames);
     }
-    // per-frame tables: same buffers, bases 0, the workspace viewed from its start
+    // per-frame tables: same buffers, bases 0, the frame's share of the same workspace (the statuses and per-tile tables
+    // from their starts, so that every run leaves the same words cleared; the frame's own slice table)
     std::vector<FrameDev> single(b->host);
     b->w_frame.resize(n_frames);
     for (uint32_t i = 0; i < n_frames; i++) {
@@ -286,10 +291,11 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         single[i].leaf_base = 0;
         single[i].live_leaf_base = 0;
         single[i].light_chunk_base = 0;
-        single[i].offs_base = 0;
         ChainWork& wf = b->w_frame[i];
-        chain_work_bind(&wf, b->work, single[i].Sx * single[i].Sy, (single[i].key_cap + VREN_SCAN_TILE - 1) / VREN_SCAN_TILE,
-                        1);
+        wf = b->w;
+        wf.slice_thr = b->w.slice_thr + (size_t)i * VREN_SLICE_TABLE;
+        wf.tile_frame = nullptr;
+        wf.total_tiles = single[i].Sx * single[i].Sy;
         wf.total_leaf_slots = b->leaf_slots[i];
         wf.max_L = single[i].L;
         wf.light_chunks = (single[i].L + VREN_LIGHT_CHUNK - 1) / VREN_LIGHT_CHUNK;
@@ -308,7 +314,9 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         st = vren_fail(ctx, VREN_EHIP, "batch: second stream or its events could not be created");
     if (!st) st = vren_upload_frames(ctx, s, b->d_table, b->host.data(), n_frames);
     if (!st) st = vren_upload_frames(ctx, s, b->d_single, single.data(), n_frames);
-    // the BVH leaf groups past each frame's last light, written once: every run of the chain skips them
+    // what depends on the frames' descriptions alone is written once, and every run of the chain skips it: the
+    // depth-slice tables and the BVH leaf groups past each frame's last light
+    if (!st) st = launch_slice_tables(ctx, s, b->d_table, n_frames, b->w);
     if (!st && leaf_base) st = launch_bvh(ctx, s, b->d_table, n_frames, leaf_base, true, nullptr, kLeavesPadding);
     if (!st && hipStreamSynchronize(s) != hipSuccess) st = vren_fail(ctx, VREN_EHIP, "batch: upload failed");
     if (st) {
@@ -343,18 +351,29 @@ VREN_EXPORT int vren_batch_run(vren_batch* b, vren_stream_t stream, int mode)
             hipGraph_t g = nullptr;
             hipError_t e = hipStreamEndCapture(b->capture, &g);
             if (st || e != hipSuccess) {
+                b->dirty = true; // nothing ran: an init that the capture recorded is gone with it
                 if (g) vren_teardown(hipGraphDestroy(g));
                 return st ? st : vren_hip_fail(ctx, e, "hipStreamEndCapture");
             }
             e = hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0);
             if (e != hipSuccess) {
                 b->exec = nullptr;
+                b->dirty = true;
                 vren_teardown(hipGraphDestroy(g));
                 return vren_hip_fail(ctx, e, "hipGraphInstantiate");
             }
             b->graph = g;
         }
-        VREN_HIP(ctx, hipGraphLaunch(b->exec, s));
+        if (b->dirty) { // an earlier run was not launched whole
+            const int st = launch_chain_init(ctx, s, b->w);
+            if (st) return st;
+            b->dirty = false;
+        }
+        const hipError_t le = hipGraphLaunch(b->exec, s);
+        if (le != hipSuccess) {
+            b->dirty = true;
+            return vren_hip_fail(ctx, le, "hipGraphLaunch");
+        }
         return VREN_OK;
     }
     return vren_fail(ctx, VREN_EINVAL, "batch_run: unknown mode %d", mode);

@@ -18,19 +18,16 @@ FrameDev* vren_next_frame_slot(vren_ctx* ctx);
 // a frame's 32x32 tiles start at a multiple of this in the flattened tile numbering of a table (the clusters kernel
 // chains its look-back over groups of this many tiles, one workgroup each); tiles of the padding do nothing
 #define VREN_TILE_GROUP 8u
-#define VREN_SCAN_TILE 4096u
 
-// look-back statuses and ticket counters of one chain launch
+// look-back statuses and ticket counter of one chain launch, and the per-tile tables between its stages
 struct ChainWork {
-    uint64_t* tile_status; // cluster compaction: one word per 32x32 tile of every frame
-    uint64_t* offs_status; // light-offset scan: one word per 4096 clusters of capacity of every frame
-    uint32_t* tickets;     // [0] cluster tiles, [1] offset tiles
+    uint64_t* tile_status; // cluster compaction: one word per group of VREN_TILE_GROUP tiles of every frame
+    uint32_t* tickets;     // [0] cluster tile groups
     float* slice_thr;      // depth-slice threshold table of every frame (VREN_SLICE_TABLE floats each)
     uint2* tile_cl;        // per 32x32 tile: (first cluster index, cluster count), written by the clusters kernel
     uint2* tile_range;     // per 32x32 tile: [begin, end) of the index-buffer entries of its clusters' light lists
     const uint32_t* tile_frame; // frame of every flattened 32x32 tile (null for a one-frame table)
     uint32_t total_tiles;
-    uint32_t total_offs_tiles;
     uint32_t total_leaf_slots;
     uint32_t max_L;
     uint32_t light_chunks;  // chunks of VREN_LIGHT_CHUNK lights over the table's frames (light_chunk_base numbering)
@@ -59,29 +56,45 @@ inline void chain_mark(const ChainWork& w, hipStream_t s)
 #define VREN_SLICE_TABLE 1024u
 
 // workspace: 256 bytes of tickets, the look-back statuses, the per-tile cluster spans and list ranges, then
-// (256-aligned) the slice tables of table_frames frames
-inline size_t chain_work_table_offset(uint32_t total_tiles, uint32_t total_offs_tiles)
+// (256-aligned) the slice tables of table_frames frames. The tickets and statuses (the first chain_work_clear_bytes)
+// are zero between runs of a chain: the light-count kernel, which follows their last use, clears them.
+inline size_t chain_work_clear_bytes(uint32_t total_tiles)
 {
-    return (256 + ((size_t)total_tiles + total_offs_tiles) * sizeof(uint64_t) + (size_t)total_tiles * 16 + 255) &
-           ~(size_t)255;
+    return 256 + ((size_t)total_tiles + VREN_TILE_GROUP - 1) / VREN_TILE_GROUP * sizeof(uint64_t);
 }
-inline size_t chain_work_bytes(uint32_t total_tiles, uint32_t total_offs_tiles, uint32_t table_frames)
+inline size_t chain_work_table_offset(uint32_t total_tiles)
 {
-    return chain_work_table_offset(total_tiles, total_offs_tiles) + (size_t)table_frames * VREN_SLICE_TABLE * 4;
+    return (chain_work_clear_bytes(total_tiles) + (size_t)total_tiles * 16 + 255) & ~(size_t)255;
 }
-void chain_work_bind(ChainWork* w, void* mem, uint32_t total_tiles, uint32_t total_offs_tiles, uint32_t table_frames);
+inline size_t chain_work_bytes(uint32_t total_tiles, uint32_t table_frames)
+{
+    return chain_work_table_offset(total_tiles) + (size_t)table_frames * VREN_SLICE_TABLE * 4;
+}
+void chain_work_bind(ChainWork* w, void* mem, uint32_t total_tiles);
 
-// stage launchers; d_frames is a device table of F FrameDev records
+// Stage launchers. d_frames is a device table of F FrameDev records; `one`, when given, is the host record of a
+// single-frame call instead, passed to the kernels by value (F = 1): the call needs no upload ahead of them.
 int launch_chain_init(vren_ctx* ctx, hipStream_t s, const ChainWork& w);
 int launch_lights(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
-                  uint32_t pad_blocks = 0);
+                  const FrameDev* one = nullptr);
 // which 32-leaf groups the leaf kernel writes: all, those holding a light, or the all-padding ones
 enum : uint32_t { kLeavesAll = 0, kLeavesLive = 1, kLeavesPadding = 2 };
 int launch_bvh(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, uint32_t total_leaf_slots,
                bool leaves_from_lights, const ChainWork* w, uint32_t span);
-int launch_clusters(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w);
-int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w);
-int launch_shade(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w);
+int launch_slice_tables(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w);
+int launch_clusters(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
+                    const FrameDev* one = nullptr);
+int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
+                  const FrameDev* one = nullptr);
+int launch_shade(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
+                 const FrameDev* one = nullptr);
+
+// device: the record that a kernel was passed by value as its first argument, where it lies: its fields are then read
+// with scalar loads from the kernel's argument segment
+__device__ __forceinline__ const FrameDev* inline_frame()
+{
+    return (const FrameDev*)(const void*)__builtin_amdgcn_kernarg_segment_ptr();
+}
 
 // device: frame of a flattened 32x32 tile: one load from the tile -> frame table (uniform across the workgroup)
 __device__ __forceinline__ uint32_t frame_of_tile(const uint32_t* tile_frame, uint32_t g)

@@ -22,7 +22,6 @@ struct FrameDev {
     uint32_t leaf_base;     // first flattened leaf slot (256-aligned) of this frame's BVH leaves
     uint32_t live_leaf_base; // the same over the light-holding leaf groups of frames of more than one light chunk
     uint32_t light_chunk_base; // first flattened chunk of VREN_LIGHT_CHUNK lights of this frame
-    uint32_t offs_base;     // first flattened tile of this frame's light-offset scan
     // camera constants
     float view[16];         // camera::get_view()
     float inv_proj[16];     // inverse(camera::get_projection()), rounded from double
@@ -80,7 +79,6 @@ struct FrameDev {
     uint32_t* assigned_total; // device u32
     uint32_t* list_slots;     // optional: VREN_LIST_SLOT entries per cluster for clusters below slot_cap
     uint32_t slot_cap;
-    uint64_t* offset_status;  // look-back statuses of the offset scan (ceil(key_cap / 4096) words)
     // output
     float* out;
     // error flags

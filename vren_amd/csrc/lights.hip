@@ -182,7 +182,7 @@ __global__ __launch_bounds__(kLT) void lights_bounds_kernel(const FrameDev* __re
 // (256 lights: 21 -> 7 us), bound by the vector issue of its one CU; 65 536 lights took 292 us in one workgroup that
 // sorted in global memory and take 36 us (bounds 6, chunks 12.5, merge 17).
 template <int BITS>
-__global__ __launch_bounds__(kLT) void lights_kernel(const FrameDev* __restrict__ frames, uint32_t F, uint32_t chunks)
+__device__ __forceinline__ void lights_body(const FrameDev* __restrict__ frames, uint32_t F, uint32_t chunks)
 {
     __shared__ uint2 s_pair[kLChunk];              // (code, light index)
     __shared__ float4 s_light[kLChunk];            // view position, radius (frames of one chunk)
@@ -356,6 +356,13 @@ __global__ __launch_bounds__(kLT) void lights_kernel(const FrameDev* __restrict_
         if (tid == 31) store_node(&fd.bvh[level2 + 32], mn, mx, level2);
     }
 }
+
+template <int BITS>
+__global__ __launch_bounds__(kLT) void lights_kernel(const FrameDev* __restrict__ frames, uint32_t F, uint32_t chunks)
+{
+    lights_body<BITS>(frames, F, chunks);
+}
+__global__ __launch_bounds__(kLT) void lights_one_kernel(const FrameDev one) { lights_body<8>(inline_frame(), 1, 1); }
 
 // Frames of more than one chunk: codes[rank] for every light of the chunks' sorted runs. A light's rank is its place in
 // its run plus, for every other run, the number of its lights that sort before it: codes up to and including the
@@ -558,19 +565,21 @@ __global__ __launch_bounds__(1024) void bvh_upper_kernel(const FrameDev* __restr
 
 } // namespace
 
-// pad_blocks: workgroups of a single-frame call that write the padding leaves of a frame of one chunk
 int launch_lights(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
-                  uint32_t pad_blocks)
+                  const FrameDev* one)
 {
     const uint32_t chunks = w.light_chunks;
-    if (chunks) {
+    if (one) { // one chunk; the workgroups past the first write the padding leaves
+        const bool padding = one->bvh_padded > ((one->L + 31u) & ~31u);
+        lights_one_kernel<<<1 + (padding ? (one->bvh_padded + kLT - 1) / kLT : 0u), kLT, 0, s>>>(*one);
+        VREN_LAUNCH_CHECK(ctx);
+    } else if (chunks) {
         if (w.max_L > kLChunk) {
             lights_bounds_kernel<<<chunks, kLT, 0, s>>>(d_frames, F);
             VREN_LAUNCH_CHECK(ctx);
         }
-        const uint32_t grid = chunks + pad_blocks;
-        if (w.light_bits == 4) lights_kernel<4><<<grid, kLT, 0, s>>>(d_frames, F, chunks);
-        else lights_kernel<8><<<grid, kLT, 0, s>>>(d_frames, F, chunks);
+        if (w.light_bits == 4) lights_kernel<4><<<chunks, kLT, 0, s>>>(d_frames, F, chunks);
+        else lights_kernel<8><<<chunks, kLT, 0, s>>>(d_frames, F, chunks);
         VREN_LAUNCH_CHECK(ctx);
         if (w.max_L > kLChunk) {
             lights_merge_kernel<<<chunks * kMergeParts, kMergeThreads, 0, s>>>(d_frames, F);
@@ -667,16 +676,15 @@ VREN_EXPORT int vren_construct_point_light_bvh(vren_ctx* ctx, vren_stream_t stre
         f.codes_tmp = static_cast<uint32_t*>(ctx->scratch);
         f.chunk_box = reinterpret_cast<uint32_t*>(static_cast<char*>(ctx->scratch) + runs);
     }
-    FrameDev* slot = vren_next_frame_slot(ctx);
-    st = vren_upload_frames(ctx, s, slot, &f, 1);
-    if (st) return st;
     ChainWork w;
     memset(&w, 0, sizeof(w));
     w.max_L = light_count;
     w.light_chunks = chunks;
-    const bool padding = chunks == 1 && f.bvh_padded > ((light_count + 31u) & ~31u);
-    st = launch_lights(ctx, s, slot, 1, w, padding ? (f.bvh_padded + kLT - 1) / kLT : 0u);
-    if (st || chunks == 1) return st;
+    if (chunks == 1) return launch_lights(ctx, s, nullptr, 1, w, &f);
+    FrameDev* slot = vren_next_frame_slot(ctx);
+    st = vren_upload_frames(ctx, s, slot, &f, 1);
+    if (!st) st = launch_lights(ctx, s, slot, 1, w);
+    if (st) return st;
     uint32_t slots = (f.bvh_padded + VREN_LEAF_ALIGN - 1) / VREN_LEAF_ALIGN * VREN_LEAF_ALIGN;
     return launch_bvh(ctx, s, slot, 1, slots, true, nullptr, kLeavesAll);
 }

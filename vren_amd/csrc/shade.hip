@@ -419,27 +419,6 @@ __device__ __forceinline__ void resolve_material(const FrameDev& fd, vf2 tc, uin
     metal = mr.z * m.metallic_factor;
 }
 
-// [begin, end) of the index-buffer entries of a tile's light lists: the tile's clusters are the consecutive indices
-// [c0, c0 + u) (clusters kernel) and their lists are consecutive in the index buffer, so the range runs from the
-// first cluster's offset to the end of the last list (both clamped to the capacities like the per-pixel lists).
-__global__ __launch_bounds__(256) void tile_range_kernel(const FrameDev* __restrict__ frames,
-                                                         const uint32_t* __restrict__ tile_frame, uint32_t total_tiles,
-                                                         const uint2* __restrict__ tile_cl, uint2* __restrict__ tile_range)
-{
-    const uint32_t g = blockIdx.x * 256 + threadIdx.x;
-    if (g >= total_tiles) return;
-    const FrameDev& fd = frames[frame_of_tile(tile_frame, g)];
-    const uint2 c = tile_cl[g];
-    uint32_t a = 0, b = 0;
-    if (g - fd.tile_base < fd.Sx * fd.Sy && fd.L > 0 && c.y > 0 && c.x < fd.key_cap) { // not a padding tile
-        const uint32_t c1 = min(c.x + c.y, fd.key_cap) - 1u;
-        a = min(fd.offsets[c.x], fd.index_cap);
-        const uint64_t e = (uint64_t)fd.offsets[c1] + fd.counts[c1];
-        b = e > fd.index_cap ? fd.index_cap : (uint32_t)e;
-    }
-    tile_range[g] = make_uint2(a, b);
-}
-
 // A 256-thread workgroup shades PPT 32x8 strips of a 32x32 tile (PPT pixels per thread, their loads issued
 // together), flattened over every frame of the table. A wave covers two whole 32-pixel rows of the tile, so each
 // 4-byte G-buffer plane is read in whole 128-byte lines: with 16-pixel-wide pieces, the other half of every line
@@ -451,10 +430,8 @@ __global__ __launch_bounds__(256) void tile_range_kernel(const FrameDev* __restr
 // caller), the workgroup first reduces the run from its pixels' lists.
 // MAT: the table may hold frames on the material path (texcoords + material index + material and texture tables)
 template <int PPT, bool MAT>
-// at most 64 VGPRs: eight waves per SIMD (the split light loops would otherwise take 66 and seven)
-__global__ __launch_bounds__(256, 8) void shade_kernel(const FrameDev* __restrict__ frames,
-                                                    const uint32_t* __restrict__ tile_frame,
-                                                    const uint2* __restrict__ tile_range, uint32_t total_tiles)
+__device__ __forceinline__ void shade_body(const FrameDev* __restrict__ frames, const uint32_t* __restrict__ tile_frame,
+                                           const uint2* __restrict__ tile_range, uint32_t total_tiles)
 {
     constexpr uint32_t BPT = 4 / PPT; // workgroups per tile
     static_assert(kFwdStage == 256, "one staged entry per thread");
@@ -598,6 +575,19 @@ __global__ __launch_bounds__(256, 8) void shade_kernel(const FrameDev* __restric
     }
 }
 
+// at most 64 VGPRs: eight waves per SIMD (the split light loops would otherwise take 66 and seven)
+template <int PPT, bool MAT>
+__global__ __launch_bounds__(256, 8) void shade_kernel(const FrameDev* __restrict__ frames,
+                                                    const uint32_t* __restrict__ tile_frame,
+                                                    const uint2* __restrict__ tile_range, uint32_t total_tiles)
+{
+    shade_body<PPT, MAT>(frames, tile_frame, tile_range, total_tiles);
+}
+template <int PPT, bool MAT>
+__global__ __launch_bounds__(256, 8) void shade_one_kernel(const FrameDev one, uint32_t total_tiles)
+{
+    shade_body<PPT, MAT>(inline_frame(), nullptr, nullptr, total_tiles);
+}
 
 // ---- adjoint ---------------------------------------------------------------------------------------------------
 
@@ -766,9 +756,9 @@ constexpr int kSumRounds = 8;  // distinct entries of one step that a wave sums;
 // when all its lanes were at one entry) and 50 us in the gradients' global atomics, seven instructions each of whose
 // lanes hit another cache line. Summing once per distinct entry and one term per lane in the global adds: 91 us.
 // Larger workgroups (two and four strips, fewer global adds) are slower, 97 and 115 us.
-__global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev* __restrict__ frames, uint32_t F,
-                                                             uint32_t total_tiles, const float* grad_out,
-                                                             float* g_pos, float* g_light, float* g_ar)
+__global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev one, uint32_t total_tiles,
+                                                             const float* grad_out, float* g_pos, float* g_light,
+                                                             float* g_ar)
 {
     __shared__ float4 s_lpos[kStage];
     __shared__ float4 s_lcol[kStage];
@@ -781,11 +771,8 @@ __global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev* __r
     const uint32_t k = blockIdx.x / 8;
     const uint32_t g = (k / 4) * 8 + blockIdx.x % 8, sub = k % 4;
     if (g >= total_tiles) return;
-    const uint32_t f = find_frame_wave(frames, F, g, [](const FrameDev& d) { return d.tile_base; });
-    const FrameDev& fd = frames[f];
-    const uint32_t t = g - fd.tile_base;
-    if (t >= fd.Sx * fd.Sy) return; // padding after the frame's tiles (the whole workgroup)
-    const uint32_t ti = t % fd.Sx, tj = t / fd.Sx;
+    const FrameDev& fd = *inline_frame();
+    const uint32_t ti = g % fd.Sx, tj = g / fd.Sx;
     const uint32_t gx = ti * 32 + (tid & 31), gy = tj * 32 + sub * 8 + (tid >> 5); // 32x8 strip `sub`
     const bool in = gx < fd.W && gy < fd.H;
     const uint64_t p = in ? (uint64_t)gy * fd.W + gx : 0;
@@ -1001,24 +988,22 @@ __global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev* __r
 
 } // namespace
 
-int launch_shade(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w)
+int launch_shade(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
+                 const FrameDev* one)
 {
-    if (w.tile_range) {
-        tile_range_kernel<<<(w.total_tiles + 255) / 256, 256, 0, s>>>(d_frames, F > 1 ? w.tile_frame : nullptr,
-                                                                    w.total_tiles, w.tile_cl, w.tile_range);
-        VREN_LAUNCH_CHECK(ctx);
-    }
     const uint32_t* tf = F > 1 ? w.tile_frame : nullptr;
-    const uint32_t rounds = (w.total_tiles + 7) / 8; // rounds of 8 tiles, one per XCD
-    if (w.shade_ppt == 2) {
-        const uint32_t grid = rounds * 8 * 2;
-        if (w.any_materials) shade_kernel<2, true><<<grid, 256, 0, s>>>(d_frames, tf, w.tile_range, w.total_tiles);
-        else shade_kernel<2, false><<<grid, 256, 0, s>>>(d_frames, tf, w.tile_range, w.total_tiles);
+    const uint2* ranges = w.max_L ? w.tile_range : nullptr; // written with the light lists
+    const uint32_t rounds = (w.total_tiles + 7) / 8;        // rounds of 8 tiles, one per XCD
+    const uint32_t grid = rounds * 8 * (4 / kShadePPT);
+    if (one) {
+        if (w.any_materials) shade_one_kernel<kShadePPT, true><<<grid, 256, 0, s>>>(*one, w.total_tiles);
+        else shade_one_kernel<kShadePPT, false><<<grid, 256, 0, s>>>(*one, w.total_tiles);
+    } else if (w.shade_ppt == 2) {
+        if (w.any_materials) shade_kernel<2, true><<<rounds * 8 * 2, 256, 0, s>>>(d_frames, tf, ranges, w.total_tiles);
+        else shade_kernel<2, false><<<rounds * 8 * 2, 256, 0, s>>>(d_frames, tf, ranges, w.total_tiles);
     } else {
-        const uint32_t grid = rounds * 8 * (4 / kShadePPT);
-        if (w.any_materials)
-            shade_kernel<kShadePPT, true><<<grid, 256, 0, s>>>(d_frames, tf, w.tile_range, w.total_tiles);
-        else shade_kernel<kShadePPT, false><<<grid, 256, 0, s>>>(d_frames, tf, w.tile_range, w.total_tiles);
+        if (w.any_materials) shade_kernel<kShadePPT, true><<<grid, 256, 0, s>>>(d_frames, tf, ranges, w.total_tiles);
+        else shade_kernel<kShadePPT, false><<<grid, 256, 0, s>>>(d_frames, tf, ranges, w.total_tiles);
     }
     VREN_LAUNCH_CHECK(ctx);
     chain_mark(w, s);
@@ -1068,13 +1053,10 @@ extern "C" VREN_EXPORT int vren_shade(vren_ctx* ctx, vren_stream_t stream, uint3
     f.dir_lights = directional_lights;
     f.n_dir = directional_light_count;
     f.out = output;
-    FrameDev* slot = vren_next_frame_slot(ctx);
-    st = vren_upload_frames(ctx, s, slot, &f, 1);
     ChainWork w;
     memset(&w, 0, sizeof(w));
     w.total_tiles = f.Sx * f.Sy;
-    if (!st) st = launch_shade(ctx, s, slot, 1, w);
-    return st;
+    return launch_shade(ctx, s, nullptr, 1, w, &f);
 }
 
 extern "C" VREN_EXPORT int vren_shade_materials(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
@@ -1122,14 +1104,11 @@ extern "C" VREN_EXPORT int vren_shade_materials(vren_ctx* ctx, vren_stream_t str
     f.dir_lights = directional_lights;
     f.n_dir = directional_light_count;
     f.out = output;
-    FrameDev* slot = vren_next_frame_slot(ctx);
-    st = vren_upload_frames(ctx, s, slot, &f, 1);
     ChainWork w;
     memset(&w, 0, sizeof(w));
     w.total_tiles = f.Sx * f.Sy;
     w.any_materials = 1;
-    if (!st) st = launch_shade(ctx, s, slot, 1, w);
-    return st;
+    return launch_shade(ctx, s, nullptr, 1, w, &f);
 }
 
 extern "C" VREN_EXPORT int vren_shade_backward(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
@@ -1173,11 +1152,8 @@ extern "C" VREN_EXPORT int vren_shade_backward(vren_ctx* ctx, vren_stream_t stre
     f.light_pos = light_positions;
     f.lights = point_lights;
     f.L = light_count;
-    FrameDev* slot = vren_next_frame_slot(ctx);
-    st = vren_upload_frames(ctx, s, slot, &f, 1);
-    if (st) return st;
     const uint32_t tiles = f.Sx * f.Sy;
-    shade_backward_kernel<<<(tiles + 7) / 8 * 32, 256, 0, s>>>(slot, 1, tiles, grad_output, grad_light_positions,
+    shade_backward_kernel<<<(tiles + 7) / 8 * 32, 256, 0, s>>>(f, tiles, grad_output, grad_light_positions,
                                                                grad_point_lights, grad_albedo_roughness);
     VREN_LAUNCH_CHECK(ctx);
     return VREN_OK;
