@@ -19,10 +19,12 @@
 namespace {
 
 constexpr uint32_t kStack = 384; // per-wave stack entries (levels are nondecreasing on the stack: <= 64 per level)
-// per-half stack entries of the counting pass: a half pops one block and pushes at most 32, so the stack holds at
-// most 31 entries of each level above the deepest and 32 of the deepest, 31 * 3 + 32 = 125 for the four block
-// levels of 2^20 lights
-constexpr uint32_t kStackHalf = 192;
+// per-half entries of the counting pass: the stack holds blocks of inner nodes (a half pops one and pushes at most 32, so
+// at most 31 entries of each level above the deepest inner one and 32 of that, 31 * 2 + 32 = 94 for 2^20 lights), the
+// leaf list blocks of leaves, which are tested when it has no room for 32 more or no inner block is left
+constexpr uint32_t kStackHalf = 96;
+constexpr uint32_t kLeafList = 128;
+constexpr int kLeafUnroll = 4; // leaf blocks per half and step: their loads overlap
 constexpr uint32_t kLevelShift = 28;
 constexpr uint32_t kAddrMask = (1u << kLevelShift) - 1u;
 
@@ -118,6 +120,30 @@ __device__ __forceinline__ bool test_leaf(const Box& c, const float4& o, float l
     return vren_sqrtf(vren_dot3(d, d)) < r;
 }
 
+// The same test against a leaf record (position, limit): the limit is the smallest squared distance whose square root
+// is not below the light's radius (leaf_limit, lights.hip), 0 for a record without a light, so sqrt(d2) < r is
+// d2 < limit exactly, without the square root and the node. The clamp as plain minimum and maximum: a NaN position
+// gives a NaN distance either way, and leaf_box takes the boxes with a NaN lower corner out.
+__device__ __forceinline__ bool test_leaf_record(const Box& c, vf4 o)
+{
+    float d[3];
+    const float oo[3] = {o.x, o.y, o.z};
+    for (int a = 0; a < 3; a++) d[a] = fmaxf(c.mn[a], fminf(oo[a], c.mx[a])) - oo[a];
+    return vren_dot3(d, d) < o.w;
+}
+
+// a cluster box for the traversal: one with a NaN in its lower corner, which no node and no leaf meets, becomes one
+// that meets none by its numbers
+__device__ __forceinline__ Box leaf_box(Box c)
+{
+    const bool nan = !(c.mn[0] == c.mn[0] && c.mn[1] == c.mn[1] && c.mn[2] == c.mn[2]);
+    for (int a = 0; a < 3; a++) {
+        c.mn[a] = nan ? VREN_F32_INF : c.mn[a];
+        c.mx[a] = nan ? -VREN_F32_INF : c.mx[a];
+    }
+    return c;
+}
+
 // Traverse the BVH for one cluster with the whole wave, setting one bit per hit light in the wave's LDS bitmask (and
 // the word's bit in the summary, one bit per bitmask word), and return the number of hit lights.
 __device__ uint32_t traverse(const FrameDev& fd, const Box& box, uint32_t* stack, uint32_t* bitmask,
@@ -127,8 +153,6 @@ __device__ uint32_t traverse(const FrameDev& fd, const Box& box, uint32_t* stack
     const uint32_t sub = lane & 31u;
     const uint32_t leaf_level = fd.bvh_levels - 1;
     const vren_bvh_node* bvh = fd.bvh;
-    const uint2* codes = reinterpret_cast<const uint2*>(fd.codes);
-    const float4* vpos = reinterpret_cast<const float4*>(fd.view_pos);
     // level 0 = the root's children (assign_lights.comp:108-119): the first child of the root
     const uint32_t root_first = __float_as_uint(reinterpret_cast<const float4*>(&bvh[fd.bvh_root])[0].w);
     uint32_t sp = 0;
@@ -152,33 +176,32 @@ __device__ uint32_t traverse(const FrameDev& fd, const Box& box, uint32_t* stack
         const bool active = e != 0xFFFFFFFFu && (e >> kLevelShift) <= leaf_level &&
                             (e & kAddrMask) + 32u <= fd.bvh_length;
         bool leaf_hit = false, push = false;
-        uint32_t child = 0, level = 0;
+        uint32_t child = 0, level = 0, li = 0xFFFFFFFFu;
         if (active) {
             level = e >> kLevelShift;
             const uint32_t addr = (e & kAddrMask) + sub;
-            const bool at_leaf = level == leaf_level && addr < fd.L;
-            // a leaf's light index and view position are addressed by the leaf slot, so they load together with
-            // the node (leaf_pos holds the positions in leaf order; without it the position needs the index)
-            uint32_t li = 0xFFFFFFFFu;
-            float4 lp = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (at_leaf) {
-                li = codes[addr].y;
-                if (fd.leaf_pos) lp = reinterpret_cast<const float4*>(fd.leaf_pos)[addr];
-            }
-            const float4* q = reinterpret_cast<const float4*>(&bvh[addr]);
-            const float4 lo = q[0], hi = q[1];
-            const uint32_t next = __float_as_uint(lo.w);
             if (level == leaf_level) {
-                if (next == VREN_BVH_LEAF_NODE && at_leaf && li < fd.L) {
-                    if (!fd.leaf_pos) lp = vpos[li];
-                    leaf_hit = test_leaf(box, lp, lo.x, hi.x);
-                    if (leaf_hit) {
-                        atomicOr(&bitmask[li >> 5], 1u << (li & 31u));
-                        atomicOr(&summary[li >> 10], 1u << ((li >> 5) & 31u));
+                if (addr < fd.L) {
+                    li = *((guint*)fd.codes + 2 * (uint64_t)addr + 1);
+                    if (fd.leaf_rec) {
+                        leaf_hit = test_leaf_record(box, *((gvf4*)fd.leaf_rec + addr));
+                    } else {
+                        const vf4 lo = *((gvf4*)&bvh[addr]), hi = *((gvf4*)&bvh[addr] + 1);
+                        if (__float_as_uint(lo.w) == VREN_BVH_LEAF_NODE && li < fd.L) {
+                            const vf4 v = *((gvf4*)fd.view_pos + li);
+                            leaf_hit = test_leaf(box, make_float4(v.x, v.y, v.z, 0.f), lo.x, hi.x);
+                        }
                     }
                 }
-            } else if (next != VREN_BVH_INVALID_NODE && next != VREN_BVH_LEAF_NODE) {
-                push = test_aabb_aabb(box, lo, hi);
+                if (leaf_hit) {
+                    atomicOr(&bitmask[li >> 5], 1u << (li & 31u));
+                    atomicOr(&summary[li >> 10], 1u << ((li >> 5) & 31u));
+                }
+            } else {
+                const vf4 lo = *((gvf4*)&bvh[addr]), hi = *((gvf4*)&bvh[addr] + 1);
+                const uint32_t next = __float_as_uint(lo.w);
+                push = next < VREN_BVH_INVALID_NODE &&
+                       test_aabb_aabb(box, make_float4(lo.x, lo.y, lo.z, 0.f), make_float4(hi.x, hi.y, hi.z, 0.f));
                 child = next | ((level + 1) << kLevelShift);
             }
         }
@@ -195,91 +218,122 @@ __device__ uint32_t traverse(const FrameDev& fd, const Box& box, uint32_t* stack
     return hits;
 }
 
-// The BVH of a frame as one half-wave's traversal needs it (per lane, so the two halves may serve two frames)
-struct TravFrame {
-    const vren_bvh_node* bvh;
-    const uint2* codes;
-    const float4* leaf_pos;
-    const float4* vpos;
-    uint32_t L, leaf_level, root, length;
-};
-
-__device__ __forceinline__ TravFrame trav_frame(const FrameDev& fd)
+// element `at` of a uniform array, at most 4 GB into it: a uniform base and a 32-bit lane offset, which one load takes
+template <typename T>
+__device__ __forceinline__ T load_at(const void* base, uint32_t at)
 {
-    return TravFrame{fd.bvh, reinterpret_cast<const uint2*>(fd.codes), reinterpret_cast<const float4*>(fd.leaf_pos),
-                     reinterpret_cast<const float4*>(fd.view_pos), fd.L, fd.bvh_levels - 1, fd.bvh_root, fd.bvh_length};
+    typedef const __attribute__((address_space(1))) char gchar;
+    typedef const __attribute__((address_space(1))) T gT;
+    return *(gT*)((gchar*)base + at * (uint32_t)sizeof(T));
 }
 
-// Two traversals at once, one per 32-lane half of the wave (lanes 0-31 and 32-63, each with its own frame, cluster
-// box, stack and hit list; a half with live = false does nothing). Each step pops one 32-node block per half and
-// tests its children with the half's 32 lanes, so the dependent node loads of two clusters overlap. Counts the hit
-// lights of each half (returned to every lane of the half) and keeps the first VREN_LIST_SLOT hit light indices of
-// each half in `list` (traversal order). Same node tests and visiting rules as traverse.
-__device__ uint32_t traverse_halves(const TravFrame& tf, const Box& box, bool live, uint32_t* stack, uint32_t* list)
+// Two traversals of one frame's BVH at once, one per 32-lane half of the wave (lanes 0-31 and 32-63, each with its own
+// cluster box, stack and lists; a half with live = false does nothing). Inner blocks are popped one per half and step, each
+// child tested by a lane of the half; the blocks of leaves that they reach wait in the half's leaf list and are tested
+// kLeafUnroll at a time, so that the two kinds of test do not share a step (a step issued both before: 96 instructions,
+// now about 60 and 30 a block) and the leaves' loads overlap. Counts the hit lights of each half (returned to every
+// lane of the half) and keeps the first VREN_LIST_SLOT of them in `list` (traversal order): the leaf's place with
+// COMPACT (leaf records; the caller looks the light index up), else the light index.
+template <bool COMPACT>
+__device__ __forceinline__ uint32_t traverse_halves(const FrameDev& fd, const Box& box, bool live, uint32_t* stack,
+                                                    uint32_t* leaves, uint32_t* list)
 {
+    const uint32_t leaf_level = fd.bvh_levels - 1, length = fd.bvh_length;
+    const vren_bvh_node* bvh = fd.bvh;
     const uint32_t lane = lane_id();
     const uint32_t sub = lane & 31u;
     const uint64_t half = lane < 32 ? 0x00000000FFFFFFFFull : 0xFFFFFFFF00000000ull;
-    // level 0 = the root's children (assign_lights.comp:108-119): the first child of the root
-    uint32_t sp = 0;
-    if (live) {
-        const uint32_t root_first = __float_as_uint(reinterpret_cast<const float4*>(&tf.bvh[tf.root])[0].w);
-        if (root_first != VREN_BVH_INVALID_NODE) {
+    // leaf blocks end by this (at least 32): the groups of 32 that hold a light (records), or the nodes
+    const uint32_t leaf_end = COMPACT ? (fd.L + 31u) & ~31u : length;
+    // level 0 = the root's children (assign_lights.comp:108-119), the 32 nodes ahead of the root in a chain's own BVH (its
+    // root is valid: there is a light); a caller's BVH says where they are
+    uint32_t sp = 0, m = 0; // the half's stack and leaf-list entries
+    const uint32_t root_first = COMPACT ? fd.bvh_root - 32u : *((guint*)&bvh[fd.bvh_root] + 3);
+    if (live && root_first != VREN_BVH_INVALID_NODE) {
+        if (leaf_level == 0) {
+            if (root_first <= leaf_end - 32u) {
+                if (sub == 0) leaves[0] = root_first;
+                m = 1;
+            }
+        } else {
             if (sub == 0) stack[0] = root_first;
             sp = 1;
         }
     }
     uint32_t hits = 0;
     __builtin_amdgcn_wave_barrier();
-    while (ballot(sp > 0)) {
-        uint32_t e = 0xFFFFFFFFu;
-        if (sp > 0) {
-            e = stack[sp - 1];
-            sp -= 1;
-        }
-        // entries always address a whole 32-node block inside the BVH; anything else is ignored
-        const bool active = e != 0xFFFFFFFFu && (e >> kLevelShift) <= tf.leaf_level &&
-                            (e & kAddrMask) + 32u <= tf.length;
-        bool leaf_hit = false, push = false;
-        uint32_t child = 0, li = 0xFFFFFFFFu;
-        if (active) {
-            const uint32_t level = e >> kLevelShift;
-            const uint32_t addr = (e & kAddrMask) + sub;
-            const bool at_leaf = level == tf.leaf_level && addr < tf.L;
-            vf4 lpv = {0.f, 0.f, 0.f, 0.f};
-            if (at_leaf) {
-                li = *((guint*)tf.codes + 2 * (uint64_t)addr + 1);
-                if (tf.leaf_pos) lpv = *((gvf4*)tf.leaf_pos + addr);
+    for (;;) {
+        // inner blocks, while both leaf lists have room
+        while (ballot(sp > 0) && !ballot(m + 32u > kLeafList)) {
+            uint32_t e = 0xFFFFFFFFu;
+            if (sp > 0) {
+                e = stack[sp - 1];
+                sp -= 1;
             }
-            const vf4 lov = *((gvf4*)&tf.bvh[addr]), hiv = *((gvf4*)&tf.bvh[addr] + 1);
-            const float4 lo = make_float4(lov.x, lov.y, lov.z, lov.w), hi = make_float4(hiv.x, hiv.y, hiv.z, hiv.w);
-            float4 lp = make_float4(lpv.x, lpv.y, lpv.z, lpv.w);
-            const uint32_t next = __float_as_uint(lo.w);
-            if (level == tf.leaf_level) {
-                if (next == VREN_BVH_LEAF_NODE && at_leaf && li < tf.L) {
-                    if (!tf.leaf_pos) {
-                        const vf4 v = *((gvf4*)tf.vpos + li);
-                        lp = make_float4(v.x, v.y, v.z, v.w);
+            const uint32_t level = e >> kLevelShift, addr = (e & kAddrMask) + sub;
+            bool push = false;
+            uint32_t next = 0;
+            // entries always address a whole 32-node block of inner nodes in the BVH; anything else is ignored
+            if (e != 0xFFFFFFFFu && level < leaf_level && (e & kAddrMask) + 32u <= length) {
+                const vf4 lo = load_at<vf4>(bvh, 2 * addr), hi = load_at<vf4>(bvh, 2 * addr + 1);
+                next = __float_as_uint(lo.w);
+                push = next < VREN_BVH_INVALID_NODE &&
+                       test_aabb_aabb(box, make_float4(lo.x, lo.y, lo.z, 0.f), make_float4(hi.x, hi.y, hi.z, 0.f));
+            }
+            const bool to_leaves = level + 1u == leaf_level; // uniform in the half
+            push = push && (!to_leaves || next <= leaf_end - 32u);
+            const uint64_t pm = ballot(push) & half;
+            const uint32_t r = mbcnt(pm), n = (uint32_t)__popcll(pm);
+            if (push) {
+                if (to_leaves) leaves[m + r] = next; // m + 32 <= kLeafList
+                else if (sp + r < kStackHalf) stack[sp + r] = next | ((level + 1u) << kLevelShift);
+            }
+            if (to_leaves) m += n;
+            else sp = min(sp + n, kStackHalf); // the level bound keeps it below kStackHalf
+            __builtin_amdgcn_wave_barrier();
+        }
+        // leaf blocks
+        for (uint32_t k = 0; ballot(k < m); k += kLeafUnroll) {
+            uint32_t addr[kLeafUnroll];
+            bool on[kLeafUnroll], hit[kLeafUnroll];
+#pragma unroll
+            for (int u = 0; u < kLeafUnroll; u++) {
+                on[u] = k + u < m;
+                addr[u] = (on[u] ? leaves[k + u] : 0u) + sub;
+            }
+            if constexpr (COMPACT) {
+                vf4 rec[kLeafUnroll];
+#pragma unroll
+                for (int u = 0; u < kLeafUnroll; u++) rec[u] = on[u] ? load_at<vf4>(fd.leaf_rec, addr[u]) : vf4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int u = 0; u < kLeafUnroll; u++) hit[u] = test_leaf_record(box, rec[u]); // limit 0: never
+            } else {
+#pragma unroll
+                for (int u = 0; u < kLeafUnroll; u++) {
+                    hit[u] = false;
+                    if (on[u] && addr[u] < fd.L) {
+                        const vf4 lo = load_at<vf4>(bvh, 2 * addr[u]), hi = load_at<vf4>(bvh, 2 * addr[u] + 1);
+                        const uint32_t li = load_at<uint32_t>(fd.codes, 2 * addr[u] + 1);
+                        addr[u] = li; // what the list keeps
+                        if (__float_as_uint(lo.w) == VREN_BVH_LEAF_NODE && li < fd.L) {
+                            const vf4 v = load_at<vf4>(fd.view_pos, li);
+                            hit[u] = test_leaf(box, make_float4(v.x, v.y, v.z, 0.f), lo.x, hi.x);
+                        }
                     }
-                    leaf_hit = test_leaf(box, lp, lo.x, hi.x);
                 }
-            } else if (next != VREN_BVH_INVALID_NODE && next != VREN_BVH_LEAF_NODE) {
-                push = test_aabb_aabb(box, lo, hi);
-                child = next | ((level + 1) << kLevelShift);
+            }
+#pragma unroll
+            for (int u = 0; u < kLeafUnroll; u++) {
+                const uint64_t all = ballot(hit[u]);
+                if (all == 0) continue; // uniform
+                const uint64_t hm = all & half;
+                const uint32_t pos = hits + mbcnt(hm);
+                if (hit[u] && pos < VREN_LIST_SLOT) list[pos] = addr[u];
+                hits += (uint32_t)__popcll(hm);
             }
         }
-        const uint64_t hm = ballot(leaf_hit) & half;
-        if (leaf_hit) {
-            const uint32_t pos = hits + mbcnt(hm);
-            if (pos < VREN_LIST_SLOT) list[pos] = li;
-        }
-        hits += (uint32_t)__popcll(hm);
-        const uint64_t pm = ballot(push) & half;
-        if (push) {
-            const uint32_t r = mbcnt(pm);
-            if (sp + r < kStackHalf) stack[sp + r] = child;
-        }
-        sp = min(sp + (uint32_t)__popcll(pm), kStackHalf); // the level bound keeps it below kStackHalf
+        m = 0;
+        if (!ballot(sp > 0)) break;
         __builtin_amdgcn_wave_barrier();
     }
     return hits;
@@ -338,8 +392,9 @@ __device__ __forceinline__ void for_each_cluster_chunk(const FrameDev* __restric
     }
 }
 
-// for_each_cluster_chunk for the paired count pass: pre(fd, c, frame) runs per lane (lane i: cluster i of the
-// chunk), then fn(k, n, cA, cB) for k = 0, 2, 4, ... with cA, cB the frame-local indices of clusters k and k + 1.
+// for_each_cluster_chunk for the paired count pass: pre(fd, c) runs per lane (lane i: cluster i of the chunk), then
+// fn(fd, k, two, cA, cB) for clusters k and, with `two`, k + 1 of the chunk, cA and cB their frame-local indices; the two
+// are of one frame, so that its record is uniform and read with scalar loads.
 template <typename Pre, typename Fn>
 __device__ __forceinline__ void for_each_cluster_chunk2(const FrameDev* __restrict__ frames, uint32_t F, uint32_t gw,
                                                         uint32_t stride, Pre pre, Fn fn)
@@ -376,11 +431,15 @@ __device__ __forceinline__ void for_each_cluster_chunk2(const FrameDev* __restri
                 if (shfl(incl, (int)(pos + step - 1)) <= c) pos += step;
             const uint32_t fl = min(pos, VREN_WAVE - 1);
             const uint32_t base = shfl(excl, (int)fl);
-            if (lane < cs && c < total) pre(frames[f0 + fl], c - base, f0 + fl);
+            if (lane < cs && c < total) pre(frames[f0 + fl], c - base);
             const uint32_t local = c - base;
             const uint32_t n = min(total - c0, cs);
-            for (uint32_t k = 0; k < n; k += 2)
-                fn(k, n, __builtin_amdgcn_readlane(local, k), __builtin_amdgcn_readlane(local, min(k + 1, n - 1)));
+            for (uint32_t k = 0; k < n;) {
+                const uint32_t k1 = min(k + 1, n - 1), f = __builtin_amdgcn_readlane(fl, k);
+                const bool two = k1 != k && (uint32_t)__builtin_amdgcn_readlane(fl, k1) == f;
+                fn(frames[f0 + f], k, two, __builtin_amdgcn_readlane(local, k), __builtin_amdgcn_readlane(local, k1));
+                k += two ? 2u : 1u;
+            }
         }
     }
 }
@@ -426,42 +485,55 @@ __device__ __forceinline__ uint32_t emit_bitmask(uint32_t* bitmask, uint32_t* su
 // counting its hit lights and keeping the first VREN_LIST_SLOT of them in the half's LDS list; a list of at most
 // VREN_LIST_SLOT lights is sorted (the rank of each index among the list) into the cluster's slot, so the writing
 // pass copies it instead of traversing again.
+template <bool COMPACT>
 __device__ __forceinline__ void assign_count_body(const FrameDev* __restrict__ frames, uint32_t F, uint32_t* s_mem)
 {
     const uint32_t wpb = blockDim.x / VREN_WAVE;
     const uint32_t wave = wave_id();
     const uint32_t lane = lane_id();
     const uint32_t hb = lane < 32 ? 0u : 1u; // half of the wave
-    uint32_t* stack = s_mem + (wave * 2 + hb) * kStackHalf;
-    uint32_t* list = s_mem + wpb * 2 * kStackHalf + (wave * 2 + hb) * VREN_LIST_SLOT;
-    Box* boxes = reinterpret_cast<Box*>(s_mem + wpb * 2 * (kStackHalf + VREN_LIST_SLOT)) + wave * VREN_WAVE;
-    uint32_t* cl_frame = s_mem + wpb * 2 * (kStackHalf + VREN_LIST_SLOT) + wpb * VREN_WAVE * 6 + wave * VREN_WAVE;
+    constexpr uint32_t kHalf = kStackHalf + kLeafList + VREN_LIST_SLOT;
+    uint32_t* stack = s_mem + (wave * 2 + hb) * kHalf;
+    uint32_t* leaves = stack + kStackHalf;
+    uint32_t* list = leaves + kLeafList;
+    Box* boxes = reinterpret_cast<Box*>(s_mem + wpb * 2 * kHalf) + wave * VREN_WAVE;
     const uint32_t gw = blockIdx.x * wpb + wave;
-    // the chunk's cluster AABBs and frames wait in LDS (one per lane) while the wave traverses two at a time
+    // the chunk's cluster AABBs wait in LDS (one per lane) while the wave traverses two at a time
     for_each_cluster_chunk2(
         frames, F, gw, gridDim.x * wpb,
-        [&](const FrameDev& fdl, uint32_t c, uint32_t f) {
-            boxes[lane] = cluster_aabb(fdl, fdl.keys[c]);
-            cl_frame[lane] = f;
-        },
-        [&](uint32_t k, uint32_t n, uint32_t cA, uint32_t cB) {
-            // half 0: cluster k of the chunk, half 1: cluster k + 1 (when the chunk has one)
+        [&](const FrameDev& fdl, uint32_t c) { boxes[lane] = leaf_box(cluster_aabb(fdl, fdl.keys[c])); },
+        [&](const FrameDev& fd, uint32_t k, bool two, uint32_t cA, uint32_t cB) {
+            // half 0: cluster k of the chunk, half 1: cluster k + 1
             __builtin_amdgcn_wave_barrier();
-            const uint32_t kk = k + hb;
-            const bool live = kk < n;
+            const bool live = hb == 0 || two;
             const uint32_t c = hb ? cB : cA;
-            const FrameDev& fd = frames[cl_frame[live ? kk : k]];
-            const Box box = boxes[live ? kk : k];
-            const uint32_t h = traverse_halves(trav_frame(fd), box, live, stack, list);
+            const Box box = boxes[live ? k + hb : k];
+            const uint32_t h = traverse_halves<COMPACT>(fd, box, live, stack, leaves, list);
             __builtin_amdgcn_wave_barrier();
-            if (live && fd.list_slots && c < fd.slot_cap && h <= VREN_LIST_SLOT) {
-                // ascending light index: each entry's rank among the (distinct) entries of the half's list, entries
-                // sub and sub + 32 on lane sub of the half
-                for (uint32_t q = lane & 31u; q < h; q += 32u) {
-                    const uint32_t li = list[q];
-                    uint32_t rank = 0;
-                    for (uint32_t j = 0; j < h; j++) rank += list[j] < li ? 1u : 0u;
-                    fd.list_slots[(size_t)c * VREN_LIST_SLOT + rank] = li;
+            const bool keep = live && fd.list_slots && c < fd.slot_cap && h <= VREN_LIST_SLOT;
+            if constexpr (COMPACT) {
+                if (keep)
+                    for (uint32_t q = lane & 31u; q < h; q += 32u) list[q] = load_at<uint32_t>(fd.codes, 2 * list[q] + 1);
+                __builtin_amdgcn_wave_barrier();
+            }
+            if (keep) {
+                // ascending light index: each entry's rank among the (distinct) entries of the half's list, entries q
+                // and q + 32 on a lane at once, four entries of the list per read (padded with one that ranks above all)
+                const uint32_t sub = lane & 31u;
+                if (sub < 4u && h + sub < VREN_LIST_SLOT) list[h + sub] = 0xFFFFFFFFu;
+                __builtin_amdgcn_wave_barrier();
+                for (uint32_t q = sub; q < h; q += 64u) {
+                    const bool two = q + 32u < h;
+                    const uint32_t l0 = list[q], l1 = two ? list[q + 32u] : 0u;
+                    uint32_t r0 = 0, r1 = 0;
+                    for (uint32_t j = 0; j < h; j += 4u) {
+                        const uint4 x = *reinterpret_cast<const uint4*>(list + j);
+                        r0 += (x.x < l0 ? 1u : 0u) + (x.y < l0 ? 1u : 0u) + (x.z < l0 ? 1u : 0u) + (x.w < l0 ? 1u : 0u);
+                        r1 += (x.x < l1 ? 1u : 0u) + (x.y < l1 ? 1u : 0u) + (x.z < l1 ? 1u : 0u) + (x.w < l1 ? 1u : 0u);
+                    }
+                    uint32_t* slot = fd.list_slots + (size_t)c * VREN_LIST_SLOT;
+                    slot[r0] = l0;
+                    if (two) slot[r1] = l1;
                 }
             }
             if (live && (lane & 31u) == 0) fd.counts[c] = h;
@@ -539,7 +611,7 @@ __device__ __forceinline__ void assign_write_body(const FrameDev* __restrict__ f
                 }
                 return;
             }
-            const Box box = cluster_aabb(fd, fd.keys[c]);
+            const Box box = leaf_box(cluster_aabb(fd, fd.keys[c]));
             traverse(fd, box, stack, bitmask, summary);
             __builtin_amdgcn_wave_barrier();
             // emit set bits in ascending light index, clearing the mask as we go
@@ -583,12 +655,12 @@ __global__ __launch_bounds__(256, 8) void assign_count_kernel(const FrameDev* __
 {
     extern __shared__ uint32_t s_mem[];
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < clear_words; i += gridDim.x * 256) clear[i] = 0u;
-    assign_count_body(frames, F, s_mem);
+    assign_count_body<true>(frames, F, s_mem);
 }
 __global__ __launch_bounds__(256, 8) void assign_count_one_kernel(const FrameDev one)
 {
     extern __shared__ uint32_t s_mem[];
-    assign_count_body(inline_frame(), 1, s_mem);
+    assign_count_body<false>(inline_frame(), 1, s_mem);
 }
 __global__ __launch_bounds__(1024) void assign_offsets_kernel(const FrameDev* __restrict__ frames) { assign_offsets_body(frames); }
 __global__ __launch_bounds__(1024) void assign_offsets_one_kernel(const FrameDev one) { assign_offsets_body(inline_frame()); }
@@ -630,8 +702,8 @@ int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32
     uint32_t wpb = 4;
     while (wpb > 1 && per_wave * wpb > 150 * 1024) wpb--;
     if (per_wave > 150 * 1024) return vren_fail(ctx, VREN_EINVAL, "assign_lights: too many lights for the LDS bitmask");
-    // two stacks and two lists per wave (one per half), the chunk's boxes and cluster frames
-    constexpr size_t count_per_wave = (size_t)2 * (kStackHalf + VREN_LIST_SLOT) * 4 + VREN_WAVE * (sizeof(float) * 6 + 4);
+    // per wave, two stacks, leaf lists and hit lists (one per half) and the chunk's boxes
+    constexpr size_t count_per_wave = (size_t)2 * (kStackHalf + kLeafList + VREN_LIST_SLOT) * 4 + VREN_WAVE * sizeof(float) * 6;
     static_assert(count_per_wave * 4 <= 160 * 1024 / 8, "assign_count: 8 workgroups of 4 waves must fit a CU's LDS");
     const uint32_t count_blocks = persistent_blocks(ctx, 4, w.assign_wpc), write_blocks = persistent_blocks(ctx, wpb, w.assign_wpc);
     if (one) {

@@ -226,7 +226,7 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         o[8] = arena; arena += a256((size_t)key_cap * 4);            // offsets
         o[9] = arena; arena += a256((size_t)index_cap * 4);          // indices
         o[10] = arena; arena += 256;                                 // assigned_total
-        o[11] = arena; arena += a256((size_t)L * 16);                // leaf_pos
+        o[11] = arena; arena += a256((((size_t)L + 31) & ~(size_t)31) * 16); // leaf_rec
         o[12] = arena; arena += a256((size_t)f.slot_cap * VREN_LIST_SLOT * 4); // list slots
     }
     hipError_t e = hipMalloc(&b->arena, std::max<size_t>(arena, 256));
@@ -267,7 +267,7 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         f.offsets = reinterpret_cast<uint32_t*>(b->arena + o[8]);
         f.indices = reinterpret_cast<uint32_t*>(b->arena + o[9]);
         f.assigned_total = reinterpret_cast<uint32_t*>(b->arena + o[10]);
-        f.leaf_pos = f.L ? reinterpret_cast<float*>(b->arena + o[11]) : nullptr;
+        f.leaf_rec = f.L ? reinterpret_cast<float*>(b->arena + o[11]) : nullptr;
         f.list_slots = f.slot_cap ? reinterpret_cast<uint32_t*>(b->arena + o[12]) : nullptr;
     }
     chain_work_bind(&b->w, b->work, tile_base);

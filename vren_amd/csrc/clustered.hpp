@@ -54,7 +54,9 @@ struct FrameDev {
     uint32_t* chunk_box;      // the chunks' view-space boxes, six words each (more than one chunk)
     vren_bvh_node* bvh;
     uint32_t bvh_padded, bvh_root, bvh_levels, bvh_length;
-    float* leaf_pos;          // optional float4[L]: view position of sorted leaf i (= view_pos[codes[i].y])
+    // optional float4[L rounded up to 32]: sorted leaf i's view position (= view_pos[codes[i].y]) and the limit of the
+    // squared distance below which it is hit (assign.hip); zeros past the last light
+    float* leaf_rec;
     // G-buffer
     const float* depth;
     const uint16_t* normals;

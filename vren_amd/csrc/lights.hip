@@ -137,6 +137,25 @@ __device__ __forceinline__ void store_invalid(vren_bvh_node* n)
     store_node(n, inf, ninf, VREN_BVH_INVALID_NODE);
 }
 
+// The smallest squared distance (a non-negative float) whose square root is not below r, so that sqrt(d2) < r is
+// d2 < limit for every float d2; 0, which nothing is below, for a radius that is not positive. r * r is within one
+// float of it (checked for radii of every magnitude), so each loop ends after at most one step.
+__device__ __forceinline__ float leaf_limit(float r)
+{
+    if (!(r > 0.0f)) return 0.0f;
+    float t = r * r;
+    while (t > 0.0f && vren_sqrtf(__uint_as_float(__float_as_uint(t) - 1u)) >= r) t = __uint_as_float(__float_as_uint(t) - 1u);
+    while (vren_sqrtf(t) < r) t = __uint_as_float(__float_as_uint(t) + 1u);
+    return t;
+}
+
+// the leaf record of a leaf box (clustered.hpp): the radius as the traversal takes it from the box
+// (assign_lights.comp:214)
+__device__ __forceinline__ float4 leaf_record(float x, float y, float z, float min_x, float max_x)
+{
+    return make_float4(x, y, z, leaf_limit((max_x - min_x) / 2.0f));
+}
+
 // the frame and the chunk of a flattened chunk number
 __device__ __forceinline__ const FrameDev& frame_of_chunk(const FrameDev* __restrict__ frames, uint32_t F, uint32_t c,
                                                           uint32_t* chunk)
@@ -293,11 +312,11 @@ __device__ __forceinline__ void lights_body(const FrameDev* __restrict__ frames,
         if (i >= groups * 32) break; // whole half-waves leave together; the others' lanes do not read them
         float mn[3] = {VREN_F32_INF, VREN_F32_INF, VREN_F32_INF};
         float mx[3] = {-VREN_F32_INF, -VREN_F32_INF, -VREN_F32_INF};
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         if (i < n) {
             const uint2 pr = s_pair[i];
-            const float4 v = s_light[pr.y];
+            v = s_light[pr.y];
             out[i] = pr;
-            if (fd.leaf_pos) reinterpret_cast<float4*>(fd.leaf_pos)[i] = v;
             mn[0] = v.x - v.w;
             mn[1] = v.y - v.w;
             mn[2] = v.z - v.w;
@@ -305,6 +324,9 @@ __device__ __forceinline__ void lights_body(const FrameDev* __restrict__ frames,
             mx[1] = v.y + v.w;
             mx[2] = v.z + v.w;
         }
+        if (fd.leaf_rec)
+            reinterpret_cast<float4*>(fd.leaf_rec)[i] = i < n ? leaf_record(v.x, v.y, v.z, mn[0], mx[0])
+                                                               : make_float4(0.f, 0.f, 0.f, 0.f);
         store_node(&fd.bvh[i], mn, mx, i < n ? VREN_BVH_LEAF_NODE : VREN_BVH_INVALID_NODE);
         half_wave_box(mn, mx);
         if ((lane & 31) == 31) {
@@ -484,14 +506,15 @@ __global__ __launch_bounds__(256) void bvh_leaf_kernel(const FrameDev* __restric
             uint32_t li = reinterpret_cast<const uint2*>(fd.codes)[i].y;
             float4 vp = reinterpret_cast<const float4*>(fd.view_pos)[li];
             float r = reinterpret_cast<const float4*>(fd.lights)[li].w;
-            if (fd.leaf_pos) reinterpret_cast<float4*>(fd.leaf_pos)[i] = vp;
             mn[0] = vp.x - r;
             mn[1] = vp.y - r;
             mn[2] = vp.z - r;
             mx[0] = vp.x + r;
             mx[1] = vp.y + r;
             mx[2] = vp.z + r;
+            if (fd.leaf_rec) reinterpret_cast<float4*>(fd.leaf_rec)[i] = leaf_record(vp.x, vp.y, vp.z, mn[0], mx[0]);
         } else {
+            if (fd.leaf_rec && i < live_end) reinterpret_cast<float4*>(fd.leaf_rec)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
             mn[0] = mn[1] = mn[2] = VREN_F32_INF;
             mx[0] = mx[1] = mx[2] = -VREN_F32_INF;
         }
