@@ -5,12 +5,12 @@
 // ballot stack, run twice (COUNT then WRITE) around a fixed 2^17-entry Blelloch scan of the counts; lists come
 // out in traversal order with reversed lanes inside each leaf block.
 // Here: persistent kernels over the clusters of every frame (their number is read on the device; it never returns
-// to the host), taken in chunks of up to 64 whose per-cluster work (the cluster AABB, the list bounds) is done one
-// cluster per lane. COUNT runs two traversals per wave, one per 32-lane half (the BVH's fan-out), each from its own
-// LDS stack, and keeps lists of at most VREN_LIST_SLOT (192) lights, sorted by rank, in per-cluster slots; one
-// workgroup per frame scans the counts into offsets; WRITE copies the kept lists and traverses again only for longer
-// ones, with the whole wave testing two BVH blocks per step, one bit per hit light in a per-wave LDS bitmask, emitted
-// in ascending light index (the canonical order) by a popcount prefix over the bitmask words.
+// to the host). COUNT takes them in chunks of up to 64 whose AABBs are computed one cluster per lane, runs two
+// traversals per wave, one per 32-lane half (the BVH's fan-out), each from its own LDS stack, and keeps lists of at most
+// VREN_LIST_SLOT (192) lights, sorted by rank, in per-cluster slots; LISTS turns the counts into offsets, copies the
+// kept lists and traverses again only for longer ones, with the whole wave testing two BVH blocks per step, one bit per
+// hit light in an LDS bitmask, emitted in ascending light index (the canonical order) by a popcount prefix over the
+// bitmask words.
 // The cluster AABB and both tests are restated operation for operation (including the inverted y range of
 // the two-corner AABB); padding leaves and invalid nodes (empty AABB) never match.
 #include "chain.hpp"
@@ -348,55 +348,13 @@ __device__ __forceinline__ uint32_t chunk_size(uint32_t total, uint32_t waves)
     return max(1u, min(VREN_WAVE, (total + 4u * waves - 1u) / (4u * waves)));
 }
 
-// Clusters of every frame of the table are processed as one flattened range, in chunks of at most 64 consecutive
+// Clusters of every frame of the table are counted as one flattened range, in chunks of at most 64 consecutive
 // clusters per wave: lane i takes cluster i of the chunk, finds its frame among 64 frames at a time (their
-// device-side cluster counts, one per lane, prefix-summed) and computes that cluster's per-lane prologue `pre` (the
-// cluster AABB, list bounds), so work that is uniform per cluster is done for a whole chunk at once. fn(fd, c, k, v)
-// then runs for each cluster k of the chunk with the whole wave (v = lane k's prologue, read with readlane).
-template <typename T, typename Pre, typename Fn>
-__device__ __forceinline__ void for_each_cluster_chunk(const FrameDev* __restrict__ frames, uint32_t F, uint32_t gw,
-                                                       uint32_t stride, Pre pre, Fn fn)
-{
-    const uint32_t lane = lane_id();
-    for (uint32_t f0 = 0; f0 < F; f0 += VREN_WAVE) {
-        const uint32_t fi = f0 + lane;
-        uint32_t nf = 0;
-        if (fi < F) {
-            const FrameDev& d = frames[fi];
-            if (d.L != 0 && d.cluster_count != nullptr) nf = min(*d.cluster_count, d.key_cap);
-        }
-        const uint32_t incl = wave_inclusive_sum(nf);
-        const uint32_t excl = incl - nf;
-        const uint32_t total = __builtin_amdgcn_readlane(incl, VREN_WAVE - 1);
-                const uint32_t cs = chunk_size(total, stride);
-        const uint32_t chunks = (total + cs - 1u) / cs;
-        for (uint32_t chunk = gw; chunk < chunks; chunk += stride) {
-            const uint32_t c0 = chunk * cs;
-            const uint32_t c = c0 + lane;
-            // frame of cluster c: the number of frames whose inclusive count is <= c (counts are non-decreasing)
-            uint32_t pos = 0;
-#pragma unroll
-            for (uint32_t step = VREN_WAVE / 2; step >= 1; step >>= 1)
-                if (shfl(incl, (int)(pos + step - 1)) <= c) pos += step;
-            const uint32_t fl = min(pos, VREN_WAVE - 1);
-            const uint32_t base = shfl(excl, (int)fl);
-            T v{};
-            if (lane < cs && c < total) v = pre(frames[f0 + fl], c - base);
-            const uint32_t n = min(total - c0, cs);
-            for (uint32_t k = 0; k < n; k++) {
-                const uint32_t fk = __builtin_amdgcn_readlane(fl, k);
-                const uint32_t bk = __builtin_amdgcn_readlane(base, k);
-                fn(frames[f0 + fk], c0 + k - bk, k, v);
-            }
-        }
-    }
-}
-
-// for_each_cluster_chunk for the paired count pass: pre(fd, c) runs per lane (lane i: cluster i of the chunk), then
-// fn(fd, k, two, cA, cB) for clusters k and, with `two`, k + 1 of the chunk, cA and cB their frame-local indices; the two
+// device-side cluster counts, one per lane, prefix-summed) and runs pre(fd, c) (the cluster AABB), so work that is
+// uniform per cluster is done for a whole chunk at once. Then the whole wave runs fn(fd, k, two, cA, cB) for clusters k and, with `two`, k + 1 of the chunk, cA and cB their frame-local indices; the two
 // are of one frame, so that its record is uniform and read with scalar loads.
 template <typename Pre, typename Fn>
-__device__ __forceinline__ void for_each_cluster_chunk2(const FrameDev* __restrict__ frames, uint32_t F, uint32_t gw,
+__device__ __forceinline__ void for_each_cluster_pair(const FrameDev* __restrict__ frames, uint32_t F, uint32_t gw,
                                                         uint32_t stride, Pre pre, Fn fn)
 {
     const uint32_t lane = lane_id();
@@ -499,7 +457,7 @@ __device__ __forceinline__ void assign_count_body(const FrameDev* __restrict__ f
     Box* boxes = reinterpret_cast<Box*>(s_mem + wpb * 2 * kHalf) + wave * VREN_WAVE;
     const uint32_t gw = blockIdx.x * wpb + wave;
     // the chunk's cluster AABBs wait in LDS (one per lane) while the wave traverses two at a time
-    for_each_cluster_chunk2(
+    for_each_cluster_pair(
         frames, F, gw, gridDim.x * wpb,
         [&](const FrameDev& fdl, uint32_t c) { boxes[lane] = leaf_box(cluster_aabb(fdl, fdl.keys[c])); },
         [&](const FrameDev& fd, uint32_t k, bool two, uint32_t cA, uint32_t cB) {
@@ -541,111 +499,153 @@ __device__ __forceinline__ void assign_count_body(const FrameDev* __restrict__ f
         });
 }
 
-// exclusive scan of counts[0 .. min(cluster_count, key_cap)) -> offsets and assigned_total: one workgroup per
-// frame walks its counts 4096 at a time with a running carry (no cross-workgroup chaining, no tickets; a frame
-// holds a few thousand clusters, at most key_cap)
-__device__ __forceinline__ void assign_offsets_body(const FrameDev* __restrict__ frames)
-{
-    __shared__ uint32_t s_wave[16];
-    const FrameDev& fd = frames[blockIdx.x];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t n = (fd.L == 0 || fd.cluster_count == nullptr) ? 0u : min(*fd.cluster_count, fd.key_cap);
-    uint32_t carry = 0;
-    for (uint32_t start = 0; start < n; start += 4096) {
-        uint32_t v[4], sum = 0;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const uint32_t i = start + tid * 4 + k;
-            v[k] = i < n ? fd.counts[i] : 0u;
-            sum += v[k];
-        }
-        uint32_t agg;
-        uint32_t run = carry + block_exclusive_sum<1024>(sum, s_wave, &agg);
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const uint32_t i = start + tid * 4 + k;
-            if (i < n) fd.offsets[i] = run;
-            run += v[k];
-        }
-        carry += agg;
-    }
-    if (tid == 0) {
-        *fd.assigned_total = carry;
-        if (carry > fd.index_cap) atomic_or_agent(fd.flags, VREN_FLAG_INDEX_CAPACITY);
-    }
-}
-
-struct ListBounds {
-    uint32_t count, offset;
-};
-
-// WRITE: each cluster's list at its offset: copied from the slot the counting pass kept, or traversed again
-// (bitmask, emitted in ascending light index) when it was longer than a slot
-__device__ __forceinline__ void assign_write_body(const FrameDev* __restrict__ frames, uint32_t F, uint32_t mask_words,
-                                                  uint32_t* s_mem)
-{
-    const uint32_t wpb = blockDim.x / VREN_WAVE;
-    const uint32_t wave = wave_id();
-    const uint32_t lane = lane_id();
-    const uint32_t summary_words = (mask_words + 31) / 32;
-    uint32_t* stack = s_mem + wave * kStack;
-    uint32_t* bitmask = s_mem + wpb * kStack + wave * mask_words;
-    uint32_t* summary = s_mem + wpb * (kStack + mask_words) + wave * summary_words;
-    for (uint32_t i = lane; i < mask_words; i += VREN_WAVE) bitmask[i] = 0u;
-    for (uint32_t i = lane; i < summary_words; i += VREN_WAVE) summary[i] = 0u;
-    __builtin_amdgcn_wave_barrier();
-    const uint32_t gw = blockIdx.x * wpb + wave;
-    for_each_cluster_chunk<ListBounds>(
-        frames, F, gw, gridDim.x * wpb,
-        [&](const FrameDev& fdl, uint32_t c) { return ListBounds{fdl.counts[c], fdl.offsets[c]}; },
-        [&](const FrameDev& fd, uint32_t c, uint32_t k, const ListBounds& mine) {
-            const uint32_t cnt = __builtin_amdgcn_readlane(mine.count, k);
-            const uint32_t out = __builtin_amdgcn_readlane(mine.offset, k);
-            if (fd.list_slots && c < fd.slot_cap && cnt <= VREN_LIST_SLOT) {
-                // the counting pass kept this list
-#pragma unroll
-                for (uint32_t r = 0; r < VREN_LIST_SLOT / VREN_WAVE; r++) {
-                    const uint32_t i = lane + r * VREN_WAVE;
-                    if (i < cnt && (uint64_t)out + i < fd.index_cap)
-                        fd.indices[out + i] = fd.list_slots[(size_t)c * VREN_LIST_SLOT + i];
-                }
-                return;
-            }
-            const Box box = leaf_box(cluster_aabb(fd, fd.keys[c]));
-            traverse(fd, box, stack, bitmask, summary);
-            __builtin_amdgcn_wave_barrier();
-            // emit set bits in ascending light index, clearing the mask as we go
-            const uint32_t room = out < fd.index_cap ? fd.index_cap - out : 0u;
-            emit_bitmask(bitmask, summary, ((fd.L + 31) / 32 + 31) / 32, fd.indices + out, room);
-            __builtin_amdgcn_wave_barrier();
-        });
-}
-
 // [begin, end) of the index-buffer entries of a tile's light lists, for shade: the tile's clusters are the consecutive
 // indices [c0, c0 + u) (clusters kernel) and their lists are consecutive in the index buffer, so the range runs from the
-// first cluster's offset to the end of the last list (both clamped to the capacities like the per-pixel lists). One
-// thread per tile, ahead of the writing pass's lists, which it does not depend on.
+// first cluster's offset to the end of the last list (both clamped to the capacities like the per-pixel lists).
 struct TileRanges {
-    const uint32_t* tile_frame;
     const uint2* tile_cl;
     uint2* tile_range; // null: no ranges
-    uint32_t total_tiles;
 };
 
-__device__ __forceinline__ void write_tile_ranges(const FrameDev* __restrict__ frames, const TileRanges& r)
+// LISTS: offsets, light lists and tile ranges in one launch. A frame's clusters are cut into `parts` runs, one workgroup
+// each, which sums the counts before its run itself (a frame holds a few thousand clusters; a launch of its own for
+// their prefix sum took longer) and takes its run 256 clusters at a time: their offsets by a block scan, then their
+// lists, which are consecutive in the index buffer, as one range of entries spread over the threads, each finding its
+// cluster among the 256 prefixes and copying it from the slot that the counting pass kept. A list longer than a slot is
+// traversed again (bitmask, emitted in ascending light index) by one of the `masks` waves that have room for a bitmask.
+// 64 frames of 1080p with 4096 lights took 6 + 54 us in two launches, the copies one cluster per wave and step with a
+// load's latency each, and take 24; one
+// frame 5 + 4.8, now 6.7; a 3840x2160 frame with 65536 lights 12 + 15, now 16.
+constexpr uint32_t kListThreads = 256;
+constexpr int kListUnroll = 4; // entries per thread and step
+
+__device__ __forceinline__ uint32_t list_sum(uint32_t v, uint32_t* s_wave)
 {
-    if (!r.tile_range) return;
-    for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < r.total_tiles; g += gridDim.x * blockDim.x) {
-        const FrameDev& fd = frames[frame_of_tile(r.tile_frame, g)];
-        const uint2 c = r.tile_cl[g];
-        uint32_t a = 0, b = 0;
-        if (g - fd.tile_base < fd.Sx * fd.Sy && fd.L > 0 && c.y > 0 && c.x < fd.key_cap) { // not a padding tile
-            const uint32_t c1 = min(c.x + c.y, fd.key_cap) - 1u;
-            a = min(fd.offsets[c.x], fd.index_cap);
-            const uint64_t e = (uint64_t)fd.offsets[c1] + fd.counts[c1];
-            b = e > fd.index_cap ? fd.index_cap : (uint32_t)e;
+    const uint32_t w = wave_sum(v);
+    if (lane_id() == 0) s_wave[wave_id()] = w;
+    __syncthreads();
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kListThreads / VREN_WAVE; i++) sum += s_wave[i];
+    __syncthreads();
+    return sum;
+}
+
+__device__ __forceinline__ void assign_lists_body(const FrameDev& fd, uint32_t part, uint32_t parts, uint32_t mask_words,
+                                                  uint32_t masks, const TileRanges ranges, uint32_t* s_mem)
+{
+    __shared__ uint32_t s_pre[kListThreads + 1]; // list starts of the 256 clusters, relative to the first one's
+    __shared__ uint32_t s_wave[kListThreads / VREN_WAVE];
+    __shared__ uint64_t s_long[kListThreads / VREN_WAVE];
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+    const uint32_t n = (fd.L == 0 || fd.cluster_count == nullptr) ? 0u : min(*fd.cluster_count, fd.key_cap);
+    const uint32_t run_len = (n + parts - 1) / parts;
+    const uint32_t begin = min(part * run_len, n), end = min(begin + run_len, n);
+    const bool last = part == parts - 1;
+    uint32_t sum = 0;
+    const uint32_t quads = (reinterpret_cast<uintptr_t>(fd.counts) & 15) == 0 ? begin / 4 : 0u;
+#pragma unroll 8
+    for (uint32_t i = tid; i < quads; i += kListThreads) {
+        const vu4 x = load_at<vu4>(fd.counts, i);
+        sum += (x.x + x.y) + (x.z + x.w);
+    }
+    for (uint32_t i = quads * 4 + tid; i < begin; i += kListThreads) sum += load_at<uint32_t>(fd.counts, i);
+    uint32_t run = list_sum(sum, s_wave);
+
+    // first clusters ascend over the frame's tiles, so 256 of them, one per thread, bracket each sub-run's tiles
+    const uint32_t tiles = ranges.tile_range ? fd.Sx * fd.Sy : 0u;
+    const uint2* tile_cl = ranges.tile_cl + fd.tile_base;
+    const uint32_t step = (tiles + kListThreads - 1) / kListThreads;
+    uint32_t sample = 0xFFFFFFFFu;
+    if (tiles) {
+        if (tid * step < tiles) sample = tile_cl[tid * step].x;
+        if (last) // a tile without clusters below the capacity (of a frame without lights, every tile) has an empty range
+            for (uint32_t t = tid; t < tiles; t += kListThreads)
+                if (!(tile_cl[t].x < n && tile_cl[t].y > 0)) ranges.tile_range[fd.tile_base + t] = make_uint2(0u, 0u);
+    }
+
+    bool cleared = false; // this wave's bitmask (which emit_bitmask leaves clear)
+    for (uint32_t c0 = begin; c0 < end; c0 += kListThreads) {
+        const uint32_t m = min(kListThreads, end - c0), c = c0 + tid;
+        const uint32_t cnt = tid < m ? load_at<uint32_t>(fd.counts, c) : 0u;
+        uint32_t total;
+        const uint32_t ex = block_exclusive_sum<kListThreads>(cnt, s_wave, &total);
+        if (tid < m) fd.offsets[c] = run + ex;
+        const bool kept = fd.list_slots != nullptr && c < fd.slot_cap && cnt <= VREN_LIST_SLOT;
+        const uint64_t longs = ballot(tid < m && !kept);
+        if (lane == 0) s_long[wave] = longs;
+        s_pre[tid] = ex;
+        if (tid == 0) s_pre[kListThreads] = total;
+        __syncthreads();
+        for (uint32_t q0 = 0; q0 < total; q0 += kListThreads * kListUnroll) { // entries whose searches and loads overlap
+            uint32_t at[kListUnroll];
+#pragma unroll
+            for (int u = 0; u < kListUnroll; u++) at[u] = 0;
+#pragma unroll
+            for (uint32_t s = kListThreads / 2; s >= 1; s >>= 1)
+#pragma unroll
+                for (int u = 0; u < kListUnroll; u++) // the last cluster whose list starts at or before the entry
+                    if (s_pre[at[u] + s] <= q0 + u * kListThreads + tid) at[u] += s;
+            uint32_t li[kListUnroll];
+            bool on[kListUnroll];
+#pragma unroll
+            for (int u = 0; u < kListUnroll; u++) {
+                const uint32_t q = q0 + u * kListThreads + tid, i = at[u];
+                on[u] = q < total && (uint64_t)run + q < fd.index_cap && !((s_long[i / VREN_WAVE] >> (i % VREN_WAVE)) & 1ull);
+                li[u] = on[u] ? fd.list_slots[(size_t)(c0 + i) * VREN_LIST_SLOT + (q - s_pre[i])] : 0u;
+            }
+#pragma unroll
+            for (int u = 0; u < kListUnroll; u++)
+                if (on[u]) fd.indices[run + q0 + u * kListThreads + tid] = li[u];
         }
-        r.tile_range[g] = make_uint2(a, b);
+        if (tiles) {
+            // tiles [t0, t1): from the last sample below c0 to the first one past the sub-run
+            const uint32_t below = list_sum(sample < c0 ? 1u : 0u, s_wave), upto = list_sum(sample < c0 + m ? 1u : 0u, s_wave);
+            const uint32_t t0 = below ? (below - 1) * step : 0u, t1 = min(upto * step, tiles);
+            for (uint32_t t = t0 + tid; t < t1; t += kListThreads) {
+                const uint2 cl = tile_cl[t];
+                if (!(cl.y > 0 && cl.x >= c0 && cl.x < c0 + m)) continue;
+                const uint32_t stop = (uint32_t)min<uint64_t>((uint64_t)cl.x + cl.y, n), in = min(stop - c0, m);
+                uint64_t e = (uint64_t)run + s_pre[in];
+                for (uint32_t k = c0 + in; k < stop; k++) e += fd.counts[k]; // clusters past the sub-run
+                const uint32_t a = min(run + s_pre[cl.x - c0], fd.index_cap);
+                ranges.tile_range[fd.tile_base + t] = make_uint2(a, e > fd.index_cap ? fd.index_cap : (uint32_t)e);
+            }
+        }
+        if (wave < masks) {
+            const uint32_t summary_words = (mask_words + 31) / 32;
+            uint32_t* stack = s_mem + wave * (kStack + mask_words + summary_words);
+            uint32_t* bitmask = stack + kStack;
+            uint32_t* summary = bitmask + mask_words;
+            uint32_t seen = 0; // long lists of the sub-run so far
+            for (uint32_t w = 0; w < kListThreads / VREN_WAVE; w++) {
+                for (uint64_t rem = s_long[w]; rem; rem &= rem - 1, seen++) {
+                    if (seen % masks != wave) continue;
+                    const uint32_t i = w * VREN_WAVE + (uint32_t)__builtin_ctzll(rem);
+                    if (s_pre[i + 1] == s_pre[i]) continue; // an empty list past the slots
+                    if (!cleared) {
+                        cleared = true;
+                        for (uint32_t k = lane; k < mask_words; k += VREN_WAVE) bitmask[k] = 0u;
+                        for (uint32_t k = lane; k < summary_words; k += VREN_WAVE) summary[k] = 0u;
+                        __builtin_amdgcn_wave_barrier();
+                    }
+                    const uint32_t out = run + s_pre[i];
+                    const Box box = leaf_box(cluster_aabb(fd, fd.keys[c0 + i]));
+                    traverse(fd, box, stack, bitmask, summary);
+                    __builtin_amdgcn_wave_barrier();
+                    // emit set bits in ascending light index, clearing the mask as we go
+                    emit_bitmask(bitmask, summary, ((fd.L + 31) / 32 + 31) / 32, fd.indices + out,
+                                 out < fd.index_cap ? fd.index_cap - out : 0u);
+                    __builtin_amdgcn_wave_barrier();
+                }
+            }
+        }
+        run += total;
+        __syncthreads(); // s_pre, s_long are rewritten
+    }
+    if (last && tid == 0) {
+        *fd.assigned_total = run;
+        if (run > fd.index_cap) atomic_or_agent(fd.flags, VREN_FLAG_INDEX_CAPACITY);
     }
 }
 
@@ -662,19 +662,18 @@ __global__ __launch_bounds__(256, 8) void assign_count_one_kernel(const FrameDev
     extern __shared__ uint32_t s_mem[];
     assign_count_body<false>(inline_frame(), 1, s_mem);
 }
-__global__ __launch_bounds__(1024) void assign_offsets_kernel(const FrameDev* __restrict__ frames) { assign_offsets_body(frames); }
-__global__ __launch_bounds__(1024) void assign_offsets_one_kernel(const FrameDev one) { assign_offsets_body(inline_frame()); }
-__global__ __launch_bounds__(256, 8) void assign_write_kernel(const FrameDev* __restrict__ frames, uint32_t F,
-                                                             uint32_t mask_words, const TileRanges ranges)
+__global__ __launch_bounds__(kListThreads) void assign_lists_kernel(const FrameDev* __restrict__ frames, uint32_t parts,
+                                                                    uint32_t mask_words, uint32_t masks,
+                                                                    const TileRanges ranges)
 {
     extern __shared__ uint32_t s_mem[];
-    write_tile_ranges(frames, ranges);
-    assign_write_body(frames, F, mask_words, s_mem);
+    assign_lists_body(frames[blockIdx.x / parts], blockIdx.x % parts, parts, mask_words, masks, ranges, s_mem);
 }
-__global__ __launch_bounds__(256, 8) void assign_write_one_kernel(const FrameDev one, uint32_t mask_words)
+__global__ __launch_bounds__(kListThreads) void assign_lists_one_kernel(const FrameDev one, uint32_t parts,
+                                                                        uint32_t mask_words, uint32_t masks)
 {
     extern __shared__ uint32_t s_mem[];
-    assign_write_body(inline_frame(), 1, mask_words, s_mem);
+    assign_lists_body(*inline_frame(), blockIdx.x, parts, mask_words, masks, TileRanges{nullptr, nullptr}, s_mem);
 }
 
 __global__ void empty_lists_kernel(uint32_t* counts, uint32_t* offsets, uint32_t n, uint32_t* total)
@@ -697,21 +696,21 @@ int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32
                   const FrameDev* one)
 {
     if (w.max_L == 0) return one ? VREN_OK : launch_chain_init(ctx, s, w); // no lists; the next run finds cleared words
+    // per wave that traverses long lists: a stack, the bitmask and its summary
     const uint32_t mask_words = (w.max_L + 31) / 32;
-    const size_t per_wave = (size_t)(kStack + mask_words + (mask_words + 31) / 32) * 4;
-    uint32_t wpb = 4;
-    while (wpb > 1 && per_wave * wpb > 150 * 1024) wpb--;
-    if (per_wave > 150 * 1024) return vren_fail(ctx, VREN_EINVAL, "assign_lights: too many lights for the LDS bitmask");
+    const size_t per_mask = (size_t)(kStack + mask_words + (mask_words + 31) / 32) * 4;
+    if (per_mask > 150 * 1024) return vren_fail(ctx, VREN_EINVAL, "assign_lights: too many lights for the LDS bitmask");
+    const uint32_t masks = (uint32_t)std::min<size_t>(kListThreads / VREN_WAVE, 150 * 1024 / per_mask);
     // per wave, two stacks, leaf lists and hit lists (one per half) and the chunk's boxes
     constexpr size_t count_per_wave = (size_t)2 * (kStackHalf + kLeafList + VREN_LIST_SLOT) * 4 + VREN_WAVE * sizeof(float) * 6;
     static_assert(count_per_wave * 4 <= 160 * 1024 / 8, "assign_count: 8 workgroups of 4 waves must fit a CU's LDS");
-    const uint32_t count_blocks = persistent_blocks(ctx, 4, w.assign_wpc), write_blocks = persistent_blocks(ctx, wpb, w.assign_wpc);
+    const uint32_t count_blocks = persistent_blocks(ctx, 4, w.assign_wpc);
+    // list runs per frame: 2048 workgroups over a batch, at most 512 and at least 8 a frame
+    const uint32_t parts = std::max<uint32_t>(8, std::min<uint32_t>(512, 2048 / F));
     if (one) {
         assign_count_one_kernel<<<count_blocks, 4 * VREN_WAVE, count_per_wave * 4, s>>>(*one);
         VREN_LAUNCH_CHECK(ctx);
-        assign_offsets_one_kernel<<<1, 1024, 0, s>>>(*one);
-        VREN_LAUNCH_CHECK(ctx);
-        assign_write_one_kernel<<<write_blocks, wpb * VREN_WAVE, per_wave * wpb, s>>>(*one, mask_words);
+        assign_lists_one_kernel<<<parts, kListThreads, per_mask * masks, s>>>(*one, parts, mask_words, masks);
         VREN_LAUNCH_CHECK(ctx);
         return VREN_OK;
     }
@@ -719,11 +718,9 @@ int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32
         d_frames, F, w.tickets, (uint32_t)(chain_work_clear_bytes(w.total_tiles) / 4));
     VREN_LAUNCH_CHECK(ctx);
     chain_mark(w, s);
-    assign_offsets_kernel<<<F, 1024, 0, s>>>(d_frames);
-    VREN_LAUNCH_CHECK(ctx);
-    chain_mark(w, s);
-    const TileRanges ranges{F > 1 ? w.tile_frame : nullptr, w.tile_cl, w.tile_range, w.total_tiles};
-    assign_write_kernel<<<write_blocks, wpb * VREN_WAVE, per_wave * wpb, s>>>(d_frames, F, mask_words, ranges);
+    chain_mark(w, s); // the offsets are written with the lists
+    assign_lists_kernel<<<F * parts, kListThreads, per_mask * masks, s>>>(d_frames, parts, mask_words, masks,
+                                                                          TileRanges{w.tile_cl, w.tile_range});
     VREN_LAUNCH_CHECK(ctx);
     chain_mark(w, s);
     return VREN_OK;
@@ -776,6 +773,15 @@ extern "C" VREN_EXPORT int vren_assign_lights(vren_ctx* ctx, vren_stream_t strea
                                                                                             key_capacity, assigned_total);
         VREN_LAUNCH_CHECK(ctx);
         return VREN_OK;
+    }
+    // list slots for the first clusters, as a batch has them; a capture that would have to grow the scratch for them does
+    // without (every list is then traversed a second time)
+    const uint32_t slot_cap = std::min<uint32_t>(key_capacity, VREN_SLOT_CLUSTERS);
+    if (vren_can_have_scratch(ctx, (size_t)slot_cap * VREN_LIST_SLOT * 4, s)) {
+        st = vren_ensure_scratch(ctx, (size_t)slot_cap * VREN_LIST_SLOT * 4, s);
+        if (st) return st;
+        f.list_slots = static_cast<uint32_t*>(ctx->scratch);
+        f.slot_cap = slot_cap;
     }
     ChainWork w;
     memset(&w, 0, sizeof(w));

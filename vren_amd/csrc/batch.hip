@@ -211,8 +211,8 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         leaf_base += slots;
         live_base += live;
         max_L = std::max(max_L, L);
-        // list slots for the first 32 768 clusters of the frame (768 B each); clusters past them are traversed again
-        const uint32_t slot_cap = std::min<uint32_t>(key_cap, 1u << 15);
+        // list slots for the first clusters of the frame; clusters past them are traversed again
+        const uint32_t slot_cap = std::min<uint32_t>(key_cap, VREN_SLOT_CLUSTERS);
         f.slot_cap = L ? slot_cap : 0u;
         size_t* o = &off[i * 14];
         o[0] = arena; arena += a256((size_t)L * 16);                 // view_pos

@@ -14,6 +14,8 @@
 // traversing those again cost 0.2 ms per batch) while the counting kernel's per-half LDS lists still let 8
 // workgroups share a CU
 #define VREN_LIST_SLOT 192u
+// clusters of a frame that have list slots (768 B each)
+#define VREN_SLOT_CLUSTERS (1u << 15)
 
 struct FrameDev {
     // sizes

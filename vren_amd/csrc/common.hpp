@@ -220,6 +220,8 @@ struct vren_ctx {
 int vren_fail(vren_ctx* ctx, int status, const char* fmt, ...);
 int vren_hip_fail(vren_ctx* ctx, hipError_t err, const char* what);
 int vren_ensure_scratch(vren_ctx* ctx, size_t bytes, hipStream_t s);
+// whether vren_ensure_scratch can give this much: always, but for a stream capture that it would have to grow in
+bool vren_can_have_scratch(vren_ctx* ctx, size_t bytes, hipStream_t s);
 int vren_noalloc_scan_setup(vren_ctx* ctx);
 
 #define VREN_HIP(ctx, expr)                                                                                            \

@@ -51,6 +51,13 @@ int vren_ensure_scratch(vren_ctx* ctx, size_t bytes, hipStream_t s)
     return VREN_OK;
 }
 
+bool vren_can_have_scratch(vren_ctx* ctx, size_t bytes, hipStream_t s)
+{
+    if (bytes <= ctx->scratch_bytes) return true;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+}
+
 extern "C" {
 
 VREN_EXPORT int vren_create(int hip_device, vren_ctx** out)
