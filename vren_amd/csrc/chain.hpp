@@ -77,6 +77,12 @@ void chain_work_bind(ChainWork* w, void* mem, uint32_t total_tiles);
 int launch_chain_init(vren_ctx* ctx, hipStream_t s, const ChainWork& w);
 int launch_lights(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
                   const FrameDev* one = nullptr);
+// the two parts of launch_lights around the chunks' sort, for frames of more than one chunk
+int launch_light_bounds(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w);
+int launch_light_merge(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w);
+// the chunks' sort and the cluster stage in one launch (front.hip), where front_fits
+bool front_fits(const vren_ctx* ctx, const ChainWork& w);
+int launch_front(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w);
 // which 32-leaf groups the leaf kernel writes: all, those holding a light, or the all-padding ones
 enum : uint32_t { kLeavesAll = 0, kLeavesLive = 1, kLeavesPadding = 2 };
 int launch_bvh(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, uint32_t total_leaf_slots,
