@@ -109,6 +109,11 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v)
     return wave_reduce_dpp(v, 0xFFFFFFFFu, [](uint32_t a, uint32_t b) { return a < b ? a : b; });
 }
 
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
+{
+    return wave_reduce_dpp(v, 0u, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+}
+
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // 128-bit streaming (non-temporal) load / store of 4 uint32 at a 16-byte aligned address
