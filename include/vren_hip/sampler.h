@@ -87,4 +87,32 @@ VREN_HD void vren_texel_axis(float s, uint32_t size, uint32_t filter, uint32_t m
     *alpha = 0.0f;
 }
 
+/* vren_texel_axis for |s * size| < 2^22 and sides up to 2^22 texels, where it picks the same texels with the same weight in
+ * 16 instructions in place of about 30: with integers x and n, |x| < 2^23, a quotient within an ulp of x / n has the
+ * floor of x / n (x / n is no integer only if it is 1 / n or more away from one, and 1 / n is more than an ulp), so
+ * neither an IEEE division nor a correction of the remainder is needed. rcp_size: 1 / size within an ulp. */
+VREN_HD void vren_texel_axis_near(float s, uint32_t size, float rcp_size, uint32_t filter, uint32_t mode, uint32_t* i0,
+                                  uint32_t* i1, float* alpha)
+{
+    const float n = (float)size;
+    const float v = filter == VREN_FILTER_LINEAR ? __builtin_fmaf(s, n, -0.5f) : s * n;
+    const float f = vren_floorf(v);
+    *alpha = filter == VREN_FILTER_LINEAR ? v - f : 0.0f;
+    if (mode == VREN_ADDRESS_CLAMP_TO_EDGE) {
+        *i0 = (uint32_t)__builtin_fminf(__builtin_fmaxf(f, 0.0f), n - 1.0f);
+        *i1 = (uint32_t)__builtin_fminf(__builtin_fmaxf(f + 1.0f, 0.0f), n - 1.0f);
+    } else {
+        const int mirrored = mode == VREN_ADDRESS_MIRRORED_REPEAT;
+        const float p = mirrored ? n + n : n, rp = mirrored ? 0.5f * rcp_size : rcp_size;
+        const uint32_t period = mirrored ? 2u * size : size;
+        const float q0 = f * rp;
+        const float q = vren_floorf(__builtin_fmaf(__builtin_fmaf(-q0, p, f), rp, q0));
+        const uint32_t t0 = (uint32_t)__builtin_fmaf(-q, p, f);
+        const uint32_t t1 = t0 + 1u == period ? 0u : t0 + 1u;
+        *i0 = mirrored && t0 >= size ? 2u * size - 1u - t0 : t0;
+        *i1 = mirrored && t1 >= size ? 2u * size - 1u - t1 : t1;
+    }
+    if (filter != VREN_FILTER_LINEAR) *i1 = *i0;
+}
+
 #endif /* VREN_HIP_SAMPLER_H_ */

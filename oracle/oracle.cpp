@@ -14,6 +14,7 @@
  *   o_rcp_f16_newton_mismatches  the planted variant (no Newton step) is reported; exact rational arithmetic
  *                        agrees (the FMA and the division here are correctly rounded by the C library)
  *   o_third_index_mismatches  a planted threshold one float off is reported
+ *   o_texel_axis_mismatches  a planted error of the reciprocal is reported
  *   o_reduce_tree_*      closed form tree[i] = op over the aligned block ending at i; totals vs numpy
  *   o_exclusive_scan_u32 numpy cumsum (uint32 wrap-around)
  *   o_stable_sort_kv     numpy argsort(kind='stable')
@@ -189,6 +190,26 @@ OEXPORT uint32_t o_third_index_mismatches(uint64_t lo, uint64_t hi, uint32_t pla
         const uint32_t cmp = planted ? (uint32_t)(u >= t1) + (uint32_t)(u >= 0x1.555556p-2f) + (uint32_t)(u >= 0x1.fffffep-1f)
                                      : vren_third_index(u);
         if (formula != cmp) bad++;
+    }
+    return bad;
+}
+
+/* Coordinates s[i] with |s size| < 2^22 for which the short form of the texel selection (vren_texel_axis_near, its reciprocal
+ * moved by `ulps` floats) differs from vren_texel_axis in a texel or in the weight's bits; `planted` moves the
+ * reciprocal by one part in 2^10, which must then be reported. */
+OEXPORT uint32_t o_texel_axis_mismatches(const float* s, uint64_t n, uint32_t size, uint32_t filter, uint32_t mode,
+                                         int32_t ulps, uint32_t planted)
+{
+    float r = vren_bits_f32(vren_f32_bits(1.0f / (float)size) + (uint32_t)ulps);
+    if (planted) r *= 1.0f + 0x1p-10f;
+    uint32_t bad = 0;
+    for (uint64_t i = 0; i < n; i++) {
+        if (!(std::fabs(s[i] * (float)size) < 0x1p22f)) continue;
+        uint32_t a0, a1, b0, b1;
+        float wa, wb;
+        vren_texel_axis(s[i], size, filter, mode, &a0, &a1, &wa);
+        vren_texel_axis_near(s[i], size, r, filter, mode, &b0, &b1, &wb);
+        bad += a0 != b0 || a1 != b1 || vren_f32_bits(wa) != vren_f32_bits(wb);
     }
     return bad;
 }

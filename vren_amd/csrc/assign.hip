@@ -218,15 +218,6 @@ __device__ uint32_t traverse(const FrameDev& fd, const Box& box, uint32_t* stack
     return hits;
 }
 
-// element `at` of a uniform array, at most 4 GB into it: a uniform base and a 32-bit lane offset, which one load takes
-template <typename T>
-__device__ __forceinline__ T load_at(const void* base, uint32_t at)
-{
-    typedef const __attribute__((address_space(1))) char gchar;
-    typedef const __attribute__((address_space(1))) T gT;
-    return *(gT*)((gchar*)base + at * (uint32_t)sizeof(T));
-}
-
 // Two traversals of one frame's BVH at once, one per 32-lane half of the wave (lanes 0-31 and 32-63, each with its own
 // cluster box, stack and lists; a half with live = false does nothing). Inner blocks are popped one per half and step, each
 // child tested by a lane of the half; the blocks of leaves that they reach wait in the half's leaf list and are tested

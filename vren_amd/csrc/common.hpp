@@ -31,6 +31,15 @@ typedef const __attribute__((address_space(1))) vf4 gvf4;
 typedef const __attribute__((address_space(1))) vu4 gvu4;
 typedef const __attribute__((address_space(1))) vu2 gvu2;
 
+// element `at` of a uniform array, at most 4 GB into it: a uniform base and a 32-bit lane offset, which one load takes
+template <typename T>
+__device__ __forceinline__ T load_at(const void* base, uint32_t at)
+{
+    typedef const __attribute__((address_space(1))) char gchar;
+    typedef const __attribute__((address_space(1))) T gT;
+    return *(gT*)((gchar*)base + at * (uint32_t)sizeof(T));
+}
+
 // index of the calling wave in its workgroup, as a wave-uniform value: the compiler then keeps what is derived
 // from it (tile and frame indices, frame-record fields) in scalar registers and reads such records with scalar loads
 __device__ __forceinline__ uint32_t wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x / VREN_WAVE); }
