@@ -236,7 +236,7 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
     }
     hipError_t e = hipMalloc(&b->arena, std::max<size_t>(arena, 256));
     if (e == hipSuccess) e = hipMemset(b->arena, 0, std::max<size_t>(arena, 256));
-    const size_t wbytes = chain_work_bytes(tile_base, n_frames);
+    const size_t wbytes = chain_work_bytes(tile_base);
     if (e == hipSuccess) e = hipMalloc(&b->work, wbytes);
     if (e == hipSuccess) e = hipMemset(b->work, 0, chain_work_clear_bytes(tile_base));
     if (e == hipSuccess) e = hipMalloc(&b->d_table, sizeof(FrameDev) * n_frames);
@@ -288,7 +288,7 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         b->size_class = batch_size_class(pixels, max_L, n_frames);
     }
     // per-frame tables: same buffers, bases 0, the frame's share of the same workspace (the statuses and per-tile tables
-    // from their starts, so that every run leaves the same words cleared; the frame's own slice table)
+    // from their starts, so that every run leaves the same words cleared)
     std::vector<FrameDev> single(b->host);
     b->w_frame.resize(n_frames);
     for (uint32_t i = 0; i < n_frames; i++) {
@@ -298,7 +298,6 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         single[i].light_chunk_base = 0;
         ChainWork& wf = b->w_frame[i];
         wf = b->w;
-        wf.slice_thr = b->w.slice_thr + (size_t)i * VREN_SLICE_TABLE;
         wf.tile_frame = nullptr;
         wf.total_tiles = single[i].Sx * single[i].Sy;
         wf.total_leaf_slots = b->leaf_slots[i];
@@ -319,9 +318,8 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         st = vren_fail(ctx, VREN_EHIP, "batch: second stream or its events could not be created");
     if (!st) st = vren_upload_frames(ctx, s, b->d_table, b->host.data(), n_frames);
     if (!st) st = vren_upload_frames(ctx, s, b->d_single, single.data(), n_frames);
-    // what depends on the frames' descriptions alone is written once, and every run of the chain skips it: the
-    // depth-slice tables and the BVH leaf groups past each frame's last light
-    if (!st) st = launch_slice_tables(ctx, s, b->d_table, n_frames, b->w);
+    // what depends on the frames' descriptions alone is written once, and every run of the chain skips it: the BVH leaf
+    // groups past each frame's last light
     if (!st && leaf_base) st = launch_bvh(ctx, s, b->d_table, n_frames, leaf_base, true, nullptr, kLeavesPadding);
     if (!st && hipStreamSynchronize(s) != hipSuccess) st = vren_fail(ctx, VREN_EHIP, "batch: upload failed");
     if (st) {

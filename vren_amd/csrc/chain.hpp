@@ -23,7 +23,6 @@ FrameDev* vren_next_frame_slot(vren_ctx* ctx);
 struct ChainWork {
     uint64_t* tile_status; // cluster compaction: one word per group of VREN_TILE_GROUP tiles of every frame
     uint32_t* tickets;     // [0] cluster tile groups
-    float* slice_thr;      // depth-slice threshold table of every frame (VREN_SLICE_TABLE floats each)
     uint2* tile_cl;        // per 32x32 tile: (first cluster index, cluster count), written by the clusters kernel
     uint2* tile_range;     // per 32x32 tile: [begin, end) of the index-buffer entries of its clusters' light lists
     const uint32_t* tile_frame; // frame of every flattened 32x32 tile (null for a one-frame table)
@@ -52,23 +51,16 @@ inline void chain_mark(const ChainWork& w, hipStream_t s)
 // kernels of one chain launch, in order (chain_mark follows each)
 #define VREN_CHAIN_KERNELS 9
 
-// floats per frame of the depth-slice threshold table (clusters.hip)
-#define VREN_SLICE_TABLE 1024u
-
-// workspace: 256 bytes of tickets, the look-back statuses, the per-tile cluster spans and list ranges, then
-// (256-aligned) the slice tables of table_frames frames. The tickets and statuses (the first chain_work_clear_bytes)
-// are zero between runs of a chain: the light-count kernel, which follows their last use, clears them.
+// workspace: 256 bytes of tickets, the look-back statuses, the per-tile cluster spans and list ranges. The tickets and
+// statuses (the first chain_work_clear_bytes) are zero between runs of a chain: the light-count kernel, which follows
+// their last use, clears them.
 inline size_t chain_work_clear_bytes(uint32_t total_tiles)
 {
     return 256 + ((size_t)total_tiles + VREN_TILE_GROUP - 1) / VREN_TILE_GROUP * sizeof(uint64_t);
 }
-inline size_t chain_work_table_offset(uint32_t total_tiles)
+inline size_t chain_work_bytes(uint32_t total_tiles)
 {
-    return (chain_work_clear_bytes(total_tiles) + (size_t)total_tiles * 16 + 255) & ~(size_t)255;
-}
-inline size_t chain_work_bytes(uint32_t total_tiles, uint32_t table_frames)
-{
-    return chain_work_table_offset(total_tiles) + (size_t)table_frames * VREN_SLICE_TABLE * 4;
+    return chain_work_clear_bytes(total_tiles) + (size_t)total_tiles * 16;
 }
 void chain_work_bind(ChainWork* w, void* mem, uint32_t total_tiles);
 
@@ -87,7 +79,6 @@ int launch_front(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_
 enum : uint32_t { kLeavesAll = 0, kLeavesLive = 1, kLeavesPadding = 2 };
 int launch_bvh(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, uint32_t total_leaf_slots,
                bool leaves_from_lights, const ChainWork* w, uint32_t span);
-int launch_slice_tables(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w);
 int launch_clusters(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
                     const FrameDev* one = nullptr);
 int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,

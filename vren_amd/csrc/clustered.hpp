@@ -40,6 +40,10 @@ struct FrameDev {
     float slice_a;          // 2 tan(fov/2) / Sy + 1
     float log_a;            // vren_logf(slice_a)
     float log_fn;           // vren_logf(far / near)
+    float slice_c1, slice_c0; // a view depth's slice is about log2(z) slice_c1 + slice_c0 (clusters_device.hpp)
+    float slice_reach;        // for |log2(z)| up to this
+    float slice_safe;         // and is that value's floor if it is nearer than this to the middle between two whole ones
+    float slice_max;          // values above this are in the last slice (sliced mode)
     float bg_threshold;     // far - 0.001
     // configuration
     uint32_t key_mode, depth_slices, aabb_mode, morton_bits, morton_aabb_mode, attenuation;

@@ -17,82 +17,26 @@
 
 namespace {
 
-// thr[k] = the smallest positive float z with slice_exact(z) >= k, for k = 1 .. kt (+inf when no finite z reaches
-// k), thr[0] = 0. slice_exact is non-decreasing in z: z / near and the division by log_a (or log_fn) are correctly
-// rounded divisions by positive constants, floor and f2u_sat are monotone, and vren_logf is non-decreasing over
-// every non-negative float (checked exhaustively by the oracle tests). So for 0 < z < thr[kt],
-// slice_exact(z) = #{k in 1 .. kt - 1 : thr[k] <= z}, and positive floats order like their bit patterns, so each
-// threshold is a search over bits (slice_exact(+inf) >= kt in both modes). The search is a chain of dependent
-// divisions and logarithms, so each step takes three points at once (their chains overlap) and keeps a quarter.
-__device__ __forceinline__ float slice_threshold(const FrameDev& fd, uint32_t k)
-{
-    if (k == 0) return 0.0f;
-    // between lo (slice < k) and hi (slice >= k), which start +-1e-5 around the real threshold near * exp(k log_a) (log
-    // mode) or near * exp(k log_fn / S) (sliced), in double: the float formula moves it by under 3e-6 at 1023 slices
-    // of a 1080p frame. Where that bracket does not hold, they start at (0, +inf].
-    const double e = fd.key_mode == VREN_KEYS_SLICED ? (double)k * (double)fd.log_fn / (double)fd.depth_slices
-                                                     : (double)k * (double)fd.log_a;
-    const double zk = (double)fd.near_plane * exp(e);
-    uint32_t lo = 0u, hi = 0x7F800000u; // slice_exact(+0) = 0 < k <= slice_exact(+inf)
-    if (zk < 3.0e38) {
-        const uint32_t blo = __float_as_uint((float)(zk * (1.0 - 1e-5)));
-        const uint32_t bhi = __float_as_uint((float)(zk * (1.0 + 1e-5)));
-        const uint32_t klo = slice_exact(fd, __uint_as_float(blo)), khi = slice_exact(fd, __uint_as_float(bhi));
-        if (klo < k && khi >= k) {
-            lo = blo;
-            hi = bhi;
-        }
-    }
-    while (hi - lo > 1u) {
-        const uint32_t quarter = max((hi - lo) / 4u, 1u);
-        const uint32_t m1 = lo + quarter, m2 = min(m1 + quarter, hi), m3 = min(m2 + quarter, hi);
-        const uint32_t k1 = slice_exact(fd, __uint_as_float(m1)), k2 = slice_exact(fd, __uint_as_float(m2));
-        const uint32_t k3 = slice_exact(fd, __uint_as_float(m3));
-        const uint32_t l = lo, h = hi;
-        hi = k1 >= k ? m1 : (k2 >= k ? m2 : (k3 >= k ? m3 : h));
-        lo = k1 >= k ? l : (k2 >= k ? m1 : (k3 >= k ? m2 : m3));
-    }
-    return __uint_as_float(hi);
-}
-
-// The tables of a batch's frames, written once when the batch is created: they depend on its cameras alone.
-__global__ __launch_bounds__(256) void slice_table_kernel(const FrameDev* __restrict__ frames, float* thr_all)
-{
-    const uint32_t f = blockIdx.x / (VREN_SLICE_TABLE / 256), k = blockIdx.x % (VREN_SLICE_TABLE / 256) * 256 + threadIdx.x;
-    const FrameDev& fd = frames[f];
-    if (k <= slice_table_kt(fd)) thr_all[(uint64_t)f * VREN_SLICE_TABLE + k] = slice_threshold(fd, k);
-}
-
-// What a single-frame call needs ahead of its clusters: its table, one wave per 64 thresholds, and cleared statuses and
-// tickets, in one launch.
-__global__ __launch_bounds__(64) void clusters_begin_kernel(const FrameDev one, float* thr, uint32_t* clear,
-                                                            uint32_t clear_words)
-{
-    const FrameDev& fd = *inline_frame();
-    const uint32_t k = blockIdx.x * 64 + threadIdx.x;
-    for (uint32_t i = k; i < clear_words; i += gridDim.x * 64) clear[i] = 0u;
-    if (k <= slice_table_kt(fd)) thr[k] = slice_threshold(fd, k);
-}
-
 __global__ void chain_init_kernel(uint32_t* clear, uint32_t clear_words)
 {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < clear_words; i += gridDim.x * blockDim.x) clear[i] = 0u;
 }
 
-__global__ __launch_bounds__(kClusterWaves * 64, 8) void clusters_kernel(const FrameDev* __restrict__ frames,
-                                                                       const uint32_t* __restrict__ tile_frame,
-                                                                       uint32_t total_tiles, uint64_t* tile_status,
-                                                                       uint32_t* ticket, const float* __restrict__ slice_thr,
-                                                                       uint2* __restrict__ tile_cl)
+template <bool DEEP>
+__global__ __launch_bounds__(kClusterWaves * 64, DEEP ? 2 : 8) void clusters_kernel(
+    const FrameDev* __restrict__ frames, const uint32_t* __restrict__ tile_frame, uint32_t total_tiles,
+    uint64_t* tile_status, uint32_t* ticket, uint2* __restrict__ tile_cl)
 {
-    clusters_body(frames, tile_frame, total_tiles, tile_status, ticket, slice_thr, tile_cl);
+    clusters_body<DEEP>(frames, tile_frame, total_tiles, tile_status, ticket, tile_cl);
 }
-__global__ __launch_bounds__(kClusterWaves * 64, 8) void clusters_one_kernel(const FrameDev one, uint32_t total_tiles,
-                                                                           uint64_t* tile_status, uint32_t* ticket,
-                                                                           const float* __restrict__ slice_thr,
-                                                                           uint2* __restrict__ tile_cl)
+template <bool DEEP>
+__global__ __launch_bounds__(kClusterWaves * 64, DEEP ? 2 : 8) void clusters_one_kernel(const FrameDev one,
+                                                                                       uint32_t total_tiles,
+                                                                                       uint64_t* tile_status,
+                                                                                       uint32_t* ticket,
+                                                                                       uint2* __restrict__ tile_cl)
 {
-    clusters_body(inline_frame(), nullptr, total_tiles, tile_status, ticket, slice_thr, tile_cl);
+    clusters_body<DEEP>(inline_frame(), nullptr, total_tiles, tile_status, ticket, tile_cl);
 }
 
 } // namespace
@@ -103,7 +47,6 @@ void chain_work_bind(ChainWork* w, void* mem, uint32_t total_tiles)
     w->tile_status = reinterpret_cast<uint64_t*>(static_cast<char*>(mem) + 256);
     w->tile_cl = reinterpret_cast<uint2*>(static_cast<char*>(mem) + chain_work_clear_bytes(total_tiles));
     w->tile_range = w->tile_cl + total_tiles;
-    w->slice_thr = reinterpret_cast<float*>(static_cast<char*>(mem) + chain_work_table_offset(total_tiles));
     w->total_tiles = total_tiles;
 }
 
@@ -117,26 +60,21 @@ int launch_chain_init(vren_ctx* ctx, hipStream_t s, const ChainWork& w)
     return VREN_OK;
 }
 
-int launch_slice_tables(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w)
-{
-    slice_table_kernel<<<F * (VREN_SLICE_TABLE / 256), 256, 0, s>>>(d_frames, w.slice_thr);
-    VREN_LAUNCH_CHECK(ctx);
-    return VREN_OK;
-}
-
 int launch_clusters(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
                     const FrameDev* one)
 {
     const uint32_t blocks = (w.total_tiles + kClusterWaves - 1) / kClusterWaves;
+    // one workgroup per CU at most: two waves per SIMD, which have the registers to load a whole tile at once
+    const bool deep = blocks <= (uint32_t)ctx->num_cus;
     if (one) {
-        const uint32_t words = (uint32_t)(chain_work_clear_bytes(w.total_tiles) / 4);
-        clusters_begin_kernel<<<VREN_SLICE_TABLE / 64, 64, 0, s>>>(*one, w.slice_thr, w.tickets, words);
-        VREN_LAUNCH_CHECK(ctx);
-        clusters_one_kernel<<<blocks, kClusterWaves * 64, 0, s>>>(*one, w.total_tiles, w.tile_status, w.tickets + 0,
-                                                                  w.slice_thr, w.tile_cl);
+        const int st = launch_chain_init(ctx, s, w);
+        if (st) return st;
+        const auto kernel = deep ? clusters_one_kernel<true> : clusters_one_kernel<false>;
+        kernel<<<blocks, kClusterWaves * 64, 0, s>>>(*one, w.total_tiles, w.tile_status, w.tickets + 0, w.tile_cl);
     } else {
-        clusters_kernel<<<blocks, kClusterWaves * 64, 0, s>>>(d_frames, F > 1 ? w.tile_frame : nullptr, w.total_tiles,
-                                                              w.tile_status, w.tickets + 0, w.slice_thr, w.tile_cl);
+        const auto kernel = deep ? clusters_kernel<true> : clusters_kernel<false>;
+        kernel<<<blocks, kClusterWaves * 64, 0, s>>>(d_frames, F > 1 ? w.tile_frame : nullptr, w.total_tiles, w.tile_status,
+                                                     w.tickets + 0, w.tile_cl);
     }
     VREN_LAUNCH_CHECK(ctx);
     chain_mark(w, s);
@@ -173,7 +111,7 @@ extern "C" VREN_EXPORT int vren_find_unique_cluster_list(vren_ctx* ctx, vren_str
     ChainWork w;
     memset(&w, 0, sizeof(w));
     uint32_t tiles = f.Sx * f.Sy;
-    st = vren_ensure_scratch(ctx, chain_work_bytes(tiles, 1), s);
+    st = vren_ensure_scratch(ctx, chain_work_bytes(tiles), s);
     if (st) return st;
     chain_work_bind(&w, ctx->scratch, tiles);
     return launch_clusters(ctx, s, nullptr, 1, w, &f);

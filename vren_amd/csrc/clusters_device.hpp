@@ -66,6 +66,49 @@ __device__ __forceinline__ uint32_t face_of_normal(const float n[3])
     return ax < 3 ? (n[ax] > 0.0f ? 1u : 0u) * 3u + ax : 0u;
 }
 
+// f16 -> f32 on the conversion unit. A key depends on a NaN component only through comparisons and through
+// f2u_sat(floor(NaN)) = 0, never on its payload, so the conversion's NaN payload need not be the oracle's.
+__device__ __forceinline__ float key_h2f(uint32_t h)
+{
+    const uint16_t b = (uint16_t)h;
+    _Float16 x;
+    __builtin_memcpy(&x, &b, 2);
+    return (float)x;
+}
+
+// the conversion as the hardware does it: a negative value and a NaN give 0
+__device__ __forceinline__ uint32_t cvt_u32(float x)
+{
+    uint32_t r;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+
+// The code of a normal (the face alone in sliced mode) without branches: right where the function returns true, for a zero
+// normal (the background of a cleared G-buffer) and wherever the largest magnitude is positive and finite; not for
+// infinities and for zeros with NaNs. The maximum drops NaNs, and no NaN equals it. The cell of u in [-1, 1] is
+// the truncation of 1.5 (u + 1), the reference's (u + 1) / 2 * 3 with its exact halving folded in.
+__device__ __forceinline__ bool normal_code(bool sliced, uint2 nb, uint32_t* code)
+{
+    const float n0 = key_h2f(nb.x & 0xFFFFu), n1 = key_h2f(nb.x >> 16), n2 = key_h2f(nb.y & 0xFFFFu);
+    const bool zero = ((nb.x & 0x7FFF7FFFu) | (nb.y & 0x7FFFu)) == 0u;
+    const float m = fmaxf(fmaxf(fabsf(n0), fabsf(n1)), fabsf(n2));
+    const bool x = fabsf(n0) == m, y = fabsf(n1) == m;
+    float d = y ? n1 : n2;
+    d = x ? n0 : d;
+    if (sliced) {
+        *code = zero ? 7u : (x ? 0u : (y ? 1u : 2u)) + (d > 0.0f ? 3u : 0u);
+    } else {
+        const float rcp = __builtin_amdgcn_rcpf(m), t = __builtin_fmaf(rcp, __builtin_fmaf(-m, rcp, 1.0f), rcp);
+        float u = y ? n2 : n0, v = y ? n0 : n1;
+        u = x ? n1 : u;
+        v = x ? n2 : v;
+        const uint32_t du = cvt_u32((u * t + 1.0f) * 1.5f), dv = cvt_u32((v * t + 1.0f) * 1.5f);
+        *code = zero ? 0x3Fu : (x ? 0u : (y ? 9u : 18u)) + (d > 0.0f ? 27u : 0u) + (du * 3u + dv);
+    }
+    return zero || __builtin_amdgcn_classf(m, 0x100); // a positive normal number
+}
+
 // The depth slice of a view depth z by the reference's formula (find_unique_clusters.comp:58-62): log mode
 // f2u_sat(floor(log(z / near) / log_a)) before the 10-bit mask, sliced mode the same over [near, far] in
 // depth_slices steps, clamped to the last slice. A non-positive or NaN z gives 0 (log of a non-positive ratio is
@@ -79,75 +122,82 @@ __device__ __forceinline__ uint32_t slice_exact(const FrameDev& fd, float z)
     return vren_f2u_sat(vren_floorf(vren_logf(z / fd.near_plane) / fd.log_a));
 }
 
-// Slices kept in the threshold table (thr[1 .. kt - 1] are looked up; z >= thr[kt] takes the formula): every
-// sliced-mode slice, log-mode slices below 1023 (the key keeps k & 0x3FF, so k >= 1023 goes through the formula)
-__device__ __forceinline__ uint32_t slice_table_kt(const FrameDev& fd)
+// A pixel's view depth (find_unique_clusters.comp:48-56) as the numerator r[0] and the denominator r[1] of the division
+// that gives it.
+__device__ __forceinline__ void pixel_view_zw(const FrameDev& fd, uint32_t gx, uint32_t gy, float depth, float r[2])
 {
-    return fd.key_mode == VREN_KEYS_SLICED ? fd.depth_slices - 1 : 1023u;
-}
-
-// view depth of a pixel (find_unique_clusters.comp:48-56)
-__device__ __forceinline__ float pixel_view_z(const FrameDev& fd, uint32_t gx, uint32_t gy, float depth)
-{
-    float r2, r3;
     if (fd.proj_zw_xy_zero) {
         // the z and w rows of inverse(P) have zero x and y coefficients: ((0 x + 0 y) + m2 depth) + m3 reduces to
         // m2 depth + m3 exactly (a zero result may only change sign, and z = 0 gives the same slice either way)
-        r2 = fd.inv_proj[2 * 4 + 2] * depth + fd.inv_proj[3 * 4 + 2];
-        r3 = fd.inv_proj[2 * 4 + 3] * depth + fd.inv_proj[3 * 4 + 3];
+        r[0] = fd.inv_proj[2 * 4 + 2] * depth + fd.inv_proj[3 * 4 + 2];
+        r[1] = fd.inv_proj[2 * 4 + 3] * depth + fd.inv_proj[3 * 4 + 3];
     } else {
         float v[4] = {(float)gx / (float)fd.W, (float)gy / (float)fd.H, depth, 1.0f};
         v[1] = 1.0f - v[1];
         v[0] = v[0] * 2.0f - 1.0f;
         v[1] = v[1] * 2.0f - 1.0f;
-        float r[4];
-        vren_mat4_mul_vec4(fd.inv_proj, v, r);
-        r2 = r[2];
-        r3 = r[3];
+        float o[4];
+        vren_mat4_mul_vec4(fd.inv_proj, v, o);
+        r[0] = o[2];
+        r[1] = o[3];
     }
-    return r2 / r3;
 }
 
-// the cluster key from its slice and normal (find_unique_clusters.comp:58-65)
-// f16 -> f32 on the conversion unit. A key depends on a NaN component only through comparisons and through
-// f2u_sat(floor(NaN)) = 0, never on its payload, so the conversion's NaN payload need not be the oracle's.
-__device__ __forceinline__ float key_h2f(uint32_t h)
+// The slice of nearly every pixel without a division, a logarithm's polynomial or a table: the floor of
+// log2(z) slice_c1 + slice_c0 with the hardware's reciprocal and logarithm, certain where that value is farther from a
+// whole number than the two formulas can lie apart and z is not far outside the planes (FrameDev's slice_*). What is not
+// certain (a few pixels in ten thousand, and any depth whose z is not a positive number) takes slice_exact.
+// Values below 0.5 are in slice 0, with everything in front of the near plane. With the branch-free normal code and the rows'
+// wide loads the cluster stage of 64 1920x1080 frames went from 580 us (an IEEE division, a search in a table of
+// thresholds in LDS and a branch per case of the normal) to 516, 16 frames with sliced keys from 218 to 139 (their
+// background, at the end of the last slice, took the formula), a 1366x769 frame from 23 and 8 for its table to 17.
+// What is left is mostly memory: 2.1 GB for the 64 frames, 452 us at the rate of a large copy.
+__device__ __forceinline__ bool slice_estimate(const FrameDev& fd, const float zw[2], uint32_t* k)
 {
-    const uint16_t b = (uint16_t)h;
-    _Float16 x;
-    __builtin_memcpy(&x, &b, 2);
-    return (float)x;
+    const float lg = __builtin_amdgcn_logf(zw[0] * __builtin_amdgcn_rcpf(zw[1]));
+    const float e = __builtin_amdgcn_fmed3f(__builtin_fmaf(lg, fd.slice_c1, fd.slice_c0), 0.5f, fd.slice_max);
+    *k = (uint32_t)e;
+    return fabsf(lg) <= fd.slice_reach && fabsf(__builtin_amdgcn_fractf(e) - 0.5f) < fd.slice_safe;
 }
 
-__device__ __forceinline__ uint32_t assemble_key(const FrameDev& fd, uint32_t ti, uint32_t tj, uint32_t k, uint2 nb)
+// the high half of a cluster key, from its slice and normal (find_unique_clusters.comp:58-65); the low half are the
+// tile's ids
+__device__ __forceinline__ uint32_t key_high(const FrameDev& fd, uint32_t k, uint32_t code)
 {
-    const float n[3] = {key_h2f(nb.x & 0xFFFFu), key_h2f(nb.x >> 16), key_h2f(nb.y & 0xFFFFu)};
-    if (fd.key_mode == VREN_KEYS_SLICED)
-        return (ti & 0xFFu) | ((tj & 0xFFu) << 8) | ((k & 0xFFu) << 16) | (face_of_normal(n) << 24);
-    return (ti & 0xFFu) | ((tj & 0xFFu) << 8) | ((k & 0x3FFu) << 16) | (discretize_normal(n) << 26);
+    return fd.key_mode == VREN_KEYS_SLICED ? (k & 0xFFu) | (code << 8) : (k & 0x3FFu) | (code << 10);
 }
 
 constexpr uint32_t kClusterWaves = 8;   // waves per workgroup, one 32x32 tile per wave (16 measured slower)
 
-// The depths and normals of lane `lane` of a tile's rows 2 h and 2 h + 1 (pixels i = 4 j + q with j = 2 h + jj,
-// stored at [4 jj + q]): pixel (x0 + q, tj * 32 + 8 j + lane / 8). A tile inside the frame with 16-byte aligned
-// rows (uniform across the wave) takes one 16-byte depth load and two 16-byte normal loads per row; other tiles
-// load per pixel, wrapping (x mod W, y mod H) like the reference's REPEAT sampler. Every load of the half is issued
-// before any is used; a tile's two halves are loaded one after the other, which keeps the register peak of a wave
-// below 64 (eight waves per SIMD).
-__device__ __forceinline__ void load_tile_half(const FrameDev& fd, uint32_t ti, uint32_t tj, uint32_t lane, uint32_t h,
-                                               float dep[8], uint2 nrm[8])
+// 16 bytes at a 4-byte boundary: one load or store, whatever the row's alignment
+typedef float vf4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t vu4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef const __attribute__((address_space(1))) vf4_a4 gvf4_a4;
+typedef const __attribute__((address_space(1))) vu4_a4 gvu4_a4;
+
+// the reference's REPEAT sampler: (x mod W, y mod H)
+__device__ __forceinline__ void wrap_pixel(const FrameDev& fd, uint32_t& x, uint32_t& y)
+{
+    if (x >= fd.W) x %= fd.W;
+    if (y >= fd.H) y %= fd.H;
+}
+
+// The depths and normals of lane `lane` of N / 4 of a tile's four 8-row groups, from group j0 on (pixels i = 4 j + q, stored
+// at [4 (j - j0) + q]): pixel (x0 + q, tj * 32 + 8 j + lane / 8). A tile inside the frame (uniform across the wave) takes
+// one 16-byte depth load and two 16-byte normal loads per row; other tiles load per pixel, wrapped. Every load is issued
+// before any is used.
+template <int N>
+__device__ __forceinline__ void load_tile(const FrameDev& fd, uint32_t ti, uint32_t tj, uint32_t lane, uint32_t j0,
+                                          float dep[N], uint2 nrm[N])
 {
     const uint32_t x0 = ti * 32 + (lane & 7) * 4;
-    const bool interior = (ti + 1) * 32 <= fd.W && (tj + 1) * 32 <= fd.H && (fd.W & 3) == 0 &&
-                          ((reinterpret_cast<uintptr_t>(fd.depth) | reinterpret_cast<uintptr_t>(fd.normals)) & 15) == 0;
-    if (interior) {
+    if ((ti + 1) * 32 <= fd.W && (tj + 1) * 32 <= fd.H) {
 #pragma unroll
-        for (int jj = 0; jj < 2; jj++) {
-            const uint64_t p0 = (uint64_t)(tj * 32 + (2 * h + jj) * 8 + (lane >> 3)) * fd.W + x0;
-            const vf4 d4 = *(gvf4*)(fd.depth + p0);
-            const vu4 n01 = *(gvu4*)(fd.normals + 4 * p0);
-            const vu4 n23 = *(gvu4*)(fd.normals + 4 * p0 + 8);
+        for (int jj = 0; jj < N / 4; jj++) {
+            const uint64_t p0 = (uint64_t)(tj * 32 + (j0 + jj) * 8 + (lane >> 3)) * fd.W + x0;
+            const vf4_a4 d4 = *(gvf4_a4*)(fd.depth + p0);
+            const vu4_a4 n01 = *(gvu4_a4*)(fd.normals + 4 * p0);
+            const vu4_a4 n23 = *(gvu4_a4*)(fd.normals + 4 * p0 + 8);
             dep[4 * jj + 0] = d4.x;
             dep[4 * jj + 1] = d4.y;
             dep[4 * jj + 2] = d4.z;
@@ -159,9 +209,10 @@ __device__ __forceinline__ void load_tile_half(const FrameDev& fd, uint32_t ti, 
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const uint32_t x = x0 + (i & 3), y = tj * 32 + (2 * h + (i >> 2)) * 8 + (lane >> 3);
-            const uint64_t p = (uint64_t)(y % fd.H) * fd.W + (x % fd.W);
+        for (int i = 0; i < N; i++) {
+            uint32_t x = x0 + (i & 3), y = tj * 32 + (j0 + (i >> 2)) * 8 + (lane >> 3);
+            wrap_pixel(fd, x, y);
+            const uint64_t p = (uint64_t)y * fd.W + x;
             dep[i] = *(gfloat*)(fd.depth + p);
             const vu2 n = *(gvu2*)(fd.normals + 4 * p);
             nrm[i] = make_uint2(n.x, n.y);
@@ -176,15 +227,15 @@ __device__ __forceinline__ void load_tile_half(const FrameDev& fd, uint32_t ti, 
 // look-back per workgroup (per tile, the walk's round trips of ~1.4 us covered 64 tiles each and could not keep up
 // with the tiles finishing). The walk waits only on groups of lower tickets, whose workgroups are already running,
 // so every wait ends. Lane l owns the pixels (4 (l % 8) + q, 8 j + l / 8), q, j = 0..3, of its tile.
+// DEEP: a tile's loads are all in flight at once (48 registers of them); otherwise its two halves are loaded one after
+// the other, which keeps the register peak of a wave below 64 (eight waves per SIMD).
+template <bool DEEP>
 __device__ __forceinline__ void clusters_body(const FrameDev* __restrict__ frames,
                                               const uint32_t* __restrict__ tile_frame, uint32_t total_tiles,
-                                              uint64_t* tile_status, uint32_t* ticket,
-                                              const float* __restrict__ slice_thr, uint2* __restrict__ tile_cl)
+                                              uint64_t* tile_status, uint32_t* ticket, uint2* __restrict__ tile_cl)
 {
     static_assert(kClusterWaves == VREN_TILE_GROUP, "one workgroup per tile group");
-    static_assert(VREN_SLICE_TABLE == 2 * kClusterWaves * 64, "two table entries per thread");
     __shared__ uint32_t s_unique[kClusterWaves][1024];
-    __shared__ float s_thr[VREN_SLICE_TABLE];
     __shared__ uint32_t s_u[kClusterWaves];
     __shared__ uint32_t s_t, s_prefix;
     const uint32_t lane = lane_id();
@@ -193,19 +244,8 @@ __device__ __forceinline__ void clusters_body(const FrameDev* __restrict__ frame
     __syncthreads();
     const uint32_t g0 = s_t * kClusterWaves;
     if (g0 >= total_tiles) return; // the whole workgroup
-    // a workgroup's tiles are one group of its frame (frame tile ranges start at multiples of VREN_TILE_GROUP), so
-    // one slice table serves them all
+    // a workgroup's tiles are one group of its frame (frame tile ranges start at multiples of VREN_TILE_GROUP)
     const FrameDev& fd = frames[frame_of_tile(tile_frame, g0)];
-    const uint32_t kt = slice_table_kt(fd);
-    {
-        // both halves of the table are requested before either is stored
-        const uint32_t i0 = threadIdx.x, i1 = threadIdx.x + kClusterWaves * 64;
-        const float* tb = slice_thr + (uint64_t)frame_of_tile(tile_frame, g0) * VREN_SLICE_TABLE;
-        const float a0 = i0 <= kt ? tb[i0] : 0.0f, a1 = i1 <= kt ? tb[i1] : 0.0f;
-        s_thr[i0] = a0;
-        s_thr[i1] = a1;
-    }
-    __syncthreads();
     uint32_t* uq = s_unique[wave];
     const uint32_t g = g0 + wave;
     const uint32_t t0 = g0 - fd.tile_base; // the group's first tile in its frame
@@ -217,67 +257,54 @@ __device__ __forceinline__ void clusters_body(const FrameDev* __restrict__ frame
     uint32_t key[16];
     uint32_t u = 0;
     if (live) {
-        const float* thr = s_thr;
-        const float thr_kt = thr[kt];
-        // slice estimate t = log2(z) c1 + c0 ~ ln(z / near) / log_a (log mode) or ln(z / near) S / log_fn (sliced):
-        // its error is orders of magnitude below one slice, so the slice is the estimate's floor k0 moved by at
-        // most one, decided by thr[k0] and thr[k0 + 1]; thr[k0 - 1] and thr[k0 + 2] confirm the move, and a pixel
-        // whose confirmation fails (or beyond the table) takes the formula
-        const float c1 = fd.key_mode == VREN_KEYS_SLICED ? 0.69314718f * (float)fd.depth_slices / fd.log_fn
-                                                          : 0.69314718f / fd.log_a;
-        const float c0 = -__builtin_amdgcn_logf(fd.near_plane) * c1;
-        const float emax = (float)(kt > 0u ? kt - 1u : 0u); // k0 <= kt - 1, so every index below is <= kt
+        constexpr int N = DEEP ? 16 : 8;
+        const bool sliced = fd.key_mode == VREN_KEYS_SLICED;
         uint32_t pend = 0u;
 #pragma unroll
-        for (uint32_t h = 0; h < 2; h++) {
-        float dep[8];
-        uint2 nrm[8];
-        load_tile_half(fd, ti, tj, lane, h, dep, nrm);
+        for (uint32_t h = 0; h < 16 / N; h++) {
+            float dep[N];
+            uint2 nrm[N];
+            load_tile<N>(fd, ti, tj, lane, h * (N / 4), dep, nrm);
 #pragma unroll
-        for (int jj = 0; jj < 2; jj++) {
-            const int j = 2 * h + jj;
-            const uint32_t y = tj * 32 + j * 8 + (lane >> 3);
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int i = 4 * j + q;
-                const float z = pixel_view_z(fd, x0 + q, y, dep[4 * jj + q]);
-                uint32_t k = 0u;
-                if (z > 0.0f) {
-                    const float e = fminf(fmaxf(__builtin_amdgcn_logf(z) * c1 + c0, 0.0f), emax);
-                    const uint32_t k0 = (uint32_t)e;
-                    const float vm = thr[k0 > 0u ? k0 - 1u : 0u], v0 = thr[k0], v1 = thr[k0 + 1u];
-                    const float v2 = thr[min(k0 + 2u, kt)];
-                    const bool dn = z < v0, up = z >= v1;
-                    k = k0 - (dn ? 1u : 0u) + (up ? 1u : 0u);
-                    const bool bad = !(z < thr_kt) || (dn && (k0 == 0u || z < vm)) || (up && z >= v2);
-                    if (bad) pend |= 1u << i;
-                }
-                key[i] = assemble_key(fd, ti, tj, k, nrm[4 * jj + q]);
+            for (int r = 0; r < N; r++) {
+                const int i = N * h + r;
+                float zw[2];
+                uint32_t k, code;
+                pixel_view_zw(fd, x0 + (i & 3), tj * 32 + (i >> 2) * 8 + (lane >> 3), dep[r], zw);
+                const bool slice_ok = slice_estimate(fd, zw, &k), code_ok = normal_code(sliced, nrm[r], &code);
+                key[i] = key_high(fd, k, code);
+                pend |= slice_ok && code_ok ? 0u : 1u << i;
+                // a pixel's key and flag are finished before the next pixel's: their temporaries together would not fit
+                asm volatile("" : "+v"(key[i]), "+v"(pend));
             }
+            // the second half's loads stay after the first half's keys (the register peak of one half)
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("" ::: "memory");
         }
-        // the second half's loads stay after the first half's keys (the register peak of one half)
-        __builtin_amdgcn_sched_barrier(0);
-        asm volatile("" ::: "memory");
-        }
-        // the formula for the flagged pixels, their depth and normal read again (rare: beyond the table)
-        if (pend) {
+        // the other pixels by the reference's formulas, one of each lane at a time, read again
+        while (ballot(pend != 0u)) {
+            if (pend) {
+                const uint32_t i = (uint32_t)__builtin_ctz(pend);
+                const uint32_t x = x0 + (i & 3), y = tj * 32 + (i >> 2) * 8 + (lane >> 3);
+                uint32_t wx = x, wy = y;
+                wrap_pixel(fd, wx, wy);
+                const uint64_t p = (uint64_t)wy * fd.W + wx;
+                float zw[2];
+                pixel_view_zw(fd, x, y, *((gfloat*)fd.depth + p), zw);
+                const vu2 nb = *(gvu2*)(fd.normals + 4 * p);
+                const float n[3] = {key_h2f(nb.x & 0xFFFFu), key_h2f(nb.x >> 16), key_h2f(nb.y & 0xFFFFu)};
+                const uint32_t code = sliced ? face_of_normal(n) : discretize_normal(n) & 0x3Fu;
+                const uint32_t exact = key_high(fd, slice_exact(fd, zw[0] / zw[1]), code);
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                if ((pend >> i) & 1u) {
-                    const uint32_t x = x0 + (i & 3), y = tj * 32 + (i >> 2) * 8 + (lane >> 3);
-                    const uint64_t p = (uint64_t)(y % fd.H) * fd.W + (x % fd.W);
-                    const float z = pixel_view_z(fd, x, y, fd.depth[p]);
-                    key[i] = assemble_key(fd, ti, tj, slice_exact(fd, z), reinterpret_cast<const uint2*>(fd.normals)[p]);
-                }
+                for (uint32_t q = 0; q < 16; q++) key[q] = q == i ? exact : key[q];
+                pend &= pend - 1u;
             }
         }
         // the tile's unique keys in ascending order, by repeated wave minima (one round per distinct key). Every
         // key of the tile has the tile's ids in its low 16 bits, so the keys compare by their high halves; a
         // pixel whose key has been emitted takes 0x10000 + the key's index in the list, above every high half
         // still pending, and keeps it as its index (no search afterwards)
-        const uint32_t low = key[0] & 0xFFFFu;
-#pragma unroll
-        for (int q = 0; q < 16; q++) key[q] >>= 16;
+        const uint32_t low = (ti & 0xFFu) | ((tj & 0xFFu) << 8);
         for (;;) {
             uint32_t mine = key[0];
 #pragma unroll
@@ -328,8 +355,8 @@ __device__ __forceinline__ void clusters_body(const FrameDev* __restrict__ frame
 #pragma unroll
         for (int q = 0; q < 4; q++) ref[q] = (prefix - 0x10000u) + key[4 * j + q]; // key = 0x10000 + index
         uint32_t* row = fd.refs + (uint64_t)y * fd.W;
-        if (x0 + 3 < fd.W && ((reinterpret_cast<uintptr_t>(row + x0) & 15) == 0)) {
-            *reinterpret_cast<uint4*>(row + x0) = make_uint4(ref[0], ref[1], ref[2], ref[3]);
+        if (x0 + 3 < fd.W) {
+            *reinterpret_cast<vu4_a4*>(row + x0) = vu4_a4{ref[0], ref[1], ref[2], ref[3]};
         } else {
 #pragma unroll
             for (int q = 0; q < 4; q++)

@@ -85,6 +85,21 @@ void vren_frame_setup(FrameDev* f, uint32_t W, uint32_t H, const vren_camera* ca
     f->slice_a = (2.0f * tan_half) / (float)f->Sy + 1.0f;
     f->log_a = vren_logf(1.0f + (2.0f * tan_half) / (float)f->Sy);
     f->log_fn = vren_logf(cam->far_plane / cam->near_plane);
+    {
+        // The cluster stage's estimate of a depth slice (clusters_device.hpp), s slices per unit of ln z. The float formula and
+        // the estimate lie within s (4e-7 + 1.2e-6 g) of each other for |log2 z| <= g, |log2 near| <= g: the roundings of
+        // z / near and of the estimate's z (under 2.5e-7 together), two ulp of vren_logf, one of the hardware's log2
+        // and the roundings of the products, all relative to values up to 2 g ln 2. slice_safe takes 1.4 times that.
+        const bool sliced = cfg->key_mode == VREN_KEYS_SLICED;
+        const double s = sliced ? (double)cfg->depth_slices / (double)f->log_fn : 1.0 / (double)f->log_a;
+        const double ln = std::log2((double)cam->near_plane), lf = std::log2((double)cam->far_plane);
+        const double g = std::max(std::fabs(ln), std::fabs(lf)) + 0.05;
+        f->slice_c1 = (float)(0.69314718055994531 * s);
+        f->slice_c0 = (float)(-ln * 0.69314718055994531 * s);
+        f->slice_reach = (float)g;
+        f->slice_safe = (float)(0.5 - s * (5.6e-7 + 1.7e-6 * g));
+        f->slice_max = sliced ? (float)cfg->depth_slices - 0.5f : 1e9f;
+    }
     f->bg_threshold = cam->far_plane - 0.001f;
     f->key_mode = cfg->key_mode;
     f->depth_slices = cfg->depth_slices;

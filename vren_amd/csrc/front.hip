@@ -1,8 +1,8 @@
 // front.hip -- the chain's two independent first stages in one launch, for tables that leave the chip mostly idle: the
 // workgroups of the light stage (a chunk of lights each) and those of the cluster stage (eight tiles each) side by side.
-// One after the other, a frame waits for one CU to sort its lights while the others have nothing to do: 21 us, as long
-// as the cluster stage of a 1920x1080 frame. Together they take 22.8 us there (44 before), and 17.9 on a 640x360 frame
-// with 256 lights (25).
+// One after the other, a frame waits for one CU to sort its lights while the others have nothing to do: 21 us for 4096.
+// Together the stages of a 1920x1080 frame take 22.9 us (44 one after the other), now bound by the lights, and those
+// of a 640x360 frame with 256 lights 13.1 (25).
 #include "clusters_device.hpp"
 #include "lights_device.hpp"
 
@@ -14,13 +14,13 @@ template <int BITS>
 __global__ __launch_bounds__(kLT) void front_kernel(const FrameDev* __restrict__ frames, uint32_t F, uint32_t chunks,
                                                     const uint32_t* __restrict__ tile_frame, uint32_t total_tiles,
                                                     uint64_t* tile_status, uint32_t* ticket,
-                                                    const float* __restrict__ slice_thr, uint2* __restrict__ tile_cl)
+                                                    uint2* __restrict__ tile_cl)
 {
     if (blockIdx.x < chunks) {
         lights_body<BITS>(frames, F, chunks);
     } else {
         if (threadIdx.x >= kClusterWaves * VREN_WAVE) return;
-        clusters_body(frames, tile_frame, total_tiles, tile_status, ticket, slice_thr, tile_cl);
+        clusters_body<true>(frames, tile_frame, total_tiles, tile_status, ticket, tile_cl);
     }
 }
 
@@ -40,10 +40,10 @@ int launch_front(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_
     const uint32_t* tf = F > 1 ? w.tile_frame : nullptr;
     if (w.light_bits == 4)
         front_kernel<4><<<grid, kLT, 0, s>>>(d_frames, F, w.light_chunks, tf, w.total_tiles, w.tile_status, w.tickets + 0,
-                                             w.slice_thr, w.tile_cl);
+                                             w.tile_cl);
     else
         front_kernel<8><<<grid, kLT, 0, s>>>(d_frames, F, w.light_chunks, tf, w.total_tiles, w.tile_status, w.tickets + 0,
-                                             w.slice_thr, w.tile_cl);
+                                             w.tile_cl);
     VREN_LAUNCH_CHECK(ctx);
     return VREN_OK;
 }
