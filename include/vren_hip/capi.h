@@ -264,6 +264,14 @@ VREN_EXPORT int vren_shade(vren_ctx* ctx, vren_stream_t stream, uint32_t width, 
                            const uint32_t* light_offsets, const uint32_t* light_indices, uint32_t index_capacity,
                            const float* light_positions, const float* point_lights, uint32_t light_count,
                            const float* directional_lights, uint32_t directional_light_count, float* output);
+/* the same into a buffer whose contents do not matter: background pixels are written as zeros instead of left alone */
+VREN_EXPORT int vren_shade_fresh(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
+                           const vren_camera* camera, const vren_cluster_cfg* cfg, const float* depth,
+                           const uint16_t* normals, const float* albedo_roughness, const float* metallic,
+                           const uint32_t* cluster_refs, uint32_t key_capacity, const uint32_t* light_counts,
+                           const uint32_t* light_offsets, const uint32_t* light_indices, uint32_t index_capacity,
+                           const float* light_positions, const float* point_lights, uint32_t light_count,
+                           const float* directional_lights, uint32_t directional_light_count, float* output);
 
 /* ---- material resolve (shade.comp:89-96) ---------------------------------------------------------------------
  * The reference's G-buffer carries a texcoord (RG32F) and a material index (R16_UINT) per pixel (gbuffer.cpp:14-27);
@@ -329,6 +337,15 @@ VREN_EXPORT int vren_shade_materials(vren_ctx* ctx, vren_stream_t stream, uint32
  * The gradient buffers must be zeroed by the caller before the first accumulation. Use VREN_ATTEN_SMOOTH: the
  * reference attenuation has a kink at d = r. */
 VREN_EXPORT int vren_shade_backward(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
+                                    const vren_camera* camera, const vren_cluster_cfg* cfg, const float* depth,
+                                    const uint16_t* normals, const float* albedo_roughness, const float* metallic,
+                                    const uint32_t* cluster_refs, uint32_t key_capacity, const uint32_t* light_counts,
+                                    const uint32_t* light_offsets, const uint32_t* light_indices,
+                                    uint32_t index_capacity, const float* light_positions, const float* point_lights,
+                                    uint32_t light_count, const float* grad_output, float* grad_light_positions,
+                                    float* grad_point_lights, float* grad_albedo_roughness);
+/* the same with the gradients written (zeros where nothing contributes) instead of added to */
+VREN_EXPORT int vren_shade_backward_fresh(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
                                     const vren_camera* camera, const vren_cluster_cfg* cfg, const float* depth,
                                     const uint16_t* normals, const float* albedo_roughness, const float* metallic,
                                     const uint32_t* cluster_refs, uint32_t key_capacity, const uint32_t* light_counts,

@@ -166,15 +166,17 @@ class Context:
             _ptr(total)))
 
     def shade(self, W, H, cam, cfg, depth, normals, albedo_rough, metallic, refs, key_cap, counts, offsets, indices,
-              index_cap, light_pos, lights, L, out, dir_lights=None, n_dir=0):
-        return self.check(self.lib.vren_shade(
+              index_cap, light_pos, lights, L, out, dir_lights=None, n_dir=0, fresh=False):
+        """`fresh`: background pixels are written as zeros instead of left alone."""
+        return self.check((self.lib.vren_shade_fresh if fresh else self.lib.vren_shade)(
             self.h, self.stream(), W, H, ctypes.byref(cam), ctypes.byref(cfg), _ptr(depth), _ptr(normals),
             _ptr(albedo_rough), _ptr(metallic), _ptr(refs), key_cap, _ptr(counts), _ptr(offsets), _ptr(indices),
             index_cap, _ptr(light_pos), _ptr(lights), L, _ptr(dir_lights), n_dir, _ptr(out)))
 
     def shade_backward(self, W, H, cam, cfg, depth, normals, albedo_rough, metallic, refs, key_cap, counts, offsets,
-                       indices, index_cap, light_pos, lights, L, grad_out, g_pos, g_lights, g_albedo_rough):
-        return self.check(self.lib.vren_shade_backward(
+                       indices, index_cap, light_pos, lights, L, grad_out, g_pos, g_lights, g_albedo_rough, fresh=False):
+        """`fresh`: the gradients are written instead of added to."""
+        return self.check((self.lib.vren_shade_backward_fresh if fresh else self.lib.vren_shade_backward)(
             self.h, self.stream(), W, H, ctypes.byref(cam), ctypes.byref(cfg), _ptr(depth), _ptr(normals),
             _ptr(albedo_rough), _ptr(metallic), _ptr(refs), key_cap, _ptr(counts), _ptr(offsets), _ptr(indices),
             index_cap, _ptr(light_pos), _ptr(lights), L, _ptr(grad_out), _ptr(g_pos), _ptr(g_lights),

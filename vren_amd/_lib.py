@@ -117,6 +117,9 @@ PROTOTYPES = {
     "vren_shade": (c_int, [c_void_p, c_void_p, c_uint32, c_uint32, P(Camera), P(ClusterCfg), c_void_p, c_void_p,
                            c_void_p, c_void_p, c_void_p, c_uint32, c_void_p, c_void_p, c_void_p, c_uint32, c_void_p,
                            c_void_p, c_uint32, c_void_p, c_uint32, c_void_p]),
+    "vren_shade_fresh": (c_int, [c_void_p, c_void_p, c_uint32, c_uint32, P(Camera), P(ClusterCfg), c_void_p, c_void_p,
+                           c_void_p, c_void_p, c_void_p, c_uint32, c_void_p, c_void_p, c_void_p, c_uint32, c_void_p,
+                           c_void_p, c_uint32, c_void_p, c_uint32, c_void_p]),
     "vren_shade_materials": (c_int, [c_void_p, c_void_p, c_uint32, c_uint32, P(Camera), P(ClusterCfg), c_void_p,
                                      c_void_p, P(MaterialSet), c_void_p, c_uint32, c_void_p, c_void_p, c_void_p,
                                      c_uint32, c_void_p, c_void_p, c_uint32, c_void_p, c_uint32, c_void_p]),
@@ -128,6 +131,10 @@ PROTOTYPES = {
                                    c_uint32, c_void_p, c_void_p, c_void_p, c_uint32, c_void_p]),
     "vren_visualize_bvh": (c_int, [c_void_p, c_void_p, c_void_p, c_uint32, c_void_p]),
     "vren_shade_backward": (c_int, [c_void_p, c_void_p, c_uint32, c_uint32, P(Camera), P(ClusterCfg), c_void_p,
+                                    c_void_p, c_void_p, c_void_p, c_void_p, c_uint32, c_void_p, c_void_p, c_void_p,
+                                    c_uint32, c_void_p, c_void_p, c_uint32, c_void_p, c_void_p, c_void_p,
+                                    c_void_p]),
+    "vren_shade_backward_fresh": (c_int, [c_void_p, c_void_p, c_uint32, c_uint32, P(Camera), P(ClusterCfg), c_void_p,
                                     c_void_p, c_void_p, c_void_p, c_void_p, c_uint32, c_void_p, c_void_p, c_void_p,
                                     c_uint32, c_void_p, c_void_p, c_uint32, c_void_p, c_void_p, c_void_p,
                                     c_void_p]),

@@ -30,6 +30,7 @@ struct ChainWork {
     uint32_t total_leaf_slots;
     uint32_t max_L;
     uint32_t light_chunks;  // chunks of VREN_LIGHT_CHUNK lights over the table's frames (light_chunk_base numbering)
+    uint32_t fresh;         // a single-frame shade call whose output holds nothing: zeros for background pixels
     uint32_t any_materials; // some frame of the table takes the material path (shade picks its kernel by it)
     // launch shape (vren_chain_shape; 0 = the default): shade strips per workgroup, persistent assignment waves
     // per CU, digit width of the light sort

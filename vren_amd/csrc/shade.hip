@@ -497,7 +497,8 @@ __device__ __forceinline__ void resolve_materials(const FrameDev& fd, bool todo,
 // the light records beside the pixels' list bounds: two dependent rounds of loads. Without it (references from the
 // caller), the workgroup first reduces the run from its pixels' lists.
 // MAT: the table may hold frames on the material path (texcoords + material index + material and texture tables)
-template <int PPT, bool MAT>
+// FRESH: background pixels are written as zeros (they are left alone otherwise)
+template <int PPT, bool MAT, bool FRESH = false>
 __device__ __forceinline__ void shade_body(const FrameDev* __restrict__ frames, const uint32_t* __restrict__ tile_frame,
                                            const uint2* __restrict__ tile_range, uint32_t total_tiles)
 {
@@ -564,6 +565,14 @@ __device__ __forceinline__ void shade_body(const FrameDev* __restrict__ frames, 
             cl_raw[q] = *((guint*)fd.refs + p[q]);
             px[q] = reconstruct(fd, gx, gy, depth);
         }
+    }
+    if constexpr (FRESH) {
+#pragma unroll
+        for (int q = 0; q < PPT; q++)
+            if (in[q] && !px[q].shaded) {
+                const vf4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                __builtin_nontemporal_store(zero, (__attribute__((address_space(1))) vf4*)fd.out + p[q]);
+            }
     }
     if (mat) {
 #pragma unroll
@@ -648,10 +657,10 @@ __global__ __launch_bounds__(256, 8) void shade_kernel(const FrameDev* __restric
 {
     shade_body<PPT, MAT>(frames, tile_frame, tile_range, total_tiles);
 }
-template <int PPT, bool MAT>
+template <int PPT, bool MAT, bool FRESH>
 __global__ __launch_bounds__(256, 8) void shade_one_kernel(const FrameDev one, uint32_t total_tiles)
 {
-    shade_body<PPT, MAT>(inline_frame(), nullptr, nullptr, total_tiles);
+    shade_body<PPT, MAT, FRESH>(inline_frame(), nullptr, nullptr, total_tiles);
 }
 
 // ---- adjoint ---------------------------------------------------------------------------------------------------
@@ -828,6 +837,8 @@ constexpr int kSumRounds = 8;  // distinct entries of one step that a wave sums;
 // leaving out the pairs behind the surface first and reducing the list ranges on the DPP network: 81 us, of which the
 // VALU is busy for about two thirds. Five waves per SIMD in place of four (a stage of 448 entries) would give 80.
 // Larger workgroups (two and four strips, fewer global adds) were slower than the 91, 97 and 115 us.
+// FRESH: the material gradient is written, zeros for the background, instead of added to.
+template <bool FRESH>
 __global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev one, uint32_t total_tiles,
                                                              const float* grad_out, float* g_pos, float* g_light,
                                                              float* g_ar)
@@ -869,8 +880,10 @@ __global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev one,
         const vf4 gv = *((gvf4*)grad_out + p);
         go = make_float4(gv.x, gv.y, gv.z, gv.w);
         cl_raw = *((guint*)fd.refs + p);
-        const vf4 gav = *((gvf4*)g_ar + p);
-        gar = make_float4(gav.x, gav.y, gav.z, gav.w);
+        if constexpr (!FRESH) {
+            const vf4 gav = *((gvf4*)g_ar + p);
+            gar = make_float4(gav.x, gav.y, gav.z, gav.w);
+        }
         px = reconstruct(fd, gx, gy, depth);
     }
     const bool has_list = px.shaded && fd.L > 0 && cl_raw < fd.key_cap;
@@ -1039,6 +1052,8 @@ __global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev one,
         gar.z += gp[2];
         gar.w += gp[3];
         reinterpret_cast<float4*>(g_ar)[p] = gar;
+    } else if (FRESH && in) {
+        reinterpret_cast<float4*>(g_ar)[p] = gar; // zero
     }
     __syncthreads();
     if (staged) {
@@ -1052,6 +1067,12 @@ __global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev one,
     }
 }
 
+__global__ void clear_light_grads_kernel(float4* a, float4* b, uint32_t n)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) a[i] = b[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+
 } // namespace
 
 int launch_shade(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
@@ -1062,8 +1083,9 @@ int launch_shade(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_
     const uint32_t rounds = (w.total_tiles + 7) / 8;        // rounds of 8 tiles, one per XCD
     const uint32_t grid = rounds * 8 * (4 / kShadePPT);
     if (one) {
-        if (w.any_materials) shade_one_kernel<kShadePPT, true><<<grid, 256, 0, s>>>(*one, w.total_tiles);
-        else shade_one_kernel<kShadePPT, false><<<grid, 256, 0, s>>>(*one, w.total_tiles);
+        if (w.any_materials) shade_one_kernel<kShadePPT, true, false><<<grid, 256, 0, s>>>(*one, w.total_tiles);
+        else if (w.fresh) shade_one_kernel<kShadePPT, false, true><<<grid, 256, 0, s>>>(*one, w.total_tiles);
+        else shade_one_kernel<kShadePPT, false, false><<<grid, 256, 0, s>>>(*one, w.total_tiles);
     } else if (w.shade_ppt == 2) {
         if (w.any_materials) shade_kernel<2, true><<<rounds * 8 * 2, 256, 0, s>>>(d_frames, tf, ranges, w.total_tiles);
         else shade_kernel<2, false><<<rounds * 8 * 2, 256, 0, s>>>(d_frames, tf, ranges, w.total_tiles);
@@ -1076,15 +1098,15 @@ int launch_shade(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_
     return VREN_OK;
 }
 
-extern "C" VREN_EXPORT int vren_shade(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
-                                      const vren_camera* camera, const vren_cluster_cfg* cfg, const float* depth,
-                                      const uint16_t* normals, const float* albedo_roughness, const float* metallic,
-                                      const uint32_t* cluster_refs, uint32_t key_capacity,
-                                      const uint32_t* light_counts, const uint32_t* light_offsets,
-                                      const uint32_t* light_indices, uint32_t index_capacity,
-                                      const float* light_positions, const float* point_lights, uint32_t light_count,
-                                      const float* directional_lights, uint32_t directional_light_count,
-                                      float* output)
+static int shade_frame(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
+                       const vren_camera* camera, const vren_cluster_cfg* cfg, const float* depth,
+                       const uint16_t* normals, const float* albedo_roughness, const float* metallic,
+                       const uint32_t* cluster_refs, uint32_t key_capacity,
+                       const uint32_t* light_counts, const uint32_t* light_offsets,
+                       const uint32_t* light_indices, uint32_t index_capacity,
+                       const float* light_positions, const float* point_lights, uint32_t light_count,
+                       const float* directional_lights, uint32_t directional_light_count,
+                       float* output, bool fresh)
 {
     if (!ctx) return VREN_EINVAL;
     int st = vren_validate_camera(ctx, camera);
@@ -1122,7 +1144,40 @@ extern "C" VREN_EXPORT int vren_shade(vren_ctx* ctx, vren_stream_t stream, uint3
     ChainWork w;
     memset(&w, 0, sizeof(w));
     w.total_tiles = f.Sx * f.Sy;
+    w.fresh = fresh ? 1 : 0;
     return launch_shade(ctx, s, nullptr, 1, w, &f);
+}
+
+extern "C" VREN_EXPORT int vren_shade(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
+                                      const vren_camera* camera, const vren_cluster_cfg* cfg, const float* depth,
+                                      const uint16_t* normals, const float* albedo_roughness, const float* metallic,
+                                      const uint32_t* cluster_refs, uint32_t key_capacity,
+                                      const uint32_t* light_counts, const uint32_t* light_offsets,
+                                      const uint32_t* light_indices, uint32_t index_capacity,
+                                      const float* light_positions, const float* point_lights, uint32_t light_count,
+                                      const float* directional_lights, uint32_t directional_light_count,
+                                      float* output)
+{
+    return shade_frame(ctx, stream, width, height, camera, cfg, depth, normals, albedo_roughness, metallic,
+                       cluster_refs, key_capacity, light_counts, light_offsets, light_indices, index_capacity,
+                       light_positions, point_lights, light_count, directional_lights, directional_light_count,
+                       output, false);
+}
+
+extern "C" VREN_EXPORT int vren_shade_fresh(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
+                                            const vren_camera* camera, const vren_cluster_cfg* cfg, const float* depth,
+                                            const uint16_t* normals, const float* albedo_roughness, const float* metallic,
+                                            const uint32_t* cluster_refs, uint32_t key_capacity,
+                                            const uint32_t* light_counts, const uint32_t* light_offsets,
+                                            const uint32_t* light_indices, uint32_t index_capacity,
+                                            const float* light_positions, const float* point_lights, uint32_t light_count,
+                                            const float* directional_lights, uint32_t directional_light_count,
+                                            float* output)
+{
+    return shade_frame(ctx, stream, width, height, camera, cfg, depth, normals, albedo_roughness, metallic,
+                       cluster_refs, key_capacity, light_counts, light_offsets, light_indices, index_capacity,
+                       light_positions, point_lights, light_count, directional_lights, directional_light_count,
+                       output, true);
 }
 
 extern "C" VREN_EXPORT int vren_shade_materials(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
@@ -1177,17 +1232,17 @@ extern "C" VREN_EXPORT int vren_shade_materials(vren_ctx* ctx, vren_stream_t str
     return launch_shade(ctx, s, nullptr, 1, w, &f);
 }
 
-extern "C" VREN_EXPORT int vren_shade_backward(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
-                                               const vren_camera* camera, const vren_cluster_cfg* cfg,
-                                               const float* depth, const uint16_t* normals,
-                                               const float* albedo_roughness, const float* metallic,
-                                               const uint32_t* cluster_refs, uint32_t key_capacity,
-                                               const uint32_t* light_counts, const uint32_t* light_offsets,
-                                               const uint32_t* light_indices, uint32_t index_capacity,
-                                               const float* light_positions, const float* point_lights,
-                                               uint32_t light_count, const float* grad_output,
-                                               float* grad_light_positions, float* grad_point_lights,
-                                               float* grad_albedo_roughness)
+static int shade_adjoint(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
+                         const vren_camera* camera, const vren_cluster_cfg* cfg,
+                         const float* depth, const uint16_t* normals,
+                         const float* albedo_roughness, const float* metallic,
+                         const uint32_t* cluster_refs, uint32_t key_capacity,
+                         const uint32_t* light_counts, const uint32_t* light_offsets,
+                         const uint32_t* light_indices, uint32_t index_capacity,
+                         const float* light_positions, const float* point_lights,
+                         uint32_t light_count, const float* grad_output,
+                         float* grad_light_positions, float* grad_point_lights,
+                         float* grad_albedo_roughness, bool fresh)
 {
     if (!ctx) return VREN_EINVAL;
     int st = vren_validate_camera(ctx, camera);
@@ -1219,8 +1274,50 @@ extern "C" VREN_EXPORT int vren_shade_backward(vren_ctx* ctx, vren_stream_t stre
     f.lights = point_lights;
     f.L = light_count;
     const uint32_t tiles = f.Sx * f.Sy;
-    shade_backward_kernel<<<(tiles + 7) / 8 * 32, 256, 0, s>>>(f, tiles, grad_output, grad_light_positions,
-                                                               grad_point_lights, grad_albedo_roughness);
+    if (fresh && light_count > 0) {
+        clear_light_grads_kernel<<<(light_count + 255) / 256, 256, 0, s>>>(
+            reinterpret_cast<float4*>(grad_light_positions), reinterpret_cast<float4*>(grad_point_lights), light_count);
+        VREN_LAUNCH_CHECK(ctx);
+    }
+    const auto kernel = fresh ? shade_backward_kernel<true> : shade_backward_kernel<false>;
+    kernel<<<(tiles + 7) / 8 * 32, 256, 0, s>>>(f, tiles, grad_output, grad_light_positions, grad_point_lights,
+                                                grad_albedo_roughness);
     VREN_LAUNCH_CHECK(ctx);
     return VREN_OK;
+}
+
+extern "C" VREN_EXPORT int vren_shade_backward(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
+                                               const vren_camera* camera, const vren_cluster_cfg* cfg,
+                                               const float* depth, const uint16_t* normals,
+                                               const float* albedo_roughness, const float* metallic,
+                                               const uint32_t* cluster_refs, uint32_t key_capacity,
+                                               const uint32_t* light_counts, const uint32_t* light_offsets,
+                                               const uint32_t* light_indices, uint32_t index_capacity,
+                                               const float* light_positions, const float* point_lights,
+                                               uint32_t light_count, const float* grad_output,
+                                               float* grad_light_positions, float* grad_point_lights,
+                                               float* grad_albedo_roughness)
+{
+    return shade_adjoint(ctx, stream, width, height, camera, cfg, depth, normals, albedo_roughness, metallic,
+                         cluster_refs, key_capacity, light_counts, light_offsets, light_indices, index_capacity,
+                         light_positions, point_lights, light_count, grad_output, grad_light_positions,
+                         grad_point_lights, grad_albedo_roughness, false);
+}
+
+extern "C" VREN_EXPORT int vren_shade_backward_fresh(vren_ctx* ctx, vren_stream_t stream, uint32_t width, uint32_t height,
+                                                     const vren_camera* camera, const vren_cluster_cfg* cfg,
+                                                     const float* depth, const uint16_t* normals,
+                                                     const float* albedo_roughness, const float* metallic,
+                                                     const uint32_t* cluster_refs, uint32_t key_capacity,
+                                                     const uint32_t* light_counts, const uint32_t* light_offsets,
+                                                     const uint32_t* light_indices, uint32_t index_capacity,
+                                                     const float* light_positions, const float* point_lights,
+                                                     uint32_t light_count, const float* grad_output,
+                                                     float* grad_light_positions, float* grad_point_lights,
+                                                     float* grad_albedo_roughness)
+{
+    return shade_adjoint(ctx, stream, width, height, camera, cfg, depth, normals, albedo_roughness, metallic,
+                         cluster_refs, key_capacity, light_counts, light_offsets, light_indices, index_capacity,
+                         light_positions, point_lights, light_count, grad_output, grad_light_positions,
+                         grad_point_lights, grad_albedo_roughness, true);
 }
