@@ -835,18 +835,18 @@ constexpr int kSumRounds = 8;  // distinct entries of one step that a wave sums;
 // when all its lanes were at one entry) and 50 us in the gradients' global atomics, seven instructions each of whose
 // lanes hit another cache line. Summing once per distinct entry and one term per lane in the global adds: 91 us;
 // leaving out the pairs behind the surface first and reducing the list ranges on the DPP network: 81 us, of which the
-// VALU is busy for about two thirds. Five waves per SIMD in place of four (a stage of 448 entries) would give 80.
+// VALU is busy for about two thirds. Five waves per SIMD in place of four, which 96 registers and 60 bytes of LDS an entry
+// (the light's index rides in its position) allow: 76 with the gradients written, 79.5 before.
 // Larger workgroups (two and four strips, fewer global adds) were slower than the 91, 97 and 115 us.
 // FRESH: the material gradient is written, zeros for the background, instead of added to.
 template <bool FRESH>
-__global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev one, uint32_t total_tiles,
+__global__ __launch_bounds__(256, 5) void shade_backward_kernel(const FrameDev one, uint32_t total_tiles,
                                                              const float* grad_out, float* g_pos, float* g_light,
                                                              float* g_ar)
 {
-    __shared__ float4 s_lpos[kStage];
+    __shared__ float4 s_lpos[kStage]; // w: the light's index
     __shared__ float4 s_lcol[kStage];
     __shared__ float s_g[kStage * 7];
-    __shared__ uint32_t s_li[kStage];
     __shared__ uint32_t s_min[4], s_max[4];
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / VREN_WAVE;
     // a tile's four strips on one XCD, consecutive tiles on consecutive XCDs (as the forward shade), the grid rounded
@@ -922,9 +922,10 @@ __global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev one,
     if (staged) {
         for (uint32_t i = tid; i < nstage; i += 256) {
             const uint32_t li = *((guint*)fd.indices + start + i);
-            s_li[i] = li;
             const bool ok = li < fd.L;
-            s_lpos[i] = ok ? lpos(li) : make_float4(0.f, 0.f, 0.f, 0.f);
+            float4 at = ok ? lpos(li) : make_float4(0.f, 0.f, 0.f, 0.f);
+            at.w = __uint_as_float(li);
+            s_lpos[i] = at;
             s_lcol[i] = ok ? lcol(li) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
         for (uint32_t i = tid; i < nstage * 7; i += 256) s_g[i] = 0.0f;
@@ -1060,7 +1061,7 @@ __global__ __launch_bounds__(256) void shade_backward_kernel(const FrameDev one,
         // one term per lane, so that a light's terms leave as neighbouring addresses of one instruction
         for (uint32_t i = tid; i < nstage * 7; i += 256) {
             const float v = s_g[i];
-            const uint32_t n = i / 7, c = i - n * 7, li = s_li[n];
+            const uint32_t n = i / 7, c = i - n * 7, li = __float_as_uint(s_lpos[n].w);
             if (v == 0.0f || li >= fd.L) continue;
             atomicAdd(c < 3 ? &g_pos[4 * li + c] : &g_light[4 * li + (c - 3)], v);
         }
