@@ -27,6 +27,10 @@ __global__ void scan_init_kernel(uint64_t* status, uint64_t n_status, uint32_t* 
     if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0u;
 }
 
+// ALONE: segments of one tile each, which nothing comes before: a workgroup takes the segment of its number, and there
+// is no ticket, no status and nothing to clear. One launch in place of two: calls on up to
+// 16384 elements, one after the other, take 5.5 us each in place of 8.4.
+template <bool ALONE>
 __global__ __launch_bounds__(kThreads) void scan_kernel(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t tiles_per_seg,
                                                         uint64_t* status, uint32_t* counter)
 {
@@ -34,11 +38,13 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const uint32_t* in, uint
     __shared__ uint32_t s_wsum[kWaves];          // each wave's total over its rows
     __shared__ uint32_t s_ticket;
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
-    if (tid == 0) s_ticket = atomic_add_agent(counter, 1u);
-    __syncthreads();
-    const uint32_t g = s_ticket;
-    const uint32_t seg = g / tiles_per_seg;
-    const uint32_t t = g - seg * tiles_per_seg;
+    if constexpr (!ALONE) {
+        if (tid == 0) s_ticket = atomic_add_agent(counter, 1u);
+        __syncthreads();
+    }
+    const uint32_t g = ALONE ? blockIdx.x : s_ticket;
+    const uint32_t seg = ALONE ? g : g / tiles_per_seg;
+    const uint32_t t = ALONE ? 0u : g - seg * tiles_per_seg;
     const uint64_t tile_start = (uint64_t)t * kTile;
     const uint64_t seg_base = (uint64_t)seg * n;
     const uint32_t cnt = (uint32_t)min<uint64_t>((uint64_t)kTile, n - tile_start);
@@ -63,19 +69,19 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const uint32_t* in, uint
     }
     // the tile's total first, published before the row scans, so that the next tiles' walks find this tile's
     // aggregate while it still scans its rows
-    {
+    if constexpr (!ALONE) {
         uint32_t tsum = 0;
 #pragma unroll
         for (int j = 0; j < kRows; j++) tsum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
         tsum = wave_sum(tsum);
         if (lane == 0) s_wsum[wave] = tsum;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        uint32_t agg = 0;
+        __syncthreads();
+        if (tid == 0) {
+            uint32_t agg = 0;
 #pragma unroll
-        for (int w = 0; w < kWaves; w++) agg += s_wsum[w];
-        wave_lookback_publish(status + (uint64_t)seg * tiles_per_seg, t, agg);
+            for (int w = 0; w < kWaves; w++) agg += s_wsum[w];
+            wave_lookback_publish(status + (uint64_t)seg * tiles_per_seg, t, agg);
+        }
     }
     uint32_t excl[kRows]; // exclusive prefix of the thread's 4 elements within its wave's segment of each row
 #pragma unroll
@@ -90,7 +96,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const uint32_t* in, uint
         const uint32_t x = s_part[lane];
         const uint32_t xi = wave_inclusive_sum(x);
         const uint32_t agg = __builtin_amdgcn_readlane(xi, VREN_WAVE - 1);
-        const uint32_t prefix = wave_lookback_walk(status + (uint64_t)seg * tiles_per_seg, t, agg);
+        const uint32_t prefix = ALONE ? 0u : wave_lookback_walk(status + (uint64_t)seg * tiles_per_seg, t, agg);
         s_part[lane] = prefix + xi - x;
     }
     __syncthreads();
@@ -132,10 +138,15 @@ int vren_scan_with_work(vren_ctx* ctx, hipStream_t s, const uint32_t* in, uint32
     uint64_t tiles = tps * blocks;
     uint32_t* counter = static_cast<uint32_t*>(work);
     uint64_t* status = reinterpret_cast<uint64_t*>(static_cast<char*>(work) + 256);
+    if (tps == 1) {
+        scan_kernel<true><<<(uint32_t)tiles, kThreads, 0, s>>>(in, out, n, 1, nullptr, nullptr);
+        VREN_LAUNCH_CHECK(ctx);
+        return VREN_OK;
+    }
     uint32_t init_blocks = (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(1, ceil_div_u64(tiles, 256)));
     scan_init_kernel<<<init_blocks, 256, 0, s>>>(status, tiles, counter);
     VREN_LAUNCH_CHECK(ctx);
-    scan_kernel<<<(uint32_t)tiles, kThreads, 0, s>>>(in, out, n, (uint32_t)tps, status, counter);
+    scan_kernel<false><<<(uint32_t)tiles, kThreads, 0, s>>>(in, out, n, (uint32_t)tps, status, counter);
     VREN_LAUNCH_CHECK(ctx);
     return VREN_OK;
 }
@@ -163,7 +174,7 @@ extern "C" VREN_EXPORT int vren_exclusive_scan_u32(vren_ctx* ctx, vren_stream_t 
 // its device current, resolves this device's address once into ctx->noalloc_scan_work, and the entry point passes
 // that. Every call on one GPU shares the array; scan_init_kernel clears the counter and the status words at the
 // start of each call, so calls in sequence on one stream are independent, and calls that overlap (other streams,
-// other contexts on the same GPU) race.
+// other contexts on the same GPU) race (but for segments of one tile, which use none of it).
 constexpr uint64_t kNoAllocTiles = 1ull << 16;
 constexpr size_t kNoAllocBytes = 256 + kNoAllocTiles * sizeof(uint64_t);
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
