@@ -21,10 +21,10 @@ uint64_t bucket_key(uint64_t n, bool vals, uint32_t key_bits)
 }
 
 // the configuration when nothing is tuned or forced: onesweep with the default tile of n keys
-int default_config(uint64_t n, int num_cus)
+int default_config(uint64_t n, bool vals, int num_cus)
 {
     const int shape[][2] = {{8, 8}, {8, 16}, {15, 16}, {23, 16}}; // (keys per thread, waves), in RadixTile order
-    const int* d = shape[vren_radix_default_tile(n, num_cus)];
+    const int* d = shape[vren_radix_default_tile(n, num_cus, vals, false)];
     for (int i = 0; i < vren_radix_config_count(); i++) {
         int b, k, w, a;
         vren_radix_config_info(i, &b, &k, &w, &a);
@@ -54,7 +54,7 @@ int vren_radix_pick_config(vren_ctx* ctx, hipStream_t s, uint64_t n, bool vals, 
     auto it = ctx->radix_tuned.find(bucket_key(n, vals, key_bits));
     if (it != ctx->radix_tuned.end()) return it->second;
     (void)s;
-    return default_config(n, ctx->num_cus);
+    return default_config(n, vals, ctx->num_cus);
 }
 
 extern "C" {

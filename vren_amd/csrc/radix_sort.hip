@@ -3,8 +3,8 @@
 // The reference runs, per 4-bit digit, six dispatches (fill, local count, 16-block reduce, global offset,
 // 16-block down-sweep, reorder) over N/1024 workgroups, i.e. 8 passes x 3 reads/writes of the keys and ~48
 // dispatches, and its reorder assumes a 32-wide subgroup (radix_sort_reorder.comp:15-17). Here:
-//   1. one histogram kernel reads the keys once and counts every pass's digit (LDS atomics, then agent-scope
-//      global atomics);
+//   1. one histogram kernel reads the keys once and counts every pass's digit (LDS atomics, one set of counts per
+//      workgroup, which a second kernel adds up and scans);
 //   2. one kernel per pass: tiles taken from a ticket counter are ranked stably in LDS with wave64 ballot
 //      matching, each tile's per-digit counts are chained across tiles by a per-digit decoupled look-back, and
 //      the tile is scattered through an LDS staging buffer so global writes go out in per-digit runs.
@@ -20,35 +20,28 @@
 
 namespace {
 
-// predecessor states read per round trip of the onesweep look-back
-constexpr int kLookback = 8;
+// predecessor states read per round trip of the onesweep look-back (2^26 keys in 15360-key tiles: 4 689 us, 8 695, 16 744)
+constexpr int kLookback = 4;
 
 // status word of (tile, digit): [31:30] state, [29:0] count
 #define RS_AGG (1u << 30)
 #define RS_INCL (2u << 30)
 #define RS_MASK ((1u << 30) - 1u)
 
-__global__ void rs_init_kernel(uint32_t* hist, uint32_t n_hist, uint32_t* counters, uint32_t n_counters)
-{
-    for (uint32_t i = threadIdx.x; i < n_hist; i += blockDim.x) hist[i] = 0u;
-    for (uint32_t i = threadIdx.x; i < n_counters; i += blockDim.x) counters[i] = 0u;
-}
-
-// one workgroup of 1024 threads per CU: the partial histograms are merged into the global one with agent-scope
-// atomics that all land in a few cache lines, so the number of workgroups is kept small
+// one workgroup of 1024 threads per CU at most, so that there are few counts to add up afterwards
 constexpr uint32_t kHistThreads = 1024;
 
 // PAIRS: the keys are the first words of interleaved (key, value) pairs (key i at keys[2 i]).
-// PARTS: every workgroup stores its own counts, pass by pass (hist[(pass * gridDim.x + blockIdx.x) * RADIX + digit]), and
-// workgroup 0 clears the passes' tile tickets; otherwise the counts are added to one histogram, which rs_init_kernel has cleared with the tickets.
-template <int BITS, bool PAIRS, bool PARTS>
+// Every workgroup stores its own counts, pass by pass (parts[(pass * gridDim.x + blockIdx.x) * RADIX + digit]), and
+// workgroup 0 clears the passes' tile tickets.
+template <int BITS, bool PAIRS>
 __global__ __launch_bounds__(kHistThreads) void rs_hist_kernel(const uint32_t* __restrict__ keys, uint64_t n,
                                                                uint32_t begin_bit, uint32_t end_bit, uint32_t passes,
-                                                               uint32_t* __restrict__ hist,
+                                                               uint32_t* __restrict__ parts,
                                                                uint32_t* __restrict__ clear, uint64_t clear_words,
                                                                uint32_t* __restrict__ counters)
 {
-    if (PARTS && blockIdx.x == 0 && threadIdx.x < passes) counters[threadIdx.x] = 0u;
+    if (blockIdx.x == 0 && threadIdx.x < passes) counters[threadIdx.x] = 0u;
     constexpr uint32_t KPV = PAIRS ? 2 : 4; // keys per 16-byte load
     constexpr int RADIX = 1 << BITS;
     __shared__ uint32_t s_h[8 * RADIX];
@@ -110,25 +103,40 @@ __global__ __launch_bounds__(kHistThreads) void rs_hist_kernel(const uint32_t* _
         count_keys(&k, 1);
     }
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < passes * RADIX; i += kHistThreads) {
-        uint32_t c = s_h[i];
-        if (PARTS) hist[(i / RADIX * gridDim.x + blockIdx.x) * RADIX + i % RADIX] = c;
-        else if (c) atomic_add_agent(&hist[i], c);
-    }
+    for (uint32_t i = threadIdx.x; i < passes * RADIX; i += kHistThreads)
+        parts[(i / RADIX * gridDim.x + blockIdx.x) * RADIX + i % RADIX] = s_h[i];
 }
 
-// exclusive scan of each pass's digit histogram in place: the digit's first output position. One workgroup.
+// The digits' first output positions of pass blockIdx.x: the n_parts workgroups' counts added up and scanned. The counts
+// were written by other XCDs, so a thread asks for many of them at once. Parts that are added up here, in place of
+// atomics on one histogram that a launch of its own cleared: 2^20 pairs 78 -> 73 us.
 template <int BITS>
-__global__ __launch_bounds__(256) void rs_hexscan_kernel(uint32_t* hist, uint32_t passes)
+__global__ __launch_bounds__(1024) void rs_hexscan_kernel(const uint32_t* __restrict__ parts, uint32_t n_parts,
+                                                          uint32_t* __restrict__ hist)
 {
-    constexpr int RADIX = 1 << BITS;
-    __shared__ uint32_t s_wave[4];
-    for (uint32_t p = 0; p < passes; p++) {
-        const uint32_t v = threadIdx.x < (uint32_t)RADIX ? hist[p * RADIX + threadIdx.x] : 0u;
-        uint32_t total;
-        const uint32_t ex = block_exclusive_sum<256>(v, s_wave, &total);
-        if (threadIdx.x < (uint32_t)RADIX) hist[p * RADIX + threadIdx.x] = ex;
+    constexpr uint32_t RADIX = 1u << BITS, GROUPS = 1024 / RADIX, U = 16;
+    __shared__ uint32_t s_sum[1024];
+    __shared__ uint32_t s_wave[16];
+    const uint32_t digit = threadIdx.x % RADIX, group = threadIdx.x / RADIX;
+    const uint32_t* src = parts + (uint64_t)blockIdx.x * n_parts * RADIX + digit;
+    uint32_t sum = 0;
+    for (uint32_t b = group; b < n_parts; b += U * GROUPS) {
+        uint32_t c[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) c[u] = src[(uint64_t)min(b + u * GROUPS, n_parts - 1u) * RADIX];
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) sum += b + u * GROUPS < n_parts ? c[u] : 0u;
     }
+    s_sum[threadIdx.x] = sum;
+    __syncthreads();
+    if (threadIdx.x < RADIX) {
+        for (uint32_t g = 1; g < GROUPS; g++) sum += s_sum[g * RADIX + threadIdx.x];
+    } else {
+        sum = 0;
+    }
+    uint32_t total;
+    const uint32_t ex = block_exclusive_sum<1024>(sum, s_wave, &total);
+    if (threadIdx.x < RADIX) hist[blockIdx.x * RADIX + threadIdx.x] = ex;
 }
 
 // Reduce-then-scan form, pass part 1: the digit counts of every tile (tiles as in the scatter pass), written
@@ -182,6 +190,20 @@ constexpr bool rs_sequential_staging()
     return VALS && 2 * WAVES * 64 * KPT * 4 > 80 * 1024;
 }
 
+// the element at a byte offset of 32 bits, which a store takes beside its scalar base
+__device__ __forceinline__ uint32_t& at32(uint32_t* p, uint32_t bytes)
+{
+    return *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(p) + bytes);
+}
+
+// tiles of 15360 keys leave room for a second workgroup on the CU, in LDS (79 KB) and, held to 64, in registers: one
+// ranks while the other waits for its loads, its look-back or its stores (2^26 keys in 15360-key tiles 947 -> 682 us; one
+// workgroup in 23552-key tiles 851 -> 775). With values that needs them read late, when the keys have left, and their
+// stores' shorter runs take back part of it: see vren_radix_default_tile. Measured and not kept: counters of 16 bits,
+// for tiles of 17408 keys (2^26 pairs 1175 -> 1398 us); workgroups that take one tile after the other and load the next
+// tile's keys during this one's stores (1077 -> 1304: the CUs fall into step).
+constexpr bool rs_two_per_cu(int kpt, int waves) { return kpt == 15 && waves == 16; }
+
 // RTS = false: onesweep (tiles from a ticket counter, per-digit decoupled look-back, digit_base = the digit's
 // first output position). RTS = true: reduce-then-scan scatter pass (tile = workgroup id; digit_base = the scanned
 // digit-major tile counts of rs_upsweep_kernel), no tickets and no waiting.
@@ -198,11 +220,11 @@ struct BucketStarts {
     uint32_t shift, mask;
 };
 
-// The histogram workgroups' counts of one pass (rs_hist_kernel with PARTS), n of them; n = 0: the pass reads scanned
+// The histogram workgroups' counts of one pass (rs_hist_kernel), n of them; n = 0: the pass reads scanned
 // digit bases. Up to kPartsMaxKeys keys, each tile sums and scans the few parts itself, beside its
-// key loads, which saves the clearing launch ahead of the histogram and the scanning one after it (2^16 pairs: 45.3
+// key loads, which saves the launch that adds them up and, with it, the clearing one that there was (2^16 pairs: 45.3
 // -> 38.9 us); tile 0 leaves the bases for whoever reads them after the pass. Above, the sum would take each tile longer
-// than the two launches take all of them.
+// than the launch takes all of them.
 struct HistParts {
     const uint32_t* counts;
     uint32_t n;
@@ -217,11 +239,10 @@ uint32_t parts_room(uint64_t n)
 {
     return (uint32_t)std::min<uint64_t>(kPartsMaxBlocks, ceil_div_u64(std::max<uint64_t>(n, 1), 4096));
 }
-uint32_t parts_blocks(uint64_t n) { return n <= kPartsMaxKeys ? parts_room(n) : 0u; }
 
 template <int BITS, int KPT, int WAVES, bool VALS, bool RTS = false, bool IN_PAIRS = false, bool OUT_PAIRS = false,
           bool BSTARTS = false>
-__global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t* __restrict__ keys_in,
+__global__ __launch_bounds__(WAVES * 64, rs_two_per_cu(KPT, WAVES) && !IN_PAIRS && !OUT_PAIRS ? 8 : 1) void rs_onesweep_kernel(const uint32_t* __restrict__ keys_in,
                                                                  const uint32_t* __restrict__ vals_in,
                                                                  uint32_t* __restrict__ keys_out,
                                                                  uint32_t* __restrict__ vals_out, uint64_t n,
@@ -235,6 +256,7 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
     constexpr int RADIX = 1 << BITS;
     constexpr int TILE = THREADS * KPT;
     constexpr bool SEQ = rs_sequential_staging<KPT, WAVES, VALS>();
+    constexpr bool LATE = VALS && !IN_PAIRS && !OUT_PAIRS && rs_two_per_cu(KPT, WAVES);
     static_assert(THREADS >= RADIX, "one thread per digit");
     static_assert(VALS || !(IN_PAIRS || OUT_PAIRS), "interleaved pairs carry values");
     static_assert(OUT_PAIRS || !BSTARTS, "bucket starts come from a pass that writes pairs");
@@ -242,18 +264,22 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
     __shared__ uint32_t s_vals[(VALS && !SEQ) ? TILE : 1];
     __shared__ uint32_t s_whist[WAVES * RADIX];
     __shared__ uint32_t s_goff[RADIX];
-    __shared__ uint32_t s_scan[THREADS / VREN_WAVE];
+    constexpr uint32_t DIGIT_WAVES = (RADIX + VREN_WAVE - 1) / VREN_WAVE;
+    __shared__ uint32_t s_scan[2 * DIGIT_WAVES];
     __shared__ uint32_t s_ticket;
 
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = lane_id();
-    const uint32_t wave = tid / VREN_WAVE;
+    uint32_t tid = threadIdx.x;
+    uint32_t lane = lane_id();
+    const uint32_t wave = wave_id();
+    uint32_t* const row = s_whist + wave * RADIX; // the wave's own counters: no other wave writes them while it ranks
     if (!RTS && tid == 0) s_ticket = atomic_add_agent(counter, 1u);
-    for (uint32_t i = tid; i < (uint32_t)(WAVES * RADIX); i += THREADS) s_whist[i] = 0u;
-    __syncthreads();
-    const uint32_t tile = RTS ? blockIdx.x : s_ticket;
+    for (uint32_t i = lane; i < (uint32_t)RADIX; i += VREN_WAVE) row[i] = 0u;
+    if (RTS) __builtin_amdgcn_wave_barrier();
+    else __syncthreads();
+    const uint32_t tile = RTS ? blockIdx.x : __builtin_amdgcn_readfirstlane(s_ticket);
     const uint64_t tile_start = (uint64_t)tile * TILE;
     const uint32_t tile_count = (uint32_t)min<uint64_t>((uint64_t)TILE, n - tile_start);
+    const bool full = tile_count == (uint32_t)TILE;
     if (!RTS && clear_next) {
         for (uint32_t i = tid; i < (uint32_t)RADIX; i += THREADS) clear_next[(uint64_t)tile * RADIX + i] = 0u;
     }
@@ -263,26 +289,47 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
     const uint32_t wbase = wave * KPT * VREN_WAVE;
     const uint32_t* kin = keys_in + tile_start + wbase + lane;
     const uint32_t* vin = vals_in + tile_start + wbase + lane;
-    uint32_t key[KPT], val[VALS ? KPT : 1], digit[KPT], local[KPT];
+    uint32_t key[KPT], val[VALS ? KPT : 1];
     if (IN_PAIRS) {
         const vu2* pin = reinterpret_cast<const vu2*>(keys_in) + tile_start + wbase + lane;
-        const bool full_tile = tile_count == (uint32_t)TILE;
+        if (full) {
 #pragma unroll
-        for (int j = 0; j < KPT; j++) {
-            vu2 q = {0xFFFFFFFFu, 0u};
-            if (full_tile || wbase + j * VREN_WAVE + lane < tile_count) q = __builtin_nontemporal_load(pin + j * VREN_WAVE);
-            key[j] = q.x;
-            val[j] = q.y;
+            for (int j = 0; j < KPT; j++) {
+                const vu2 q = __builtin_nontemporal_load(pin + j * VREN_WAVE);
+                key[j] = q.x;
+                val[j] = q.y;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < KPT; j++) {
+                const uint32_t i = wbase + j * VREN_WAVE + lane;
+                const vu2 q = reinterpret_cast<const vu2*>(keys_in)[tile_start + min(i, tile_count - 1u)];
+                key[j] = i < tile_count ? q.x : 0xFFFFFFFFu;
+                val[j] = q.y;
+            }
         }
-    } else if (tile_count == (uint32_t)TILE) {
+    } else if (full) {
 #pragma unroll
         for (int j = 0; j < KPT; j++) key[j] = __builtin_nontemporal_load(kin + j * VREN_WAVE);
     } else {
 #pragma unroll
-        for (int j = 0; j < KPT; j++)
-            key[j] = wbase + j * VREN_WAVE + lane < tile_count ? __builtin_nontemporal_load(kin + j * VREN_WAVE)
-                                                               : 0xFFFFFFFFu;
+        for (int j = 0; j < KPT; j++) {
+            const uint32_t i = wbase + j * VREN_WAVE + lane;
+            const uint32_t k = keys_in[tile_start + min(i, tile_count - 1u)];
+            key[j] = i < tile_count ? k : 0xFFFFFFFFu;
+        }
     }
+    const auto load_vals = [&]() {
+        if (full) {
+#pragma unroll
+            for (int j = 0; j < KPT; j++) val[j] = __builtin_nontemporal_load(vin + j * VREN_WAVE);
+        } else {
+#pragma unroll
+            for (int j = 0; j < KPT; j++)
+                val[j] = vals_in[tile_start + min(wbase + j * VREN_WAVE + lane, tile_count - 1u)];
+        }
+    };
+    uint32_t digit[KPT], local[KPT];
     // the histogram's parts of this thread's digit are requested with the keys and summed after the ranking
     constexpr bool PARTS = !RTS && takes_parts(KPT);
     uint32_t part[PARTS ? kPartsMaxBlocks : 1];
@@ -293,48 +340,56 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
     }
 #pragma unroll
     for (int j = 0; j < KPT; j++) digit[j] = __builtin_amdgcn_ubfe(key[j], shift, width);
-    rank_wave_keys<BITS, KPT, false>(digit, wbase, tile_count, &s_whist[wave * RADIX], local);
+    rank_wave_keys<BITS, KPT, false>(digit, wbase, tile_count, row, local);
     // the values are read after the ranking: their loads overlap the counts, the look-back and the key stores
-    if (VALS && !IN_PAIRS) {
-#pragma unroll
-        for (int j = 0; j < KPT; j++)
-            val[j] = wbase + j * VREN_WAVE + lane < tile_count ? __builtin_nontemporal_load(vin + j * VREN_WAVE) : 0u;
-    }
+    if (VALS && !IN_PAIRS && !LATE) load_vals();
     __syncthreads();
     // per digit: tile count, then the exclusive prefix across waves offset by the digit's tile-local start, so a
-    // key's staged position is s_whist[wave][d] + local
-    uint32_t dcount = 0;
-    uint32_t wc[WAVES];
-    if (tid < (uint32_t)RADIX) {
+    // key's staged position is s_whist[wave][d] + local. The waves of the digits do it, each 64 of them.
+    uint32_t dcount = 0, dstart = 0, base = 0;
+    if (wave < DIGIT_WAVES) {
+        if (tid < (uint32_t)RADIX) {
 #pragma unroll
-        for (int w = 0; w < WAVES; w++) {
-            wc[w] = s_whist[w * RADIX + tid];
-            dcount += wc[w];
+            for (int w = 0; w < WAVES; w++) dcount += s_whist[w * RADIX + tid];
+            // onesweep: the tile's per-digit counts (the padding of a partial tile included: only the last tile has
+            // padding, and no tile looks back at the last one) are published before they are scanned
+            if (!RTS) st_agent_u32(status + (uint64_t)tile * RADIX + tid, (tile == 0 ? RS_INCL : RS_AGG) | dcount);
+        }
+        dstart = wave_inclusive_sum(dcount);
+        if (lane == VREN_WAVE - 1) s_scan[wave] = dstart;
+        if constexpr (PARTS) {
+            if (parts.n) {
+                uint32_t c = 0;
+#pragma unroll
+                for (uint32_t b = 0; b < kPartsMaxBlocks; b++) c += part[b];
+                base = wave_inclusive_sum(c);
+                if (lane == VREN_WAVE - 1) s_scan[DIGIT_WAVES + wave] = base;
+                base -= c;
+            }
         }
     }
-    // onesweep: the tile's per-digit counts (the padding of a partial tile included: only the last tile has
-    // padding, and no tile looks back at the last one) are published before the block scan
-    if (!RTS && tid < (uint32_t)RADIX)
-        st_agent_u32(status + (uint64_t)tile * RADIX + tid, (tile == 0 ? RS_INCL : RS_AGG) | dcount);
-    uint32_t total, base = 0;
-    uint32_t dstart = block_exclusive_sum<THREADS>(dcount, s_scan, &total);
-    if constexpr (PARTS) {
-        if (parts.n) {
-            uint32_t c = 0;
-#pragma unroll
-            for (uint32_t b = 0; b < kPartsMaxBlocks; b++) c += part[b];
-            base = block_exclusive_sum<THREADS>(c, s_scan, &total);
-            if (tile == 0 && tid < (uint32_t)RADIX) digit_base[tid] = base;
+    __syncthreads();
+    if (wave < DIGIT_WAVES && tid < (uint32_t)RADIX) {
+        dstart -= dcount;
+        for (uint32_t w = 0; w < wave; w++) dstart += s_scan[w];
+        if constexpr (PARTS) {
+            if (parts.n) {
+                for (uint32_t w = 0; w < wave; w++) base += s_scan[DIGIT_WAVES + w];
+                if (tile == 0) digit_base[tid] = base;
+            }
         }
-    }
-    uint32_t prefix = 0;
-    if (tid < (uint32_t)RADIX) {
         uint32_t run = dstart;
 #pragma unroll
         for (int w = 0; w < WAVES; w++) {
+            const uint32_t c = s_whist[w * RADIX + tid];
             s_whist[w * RADIX + tid] = run;
-            run += wc[w];
+            run += c;
         }
+    }
+    __syncthreads();
+    // the waves that hold the digits look back while the others already scatter
+    if (tid < (uint32_t)RADIX) {
+        uint32_t prefix = 0;
         if (!RTS && tile != 0) {
             // windowed decoupled look-back on this digit: the states of the kLookback nearest unread predecessors
             // are loaded at once and their counts summed up to the first inclusive one; an unpublished state is
@@ -363,18 +418,15 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
         }
         // global destination of staged position i = s_goff[digit] + i: RTS from the scanned digit-major tile
         // counts, onesweep from the pass histogram's exclusive scan (rs_hexscan_kernel) plus the look-back prefix
-        if (RTS) {
-            const uint32_t tiles = (uint32_t)((n + TILE - 1) / TILE);
-            s_goff[tid] = digit_base[(uint64_t)tid * tiles + tile] - dstart;
-        } else {
-            s_goff[tid] = (PARTS && parts.n ? base : digit_base[tid]) + prefix - dstart;
-        }
+        if (RTS) s_goff[tid] = digit_base[(uint64_t)tid * ((n + TILE - 1) / TILE) + tile] - dstart;
+        else s_goff[tid] = (PARTS && parts.n ? base : digit_base[tid]) + prefix - dstart;
     }
-    __syncthreads();
     // scatter into LDS in tile-local sorted order (every staged position is < TILE, padding included)
+    uint32_t sh = shift;
+    asm volatile("" : "+s"(sh)); // the digits again from the keys: kept since the ranking, they would take a register a key
 #pragma unroll
     for (int j = 0; j < KPT; j++) {
-        local[j] += s_whist[wave * RADIX + digit[j]];
+        local[j] += row[__builtin_amdgcn_ubfe(key[j], sh, width)];
         s_keys[local[j]] = key[j];
         if (VALS && !SEQ) s_vals[local[j]] = val[j];
     }
@@ -382,7 +434,6 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
     // staged position i = tid + j * THREADS goes to s_goff[digit] + i (< n: the digit's count over the tiles up to
     // this one never exceeds its count in the pass histogram). A full tile reads all its staged keys before the
     // first store, so the LDS reads overlap.
-    const bool full = tile_count == (uint32_t)TILE;
     if constexpr (OUT_PAIRS) {
         // keys and values of staged position i leave together as one 8-byte pair (positions past the end of a
         // partial tile hold padding and are not stored)
@@ -421,25 +472,25 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
             if (full || tid + j * THREADS < tile_count) pout[o[j]] = vu2{k[j], v[j]};
         return;
     }
-    uint32_t o[KPT];
+    uint32_t o[KPT]; // in bytes: n < 2^30
     if (full) {
         uint32_t k[KPT];
 #pragma unroll
         for (int j = 0; j < KPT; j++) k[j] = s_keys[tid + j * THREADS];
 #pragma unroll
-        for (int j = 0; j < KPT; j++) o[j] = s_goff[__builtin_amdgcn_ubfe(k[j], shift, width)] + tid + j * THREADS;
+        for (int j = 0; j < KPT; j++) o[j] = (s_goff[__builtin_amdgcn_ubfe(k[j], shift, width)] + tid + j * THREADS) * 4u;
         if (VALS && !SEQ) {
             uint32_t v[KPT];
 #pragma unroll
             for (int j = 0; j < KPT; j++) v[j] = s_vals[tid + j * THREADS];
 #pragma unroll
             for (int j = 0; j < KPT; j++) {
-                keys_out[o[j]] = k[j];
-                vals_out[o[j]] = v[j];
+                at32(keys_out, o[j]) = k[j];
+                at32(vals_out, o[j]) = v[j];
             }
         } else {
 #pragma unroll
-            for (int j = 0; j < KPT; j++) keys_out[o[j]] = k[j];
+            for (int j = 0; j < KPT; j++) at32(keys_out, o[j]) = k[j];
         }
     } else {
 #pragma unroll
@@ -448,12 +499,13 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
             o[j] = 0u;
             if (i < tile_count) {
                 const uint32_t k = s_keys[i];
-                o[j] = s_goff[__builtin_amdgcn_ubfe(k, shift, width)] + i;
-                keys_out[o[j]] = k;
-                if (VALS && !SEQ) vals_out[o[j]] = s_vals[i];
+                o[j] = (s_goff[__builtin_amdgcn_ubfe(k, shift, width)] + i) * 4u;
+                at32(keys_out, o[j]) = k;
+                if (VALS && !SEQ) at32(vals_out, o[j]) = s_vals[i];
             }
         }
     }
+    if (LATE) load_vals(); // the key stores are on their way, and most registers free
     if (SEQ) {
         // the values through the same staging buffer, to the destinations kept from the keys
         __syncthreads();
@@ -463,7 +515,7 @@ __global__ __launch_bounds__(WAVES * 64) void rs_onesweep_kernel(const uint32_t*
 #pragma unroll
         for (int j = 0; j < KPT; j++) {
             const uint32_t i = tid + j * THREADS;
-            if (full || i < tile_count) vals_out[o[j]] = s_keys[i];
+            if (full || i < tile_count) at32(vals_out, o[j]) = s_keys[i];
         }
     }
 }
@@ -554,22 +606,19 @@ int run_hist(vren_ctx* ctx, hipStream_t s, const uint32_t* keys, uint64_t n, uin
     uint32_t* hist = reinterpret_cast<uint32_t*>(scratch + L.hist);
     uint32_t* counters = reinterpret_cast<uint32_t*>(scratch + L.counters);
     uint32_t* status = reinterpret_cast<uint32_t*>(scratch + L.status_a);
-    const uint32_t blocks = takes_parts(KPT) ? parts_blocks(n) : 0u;
-    if (blocks) {
-        uint32_t* counts = reinterpret_cast<uint32_t*>(scratch + L.parts);
-        rs_hist_kernel<BITS, PAIRS, true><<<blocks, kHistThreads, 0, s>>>(keys, n, begin_bit, end_bit, passes, counts, status,
-                                                                          tiles * RADIX, counters);
-        VREN_LAUNCH_CHECK(ctx);
+    // up to kPartsMaxKeys keys the scratch holds the parts in a place of their own, above in the first pass's output,
+    // which is longer (n / 16384 parts of 4 KB at most) and not written before they are added up
+    const bool few = n <= kPartsMaxKeys;
+    const uint32_t blocks = few ? parts_room(n) : (uint32_t)std::min<uint64_t>((uint64_t)ctx->num_cus, n / 16384);
+    uint32_t* counts = reinterpret_cast<uint32_t*>(scratch + (few ? L.parts : L.tmp_keys));
+    rs_hist_kernel<BITS, PAIRS><<<blocks, kHistThreads, 0, s>>>(keys, n, begin_bit, end_bit, passes, counts, status,
+                                                                tiles * RADIX, counters);
+    VREN_LAUNCH_CHECK(ctx);
+    if (few && takes_parts(KPT)) {
         *parts = HistParts{counts, blocks};
         return VREN_OK;
     }
-    rs_init_kernel<<<1, 256, 0, s>>>(hist, passes * RADIX, counters, passes);
-    VREN_LAUNCH_CHECK(ctx);
-    const uint32_t hb = (uint32_t)std::min<uint64_t>((uint64_t)ctx->num_cus, std::max<uint64_t>(1, ceil_div_u64(n, 16384)));
-    rs_hist_kernel<BITS, PAIRS, false><<<hb, kHistThreads, 0, s>>>(keys, n, begin_bit, end_bit, passes, hist, status,
-                                                                   tiles * RADIX, counters);
-    VREN_LAUNCH_CHECK(ctx);
-    rs_hexscan_kernel<BITS><<<1, 256, 0, s>>>(hist, passes);
+    rs_hexscan_kernel<BITS><<<passes, 1024, 0, s>>>(counts, blocks, hist);
     VREN_LAUNCH_CHECK(ctx);
     *parts = HistParts{nullptr, 0};
     return VREN_OK;
@@ -817,13 +866,19 @@ const SortConfig kConfigs[] = {
 // longest stores. The smallest one stops at half the CUs, since the look-back over more tiles costs what the tile saves.
 // 2^16 pairs on 32 bits: 38.9 us in 4096-key tiles, 45.6 in 8192, 83.5 in 23552; 2^20: 79.5, 76.6, 101; 3 M: 142, 125,
 // 115 and 103 in 15360; 4.2 M: 173, 147, 123 and 148.
-RadixTile vren_radix_default_tile(uint64_t n, int num_cus)
+//
+// Above one 23552-key tile per CU: keys alone in 15360-key tiles, two workgroups to a CU (2^24 keys 224 us, in 23552-key
+// tiles 241; 2^26 682, 775); with values up to 20 M too (2^23 pairs 183, 192; 2^24 279, 288), above in 23552-key tiles,
+// whose digit runs fill more of a cache line in each of the two stores (25 M pairs 428, 423; 2^26 1175, 1072). Interleaved
+// pairs need more registers than two workgroups have.
+RadixTile vren_radix_default_tile(uint64_t n, int num_cus, bool vals, bool interleaved)
 {
     const uint64_t cus = (uint64_t)num_cus;
     if (n <= 4096 * cus / 2) return kRadixTile4096;
     if (n <= 8192 * cus) return kRadixTile8192;
     if (n <= 15360 * cus) return kRadixTile15360;
-    return kRadixTile23552;
+    if (n <= 23552 * cus || interleaved || (vals && n > 5u << 22)) return kRadixTile23552;
+    return kRadixTile15360;
 }
 
 int vren_radix_config_count() { return (int)(sizeof(kConfigs) / sizeof(kConfigs[0])); }
@@ -877,7 +932,7 @@ int vren_radix_sort_pairs_interleaved(vren_ctx* ctx, hipStream_t s, const uint32
         const auto sort = [&](auto run) {
             return run(ctx, s, in_pairs, out_pairs, n, begin_bit, end_bit, static_cast<char*>(scratch), L, starts, n_buckets);
         };
-        switch (vren_radix_default_tile(n, ctx->num_cus)) {
+        switch (vren_radix_default_tile(n, ctx->num_cus, true, true)) {
         case kRadixTile4096: st = sort(run_sort_pairs<8, 8, 8>); break;
         case kRadixTile8192: st = sort(run_sort_pairs<8, 8, 16>); break;
         case kRadixTile15360: st = sort(run_sort_pairs<8, 15, 16>); break;

@@ -5,7 +5,7 @@
 
 // keys per tile of an untuned sort: 8 keys per thread in 8 and 16 waves, 15 and 23 in 16 waves
 enum RadixTile { kRadixTile4096, kRadixTile8192, kRadixTile15360, kRadixTile23552 };
-RadixTile vren_radix_default_tile(uint64_t n, int num_cus);
+RadixTile vren_radix_default_tile(uint64_t n, int num_cus, bool vals, bool interleaved);
 
 int vren_radix_config_count();
 void vren_radix_config_info(int i, int* bits, int* kpt, int* waves, int* algorithm);
