@@ -124,6 +124,8 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
 }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// four words at any word's address: the hardware's wide accesses need 4-byte alignment
+typedef uint32_t vu4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 // 128-bit streaming (non-temporal) load / store of 4 uint32 at a 16-byte aligned address
 __device__ __forceinline__ uint4 ntload4(const void* p)

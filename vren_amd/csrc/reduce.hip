@@ -52,24 +52,26 @@ __device__ __forceinline__ float4 shfl_up_t<float4>(float4 v, unsigned d)
 
 constexpr int kThreads = 256; // scalar total
 
-// Up-sweep tile: kRows rows of kTreeThreads x E elements, E = 16 / sizeof(T), so that every thread loads and stores
+// Up-sweep tile: ROWS rows of THREADS x E elements, E = 16 / sizeof(T), so that every thread loads and stores
 // E consecutive elements of each row with one 16-byte access (coalesced across the wave). The tree levels inside
 // a thread's E elements are formed in registers, the next six across the lanes with shuffles (a wave covers an
-// aligned run of 64 E elements of a row), and the last six across the tile's 64 (row, wave) runs by one wave.
-constexpr int kTreeThreads = 512;
-constexpr int kTreeWaves = kTreeThreads / VREN_WAVE;
-constexpr int kRows = 8;
-static_assert(kRows * kTreeWaves == VREN_WAVE, "one run per lane of the finishing wave");
+// aligned run of 64 E elements of a row), and the last ones across the tile's (row, wave) runs by one wave.
+// Tiles have eight rows of 512 threads; a last pass, or an input, of at most one row of 1024 threads takes that: its time
+// is its latency, which eight rows of guarded accesses lengthen. With that and 16-byte accesses wherever four values are
+// inside the input, not in whole tiles alone: 2^20 values 12.0 -> 9.4 us, 2^22 15.0 -> 12.0, 10000001 22.7 -> 18.5.
+constexpr int kTreeThreads = 512, kTreeRows = 8, kSmallThreads = 1024;
 
 template <typename T>
-constexpr uint64_t tree_tile() { return (uint64_t)kTreeThreads * (16 / sizeof(T)) * kRows; }
+constexpr uint64_t tree_tile() { return (uint64_t)kTreeThreads * (16 / sizeof(T)) * kTreeRows; }
+template <typename T>
+constexpr uint64_t small_tile() { return (uint64_t)kSmallThreads * (16 / sizeof(T)); }
 
 // One tile of the view: elements e = tile * TILE + i, read from in[in_offset + e * in_stride] (identity at and
 // beyond `valid`) and written to out[offset + e * stride] (e < count). With `totals`, the tile's total (the node
 // at its last element) is also written to totals[segment * gridDim.x + tile], a compact array that the next pass
 // reads instead of the totals' strided places in the tree.
-template <typename T, typename Op>
-__global__ __launch_bounds__(kTreeThreads) void upsweep_tile_kernel(const T* in, T* out,
+template <typename T, typename Op, int THREADS, int ROWS>
+__global__ __launch_bounds__(THREADS) void upsweep_tile_kernel(const T* in, T* out,
                                                                     uint64_t in_seg_stride, uint64_t out_seg_stride,
                                                                     uint64_t valid, uint64_t count,
                                                                     uint64_t in_offset, uint64_t in_stride,
@@ -77,36 +79,44 @@ __global__ __launch_bounds__(kTreeThreads) void upsweep_tile_kernel(const T* in,
                                                                     T* __restrict__ totals)
 {
     constexpr int E = 16 / sizeof(T);
-    constexpr uint64_t TILE = tree_tile<T>();
-    static_assert(E * sizeof(T) == 16, "16-byte groups");
-    __shared__ T s_run[kRows * kTreeWaves];
+    constexpr int WAVES = THREADS / VREN_WAVE, RUNS = ROWS * WAVES;
+    constexpr uint64_t TILE = (uint64_t)THREADS * E * ROWS;
+    static_assert(E * sizeof(T) == 16 && RUNS <= VREN_WAVE, "16-byte groups; one run per lane of the finishing wave");
+    __shared__ T s_run[RUNS];
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
     const uint64_t seg = blockIdx.y;
     const T* src = in + seg * in_seg_stride;
     T* dst = out + seg * out_seg_stride;
     const uint64_t tile_start = (uint64_t)blockIdx.x * TILE;
-    const bool vin = in_stride == 1 && in_offset == 0 && tile_start + TILE <= valid &&
-                     (reinterpret_cast<uintptr_t>(src + tile_start) & 15) == 0;
-    const bool vout = stride == 1 && offset == 0 && tile_start + TILE <= count &&
-                      (reinterpret_cast<uintptr_t>(dst + tile_start) & 15) == 0;
+    const bool vin = in_stride == 1 && in_offset == 0, vout = stride == 1 && offset == 0;
+    const bool full_out = tile_start + TILE <= count;
 
-    T v[kRows][E];
+    T v[ROWS][E];
+    if (vin && tile_start + TILE <= valid) { // uniform: the loads of all rows in flight together
 #pragma unroll
-    for (int j = 0; j < kRows; j++) {
-        const uint64_t first = tile_start + ((uint64_t)j * kTreeThreads + tid) * E;
-        if (vin) {
-            const uint4 q = *reinterpret_cast<const uint4*>(src + first);
+        for (int j = 0; j < ROWS; j++) {
+            const vu4_any q = *reinterpret_cast<const vu4_any*>(src + tile_start + ((uint64_t)j * THREADS + tid) * E);
             memcpy(&v[j][0], &q, 16);
-        } else {
+        }
+    } else {
 #pragma unroll
-            for (int c = 0; c < E; c++) {
-                const uint64_t e = first + c;
-                v[j][c] = e < valid ? src[in_offset + e * in_stride] : Op::identity();
+        for (int j = 0; j < ROWS; j++) {
+            const uint64_t first = tile_start + ((uint64_t)j * THREADS + tid) * E;
+#pragma unroll
+            for (int c = 0; c < E; c++) v[j][c] = Op::identity();
+            if (first >= valid) continue;
+            if (vin && first + E <= valid) {
+                const vu4_any q = *reinterpret_cast<const vu4_any*>(src + first);
+                memcpy(&v[j][0], &q, 16);
+            } else {
+#pragma unroll
+                for (int c = 0; c < E; c++)
+                    if (first + c < valid) v[j][c] = src[in_offset + (first + c) * in_stride];
             }
         }
     }
 #pragma unroll
-    for (int j = 0; j < kRows; j++) {
+    for (int j = 0; j < ROWS; j++) {
         // levels inside the thread's E elements
 #pragma unroll
         for (int l = 1; l < E; l <<= 1) {
@@ -122,32 +132,32 @@ __global__ __launch_bounds__(kTreeThreads) void upsweep_tile_kernel(const T* in,
             if ((lane & (2 * l - 1)) == 2 * l - 1) x = Op::apply(x, o);
         }
         v[j][E - 1] = x;
-        if (lane == VREN_WAVE - 1) s_run[j * kTreeWaves + wave] = x;
+        if (lane == VREN_WAVE - 1) s_run[j * WAVES + wave] = x;
     }
     __syncthreads();
     if (wave == 0) {
-        // levels across the 64 runs, in element order (row-major over (row, wave))
-        T x = s_run[lane];
+        // levels across the runs, in element order (row-major over (row, wave))
+        T x = s_run[lane % RUNS];
 #pragma unroll
-        for (unsigned l = 1; l < VREN_WAVE; l <<= 1) {
+        for (unsigned l = 1; l < RUNS; l <<= 1) {
             T o = shfl_up_t(x, l);
             if ((lane & (2 * l - 1)) == 2 * l - 1) x = Op::apply(x, o);
         }
-        s_run[lane] = x;
+        if (lane < RUNS) s_run[lane] = x;
     }
     __syncthreads();
-    if (totals && tid == 0) totals[seg * gridDim.x + blockIdx.x] = s_run[kRows * kTreeWaves - 1];
+    if (totals && tid == 0) totals[seg * gridDim.x + blockIdx.x] = s_run[RUNS - 1];
     if (lane == VREN_WAVE - 1) {
 #pragma unroll
-        for (int j = 0; j < kRows; j++) v[j][E - 1] = s_run[j * kTreeWaves + wave];
+        for (int j = 0; j < ROWS; j++) v[j][E - 1] = s_run[j * WAVES + wave];
     }
 #pragma unroll
-    for (int j = 0; j < kRows; j++) {
-        const uint64_t first = tile_start + ((uint64_t)j * kTreeThreads + tid) * E;
-        if (vout) {
-            uint4 q;
+    for (int j = 0; j < ROWS; j++) {
+        const uint64_t first = tile_start + ((uint64_t)j * THREADS + tid) * E;
+        if (vout && (full_out || first + E <= count)) {
+            vu4_any q;
             memcpy(&q, &v[j][0], 16);
-            *reinterpret_cast<uint4*>(dst + first) = q;
+            *reinterpret_cast<vu4_any*>(dst + first) = q;
         } else {
 #pragma unroll
             for (int c = 0; c < E; c++) {
@@ -178,12 +188,14 @@ int reduce_tree(vren_ctx* ctx, hipStream_t s, const T* in, uint32_t n, T* out, u
         const uint64_t tiles = ceil_div_u64(count, TILE);
         const dim3 grid((uint32_t)tiles, blocks);
         T* totals = count > TILE ? buf[pass & 1] : nullptr;
-        if (pass == 0) {
-            upsweep_tile_kernel<T, Op><<<grid, kTreeThreads, 0, s>>>(in, out, n, p, n, count, 0, 1, 0, 1, totals);
-        } else {
-            upsweep_tile_kernel<T, Op><<<grid, kTreeThreads, 0, s>>>(buf[(pass - 1) & 1], out, count, p, count, count,
-                                                                     0, 1, offset, stride, totals);
-        }
+        const T* from = pass == 0 ? in : buf[(pass - 1) & 1];
+        const uint64_t valid = pass == 0 ? n : count, from_seg = valid;
+        if (count <= small_tile<T>())
+            upsweep_tile_kernel<T, Op, kSmallThreads, 1><<<grid, kSmallThreads, 0, s>>>(from, out, from_seg, p, valid, count, 0,
+                                                                                        1, offset, stride, totals);
+        else
+            upsweep_tile_kernel<T, Op, kTreeThreads, kTreeRows><<<grid, kTreeThreads, 0, s>>>(
+                from, out, from_seg, p, valid, count, 0, 1, offset, stride, totals);
         VREN_LAUNCH_CHECK(ctx);
         if (count <= TILE) break;
         // next view: the tile totals

@@ -16,9 +16,6 @@ namespace {
 // for 16384-element tiles took as long as the copy did.
 constexpr uint32_t kTile = 16384; // of the smallest tile
 
-// four elements at any element's address: the hardware's wide accesses need 4-byte alignment
-typedef uint32_t vu4_any __attribute__((ext_vector_type(4), aligned(4)));
-
 __global__ void scan_init_kernel(uint64_t* status, uint64_t n_status, uint32_t* counter)
 {
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
