@@ -205,6 +205,22 @@ VREN_HD uint32_t vren_third_index(float u)
     return (uint32_t)(u >= -0x1.555554p-2f) + (uint32_t)(u >= 0x1.555556p-2f) + (uint32_t)(u >= 0x1.fffffep-1f);
 }
 
+/* r / ext for 0 <= |r| <= ext, with rec = 1 / ext correctly rounded, by two fused steps in place of a division, wherever
+ * vren_unit_quotient_holds: the floor of the quotient times a power of two up to 2^10 is that of the correctly rounded
+ * quotient (for a positive one its float too: every divisor mantissa was compared at the dividends next to every
+ * multiple of 2^-10). A dividend above the extent takes the division: the product r * rec could overflow, and the
+ * residual would make a NaN of it. Extents under 2^-60 take it too: their residuals could be too small for a float. */
+VREN_HD int vren_unit_quotient_holds(float r, float ext)
+{
+    return ext > 0x1p-60f && ext < 0x1p100f && __builtin_fabsf(r) <= ext;
+}
+
+VREN_HD float vren_unit_quotient(float r, float ext, float rec)
+{
+    const float q = r * rec;
+    return __builtin_fmaf(__builtin_fmaf(-q, ext, r), rec, q);
+}
+
 VREN_HD float vren_dot3(const float a[3], const float b[3])
 {
     return (a[0] * b[0] + a[1] * b[1]) + a[2] * b[2];

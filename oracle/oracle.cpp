@@ -15,6 +15,7 @@
  *                        agrees (the FMA and the division here are correctly rounded by the C library)
  *   o_third_index_mismatches  a planted threshold one float off is reported
  *   o_texel_axis_mismatches  a planted error of the reciprocal is reported
+ *   o_unit_quotient_mismatches  a planted error of the reciprocal is reported
  *   o_reduce_tree_*      closed form tree[i] = op over the aligned block ending at i; totals vs numpy
  *   o_exclusive_scan_u32 numpy cumsum (uint32 wrap-around)
  *   o_stable_sort_kv     numpy argsort(kind='stable')
@@ -210,6 +211,27 @@ OEXPORT uint32_t o_texel_axis_mismatches(const float* s, uint64_t n, uint32_t si
         vren_texel_axis(s[i], size, filter, mode, &a0, &a1, &wa);
         vren_texel_axis_near(s[i], size, r, filter, mode, &b0, &b1, &wb);
         bad += a0 != b0 || a1 != b1 || vren_f32_bits(wa) != vren_f32_bits(wb);
+    }
+    return bad;
+}
+
+/* Pairs (r[i], ext[i]) for which the fused quotient (vren_unit_quotient, where it holds; else the division, as the light
+ * stage takes it) and the division fall into different cells of 2^bits; `planted` moves the reciprocal by one part in
+ * 2^20, which must then be reported. *fused receives the number of pairs that took the fused form. */
+OEXPORT uint32_t o_unit_quotient_mismatches(const float* r, const float* ext, uint64_t n, uint32_t bits, uint32_t planted,
+                                            uint64_t* fused)
+{
+    const float scale = (float)(1u << bits);
+    uint32_t bad = 0;
+    *fused = 0;
+    for (uint64_t i = 0; i < n; i++) {
+        const float d = r[i] / ext[i];
+        float rec = 1.0f / ext[i];
+        if (planted) rec *= 1.0f - 0x1p-20f;
+        const int holds = vren_unit_quotient_holds(r[i], ext[i]);
+        const float t = holds ? (planted ? r[i] * rec : vren_unit_quotient(r[i], ext[i], rec)) : d;
+        *fused += holds ? 1 : 0;
+        bad += vren_f2u_sat(vren_floorf(t * scale)) != vren_f2u_sat(vren_floorf(d * scale));
     }
     return bad;
 }

@@ -256,26 +256,25 @@ __device__ __forceinline__ void lights_body(const FrameDev* __restrict__ frames,
     // Morton codes (discretize_point_light_positions.comp:26-43), paired with the light index
     const uint32_t bits = fd.morton_bits, total_bits = 3 * bits;
     const float scale = (float)(1u << bits);
-    // The quotients (r - lo) / (hi - lo) by one correctly rounded reciprocal per axis and two fused steps, which give
-    // the division's own result (Markstein) while nothing over- or underflows; a quotient too small for that quantises
-    // to 0 either way. Extents or positions beyond 2^100 take the division.
+    // The quotients (r - lo) / (hi - lo) by one correctly rounded reciprocal per axis and two fused steps (vmath.h), if every
+    // light of the wave is inside the box on every axis, as all are in the lights' own box; a given box takes the
+    // division where one is not.
     float ext[3], rec[3];
-    bool plain = true;
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         ext[a] = hi[a] - lo[a];
         rec[a] = 1.0f / ext[a];
-        plain = plain && ext[a] > 0x1p-100f && ext[a] < 0x1p100f;
     }
+    bool inside = true;
 #pragma unroll
     for (int j = 0; j < kLKPT; j++)
         if (j < (int)kpt && wbase + j * VREN_WAVE + lane < n)
 #pragma unroll
             for (int a = 0; a < 3; a++) {
                 r[j][a] = r[j][a] - lo[a];
-                plain = plain && __builtin_fabsf(r[j][a]) < 0x1p100f;
+                inside = inside && vren_unit_quotient_holds(r[j][a], ext[a]);
             }
-    const bool fused = ballot(!plain) == 0;
+    const bool fused = ballot(!inside) == 0;
     uint2 e[kLKPT];
 #pragma unroll
     for (int j = 0; j < kLKPT; j++) {
@@ -286,12 +285,8 @@ __device__ __forceinline__ void lights_body(const FrameDev* __restrict__ frames,
 #pragma unroll
             for (int a = 0; a < 3; a++) {
                 float t;
-                if (fused) { // uniform
-                    const float q0 = r[j][a] * rec[a];
-                    t = __builtin_fmaf(__builtin_fmaf(-q0, ext[a], r[j][a]), rec[a], q0);
-                } else {
-                    t = r[j][a] / ext[a];
-                }
+                if (fused) t = vren_unit_quotient(r[j][a], ext[a], rec[a]); // uniform
+                else t = r[j][a] / ext[a];
                 q[a] = floor_u32_sat(t * scale);
             }
             e[j] = make_uint2(morton_interleave(q[0], q[1], q[2], bits), first + i);
