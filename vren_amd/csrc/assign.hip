@@ -775,15 +775,9 @@ extern "C" VREN_EXPORT int vren_assign_lights(vren_ctx* ctx, vren_stream_t strea
         VREN_LAUNCH_CHECK(ctx);
         return VREN_OK;
     }
-    // list slots for the first clusters, as a batch has them; a capture that would have to grow the scratch for them does
-    // without (every list is then traversed a second time)
-    const uint32_t slot_cap = std::min<uint32_t>(key_capacity, VREN_SLOT_CLUSTERS);
-    if (vren_can_have_scratch(ctx, (size_t)slot_cap * VREN_LIST_SLOT * 4, s)) {
-        st = vren_ensure_scratch(ctx, (size_t)slot_cap * VREN_LIST_SLOT * 4, s);
-        if (st) return st;
-        f.list_slots = static_cast<uint32_t*>(ctx->scratch);
-        f.slot_cap = slot_cap;
-    }
+    // list slots for the first clusters, as a batch has them (without them every list is traversed a second time)
+    f.list_slots = ctx->list_slots;
+    f.slot_cap = ctx->list_slots ? std::min<uint32_t>(key_capacity, VREN_SLOT_CLUSTERS) : 0u;
     ChainWork w;
     memset(&w, 0, sizeof(w));
     w.max_L = light_count;

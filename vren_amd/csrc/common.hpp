@@ -219,6 +219,9 @@ struct vren_ctx {
     // grow-only device scratch for primitives that do not take a caller scratch buffer
     void* scratch = nullptr;
     size_t scratch_bytes = 0;
+    // list slots of vren_assign_lights (VREN_SLOT_CLUSTERS clusters), made with the context and never moved, so that a
+    // captured call's address stays good; null where there was no memory for them
+    uint32_t* list_slots = nullptr;
     // ring of device frame-descriptor slots for the single-frame stage entry points
     FrameDev* frame_slots = nullptr;
     uint32_t frame_slot_next = 0;
@@ -236,8 +239,6 @@ struct vren_ctx {
 int vren_fail(vren_ctx* ctx, int status, const char* fmt, ...);
 int vren_hip_fail(vren_ctx* ctx, hipError_t err, const char* what);
 int vren_ensure_scratch(vren_ctx* ctx, size_t bytes, hipStream_t s);
-// whether vren_ensure_scratch can give this much: always, but for a stream capture that it would have to grow in
-bool vren_can_have_scratch(vren_ctx* ctx, size_t bytes, hipStream_t s);
 int vren_noalloc_scan_setup(vren_ctx* ctx);
 
 #define VREN_HIP(ctx, expr)                                                                                            \

@@ -51,13 +51,6 @@ int vren_ensure_scratch(vren_ctx* ctx, size_t bytes, hipStream_t s)
     return VREN_OK;
 }
 
-bool vren_can_have_scratch(vren_ctx* ctx, size_t bytes, hipStream_t s)
-{
-    if (bytes <= ctx->scratch_bytes) return true;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
-}
-
 extern "C" {
 
 VREN_EXPORT int vren_create(int hip_device, vren_ctx** out)
@@ -84,6 +77,10 @@ VREN_EXPORT int vren_create(int hip_device, vren_ctx** out)
     if (e == hipSuccess) e = hipMalloc(&ctx->frame_slots, sizeof(FrameDev) * VREN_FRAME_SLOTS);
     if (e == hipSuccess && vren_noalloc_scan_setup(ctx) != VREN_OK) e = hipErrorInvalidSymbol;
     if (e == hipSuccess) e = hipDeviceSynchronize();
+    if (e == hipSuccess && hipMalloc(&ctx->list_slots, (size_t)VREN_SLOT_CLUSTERS * VREN_LIST_SLOT * 4) != hipSuccess) {
+        ctx->list_slots = nullptr; // vren_assign_lights does without
+        (void)hipGetLastError();
+    }
     if (e != hipSuccess) {
         vren_destroy(ctx);
         return e == hipErrorOutOfMemory ? VREN_ENOMEM : VREN_EHIP;
@@ -103,6 +100,7 @@ VREN_EXPORT void vren_destroy(vren_ctx* ctx)
     vren_teardown(hipDeviceSynchronize());
     if (ctx->d_flags) vren_teardown(hipFree(ctx->d_flags));
     if (ctx->scratch) vren_teardown(hipFree(ctx->scratch));
+    if (ctx->list_slots) vren_teardown(hipFree(ctx->list_slots));
     if (ctx->frame_slots) vren_teardown(hipFree(ctx->frame_slots));
     delete ctx;
 }
