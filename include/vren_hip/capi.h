@@ -11,7 +11,8 @@
  *   - a vren_ctx is not thread-safe (one per host thread), mirroring single-threaded command recording, and is
  *     used from one stream at a time: the primitives that take no caller scratch share the context's scratch
  *     buffer. Growing it synchronises the device, so a call that would grow it during a stream capture fails
- *     with VREN_EINVAL (make the same call once outside the capture first), and a graph captured over it is
+ *     with VREN_EINVAL (make the same call once outside the capture first). Blocks of up
+ *     to 64 MB that it outgrows are kept for the graphs captured over them; a graph captured over a larger one is
  *     replayed only while it has not grown since. vren_assign_lights takes nothing from it: its 25 MB of list
  *     slots are made with the context;
  *   - capacity overflows that only the device can see (unique clusters, assigned lights) never write out of

@@ -219,6 +219,9 @@ struct vren_ctx {
     // grow-only device scratch for primitives that do not take a caller scratch buffer
     void* scratch = nullptr;
     size_t scratch_bytes = 0;
+    // scratch blocks that it has outgrown (vren_ensure_scratch): 1 MB, 2, 4, .. 64 at least
+    void* kept_scratch[8] = {};
+    uint32_t kept_scratch_count = 0;
     // list slots of vren_assign_lights (VREN_SLOT_CLUSTERS clusters), made with the context and never moved, so that a
     // captured call's address stays good; null where there was no memory for them
     uint32_t* list_slots = nullptr;

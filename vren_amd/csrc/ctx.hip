@@ -1,4 +1,5 @@
 // ctx.hip -- context lifetime, status reporting and the host-only helpers of the C ABI.
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
@@ -24,10 +25,25 @@ int vren_hip_fail(vren_ctx* ctx, hipError_t err, const char* what)
 }
 
 // The context's scratch serves one stream at a time (a context is used from one stream, like the reference's
-// single command buffer per recording thread). Growing it synchronises the device and frees the old buffer, which
-// must not happen while `s` is being captured: the capture would break, and a graph captured earlier would keep a
-// pointer into freed memory. A capture therefore needs the scratch already grown by an earlier call of the same
-// size outside the capture.
+// single command buffer per recording thread). It must not grow while `s` is being captured: a capture needs it
+// already grown by an earlier call of the same size outside the capture.
+// A graph captured earlier keeps the address of the scratch that it was captured with. A call a little larger than
+// those before it (a bucket sort of 113 000 pairs is the first past the first megabyte) must not free that memory
+// under the graph, so blocks up to kKeptScratch are kept until the context is destroyed; each is at least twice as large
+// as the one before, which bounds them to 128 MB in all. Larger ones are freed when the device is done with them.
+static constexpr size_t kFirstScratch = 1u << 20, kKeptScratch = 64u << 20;
+
+static hipError_t free_kept_scratch(vren_ctx* ctx)
+{
+    hipError_t e = hipSuccess;
+    for (void*& p : ctx->kept_scratch) {
+        if (p && e == hipSuccess) e = hipFree(p);
+        p = nullptr;
+    }
+    ctx->kept_scratch_count = 0;
+    return e;
+}
+
 int vren_ensure_scratch(vren_ctx* ctx, size_t bytes, hipStream_t s)
 {
     if (bytes <= ctx->scratch_bytes) return VREN_OK;
@@ -38,15 +54,31 @@ int vren_ensure_scratch(vren_ctx* ctx, size_t bytes, hipStream_t s)
                          "context scratch must grow to %zu bytes during a stream capture; make the same call once "
                          "outside the capture first",
                          bytes);
-    if (ctx->scratch) {
+    const bool keep = ctx->scratch && ctx->scratch_bytes <= kKeptScratch;
+    if (ctx->scratch && !keep) {
         // a grown scratch replaces the old one only after the device is done with it
         VREN_HIP(ctx, hipDeviceSynchronize());
         VREN_HIP(ctx, hipFree(ctx->scratch));
         ctx->scratch = nullptr;
         ctx->scratch_bytes = 0;
     }
-    size_t sz = bytes < (1u << 20) ? (1u << 20) : bytes;
-    VREN_HIP(ctx, hipMalloc(&ctx->scratch, sz));
+    size_t sz = std::max(bytes, keep ? 2 * ctx->scratch_bytes : kFirstScratch);
+    void* block = nullptr;
+    hipError_t e = hipMalloc(&block, sz);
+    if (e != hipSuccess && keep) {
+        // no memory beside the old blocks: in place of them
+        (void)hipGetLastError();
+        VREN_HIP(ctx, hipDeviceSynchronize());
+        VREN_HIP(ctx, free_kept_scratch(ctx));
+        VREN_HIP(ctx, hipFree(ctx->scratch));
+        ctx->scratch = nullptr;
+        ctx->scratch_bytes = 0;
+        sz = bytes;
+        e = hipMalloc(&block, sz);
+    }
+    VREN_HIP(ctx, e);
+    if (ctx->scratch) ctx->kept_scratch[ctx->kept_scratch_count++] = ctx->scratch;
+    ctx->scratch = block;
     ctx->scratch_bytes = sz;
     return VREN_OK;
 }
@@ -100,6 +132,7 @@ VREN_EXPORT void vren_destroy(vren_ctx* ctx)
     vren_teardown(hipDeviceSynchronize());
     if (ctx->d_flags) vren_teardown(hipFree(ctx->d_flags));
     if (ctx->scratch) vren_teardown(hipFree(ctx->scratch));
+    vren_teardown(free_kept_scratch(ctx));
     if (ctx->list_slots) vren_teardown(hipFree(ctx->list_slots));
     if (ctx->frame_slots) vren_teardown(hipFree(ctx->frame_slots));
     delete ctx;
