@@ -343,7 +343,18 @@ VREN_EXPORT int vren_batch_run(vren_batch* b, vren_stream_t stream, int mode)
         }
         return VREN_OK;
     }
-    if (mode == VREN_RUN_BATCHED) return run_chain(b, s, b->d_table, b->F, b->w, b->total_live_slots);
+    if (mode == VREN_RUN_BATCHED) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cs) != hipSuccess) (void)hipGetLastError();
+        if (cs == hipStreamCaptureStatusNone) return run_chain(b, s, b->d_table, b->F, b->w, b->total_live_slots);
+        // recorded into the caller's graph: it clears the work memory itself, whatever runs between its replays, and
+        // what the memory holds now does not change
+        const bool dirty = b->dirty;
+        b->dirty = true;
+        const int st = run_chain(b, s, b->d_table, b->F, b->w, b->total_live_slots);
+        b->dirty = dirty;
+        return st;
+    }
     if (mode == VREN_RUN_GRAPH) {
         if (!b->exec) {
             // the capture stream lives as long as the batch (created once, destroyed by vren_batch_destroy); a
