@@ -512,11 +512,17 @@ struct TileRanges {
 // each, which sums the counts before its run itself (a frame holds a few thousand clusters; a launch of its own for
 // their prefix sum took longer) and takes its run 256 clusters at a time: their offsets by a block scan, then their
 // lists, which are consecutive in the index buffer, as one range of entries spread over the threads, each finding its
-// cluster among the 256 prefixes and copying it from the slot that the counting pass kept. A list longer than a slot is
-// traversed again (bitmask, emitted in ascending light index) by one of the `masks` waves that have room for a bitmask.
+// cluster among the 256 prefixes and copying it from the slot that the counting pass kept.
+// A list that has no slot or is longer than one is traversed again (bitmask, emitted in ascending light index) by a
+// wave with room for a bitmask, `masks` of a workgroup. The clusters that meet many lights sit together in the image, so
+// a run has a `team` of workgroups for them: the first also writes the run's offsets, copies and ranges, the helpers
+// traverse their share of the long lists, and leave at once where there are none. One workgroup a run made frames of
+// long lists slower than a pass of their own had been; with teams (us, counting, offsets and lists, then | in one pass each |
+// one workgroup | team): 1920x1080 with 4096 lights of six times the radius 201 | 213 | 121, 3840x2160 with 65536 of twice
+// the radius 507 | 522 | 376, 8192x8192 with 110 k clusters 328 | 444 | 231; a frame without long lists takes what it took
+// (640x360 42.6 a frame, 3840x2160 with 65536 lights 563), since a helper leaves as soon as it sees that it has no share.
 // 64 frames of 1080p with 4096 lights took 6 + 54 us in two launches, the copies one cluster per wave and step with a
-// load's latency each, and take 24; one
-// frame 5 + 4.8, now 6.7; a 3840x2160 frame with 65536 lights 12 + 15, now 16.
+// load's latency each, and take 24; one frame 5 + 4.8, now 6.7; a 3840x2160 frame with 65536 lights 12 + 15, now 16.
 constexpr uint32_t kListThreads = 256;
 constexpr int kListUnroll = 4; // entries per thread and step
 
@@ -532,8 +538,9 @@ __device__ __forceinline__ uint32_t list_sum(uint32_t v, uint32_t* s_wave)
     return sum;
 }
 
-__device__ __forceinline__ void assign_lists_body(const FrameDev& fd, uint32_t part, uint32_t parts, uint32_t mask_words,
-                                                  uint32_t masks, const TileRanges ranges, uint32_t* s_mem)
+__device__ __forceinline__ void assign_lists_body(const FrameDev& fd, uint32_t part, uint32_t parts, uint32_t helper,
+                                                  uint32_t team, uint32_t mask_words, uint32_t masks,
+                                                  const TileRanges ranges, uint32_t* s_mem)
 {
     __shared__ uint32_t s_pre[kListThreads + 1]; // list starts of the 256 clusters, relative to the first one's
     __shared__ uint32_t s_wave[kListThreads / VREN_WAVE];
@@ -542,7 +549,16 @@ __device__ __forceinline__ void assign_lists_body(const FrameDev& fd, uint32_t p
     const uint32_t n = (fd.L == 0 || fd.cluster_count == nullptr) ? 0u : min(*fd.cluster_count, fd.key_cap);
     const uint32_t run_len = (n + parts - 1) / parts;
     const uint32_t begin = min(part * run_len, n), end = min(begin + run_len, n);
-    const bool last = part == parts - 1;
+    const bool last = part == parts - 1 && helper == 0;
+    const auto kept = [&](uint32_t c, uint32_t cnt) {
+        return fd.list_slots != nullptr && c < fd.slot_cap && cnt <= VREN_LIST_SLOT;
+    };
+    if (helper) {
+        if (run_len <= helper * masks) return; // the waves before these take every list of a run
+        bool any = false;
+        for (uint32_t c = begin + tid; c < end; c += kListThreads) any = any || !kept(c, load_at<uint32_t>(fd.counts, c));
+        if (!__syncthreads_or(any)) return; // the whole workgroup
+    }
     uint32_t sum = 0;
     const uint32_t quads = (reinterpret_cast<uintptr_t>(fd.counts) & 15) == 0 ? begin / 4 : 0u;
 #pragma unroll 8
@@ -554,7 +570,7 @@ __device__ __forceinline__ void assign_lists_body(const FrameDev& fd, uint32_t p
     uint32_t run = list_sum(sum, s_wave);
 
     // first clusters ascend over the frame's tiles, so 256 of them, one per thread, bracket each sub-run's tiles
-    const uint32_t tiles = ranges.tile_range ? fd.Sx * fd.Sy : 0u;
+    const uint32_t tiles = ranges.tile_range && helper == 0 ? fd.Sx * fd.Sy : 0u;
     const uint2* tile_cl = ranges.tile_cl + fd.tile_base;
     const uint32_t step = (tiles + kListThreads - 1) / kListThreads;
     uint32_t sample = 0xFFFFFFFFu;
@@ -571,14 +587,14 @@ __device__ __forceinline__ void assign_lists_body(const FrameDev& fd, uint32_t p
         const uint32_t cnt = tid < m ? load_at<uint32_t>(fd.counts, c) : 0u;
         uint32_t total;
         const uint32_t ex = block_exclusive_sum<kListThreads>(cnt, s_wave, &total);
-        if (tid < m) fd.offsets[c] = run + ex;
-        const bool kept = fd.list_slots != nullptr && c < fd.slot_cap && cnt <= VREN_LIST_SLOT;
-        const uint64_t longs = ballot(tid < m && !kept);
+        if (tid < m && helper == 0) fd.offsets[c] = run + ex;
+        const uint64_t longs = ballot(tid < m && !kept(c, cnt));
         if (lane == 0) s_long[wave] = longs;
         s_pre[tid] = ex;
         if (tid == 0) s_pre[kListThreads] = total;
         __syncthreads();
-        for (uint32_t q0 = 0; q0 < total; q0 += kListThreads * kListUnroll) { // entries whose searches and loads overlap
+        const uint32_t copied = helper == 0 ? total : 0u;
+        for (uint32_t q0 = 0; q0 < copied; q0 += kListThreads * kListUnroll) { // entries whose searches and loads overlap
             uint32_t at[kListUnroll];
 #pragma unroll
             for (int u = 0; u < kListUnroll; u++) at[u] = 0;
@@ -621,7 +637,7 @@ __device__ __forceinline__ void assign_lists_body(const FrameDev& fd, uint32_t p
             uint32_t seen = 0; // long lists of the sub-run so far
             for (uint32_t w = 0; w < kListThreads / VREN_WAVE; w++) {
                 for (uint64_t rem = s_long[w]; rem; rem &= rem - 1, seen++) {
-                    if (seen % masks != wave) continue;
+                    if (seen % (masks * team) != helper * masks + wave) continue;
                     const uint32_t i = w * VREN_WAVE + (uint32_t)__builtin_ctzll(rem);
                     if (s_pre[i + 1] == s_pre[i]) continue; // an empty list past the slots
                     if (!cleared) {
@@ -663,18 +679,21 @@ __global__ __launch_bounds__(256, 8) void assign_count_one_kernel(const FrameDev
     extern __shared__ uint32_t s_mem[];
     assign_count_body<false>(inline_frame(), 1, s_mem);
 }
-__global__ __launch_bounds__(kListThreads) void assign_lists_kernel(const FrameDev* __restrict__ frames, uint32_t parts,
-                                                                    uint32_t mask_words, uint32_t masks,
-                                                                    const TileRanges ranges)
+// grid: the first workgroups of all runs, then the helpers
+__global__ __launch_bounds__(kListThreads) void assign_lists_kernel(const FrameDev* __restrict__ frames, uint32_t runs,
+                                                                    uint32_t parts, uint32_t team, uint32_t mask_words,
+                                                                    uint32_t masks, const TileRanges ranges)
 {
     extern __shared__ uint32_t s_mem[];
-    assign_lists_body(frames[blockIdx.x / parts], blockIdx.x % parts, parts, mask_words, masks, ranges, s_mem);
+    const uint32_t helper = blockIdx.x / runs, r = blockIdx.x - helper * runs;
+    assign_lists_body(frames[r / parts], r % parts, parts, helper, team, mask_words, masks, ranges, s_mem);
 }
-__global__ __launch_bounds__(kListThreads) void assign_lists_one_kernel(const FrameDev one, uint32_t parts,
+__global__ __launch_bounds__(kListThreads) void assign_lists_one_kernel(const FrameDev one, uint32_t parts, uint32_t team,
                                                                         uint32_t mask_words, uint32_t masks)
 {
     extern __shared__ uint32_t s_mem[];
-    assign_lists_body(*inline_frame(), blockIdx.x, parts, mask_words, masks, TileRanges{nullptr, nullptr}, s_mem);
+    assign_lists_body(*inline_frame(), blockIdx.x % parts, parts, blockIdx.x / parts, team, mask_words, masks,
+                      TileRanges{nullptr, nullptr}, s_mem);
 }
 
 __global__ void empty_lists_kernel(uint32_t* counts, uint32_t* offsets, uint32_t n, uint32_t* total)
@@ -708,10 +727,13 @@ int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32
     const uint32_t count_blocks = persistent_blocks(ctx, 4, w.assign_wpc);
     // list runs per frame: 2048 workgroups over a batch, at most 512 and at least 8 a frame
     const uint32_t parts = std::max<uint32_t>(8, std::min<uint32_t>(512, 2048 / F));
+    // and up to 4096 workgroups, four a run at most, for the long lists (64 frames of 1920x1080 with 4096 lights of four
+    // times the radius: lists 740 us with one a run, 445 with two)
+    const uint32_t runs = F * parts, team = std::max<uint32_t>(1, std::min<uint32_t>(4, 4096 / runs));
     if (one) {
         assign_count_one_kernel<<<count_blocks, 4 * VREN_WAVE, count_per_wave * 4, s>>>(*one);
         VREN_LAUNCH_CHECK(ctx);
-        assign_lists_one_kernel<<<parts, kListThreads, per_mask * masks, s>>>(*one, parts, mask_words, masks);
+        assign_lists_one_kernel<<<runs * team, kListThreads, per_mask * masks, s>>>(*one, parts, team, mask_words, masks);
         VREN_LAUNCH_CHECK(ctx);
         return VREN_OK;
     }
@@ -720,8 +742,8 @@ int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32
     VREN_LAUNCH_CHECK(ctx);
     chain_mark(w, s);
     chain_mark(w, s); // the offsets are written with the lists
-    assign_lists_kernel<<<F * parts, kListThreads, per_mask * masks, s>>>(d_frames, parts, mask_words, masks,
-                                                                          TileRanges{w.tile_cl, w.tile_range});
+    assign_lists_kernel<<<runs * team, kListThreads, per_mask * masks, s>>>(d_frames, runs, parts, team, mask_words, masks,
+                                                                            TileRanges{w.tile_cl, w.tile_range});
     VREN_LAUNCH_CHECK(ctx);
     chain_mark(w, s);
     return VREN_OK;
