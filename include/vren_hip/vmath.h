@@ -210,9 +210,14 @@ VREN_HD uint32_t vren_third_index(float u)
  * quotient (for a positive one its float too: every divisor mantissa was compared at the dividends next to every
  * multiple of 2^-10). A dividend above the extent takes the division: the product r * rec could overflow, and the
  * residual would make a NaN of it. Extents under 2^-60 take it too: their residuals could be too small for a float. */
+VREN_HD int vren_unit_quotient_extent(float ext)
+{
+    return ext > 0x1p-60f && ext < 0x1p100f;
+}
+
 VREN_HD int vren_unit_quotient_holds(float r, float ext)
 {
-    return ext > 0x1p-60f && ext < 0x1p100f && __builtin_fabsf(r) <= ext;
+    return vren_unit_quotient_extent(ext) && __builtin_fabsf(r) <= ext;
 }
 
 VREN_HD float vren_unit_quotient(float r, float ext, float rec)

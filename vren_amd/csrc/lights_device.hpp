@@ -260,19 +260,20 @@ __device__ __forceinline__ void lights_body(const FrameDev* __restrict__ frames,
     // light of the wave is inside the box on every axis, as all are in the lights' own box; a given box takes the
     // division where one is not.
     float ext[3], rec[3];
+    bool inside = true;
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         ext[a] = hi[a] - lo[a];
         rec[a] = 1.0f / ext[a];
+        inside = inside && vren_unit_quotient_extent(ext[a]);
     }
-    bool inside = true;
 #pragma unroll
     for (int j = 0; j < kLKPT; j++)
         if (j < (int)kpt && wbase + j * VREN_WAVE + lane < n)
 #pragma unroll
             for (int a = 0; a < 3; a++) {
                 r[j][a] = r[j][a] - lo[a];
-                inside = inside && vren_unit_quotient_holds(r[j][a], ext[a]);
+                inside = inside && __builtin_fabsf(r[j][a]) <= ext[a];
             }
     const bool fused = ballot(!inside) == 0;
     uint2 e[kLKPT];
