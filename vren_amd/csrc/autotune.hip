@@ -20,15 +20,16 @@ uint64_t bucket_key(uint64_t n, bool vals, uint32_t key_bits)
     return ((uint64_t)ilog2_u64(n) << 8) | ((uint64_t)(vals ? 1 : 0) << 7) | key_bits;
 }
 
-// the configuration when nothing is tuned or forced: onesweep with the default tile of n keys
+// the configuration when nothing is tuned or forced: one workgroup, or onesweep with the default tile of n keys
 int default_config(uint64_t n, bool vals, int num_cus)
 {
     const int shape[][2] = {{8, 8}, {8, 16}, {15, 16}, {23, 16}}; // (keys per thread, waves), in RadixTile order
     const int* d = shape[vren_radix_default_tile(n, num_cus, vals, false)];
+    const bool one = n <= kRadixOneWorkgroupMax;
     for (int i = 0; i < vren_radix_config_count(); i++) {
         int b, k, w, a;
         vren_radix_config_info(i, &b, &k, &w, &a);
-        if (b == 8 && k == d[0] && w == d[1] && a == 0) return i;
+        if (one ? a == kRadixOneWorkgroup : b == 8 && k == d[0] && w == d[1] && a == kRadixOnesweep) return i;
     }
     return 0;
 }
@@ -110,6 +111,9 @@ VREN_EXPORT int vren_autotune_radix_sort(vren_ctx* ctx, vren_stream_t stream, ui
     }
     const int reps = 3;
     for (int c = 0; c < vren_radix_config_count() && status == VREN_OK; c++) {
+        int bits, kpt, waves, algorithm;
+        vren_radix_config_info(c, &bits, &kpt, &waves, &algorithm);
+        if (algorithm == kRadixOneWorkgroup && n > kRadixOneWorkgroupMax) continue; // another configuration's tile there
         float acc = 0.f;
         for (int r = 0; r <= reps && status == VREN_OK; r++) {
             fill_random_kernel<<<1024, 256, 0, s>>>(keys, vals, n, (uint32_t)(c * 16 + r));

@@ -774,10 +774,9 @@ int run_sort_pairs(vren_ctx* ctx, hipStream_t s, const uint32_t* in, uint32_t* o
 }
 
 // ---- a few thousand keys: one workgroup, one launch ----------------------------------------------------------------
-// Every pass in LDS (block_sort). Up to kBlockSortMax keys the launches of the multi-tile sort, each with its own loads
+// Every pass in LDS (block_sort). Up to kRadixOneWorkgroupMax keys the launches of the multi-tile sort, each with its own loads
 // and its own wait for the previous one, take longer than one CU takes to rank the keys: 4096 pairs on 32 bits 64.7 us
 // (29.2 with its best configuration) -> 13.7, 8192 pairs 66.1 (30.4) -> 21.7.
-constexpr uint32_t kBlockSortMax = 8192;
 constexpr int kBlockSortThreads = 1024, kBlockSortWaves = kBlockSortThreads / VREN_WAVE;
 
 template <int KPT, bool VALS>
@@ -840,16 +839,39 @@ __global__ __launch_bounds__(kBlockSortThreads) void rs_block_pairs_kernel(const
     }
 }
 
+int run_sort_one_workgroup(vren_ctx* ctx, hipStream_t s, uint32_t* keys, uint32_t* vals, uint64_t n, uint32_t begin_bit,
+                           uint32_t end_bit, char* scratch, const Layout& L)
+{
+    if (n > kRadixOneWorkgroupMax) {
+        switch (vren_radix_default_tile(n, ctx->num_cus, vals != nullptr, false)) {
+        case kRadixTile4096: return run_sort<8, 8, 8>(ctx, s, keys, vals, n, begin_bit, end_bit, scratch, L);
+        case kRadixTile8192: return run_sort<8, 8, 16>(ctx, s, keys, vals, n, begin_bit, end_bit, scratch, L);
+        case kRadixTile15360: return run_sort<8, 15, 16>(ctx, s, keys, vals, n, begin_bit, end_bit, scratch, L);
+        default: return run_sort<8, 23, 16>(ctx, s, keys, vals, n, begin_bit, end_bit, scratch, L);
+        }
+    }
+    const uint32_t m = (uint32_t)n;
+    if (vals) {
+        if (m <= 2048) rs_block_kernel<2, true><<<1, kBlockSortThreads, 0, s>>>(keys, vals, m, begin_bit, end_bit);
+        else rs_block_kernel<8, true><<<1, kBlockSortThreads, 0, s>>>(keys, vals, m, begin_bit, end_bit);
+    } else {
+        if (m <= 2048) rs_block_kernel<2, false><<<1, kBlockSortThreads, 0, s>>>(keys, vals, m, begin_bit, end_bit);
+        else rs_block_kernel<8, false><<<1, kBlockSortThreads, 0, s>>>(keys, vals, m, begin_bit, end_bit);
+    }
+    VREN_LAUNCH_CHECK(ctx);
+    return VREN_OK;
+}
+
 typedef int (*sort_fn)(vren_ctx*, hipStream_t, uint32_t*, uint32_t*, uint64_t, uint32_t, uint32_t, char*, const Layout&);
 
 struct SortConfig {
     int bits, kpt, waves;
     sort_fn fn;
-    int algorithm; // 0 onesweep with look-back, 1 reduce-then-scan
+    int algorithm; // RadixAlgorithm
 };
 
-#define RS_CFG(B, K, W) {B, K, W, &run_sort<B, K, W>, 0}
-#define RS_CFG_RTS(B, K, W) {B, K, W, &run_sort_rts<B, K, W>, 1}
+#define RS_CFG(B, K, W) {B, K, W, &run_sort<B, K, W>, kRadixOnesweep}
+#define RS_CFG_RTS(B, K, W) {B, K, W, &run_sort_rts<B, K, W>, kRadixReduceThenScan}
 const SortConfig kConfigs[] = {
     RS_CFG(8, 8, 4),  RS_CFG(8, 15, 4), RS_CFG(8, 23, 4), RS_CFG(8, 8, 8),  RS_CFG(8, 15, 8),
     RS_CFG(8, 23, 8), RS_CFG(8, 8, 16), RS_CFG(8, 15, 16), RS_CFG(8, 23, 16), RS_CFG(6, 8, 4),  RS_CFG(6, 15, 4), RS_CFG(6, 23, 4),
@@ -857,11 +879,12 @@ const SortConfig kConfigs[] = {
     RS_CFG(4, 15, 4), RS_CFG(4, 23, 4), RS_CFG(4, 8, 8),  RS_CFG(4, 15, 8), RS_CFG(4, 23, 8),
     RS_CFG(4, 8, 16),
     RS_CFG_RTS(8, 15, 8), RS_CFG_RTS(8, 23, 8), RS_CFG_RTS(8, 8, 16), RS_CFG_RTS(8, 15, 16), RS_CFG_RTS(8, 23, 4),
+    {8, 8, 16, &run_sort_one_workgroup, kRadixOneWorkgroup},
 };
 
 } // namespace
 
-// Untuned sorts use 8-bit digits and the smallest tile that still gives no CU more than one tile per pass: a pass then
+// Untuned sorts of up to kRadixOneWorkgroupMax keys take one workgroup. Above, they use 8-bit digits and the smallest tile that still gives no CU more than one tile per pass: a pass then
 // takes one tile's time, which is what its size makes it, and above that the largest tile, whose digit runs are the
 // longest stores. The smallest one stops at half the CUs, since the look-back over more tiles costs what the tile saves.
 // 2^16 pairs on 32 bits: 38.9 us in 4096-key tiles, 45.6 in 8192, 83.5 in 23552; 2^20: 79.5, 76.6, 101; 3 M: 142, 125,
@@ -919,7 +942,7 @@ int vren_radix_sort_pairs_interleaved(vren_ctx* ctx, hipStream_t s, const uint32
     uint32_t* starts = search ? nullptr : bucket_offsets;
     const BucketStarts bs{bucket_offsets, begin_bit, n_buckets ? n_buckets - 1u : 0u};
     int st = VREN_OK;
-    if (n <= kBlockSortMax) {
+    if (n <= kRadixOneWorkgroupMax) {
         const uint2* in = reinterpret_cast<const uint2*>(in_pairs);
         uint2* out = reinterpret_cast<uint2*>(out_pairs);
         const BucketStarts own{starts, bs.shift, bs.mask};
@@ -963,19 +986,6 @@ VREN_EXPORT int vren_radix_sort(vren_ctx* ctx, vren_stream_t stream, uint32_t* k
         return vren_fail(ctx, VREN_EINVAL, "radix_sort: scratch of %zu bytes, %zu required", scratch_bytes,
                          vren_radix_sort_scratch_bytes(n, vals != nullptr));
     if (ctx->device < 0) return vren_fail(ctx, VREN_EINVAL, "radix_sort: context has no device");
-    if (n <= kBlockSortMax && begin_bit < end_bit && ctx->radix_forced < 0) {
-        hipStream_t s = (hipStream_t)stream;
-        const uint32_t m = (uint32_t)n;
-        if (vals) {
-            if (m <= 2048) rs_block_kernel<2, true><<<1, kBlockSortThreads, 0, s>>>(keys, vals, m, begin_bit, end_bit);
-            else rs_block_kernel<8, true><<<1, kBlockSortThreads, 0, s>>>(keys, vals, m, begin_bit, end_bit);
-        } else {
-            if (m <= 2048) rs_block_kernel<2, false><<<1, kBlockSortThreads, 0, s>>>(keys, vals, m, begin_bit, end_bit);
-            else rs_block_kernel<8, false><<<1, kBlockSortThreads, 0, s>>>(keys, vals, m, begin_bit, end_bit);
-        }
-        VREN_LAUNCH_CHECK(ctx);
-        return VREN_OK;
-    }
     int cfg = vren_radix_pick_config(ctx, (hipStream_t)stream, n, vals != nullptr, end_bit - begin_bit);
     return vren_radix_sort_with_config(ctx, (hipStream_t)stream, cfg, keys, vals, n, begin_bit, end_bit, scratch,
                                        scratch_bytes);

@@ -7,6 +7,11 @@
 enum RadixTile { kRadixTile4096, kRadixTile8192, kRadixTile15360, kRadixTile23552 };
 RadixTile vren_radix_default_tile(uint64_t n, int num_cus, bool vals, bool interleaved);
 
+// the algorithms of a configuration
+enum RadixAlgorithm { kRadixOnesweep = 0, kRadixReduceThenScan = 1, kRadixOneWorkgroup = 2 };
+// the largest sort of one workgroup; more keys under that configuration take the untuned sort's tile
+constexpr uint32_t kRadixOneWorkgroupMax = 8192;
+
 int vren_radix_config_count();
 void vren_radix_config_info(int i, int* bits, int* kpt, int* waves, int* algorithm);
 int vren_radix_sort_with_config(vren_ctx* ctx, hipStream_t s, int cfg, uint32_t* keys, uint32_t* vals, uint64_t n,
