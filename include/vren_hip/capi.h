@@ -410,10 +410,13 @@ enum {
 VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, uint32_t n_frames,
                                   const vren_cluster_cfg* cfg, vren_batch** out);
 VREN_EXPORT int vren_batch_run(vren_batch* batch, vren_stream_t stream, int mode);
-/* VREN_RUN_BATCHED with a HIP event after every kernel; kernel_ms[VREN_CHAIN_KERNEL_COUNT] receives the
+/* VREN_RUN_BATCHED with a HIP event after every stage; kernel_ms[VREN_CHAIN_KERNEL_COUNT] receives the
  * durations of chain init, lights, BVH leaves, BVH upper levels, clusters, light counts, light offsets,
  * light lists and shade (the reference's GPU timestamp profiler, profiler.cpp:32-104, has no slot wired on
- * this path). Synchronises the stream. */
+ * this path), 0 for a stage that launches nothing of its own: chain init, unless the run before failed; the BVH levels,
+ * unless a frame has more than 4096 lights; clusters where tables that fit the chip find them in the lights' launch,
+ * whose time then holds both; and light offsets, which are written with the lists. A light stage beside the clusters
+ * (vren_chain_shape) is timed before them. Synchronises the stream. */
 #define VREN_CHAIN_KERNEL_COUNT 9
 VREN_EXPORT int vren_batch_run_profiled(vren_batch* batch, vren_stream_t stream, float* kernel_ms);
 VREN_EXPORT int vren_batch_frame_outputs(vren_batch* batch, uint32_t frame, vren_frame_outputs* out);

@@ -715,7 +715,13 @@ uint32_t persistent_blocks(vren_ctx* ctx, uint32_t wpb, uint32_t waves_per_cu)
 int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
                   const FrameDev* one)
 {
-    if (w.max_L == 0) return one ? VREN_OK : launch_chain_init(ctx, s, w); // no lists; the next run finds cleared words
+    if (w.max_L == 0) { // no lists; the next run finds cleared words
+        const int st = one ? VREN_OK : launch_chain_init(ctx, s, w);
+        chain_mark(w, s, !one);
+        chain_mark(w, s, false);
+        chain_mark(w, s, false);
+        return st;
+    }
     // per wave that traverses long lists: a stack, the bitmask and its summary
     const uint32_t mask_words = (w.max_L + 31) / 32;
     const size_t per_mask = (size_t)(kStack + mask_words + (mask_words + 31) / 32) * 4;
@@ -741,7 +747,7 @@ int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32
         d_frames, F, w.tickets, (uint32_t)(chain_work_clear_bytes(w.total_tiles) / 4));
     VREN_LAUNCH_CHECK(ctx);
     chain_mark(w, s);
-    chain_mark(w, s); // the offsets are written with the lists
+    chain_mark(w, s, false); // the offsets are written with the lists
     assign_lists_kernel<<<runs * team, kListThreads, per_mask * masks, s>>>(d_frames, runs, parts, team, mask_words, masks,
                                                                             TileRanges{w.tile_cl, w.tile_range});
     VREN_LAUNCH_CHECK(ctx);

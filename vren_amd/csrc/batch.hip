@@ -100,9 +100,10 @@ int run_chain(vren_batch* b, hipStream_t s, const FrameDev* table, uint32_t F, c
 {
     vren_ctx* ctx = b->ctx;
     // a run leaves the tickets and statuses cleared for the next one (launch_assign); one that failed half-way may not
-    int st = b->dirty ? launch_chain_init(ctx, s, b->w) : VREN_OK;
+    const bool init = b->dirty;
+    int st = init ? launch_chain_init(ctx, s, b->w) : VREN_OK;
     b->dirty = true;
-    chain_mark(w, s);
+    chain_mark(w, s, init);
     if (!st && w.light_concurrent && !w.events && b->side) {
         VREN_HIP(ctx, hipEventRecord(b->fork, s));
         VREN_HIP(ctx, hipStreamWaitEvent(b->side, b->fork, 0));
@@ -112,11 +113,13 @@ int run_chain(vren_batch* b, hipStream_t s, const FrameDev* table, uint32_t F, c
         st = launch_clusters(ctx, s, table, F, w);
         VREN_HIP(ctx, hipStreamWaitEvent(s, b->join, 0));
         if (!st) st = sl;
-    } else if (!w.events && front_fits(ctx, w)) {
+    } else if (front_fits(ctx, w)) {
         if (!st) st = launch_light_bounds(ctx, s, table, F, w);
         if (!st) st = launch_front(ctx, s, table, F, w);
         if (!st) st = launch_light_merge(ctx, s, table, F, w);
+        chain_mark(w, s);
         if (!st) st = launch_bvh(ctx, s, table, F, live_slots, true, &w, kLeavesLive);
+        chain_mark(w, s, false); // the clusters were found in the lights' launch
     } else {
         if (!st) st = launch_lights(ctx, s, table, F, w);
         if (!st) st = launch_bvh(ctx, s, table, F, live_slots, true, &w, kLeavesLive);
@@ -400,17 +403,21 @@ VREN_EXPORT int vren_batch_run_profiled(vren_batch* b, vren_stream_t stream, flo
     hipStream_t s = (hipStream_t)stream;
     hipEvent_t ev[VREN_CHAIN_KERNELS + 1];
     for (int i = 0; i <= VREN_CHAIN_KERNELS; i++) VREN_HIP(ctx, hipEventCreate(&ev[i]));
-    int n = 0;
+    int n = 0, last = 0; // the last event recorded
+    uint32_t launched = 0;
     ChainWork w = b->w;
     w.events = ev + 1;
     w.n_events = &n;
+    w.launched = &launched;
     VREN_HIP(ctx, hipEventRecord(ev[0], s));
     int st = run_chain(b, s, b->d_table, b->F, w, b->total_live_slots);
-    if (!st) VREN_HIP(ctx, hipEventSynchronize(ev[n]));
+    if (!st) VREN_HIP(ctx, hipStreamSynchronize(s));
     for (int i = 0; i < VREN_CHAIN_KERNELS; i++) {
         kernel_ms[i] = 0.0f;
-        if (!st && i < n && hipEventElapsedTime(&kernel_ms[i], ev[i], ev[i + 1]) != hipSuccess)
-            st = vren_fail(ctx, VREN_EHIP, "batch_run_profiled: no time between events %d and %d", i, i + 1);
+        if (st || i >= n || !((launched >> i) & 1u)) continue;
+        if (hipEventElapsedTime(&kernel_ms[i], ev[last], ev[i + 1]) != hipSuccess)
+            st = vren_fail(ctx, VREN_EHIP, "batch_run_profiled: no time between events %d and %d", last, i + 1);
+        last = i + 1;
     }
     for (int i = 0; i <= VREN_CHAIN_KERNELS; i++) vren_teardown(hipEventDestroy(ev[i]));
     return st;

@@ -38,18 +38,24 @@ struct ChainWork {
     uint32_t assign_wpc = 0;
     uint32_t light_bits = 0;
     uint32_t light_concurrent = 0; // batched runs: the light BVH on a second stream beside the cluster stage
-    // optional per-kernel timing: an event is recorded after every kernel of the chain
+    // optional per-stage timing: an event is recorded after every stage of the chain that launches something
     hipEvent_t* events = nullptr;
-    int* n_events = nullptr;
+    int* n_events = nullptr;    // stages so far
+    uint32_t* launched = nullptr; // one bit per stage
 };
 
-// a failed record surfaces at the checked synchronisation on the last event (vren_batch_run_profiled)
-inline void chain_mark(const ChainWork& w, hipStream_t s)
+// the end of the chain's next stage; one that launches nothing in this run has no event and no time. A failed record
+// surfaces at the checked synchronisation on the last event (vren_batch_run_profiled).
+inline void chain_mark(const ChainWork& w, hipStream_t s, bool launched = true)
 {
-    if (w.events) vren_teardown(hipEventRecord(w.events[(*w.n_events)++], s));
+    if (!w.events) return;
+    const int i = (*w.n_events)++;
+    if (!launched) return;
+    *w.launched |= 1u << i;
+    vren_teardown(hipEventRecord(w.events[i], s));
 }
 
-// kernels of one chain launch, in order (chain_mark follows each)
+// stages of one chain launch, in order (chain_mark follows each)
 #define VREN_CHAIN_KERNELS 9
 
 // workspace: 256 bytes of tickets, the look-back statuses, the per-tile cluster spans and list ranges. The tickets and
@@ -70,7 +76,8 @@ void chain_work_bind(ChainWork* w, void* mem, uint32_t total_tiles);
 int launch_chain_init(vren_ctx* ctx, hipStream_t s, const ChainWork& w);
 int launch_lights(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w,
                   const FrameDev* one = nullptr);
-// the two parts of launch_lights around the chunks' sort, for frames of more than one chunk
+// the two parts of launch_lights around the chunks' sort, for frames of more than one chunk; launch_lights, but not these,
+// marks the stage
 int launch_light_bounds(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w);
 int launch_light_merge(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t F, const ChainWork& w);
 // the chunks' sort and the cluster stage in one launch (front.hip), where front_fits

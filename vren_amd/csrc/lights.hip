@@ -292,7 +292,7 @@ int launch_lights(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32
         st = launch_light_merge(ctx, s, d_frames, F, w);
         if (st) return st;
     }
-    chain_mark(w, s);
+    chain_mark(w, s, chunks || one);
     return VREN_OK;
 }
 
@@ -306,12 +306,12 @@ int launch_bvh(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32_t 
         VREN_LAUNCH_CHECK(ctx);
     }
     if (span == kLeavesPadding) return VREN_OK;
-    if (w) chain_mark(*w, s);
+    if (w) chain_mark(*w, s, total_leaf_slots);
     if (total_leaf_slots) {
         bvh_upper_kernel<<<F, 1024, 0, s>>>(d_frames, leaves_from_lights);
         VREN_LAUNCH_CHECK(ctx);
     }
-    if (w) chain_mark(*w, s);
+    if (w) chain_mark(*w, s, total_leaf_slots);
     return VREN_OK;
 }
 
