@@ -121,7 +121,7 @@ __device__ __forceinline__ bool test_leaf(const Box& c, const float4& o, float l
 }
 
 // The same test against a leaf record (position, limit): the limit is the smallest squared distance whose square root
-// is not below the light's radius (leaf_limit, lights.hip), 0 for a record without a light, so sqrt(d2) < r is
+// is not below the light's radius (leaf_limit, lights_device.hpp), 0 for a record without a light, so sqrt(d2) < r is
 // d2 < limit exactly, without the square root and the node. The clamp as plain minimum and maximum: a NaN position
 // gives a NaN distance either way, and leaf_box takes the boxes with a NaN lower corner out.
 __device__ __forceinline__ bool test_leaf_record(const Box& c, vf4 o)
@@ -145,8 +145,8 @@ __device__ __forceinline__ Box leaf_box(Box c)
 }
 
 // Traverse the BVH for one cluster with the whole wave, setting one bit per hit light in the wave's LDS bitmask (and
-// the word's bit in the summary, one bit per bitmask word), and return the number of hit lights.
-__device__ uint32_t traverse(const FrameDev& fd, const Box& box, uint32_t* stack, uint32_t* bitmask,
+// the word's bit in the summary, one bit per bitmask word).
+__device__ void traverse(const FrameDev& fd, const Box& box, uint32_t* stack, uint32_t* bitmask,
                              uint32_t* summary)
 {
     const uint32_t lane = lane_id();
@@ -156,10 +156,9 @@ __device__ uint32_t traverse(const FrameDev& fd, const Box& box, uint32_t* stack
     // level 0 = the root's children (assign_lights.comp:108-119): the first child of the root
     const uint32_t root_first = __float_as_uint(reinterpret_cast<const float4*>(&bvh[fd.bvh_root])[0].w);
     uint32_t sp = 0;
-    if (root_first == VREN_BVH_INVALID_NODE) return 0u;
+    if (root_first == VREN_BVH_INVALID_NODE) return;
     if (lane == 0) stack[0] = root_first; // level 0
     sp = 1;
-    uint32_t hits = 0;
     __builtin_amdgcn_wave_barrier();
     while (sp > 0) {
         uint32_t e0, e1 = 0xFFFFFFFFu;
@@ -205,7 +204,6 @@ __device__ uint32_t traverse(const FrameDev& fd, const Box& box, uint32_t* stack
                 child = next | ((level + 1) << kLevelShift);
             }
         }
-        hits += (uint32_t)__popcll(ballot(leaf_hit));
         const uint64_t pm = ballot(push);
         if (pm) {
             const uint32_t r = mbcnt(pm);
@@ -215,7 +213,6 @@ __device__ uint32_t traverse(const FrameDev& fd, const Box& box, uint32_t* stack
         }
         __builtin_amdgcn_wave_barrier();
     }
-    return hits;
 }
 
 // Two traversals of one frame's BVH at once, one per 32-lane half of the wave (lanes 0-31 and 32-63, each with its own
@@ -352,8 +349,9 @@ __device__ __forceinline__ uint32_t chunk_size(uint32_t total, uint32_t waves)
 // Clusters of every frame of the table are counted as one flattened range, in chunks of at most 64 consecutive
 // clusters per wave: lane i takes cluster i of the chunk, finds its frame among 64 frames at a time (their
 // device-side cluster counts, one per lane, prefix-summed) and runs pre(fd, c) (the cluster AABB), so work that is
-// uniform per cluster is done for a whole chunk at once. Then the whole wave runs fn(fd, k, two, cA, cB) for clusters k and, with `two`, k + 1 of the chunk, cA and cB their frame-local indices; the two
-// are of one frame, so that its record is uniform and read with scalar loads.
+// uniform per cluster is done for a whole chunk at once. Then the whole wave runs fn(fd, k, two, cA, cB) for clusters
+// k and, with `two`, k + 1 of the chunk, cA and cB their frame-local indices; the two are of one frame, so that its record
+// is uniform and read with scalar loads.
 template <typename Pre, typename Fn>
 __device__ __forceinline__ void for_each_cluster_pair(const FrameDev* __restrict__ frames, uint32_t F, uint32_t gw,
                                                         uint32_t stride, Pre pre, Fn fn)
@@ -404,13 +402,12 @@ __device__ __forceinline__ void for_each_cluster_pair(const FrameDev* __restrict
 }
 
 
-
-// Emits the lights set in a wave's bitmask in ascending index to dst[0 ..) (nothing when dst is null), clearing
-// the bitmask and its summary, and returns their number. Only the words the summary marks are read: lane l of a
+// Emits the lights set in a wave's bitmask in ascending index to dst[0 .. cap), clearing the bitmask and its summary.
+// Only the words the summary marks are read: lane l of a
 // step takes summary word s0 + l (bitmask words 32 (s0 + l) ..), counts its lights, and writes them after the
 // lights of the lanes before it, so a cluster's list costs its hit words, not the L / 32 words of the mask.
-__device__ __forceinline__ uint32_t emit_bitmask(uint32_t* bitmask, uint32_t* summary, uint32_t summary_words,
-                                                 uint32_t* dst, uint32_t cap)
+__device__ __forceinline__ void emit_bitmask(uint32_t* bitmask, uint32_t* summary, uint32_t summary_words, uint32_t* dst,
+                                             uint32_t cap)
 {
     const uint32_t lane = lane_id();
     uint32_t out = 0;
@@ -426,18 +423,15 @@ __device__ __forceinline__ uint32_t emit_bitmask(uint32_t* bitmask, uint32_t* su
             const uint32_t wi = si * 32u + (uint32_t)__builtin_ctz(m);
             uint32_t bits = bitmask[wi];
             bitmask[wi] = 0u;
-            if (dst) {
-                while (bits) {
-                    const uint32_t b = (uint32_t)__builtin_ctz(bits);
-                    bits &= bits - 1u;
-                    if (pos < cap) dst[pos] = wi * 32u + b;
-                    pos++;
-                }
+            while (bits) {
+                const uint32_t b = (uint32_t)__builtin_ctz(bits);
+                bits &= bits - 1u;
+                if (pos < cap) dst[pos] = wi * 32u + b;
+                pos++;
             }
         }
         out += __builtin_amdgcn_readlane(incl, VREN_WAVE - 1);
     }
-    return out;
 }
 
 // COUNT (assign_lights.comp, count pass): two clusters per wave at a time (one per half, traverse_halves), each

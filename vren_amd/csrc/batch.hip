@@ -4,8 +4,9 @@
 // once at fixed maxima (1920x1080, 2^17 clusters, 2^23 assignments; clustered_shading.cpp:817-922). A batch
 // here owns one device arena with every frame's intermediates sized for that frame, a device table of FrameDev
 // records, and the look-back workspace. The chain is the same kernels for one frame or for all of them:
-//   chain init -> lights -> BVH leaves + first level -> BVH upper levels -> clusters -> light counts ->
-//   light offsets -> light lists -> shade
+//   lights (and the BVHs of frames of up to 4096) -> BVH leaves + first level and upper levels of larger frames ->
+//   clusters -> light counts -> light lists and offsets -> shade
+// with lights and clusters in one launch where both fit the chip (front.hip).
 // VREN_RUN_PER_FRAME launches it once per frame (with that frame's one-entry table) and synchronises the stream
 // after each frame; VREN_RUN_BATCHED launches it once for all frames; VREN_RUN_GRAPH captures the batched launches
 // into a hipGraph on first use and replays it.
@@ -25,7 +26,6 @@ struct vren_batch {
     void* work = nullptr;           // ChainWork memory
     ChainWork w;                    // batch-wide
     std::vector<ChainWork> w_frame; // per-frame views of the same memory
-    std::vector<uint32_t> leaf_slots;
     std::vector<uint32_t> live_slots; // per frame: leaf slots of the leaf kernel (256-aligned; none for one chunk)
     uint32_t total_live_slots = 0;
     uint32_t* d_tile_frame = nullptr; // frame of every flattened tile
@@ -166,7 +166,6 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
     b->ctx = ctx;
     b->F = n_frames;
     b->host.resize(n_frames);
-    b->leaf_slots.resize(n_frames);
     b->live_slots.resize(n_frames);
     // sizes and arena layout
     uint32_t tile_base = 0, leaf_base = 0, live_base = 0, chunk_base = 0, max_L = 0, any_materials = 0;
@@ -211,7 +210,6 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         f.bvh_levels = L ? vren_calc_bvh_level_count(L) : 0;
         f.bvh_length = L ? vren_calc_bvh_buffer_length(L) : 0;
         const uint32_t slots = L ? (f.bvh_padded + VREN_LEAF_ALIGN - 1) / VREN_LEAF_ALIGN * VREN_LEAF_ALIGN : 0;
-        b->leaf_slots[i] = slots;
         const uint32_t live = chunks <= 1 ? 0u // lights_kernel writes these frames' leaves
             : (std::min(slots, (L + 31u) & ~31u) + VREN_LEAF_ALIGN - 1) / VREN_LEAF_ALIGN * VREN_LEAF_ALIGN;
         b->live_slots[i] = live;
@@ -280,7 +278,6 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
     }
     chain_work_bind(&b->w, b->work, tile_base);
     b->w.tile_frame = b->d_tile_frame;
-    b->w.total_leaf_slots = leaf_base;
     b->total_live_slots = live_base;
     b->w.max_L = max_L;
     b->w.light_chunks = chunk_base;
@@ -303,7 +300,6 @@ VREN_EXPORT int vren_batch_create(vren_ctx* ctx, const vren_frame_desc* frames, 
         wf = b->w;
         wf.tile_frame = nullptr;
         wf.total_tiles = single[i].Sx * single[i].Sy;
-        wf.total_leaf_slots = b->leaf_slots[i];
         wf.max_L = single[i].L;
         wf.light_chunks = (single[i].L + VREN_LIGHT_CHUNK - 1) / VREN_LIGHT_CHUNK;
         wf.any_materials = single[i].texcoords != nullptr;

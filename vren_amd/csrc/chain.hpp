@@ -27,7 +27,6 @@ struct ChainWork {
     uint2* tile_range;     // per 32x32 tile: [begin, end) of the index-buffer entries of its clusters' light lists
     const uint32_t* tile_frame; // frame of every flattened 32x32 tile (null for a one-frame table)
     uint32_t total_tiles;
-    uint32_t total_leaf_slots;
     uint32_t max_L;
     uint32_t light_chunks;  // chunks of VREN_LIGHT_CHUNK lights over the table's frames (light_chunk_base numbering)
     uint32_t fresh;         // a single-frame shade call whose output holds nothing: zeros for background pixels

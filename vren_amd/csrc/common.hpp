@@ -28,7 +28,6 @@ typedef uint32_t vu2 __attribute__((ext_vector_type(2)));
 typedef const __attribute__((address_space(1))) float gfloat;
 typedef const __attribute__((address_space(1))) uint32_t guint;
 typedef const __attribute__((address_space(1))) vf4 gvf4;
-typedef const __attribute__((address_space(1))) vu4 gvu4;
 typedef const __attribute__((address_space(1))) vu2 gvu2;
 
 // element `at` of a uniform array, at most 4 GB into it: a uniform base and a 32-bit lane offset, which one load takes
@@ -127,16 +126,11 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // four words at any word's address: the hardware's wide accesses need 4-byte alignment
 typedef uint32_t vu4_any __attribute__((ext_vector_type(4), aligned(4)));
 
-// 128-bit streaming (non-temporal) load / store of 4 uint32 at a 16-byte aligned address
+// 128-bit streaming (non-temporal) load of 4 uint32 at a 16-byte aligned address
 __device__ __forceinline__ uint4 ntload4(const void* p)
 {
     u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
     return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ void ntstore4(void* p, uint4 q)
-{
-    u32x4 v = {q.x, q.y, q.z, q.w};
-    __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -169,16 +163,6 @@ __device__ __forceinline__ uint32_t atomic_add_agent(uint32_t* p, uint32_t v)
 __device__ __forceinline__ void atomic_or_agent(uint32_t* p, uint32_t v)
 {
     __hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// f16 -> f32 on the conversion unit (exact); Inf/NaN halves take the shared software path, whose NaN payload
-// handling is the oracle's
-__device__ __forceinline__ float vren_h2f(uint16_t h)
-{
-    if ((h & 0x7C00u) == 0x7C00u) return vren_half_to_float(h);
-    _Float16 x;
-    __builtin_memcpy(&x, &h, 2);
-    return (float)x;
 }
 
 // min / max in the total order -0 < +0 (order-independent, so any reduction tree gives the same bits)

@@ -67,33 +67,23 @@ __device__ __forceinline__ void match_digit(uint32_t d, uint32_t& lo, uint32_t& 
     }
 }
 
-// s_whist: WAVES * RADIX counters, zeroed before the call (and a __syncthreads() after zeroing).
-// Writes local[j] = rank of key j among the same-digit keys of this wave that precede it.
-// CHECK = true: positions at or past tile_count are excluded (neither ranked nor counted). CHECK = false: every
-// lane takes part; a caller padding a partial tile gives its padding the largest digit, so that the padding ranks
-// after every real key of the tile and the real keys keep positions [0, tile_count).
-template <int BITS, int KPT, bool CHECK = true>
-__device__ __forceinline__ void rank_wave_keys(const uint32_t (&digit)[KPT], uint32_t valid_count_base,
-                                               uint32_t tile_count, uint32_t* s_wave_row, uint32_t (&local)[KPT])
+// s_wave_row: the wave's RADIX counters, zero before the call. Writes local[j] = rank of key j among the same-digit keys
+// of this wave that precede it. Every lane takes part: a caller padding a partial tile gives its padding the largest
+// digit, so that the padding ranks after every real key of the tile, which keep the positions from 0.
+template <int BITS, int KPT>
+__device__ __forceinline__ void rank_wave_keys(const uint32_t (&digit)[KPT], uint32_t* s_wave_row, uint32_t (&local)[KPT])
 {
     const uint32_t lane = lane_id();
 #pragma unroll
     for (int j = 0; j < KPT; j++) {
         const uint32_t d = digit[j];
-        bool valid = true;
-        uint32_t lo = 0xFFFFFFFFu, hi = 0xFFFFFFFFu;
-        if (CHECK) {
-            valid = valid_count_base + (uint32_t)j * VREN_WAVE + lane < tile_count;
-            const uint64_t v = ballot(valid);
-            lo = (uint32_t)v;
-            hi = (uint32_t)(v >> 32);
-        }
-        const uint32_t before = valid ? s_wave_row[d] : 0u;
-        match_digit<BITS, !CHECK>(d, lo, hi);
+        uint32_t lo, hi;
+        const uint32_t before = s_wave_row[d];
+        match_digit<BITS, true>(d, lo, hi);
         const uint32_t rank = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
         const uint64_t peers = ((uint64_t)hi << 32) | lo;
         // the highest peer lane publishes the new running count
-        if (valid && (peers >> lane) == 1ull) s_wave_row[d] = before + rank + 1u;
+        if ((peers >> lane) == 1ull) s_wave_row[d] = before + rank + 1u;
         local[j] = before + rank;
         __builtin_amdgcn_wave_barrier();
     }

@@ -340,7 +340,7 @@ __global__ __launch_bounds__(WAVES * 64, rs_two_per_cu(KPT, WAVES) && !IN_PAIRS 
     }
 #pragma unroll
     for (int j = 0; j < KPT; j++) digit[j] = __builtin_amdgcn_ubfe(key[j], shift, width);
-    rank_wave_keys<BITS, KPT, false>(digit, wbase, tile_count, row, local);
+    rank_wave_keys<BITS, KPT>(digit, row, local);
     // the values are read after the ranking: their loads overlap the counts, the look-back and the key stores
     if (VALS && !IN_PAIRS && !LATE) load_vals();
     __syncthreads();

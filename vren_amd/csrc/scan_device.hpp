@@ -1,5 +1,5 @@
 // scan_device.hpp -- block-level scan pieces and the single-pass decoupled look-back (Merrill & Garland 2016)
-// shared by the exclusive scan primitive, cluster compaction and the light-offset scan.
+// shared by the exclusive scan primitive and cluster compaction.
 #pragma once
 
 #include "common.hpp"
@@ -65,11 +65,4 @@ __device__ __forceinline__ uint32_t wave_lookback_walk(uint64_t* status, uint32_
     }
     if (lane == 0) st_agent_u64(&status[t], VREN_LB_INCL | (uint32_t)(prefix + agg));
     return prefix;
-}
-
-// both steps at once (nothing between publishing the aggregate and walking)
-__device__ __forceinline__ uint32_t wave_lookback(uint64_t* status, uint32_t t, uint32_t agg)
-{
-    if (lane_id() == 0) wave_lookback_publish(status, t, agg);
-    return wave_lookback_walk(status, t, agg);
 }

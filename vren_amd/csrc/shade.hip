@@ -986,8 +986,8 @@ __global__ __launch_bounds__(256, 5) void shade_backward_kernel(const FrameDev o
         len = end > off ? end - off : 0u;
     }
     // pass 2: adjoint of every contribution, in a loop that is uniform over the wave (iteration k handles entry
-    // off + k of every lane whose list is that long), so that when every such lane is at the same entry -- the
-    // lanes of one cluster -- the wave sums its 7 light-gradient terms and one lane adds them to the staged slot
+    // off + k of every lane whose list is that long), so that the wave sums the 7 light-gradient terms of the lanes at one
+    // entry -- those of one cluster -- and seven lanes add them to the staged slot
     const uint32_t kmax = wave_max_u32(len);
     for (uint32_t k = 0; k < kmax; k++) {
         const bool act = k < len;
