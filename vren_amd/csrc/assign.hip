@@ -23,8 +23,12 @@ constexpr uint32_t kStack = 384; // per-wave stack entries (levels are nondecrea
 // at most 31 entries of each level above the deepest inner one and 32 of that, 31 * 2 + 32 = 94 for 2^20 lights), the
 // leaf list blocks of leaves, which are tested when it has no room for 32 more or no inner block is left
 constexpr uint32_t kStackHalf = 96;
+// (128 entries and 64 take the same time)
 constexpr uint32_t kLeafList = 128;
-constexpr int kLeafUnroll = 4; // leaf blocks per half and step: their loads overlap
+// leaf blocks per half and step, whose loads overlap: a 1920x1080 frame with 4096 lights takes 77.0 us with 2, 76.7 with 4 and
+// 81.9 with 8, the stage calls of a 1366x769 frame 66.1, 66.7 and 79.7 (eight blocks' nodes and positions do not fit the
+// registers of eight waves per SIMD)
+constexpr int kLeafUnroll = 4;
 constexpr uint32_t kLevelShift = 28;
 constexpr uint32_t kAddrMask = (1u << kLevelShift) - 1u;
 
@@ -518,7 +522,7 @@ struct TileRanges {
 // 64 frames of 1080p with 4096 lights took 6 + 54 us in two launches, the copies one cluster per wave and step with a
 // load's latency each, and take 24; one frame 5 + 4.8, now 6.7; a 3840x2160 frame with 65536 lights 12 + 15, now 16.
 constexpr uint32_t kListThreads = 256;
-constexpr int kListUnroll = 4; // entries per thread and step
+constexpr int kListUnroll = 4; // entries per thread and step (2 is within 1 %)
 
 __device__ __forceinline__ uint32_t list_sum(uint32_t v, uint32_t* s_wave)
 {
@@ -725,7 +729,8 @@ int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32
     constexpr size_t count_per_wave = (size_t)2 * (kStackHalf + kLeafList + VREN_LIST_SLOT) * 4 + VREN_WAVE * sizeof(float) * 6;
     static_assert(count_per_wave * 4 <= 160 * 1024 / 8, "assign_count: 8 workgroups of 4 waves must fit a CU's LDS");
     const uint32_t count_blocks = persistent_blocks(ctx, 4, w.assign_wpc);
-    // list runs per frame: 2048 workgroups over a batch, at most 512 and at least 8 a frame
+    // list runs per frame: 2048 over a batch, at most 512 and at least 8 a frame (a 3840x2160 frame with 65536 lights 567 us;
+    // 574 with half as many runs, 572 with twice; smaller frames and batches within the spread)
     const uint32_t parts = std::max<uint32_t>(8, std::min<uint32_t>(512, 2048 / F));
     // and up to 4096 workgroups, four a run at most, for the long lists (64 frames of 1920x1080 with 4096 lights of four
     // times the radius: lists 740 us with one a run, 445 with two)

@@ -828,7 +828,9 @@ __device__ __forceinline__ float wave_sum_components(const float g[7])
     return w;
 }
 
-constexpr int kSumRounds = 8;  // distinct entries of one step that a wave sums; lanes past them add one by one
+// distinct entries of one step that a wave sums; lanes past them add one by one (1920x1080 with 4096 lights 83.8 us with one
+// round, 77.0 with 4, 77.1 with 8, 77.4 with 16)
+constexpr int kSumRounds = 8;
 
 // One 32x8 strip of a tile per workgroup. On a 1920x1080 frame with 4096 lights (4.7 M pairs) it took 228 us: 95 us in
 // LDS adds of 64 lanes to one slot (every wave that covers two clusters took them, since it summed over the wave only
