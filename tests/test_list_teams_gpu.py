@@ -1,4 +1,4 @@
-"""Light lists of a batch whose runs are shared by a team of four, two or one workgroups: lists longer than a slot beside
+"""Light lists of a batch whose runs are shared by a team of four or two workgroups, or taken by one: lists longer than a slot beside
 short ones and frames without lights, bit for bit against the oracle, and the same image as from one frame at a time."""
 import numpy as np
 import pytest

@@ -516,8 +516,8 @@ struct TileRanges {
 // a run has a `team` of workgroups for them: the first also writes the run's offsets, copies and ranges, the helpers
 // traverse their share of the long lists, and leave at once where there are none. One workgroup a run made frames of
 // long lists slower than a pass of their own had been; with teams (us, counting, offsets and lists, then | in one pass each |
-// one workgroup | team): 1920x1080 with 4096 lights of six times the radius 201 | 213 | 121, 3840x2160 with 65536 of twice
-// the radius 507 | 522 | 376, 8192x8192 with 110 k clusters 328 | 444 | 231; a frame without long lists takes what it took
+// one workgroup | team): 1920x1080 with 4096 lights of six times the radius 200 | 209 | 115, 3840x2160 with 65536 of twice
+// the radius 508 | 517 | 372, 8192x8192 with 110 k clusters 327 | 438 | 225; a frame without long lists takes what it took
 // (640x360 42.6 a frame, 3840x2160 with 65536 lights 563), since a helper leaves as soon as it sees that it has no share.
 // 64 frames of 1080p with 4096 lights took 6 + 54 us in two launches, the copies one cluster per wave and step with a
 // load's latency each, and take 24; one frame 5 + 4.8, now 6.7; a 3840x2160 frame with 65536 lights 12 + 15, now 16.
@@ -733,7 +733,7 @@ int launch_assign(vren_ctx* ctx, hipStream_t s, const FrameDev* d_frames, uint32
     // 574 with half as many runs, 572 with twice; smaller frames and batches within the spread)
     const uint32_t parts = std::max<uint32_t>(8, std::min<uint32_t>(512, 2048 / F));
     // and up to 4096 workgroups, four a run at most, for the long lists (64 frames of 1920x1080 with 4096 lights of four
-    // times the radius: lists 740 us with one a run, 445 with two)
+    // times the radius: lists 735 us with one a run, 445 with two; short lists take the same with both)
     const uint32_t runs = F * parts, team = std::max<uint32_t>(1, std::min<uint32_t>(4, 4096 / runs));
     if (one) {
         assign_count_one_kernel<<<count_blocks, 4 * VREN_WAVE, count_per_wave * 4, s>>>(*one);
