@@ -16,7 +16,8 @@ INIT, LIGHTS, LEAVES, UPPER, CLUSTERS, COUNTS, OFFSETS, LISTS, SHADE = range(9)
     (2560, 1440, 300, (LIGHTS, CLUSTERS, COUNTS, LISTS, SHADE)),
     (2560, 1440, 4100, (LIGHTS, LEAVES, UPPER, CLUSTERS, COUNTS, LISTS, SHADE)),
     (320, 180, 0, (CLUSTERS, COUNTS, SHADE))])
-def test_stages_of_a_run(vctx, W, H, L, stages):
+@pytest.mark.parametrize("concurrent", [0, 1])
+def test_stages_of_a_run(vctx, W, H, L, stages, concurrent):
     import torch
     import vren_amd
     cam = ol.camera(W, H)
@@ -35,6 +36,9 @@ def test_stages_of_a_run(vctx, W, H, L, stages):
         d.light_positions, d.point_lights, d.light_count = t["pos"].data_ptr(), t["lig"].data_ptr(), L
     torch.cuda.synchronize()
     batch = vren_amd.Batch(vctx, [d], ol.cfg())
+    if concurrent and L:  # lights on the second stream: a launch of their own, timed ahead of the clusters'
+        batch.set_shape(1, 32, 8, 1)
+        stages = sorted({*stages, CLUSTERS})
     for _ in range(2):
         t["out"].zero_()
         ms = batch.run_profiled()

@@ -113,7 +113,7 @@ int run_chain(vren_batch* b, hipStream_t s, const FrameDev* table, uint32_t F, c
         st = launch_clusters(ctx, s, table, F, w);
         VREN_HIP(ctx, hipStreamWaitEvent(s, b->join, 0));
         if (!st) st = sl;
-    } else if (front_fits(ctx, w)) {
+    } else if (!w.light_concurrent && front_fits(ctx, w)) {
         if (!st) st = launch_light_bounds(ctx, s, table, F, w);
         if (!st) st = launch_front(ctx, s, table, F, w);
         if (!st) st = launch_light_merge(ctx, s, table, F, w);
